@@ -887,6 +887,22 @@ def test_out_residual_decode_strides_alignment_and_absent_operands(gpu, rows, fp
         assert torch.all(out[:, 2880:] == 7.0) and torch.all(buf[:shift] == 7.0) and torch.all(buf[shift + rows * stride:] == 7.0)
 
 
+@pytest.mark.parametrize("in_dim,out_dim", [(32, 1), (608, 17), (1056, 100), (4096, 4096), (100, 30)])
+@pytest.mark.parametrize("rows", [1, 8, 9, 33])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_out_residual_general_stream(gpu, in_dim, out_dim, rows, fp8):
+    """The general out-projection stream at its edges: one k32 step, K that ends inside a wavefront's phase, fewer output
+    features than a tile and ragged last tiles, both activation-row forms and a ragged last chunk; in_dim 100 is the
+    plain kernel behind it."""
+    d = _out_inputs(rows, 7000 + in_dim + rows, in_dim=in_dim, out_dim=out_dim)
+    w, ws, ref = d["w"].to(gpu), None, d["w"]
+    if fp8:
+        w, ws = T.quantize_fp8_rows(w)
+        ref = O.dequant_fp8_ref(w.cpu(), ws.cpu())
+    out = T.out_residual_decode_forward(d["x"].view(rows, 1, in_dim).to(gpu), w, d["b"].to(gpu), d["r"].view(rows, 1, out_dim).to(gpu), weight_scale=ws)
+    close(out.view(rows, out_dim), O.out_residual_ref(d["x"], ref, d["b"], d["r"]))
+
+
 def test_out_residual_other_shapes_module_and_errors(gpu, monkeypatch):
     # a shape the streaming kernel does not serve (in_dim != 4096): the plain kernel, bf16 and fp8
     d = _out_inputs(5, 61, in_dim=320, out_dim=100)

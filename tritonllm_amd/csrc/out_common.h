@@ -1,4 +1,4 @@
-// Argument block shared by the decode out-projection kernels (out_decode.hip, out_decode_r8.hip, out_decode_r32.hip).
+// Argument block shared by the decode out-projection kernels (out_decode.hip, out_decode_r8.hip, out_decode_r32.hip, decode_general.hip).
 #pragma once
 #include "common.h"
 
@@ -22,5 +22,8 @@ void launch_out_decode_r8(dim3 grid, hipStream_t st, const OutArgs& a);
 // in_dim 4096, out_dim % 12 == 0, bf16 or fp8 weight, any number of rows in chunks of 32; grid = (out_dim / 12, ceil(rows / 32)) as
 // the caller counts chunks -- the launch itself gives a workgroup up to four of them
 void launch_out_decode_r32(dim3 grid, hipStream_t st, const OutArgs& a);
+
+// any in_dim % 32 == 0 and out_dim, bf16 or fp8 weight, any rows in chunks of 8 or 16; x and W 16-byte aligned
+int launch_out_decode_general(const char* what, const OutArgs& a, hipStream_t st);
 
 }  // namespace tllm

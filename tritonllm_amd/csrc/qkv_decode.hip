@@ -10,8 +10,7 @@
 //   qkv_decode_r32_kernel  hidden == 2880, 9..32 rows per workgroup, bf16 or fp8 weight, no fused norm: qkv_decode_r32.hip.
 //   qkv_decode_rows_kernel hidden == 2880, more than 32 rows: the weight read once and held, the rows streamed past it:
 //                          qkv_decode_rows.hip.
-//   qkv_decode_kernel      head_dim == 64, hidden % 32 == 0: operands loaded straight into MFMA
-//                          layout (simple, ~1.8x slower: every lane is its own cache-line request).
+//   qkv_decode_general_kernel  any hidden % 32 == 0, head_dim % 16 == 0, bf16 or fp8 weight: decode_general.hip.
 //   qkv_generic_kernel     anything else: shuffle-reduced dot products.
 #include "qkv_common.h"
 
@@ -113,138 +112,6 @@ void launch_qkv_generic(const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& f
   const int heads = a.n_q_heads + 2 * a.n_kv_heads;
   const unsigned gy = static_cast<unsigned>(a.rows < 65535 ? a.rows : 65535);   // rows beyond grid.y are looped in-kernel
   hipLaunchKernelGGL(qkv_generic_kernel, dim3((unsigned)heads, gy), dim3(256), 0, st, a, ra, fr);
-}
-
-// ------------------------------------------------------------------------------------------------
-// MFMA kernel for any hidden % 32 == 0 and head_dim % 16 == 0 (the reference's decode kernel is generic over both,
-// triton_kernels.py:1127-1158). A workgroup owns 16 weight rows of one head -- dims [8p, 8p+8) and their partners
-// [half+8p, half+8p+8), half = head_dim / 2 -- and up to 16 activation rows; its wavefronts
-// split K in runs of SPW k32-steps whose loads are all issued before the first multiply.
-// v_mfma_f32_16x16x32_bf16: tile row 4*qd + i is dim 8p + 2*qd + (i & 1), plus half when i >= 2, so
-// each lane's four accumulators are two complete (lo, hi) pairs.
-// W8: the weight is fp8 (OCP e4m3) with one fp32 scale per output row (the reference's fp8 branch is as generic as its
-// bf16 one, triton_kernels.py:927-940): eight bytes per lane and step, widened to bf16 in registers (exact), the row
-// scale applied to the finished sum.
-// A run's 16 weight rows x SPW steps arrive row by row -- one load instruction = one row's contiguous run, 64 lanes x 16
-// bytes (fp8: x 8) -- and pass a wavefront-private LDS patch on their way into A-operand layout (loaded straight into
-// that layout every lane's bytes are a request of their own, and the memory side serves such a stream at three
-// quarters of the rate).
-template <int NW, int SPW, bool W8 = false>
-__global__ __launch_bounds__(NW * 64) void qkv_decode_kernel(QkvArgs a, RopeArgs ra, YarnFreqs fr) {
-  __shared__ float red[NW][4][64];
-  constexpr int WROW = SPW * (W8 ? 32 : 64) + 16;           // patch row: a run's bytes of one weight row + padding (conflict-free fragment reads)
-  extern __shared__ __align__(16) unsigned char wpatch_all[];   // [NW][16][WROW]
-  static_assert(SPW == 16, "a load instruction covers one row's run of 16 steps");
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int half = a.head_dim >> 1, pieces = half >> 3;
-  const int head = blockIdx.x / pieces, piece = blockIdx.x - head * pieces;
-  const int64_t row0 = static_cast<int64_t>(blockIdx.y) * 16;
-  const int kvec = a.hidden >> 3;       // 16-byte vectors per row
-  const int nsteps = a.hidden >> 5;     // MFMA k-steps of 32
-  const int m = lane & 15, g = lane >> 4;
-
-  typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u32x2;
-  // Lanes past the last activation row re-read a live lane's row (same addresses, no extra traffic);
-  // their output column is dropped.
-  const int64_t xrow_idx = row0 + m;
-  const bool xvalid = xrow_idx < a.rows;
-  const int nvalid = static_cast<int>(a.rows - row0 < 16 ? a.rows - row0 : 16);
-  const bf16x8* xrow = reinterpret_cast<const bf16x8*>(a.x) + (row0 + (xvalid ? m : m % nvalid)) * kvec + g;
-  const bool rotate = a.has_rope && head < a.n_q_heads + a.n_kv_heads;
-
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = wave * SPW; s0 < nsteps; s0 += NW * SPW) {
-    bf16x8 wa[SPW], xb[SPW];
-    u32x2 wa8[SPW];
-#pragma unroll
-    for (int i = 0; i < SPW; ++i) {       // clamped, never predicated: a tail step re-reads the last one and is masked below
-      const int step = s0 + i < nsteps ? s0 + i : nsteps - 1;
-      // load i = tile row i: lane l fetches chunk s0 * 4 + l of that row -- 16 bytes of a bf16 row, 8 of an fp8 row, either
-      // way the lane's share of the run's 16 steps -- clamped at the row's end (a tail run re-reads the last chunk; those
-      // steps are masked below)
-      const int chunk = s0 * 4 + lane < kvec ? s0 * 4 + lane : kvec - 1;
-      const int dim_i = 8 * piece + 2 * (i >> 2) + (i & 1) + ((i & 2) ? half : 0);
-      const int64_t wrow_i = static_cast<int64_t>(head) * a.head_dim + dim_i;
-      if constexpr (W8) {
-        wa8[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(reinterpret_cast<const unsigned char*>(a.W) + wrow_i * a.hidden) + chunk);
-      } else {
-        wa[i] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(a.W) + wrow_i * kvec + chunk);
-      }
-      xb[i] = xrow[step * 4];
-    }
-    unsigned char* wp = wpatch_all + wave * (16 * WROW);
-#pragma unroll
-    for (int i = 0; i < SPW; ++i) {
-      if constexpr (W8) *reinterpret_cast<u32x2*>(wp + i * WROW + lane * 8) = wa8[i];
-      else *reinterpret_cast<bf16x8*>(wp + i * WROW + lane * 16) = wa[i];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int i = 0; i < SPW; ++i) {
-      if constexpr (W8) wa8[i] = *reinterpret_cast<const u32x2*>(wp + m * WROW + (4 * i + g) * 8);
-      else wa[i] = *reinterpret_cast<const bf16x8*>(wp + m * WROW + (4 * i + g) * 16);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the next run's writes come after these reads
-    __builtin_amdgcn_wave_barrier();
-    if constexpr (W8) {
-#pragma unroll
-      for (int i = 0; i < SPW; ++i) wa[i] = fp8x8_to_bf16x8(wa8[i][0], wa8[i][1]);
-    }
-#pragma unroll
-    for (int i = 0; i < SPW; ++i) {
-      if (s0 + i < nsteps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[i], xb[i], acc, 0, 0, 0);
-    }
-  }
-
-#pragma unroll
-  for (int i = 0; i < 4; ++i) red[wave][i][lane] = acc[i];
-  __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int w = 1; w < NW; ++w) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] += red[w][i][lane];
-  }
-  if (!xvalid) return;
-
-  // the lane holds activation row xrow_idx and dims d0, d0 + 1 (acc[0], acc[1]) with their partners (acc[2], acc[3])
-  const int d0 = 8 * piece + 2 * g;
-  const int col = head * a.head_dim + d0;
-  float lo0 = acc[0], lo1 = acc[1], hi0 = acc[2], hi1 = acc[3];
-  if constexpr (W8) {
-    lo0 *= a.w_scale[col];
-    lo1 *= a.w_scale[col + 1];
-    hi0 *= a.w_scale[col + half];
-    hi1 *= a.w_scale[col + half + 1];
-  }
-  if (a.bias) {
-    lo0 += static_cast<float>(a.bias[col]);
-    lo1 += static_cast<float>(a.bias[col + 1]);
-    hi0 += static_cast<float>(a.bias[col + half]);
-    hi1 += static_cast<float>(a.bias[col + half + 1]);
-  }
-  if (rotate) {
-    const int64_t pos = rope_position(ra, xrow_idx);
-    float c0, s0, c1, s1;
-    rope_cos_sin(ra, fr, pos, d0, &c0, &s0);
-    rope_cos_sin(ra, fr, pos, d0 + 1, &c1, &s1);
-    const float r0 = lo0 * c0 - hi0 * s0, r1 = lo1 * c1 - hi1 * s1;
-    const float r2 = hi0 * c0 + lo0 * s0, r3 = hi1 * c1 + lo1 * s1;
-    lo0 = r0;
-    lo1 = r1;
-    hi0 = r2;
-    hi1 = r3;
-  }
-  bf16* out = qkv_out_ptr(a, qkv_slot(a, ra), xrow_idx, head);
-  bf16x2 plo, phi;
-  plo[0] = static_cast<bf16>(lo0);
-  plo[1] = static_cast<bf16>(lo1);
-  phi[0] = static_cast<bf16>(hi0);
-  phi[1] = static_cast<bf16>(hi1);
-  *reinterpret_cast<bf16x2*>(out + d0) = plo;
-  *reinterpret_cast<bf16x2*>(out + d0 + half) = phi;
 }
 
 }  // namespace tllm
@@ -370,6 +237,7 @@ extern "C" int tllm_qkv_rope_decode_w8_bf16(const void* x, const void* norm_scal
                "qkv_rope_decode_w8: the fused RMSNorm exists for hidden 2880 / head_dim 64 only: call tllm_rmsnorm_bf16 first");
   TLLM_REQUIRE(head_dim % 16 == 0 && hidden % 32 == 0, TLLM_E_SHAPE,
                "qkv_rope_decode_w8: head_dim %d must be a multiple of 16 and hidden %lld of 32", head_dim, (long long)hidden);
+  TLLM_REQUIRE(static_cast<int64_t>(head_dim) * hidden < (1ll << 31), TLLM_E_SHAPE, "qkv_rope_decode_w8: a head's rows of the weight exceed 2 GiB");
   TLLM_REQUIRE(aligned16(x) && aligned16(W8), TLLM_E_ALIGN, "qkv_rope_decode_w8: x and W must be 16-byte aligned");
   TLLM_REQUIRE(w_scale != nullptr && reinterpret_cast<uintptr_t>(w_scale) % 4 == 0, TLLM_E_ARG,
                "qkv_rope_decode_w8: w_scale must be a 4-byte aligned device pointer");
@@ -380,16 +248,7 @@ extern "C" int tllm_qkv_rope_decode_w8_bf16(const void* x, const void* norm_scal
   a.bias = (const bf16*)b;
   a.w_scale = w_scale;
   if (rows == 0) return TLLM_OK;
-  const int heads = n_q_heads + 2 * n_kv_heads;
-  const int64_t chunks = (rows + 15) / 16;
-  TLLM_REQUIRE(chunks <= 65535, TLLM_E_SHAPE, "qkv_rope_decode_w8: rows %lld too many for the decode kernel", (long long)rows);
-  // wavefronts per workgroup 1 / 2 / 4 / 8: 16.2 / 13.0 / 13.6 / 14.0 us at hidden 4096, 8 or 16 rows (a run is half the bytes of
-  // a bf16 run, so two wavefronts keep as much in flight as one does there); loaded straight into operand layout, four
-  // wavefronts: 19.6 us
-  constexpr int GNW = 2;
-  hipLaunchKernelGGL((qkv_decode_kernel<GNW, 16, true>), dim3((unsigned)(heads * (head_dim / 16)), (unsigned)chunks), dim3(GNW * 64),
-                     GNW * 16 * (16 * 32 + 16), static_cast<hipStream_t>(stream), a, ra, fr);
-  return check_launch("qkv_rope_decode_w8");
+  return launch_qkv_decode_general("qkv_rope_decode_w8", a, ra, fr, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tllm_qkv_rope_decode_bf16(const void* x, const void* W, const void* b, void* q, void* k, void* v, int64_t q_row_stride,
@@ -414,25 +273,9 @@ extern "C" int tllm_qkv_rope_decode_bf16(const void* x, const void* W, const voi
   const bool out4 = (reinterpret_cast<uintptr_t>(q) % 4 == 0) && (reinterpret_cast<uintptr_t>(k) % 4 == 0) &&
                     (reinterpret_cast<uintptr_t>(v) % 4 == 0) && q_row_stride % 2 == 0 && k_row_stride % 2 == 0 &&
                     v_row_stride % 2 == 0 && kv_slot_stride % 2 == 0;
-  if (mfma_ok && out4) {
-    const int64_t chunks = (rows + 15) / 16;
-    TLLM_REQUIRE(chunks <= 65535, TLLM_E_SHAPE, "qkv_rope_decode: rows %lld too many for the decode kernel", (long long)rows);
-    // wavefronts per workgroup 1 / 2 / 4 / 8: 14.0 / 14.7 / 15.5 / 17.2 us at hidden 4096, 8 rows (one wavefront then walks K in
-    // runs of 512, one after the other; two register sets taken in turn, so that the next run's loads are out while a run is
-    // multiplied, changed nothing: 14.1 us, at 292 registers one wavefront per SIMD)
-    constexpr int GNW = 1;
-    constexpr size_t kPatchBytes = GNW * 16 * (16 * 64 + 16);   // the wavefronts' weight patches
-    static bool attr_set = false;   // raising the dynamic-LDS limit is idempotent; a benign race at worst repeats it
-    if (!attr_set) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(qkv_decode_kernel<GNW, 16>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)kPatchBytes);
-      TLLM_REQUIRE(e == hipSuccess, TLLM_E_LAUNCH, "qkv_rope_decode: cannot raise LDS limit: %s", hipGetErrorString(e));
-      attr_set = true;
-    }
-    hipLaunchKernelGGL((qkv_decode_kernel<GNW, 16>), dim3((unsigned)(heads * (head_dim / 16)), (unsigned)chunks), dim3(GNW * 64), kPatchBytes, st, a, ra,
-                       fr);
-    return check_launch("qkv_rope_decode");
-  }
+  // (the general kernel addresses a head's rows of the weight with 32-bit byte offsets)
+  if (mfma_ok && out4 && static_cast<int64_t>(head_dim) * hidden * 2 < (1ll << 31))
+    return launch_qkv_decode_general("qkv_rope_decode", a, ra, fr, st);
   launch_qkv_generic(a, ra, fr, st);
   return check_launch("qkv_rope_decode(generic)");
 }
