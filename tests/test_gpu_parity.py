@@ -9,7 +9,7 @@ import torch
 
 import tritonllm_amd as T
 from oracle import layers as O
-from tritonllm_amd import scratch_pool
+from tritonllm_amd import ops, scratch_pool
 
 pytestmark = pytest.mark.gpu
 
@@ -708,6 +708,67 @@ def test_qkv_decode_fp8_weight_other_shapes(gpu, hd, nq, nkv, rows):
     close(q, qr)
     close(k, kr)
     close(v, vr)
+
+
+@pytest.mark.parametrize("rows,hidden,nq,nkv", [(1, 64, 3, 1), (65, 128, 2, 1), (97, 2880, 64, 8), (130, 192, 40, 8), (200, 320, 64, 8),
+                                                (333, 640, 64, 8), (450, 2880, 64, 8), (600, 704, 64, 8), (999, 448, 64, 8),
+                                                (1100, 576, 64, 8), (1400, 512, 64, 8), (1500, 1024, 64, 8)])
+@pytest.mark.parametrize("how", ["positions", "offset", "wrap", "table", "plain"])
+def test_qkv_tile_gemm(gpu, rows, hidden, nq, nkv, how):
+    """The GEMM tiles at sizes that take each of them (64 x 32 .. 128 x 256): fewer K slices than ring stages, odd and even
+    slice counts (tiles that split a stage's two slices between their wavefronts), ragged last row and column tiles, and
+    every source of the rotary positions: a tensor, one sequence behind an offset, several sequences with wrap-around, a
+    cos / sin table, no rotation."""
+    g = torch.Generator().manual_seed(40 + rows)
+    x = torch.randn(rows, hidden, generator=g).bfloat16()
+    w = (0.05 * torch.randn((nq + 2 * nkv) * 64, hidden, generator=g)).bfloat16()
+    b = (0.05 * torch.randn((nq + 2 * nkv) * 64, generator=g)).bfloat16()
+    kw, pos = {}, torch.randint(0, 8192, (rows,), generator=g)
+    if how == "positions":
+        kw = dict(yarn=T.gpt_oss_yarn(), positions=pos.to(gpu))
+    elif how == "offset":
+        pos = 37 + torch.arange(rows)
+        kw = dict(yarn=T.gpt_oss_yarn(), offset=torch.tensor([37], device=gpu))
+    elif how == "wrap":
+        pos = (90 + torch.arange(rows) % 100) % 150
+        kw = dict(yarn=T.gpt_oss_yarn(), offset=torch.tensor([90], device=gpu), tokens_per_batch=100, max_context_length=150)
+    elif how == "table":
+        cos, sin = O.yarn_cos_sin(torch.arange(8192))
+        kw = dict(cos=cos.to(gpu), sin=sin.to(gpu), positions=pos.to(gpu), max_context_length=8192)
+    else:
+        kw = dict(rotate=False)
+    q, k, v = T.qkv_rope_forward(x.to(gpu), w.to(gpu), b.to(gpu), nq, nkv, 64, mode="prefill", **kw)
+    if how == "plain":
+        want = O.linear_ref(x, w, b)
+        qr, kr, vr = want[:, :nq * 64], want[:, nq * 64:(nq + nkv) * 64], want[:, (nq + nkv) * 64:]
+    else:
+        qr, kr, vr = O.qkv_rope_ref(x, w, b, pos, nq, nkv, 64)
+    close(q, qr)
+    close(k, kr)
+    close(v, vr)
+
+
+@pytest.mark.parametrize("rows,k,n", [(1, 64, 16), (3, 4096, 2880), (97, 4096, 2880), (200, 448, 2880), (333, 576, 2880), (512, 640, 2880),
+                                      (999, 320, 2880), (1400, 256, 2880), (2048, 192, 2880), (70, 128, 48)])
+def test_linear_tile_gemm(gpu, rows, k, n):
+    """OUT.forward of a prompt against the oracle, through the module, and where it hands over to the library: a gradient
+    wanted, and more rows than one round of tiles."""
+    g = torch.Generator().manual_seed(900 + rows)
+    x = torch.randn(1, rows, k, generator=g).bfloat16()
+    mod = T.OUT(k, n, device=gpu).requires_grad_(False)
+    mod.weight.copy_((0.05 * torch.randn(n, k, generator=g)).bfloat16())
+    mod.bias.copy_((0.05 * torch.randn(n, generator=g)).bfloat16())
+    want = O.linear_ref(x[0], mod.weight.cpu(), mod.bias.cpu())
+    assert ops.linear_fits(x.to(gpu), mod.weight, mod.bias)
+    out = mod(x.to(gpu))
+    assert out.shape == (1, rows, n)
+    close(out[0], want)
+    assert not ops.linear_fits(torch.empty(128 * 256 + 1, k, dtype=torch.bfloat16, device=gpu), mod.weight, mod.bias)
+    mod.weight.requires_grad_(True)
+    assert not ops.linear_fits(x.to(gpu), mod.weight, mod.bias)
+    y = mod(x.to(gpu))
+    assert y.requires_grad
+    close(y.detach()[0], want)
 
 
 def test_qkv_generic_shapes(gpu):

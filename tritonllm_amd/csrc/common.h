@@ -1,5 +1,6 @@
 // Shared device/host helpers for the gfx950 layer kernels.
 #pragma once
+#include <atomic>
 #include <type_traits>
 
 #include <hip/hip_runtime.h>
@@ -29,6 +30,17 @@ int check_launch(const char* what);
       return (code);                       \
     }                                      \
   } while (0)
+
+// More than 64 KB of dynamic LDS has to be asked for once per kernel and device; `done` (one per kernel) remembers where.
+static inline hipError_t raise_lds_limit(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
+  int dev = 0;
+  if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+  const uint64_t bit = 1ull << (dev & 63);
+  if (dev < 64 && (done.load(std::memory_order_relaxed) & bit)) return hipSuccess;
+  const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e == hipSuccess) done.fetch_or(bit, std::memory_order_relaxed);
+  return e;
+}
 
 static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -167,7 +179,8 @@ __device__ __forceinline__ void sincos_reduced(float x, float* s, float* c) {
 // cos/sin of the rotary angle for (position, frequency), scaled by the concentration. The angle is
 // the single fp32 product float(pos) * inv_freq, exactly as the reference's table construction forms
 // it (angles reach 1.3e5 rad at the end of the context: the fast hardware sin/cos are useless here).
-__device__ __forceinline__ void yarn_cos_sin(int64_t pos, float inv_freq, float concentration, float* c, float* s) {
+template <class Int>
+__device__ __forceinline__ void yarn_cos_sin(Int pos, float inv_freq, float concentration, float* c, float* s) {
   const float angle = __fmul_rn(static_cast<float>(pos), inv_freq);
   float sv, cv;
   sincos_reduced(angle, &sv, &cv);

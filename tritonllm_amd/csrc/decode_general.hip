@@ -131,12 +131,12 @@ __global__ __launch_bounds__(320) void out_decode_general_kernel(OutArgs a, int 
 }
 
 namespace {
-template <class Kernel, class... Args>
-int launch(const char* what, Kernel kernel, int lds, unsigned gx, int64_t gy, hipStream_t st, const Args&... args) {
+template <auto kernel, class... Args>
+int launch(const char* what, int lds, unsigned gx, int64_t gy, hipStream_t st, const Args&... args) {
   TLLM_REQUIRE(gy <= 65535, TLLM_E_SHAPE, "%s: too many rows for the decode kernel", what);
-  // above 64 KB of dynamic LDS a kernel has to say so once per device; idempotent and cheap next to a launch
   if (lds > 64 * 1024) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    static std::atomic<uint64_t> done{0};
+    hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds, done);
     TLLM_REQUIRE(e == hipSuccess, TLLM_E_LAUNCH, "%s: cannot raise LDS limit: %s", what, hipGetErrorString(e));
   }
   hipLaunchKernelGGL(kernel, dim3(gx, (unsigned)gy), dim3(320), (size_t)lds, st, args...);
@@ -149,10 +149,10 @@ int launch_qkv_decode_general(const char* what, const QkvArgs& a, const RopeArgs
   const bool few = a.rows <= 8;
   const int64_t gy = few ? 1 : (a.rows + 15) / 16;
   if (a.w_scale)
-    return few ? launch(what, qkv_decode_general_kernel<8, true>, DecodeGeneralStream<8, true>::LDS, gx, gy, st, a, ra, fr)
-               : launch(what, qkv_decode_general_kernel<16, true>, DecodeGeneralStream<16, true>::LDS, gx, gy, st, a, ra, fr);
-  return few ? launch(what, qkv_decode_general_kernel<8, false>, DecodeGeneralStream<8, false>::LDS, gx, gy, st, a, ra, fr)
-             : launch(what, qkv_decode_general_kernel<16, false>, DecodeGeneralStream<16, false>::LDS, gx, gy, st, a, ra, fr);
+    return few ? launch<qkv_decode_general_kernel<8, true>>(what, DecodeGeneralStream<8, true>::LDS, gx, gy, st, a, ra, fr)
+               : launch<qkv_decode_general_kernel<16, true>>(what, DecodeGeneralStream<16, true>::LDS, gx, gy, st, a, ra, fr);
+  return few ? launch<qkv_decode_general_kernel<8, false>>(what, DecodeGeneralStream<8, false>::LDS, gx, gy, st, a, ra, fr)
+             : launch<qkv_decode_general_kernel<16, false>>(what, DecodeGeneralStream<16, false>::LDS, gx, gy, st, a, ra, fr);
 }
 
 int launch_out_decode_general(const char* what, const OutArgs& a, hipStream_t st) {
@@ -162,10 +162,10 @@ int launch_out_decode_general(const char* what, const OutArgs& a, hipStream_t st
   const bool few = a.rows <= 8;
   const int64_t gy = few ? 1 : (a.rows + 15) / 16;
   if (a.w_scale)
-    return few ? launch(what, out_decode_general_kernel<8, true>, DecodeGeneralStream<8, true>::LDS, gx, gy, st, a, vec8)
-               : launch(what, out_decode_general_kernel<16, true>, DecodeGeneralStream<16, true>::LDS, gx, gy, st, a, vec8);
-  return few ? launch(what, out_decode_general_kernel<8, false>, DecodeGeneralStream<8, false>::LDS, gx, gy, st, a, vec8)
-             : launch(what, out_decode_general_kernel<16, false>, DecodeGeneralStream<16, false>::LDS, gx, gy, st, a, vec8);
+    return few ? launch<out_decode_general_kernel<8, true>>(what, DecodeGeneralStream<8, true>::LDS, gx, gy, st, a, vec8)
+               : launch<out_decode_general_kernel<16, true>>(what, DecodeGeneralStream<16, true>::LDS, gx, gy, st, a, vec8);
+  return few ? launch<out_decode_general_kernel<8, false>>(what, DecodeGeneralStream<8, false>::LDS, gx, gy, st, a, vec8)
+             : launch<out_decode_general_kernel<16, false>>(what, DecodeGeneralStream<16, false>::LDS, gx, gy, st, a, vec8);
 }
 
 }  // namespace tllm

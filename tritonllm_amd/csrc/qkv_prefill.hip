@@ -34,7 +34,7 @@
 // the stages, it is built inside the idle ring after the K loop); every lane adds the bias to its fp32 accumulators,
 // rotates q/k pairs, rounds once to bf16 into an LDS image of the tile, and the image leaves as coalesced 128-bit
 // stores straight into the separate q / k / v outputs (no split / contiguous copies afterwards).
-#include "qkv_common.h"
+#include "qkv_prefill.h"
 
 namespace tllm {
 
@@ -64,10 +64,6 @@ static_assert(IMG_BYTES + CS_BYTES <= ring_bytes(128) && IMG_BYTES + CS_BYTES <=
 static_assert(prefill_smem(128) <= 160 * 1024 && prefill_smem(256) <= 160 * 1024, "LDS per workgroup");
 static_assert(W_STAGE % 8192 == 0 && x_stage(128) % 8192 == 0 && CHUNKS == 8 && XS == 2, "the schedules and the swizzle below are written for BK = 64");
 }  // namespace
-
-// Chunk swizzle of LDS row r: the 16-byte chunk c of the row is stored at chunk position c ^ swz(r). Eight consecutive
-// rows of one chunk land on the eight chunk positions, and rows r, r + 8 on positions that differ in bit 0.
-__device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 
 // Tile of a workgroup, XCD-aware: consecutive block ids go to different XCDs (8 of them, each with its own L2), so
 // every XCD gets a compact super-block of `swizzle` x (32 / swizzle) tiles (token tiles x column tiles).
@@ -133,29 +129,6 @@ __device__ __forceinline__ void w_tile_row_quads(int i, int* head_local, int* di
   const int b = i >> 4, i16 = i & 15;
   *head_local = b >> 2;
   *dim = 8 * (b & 3) + 2 * (i16 >> 2) + (i16 & 1) + 32 * ((i16 >> 1) & 1);
-}
-
-// Unwrapped rotary positions of 16 consecutive rows starting at row g0 (the same in every lane; rows past the last one
-// repeat it), read through the scalar cache: positions and offset were written before this kernel started and nothing
-// writes them while it runs, and a scalar load does not involve the vector-memory counter the look-ahead loads are
-// waited for with. Without a positions tensor the result is offset[0] alone and the caller adds row % tokens_per_batch.
-__device__ __forceinline__ void rope_positions_16_uniform(const RopeArgs& r, const void* any_valid, int64_t g0, int64_t rows, int64_t (&pos_even)[8],
-                                                          int64_t (&pos_odd)[8]) {
-  typedef const int64_t __attribute__((address_space(4))) * const_i64_ptr;
-  // branch-free (an absent tensor reads a valid dummy address), so that the sixteen values stay in scalar registers
-  const_i64_ptr pp = reinterpret_cast<const_i64_ptr>(reinterpret_cast<uintptr_t>(r.positions ? static_cast<const void*>(r.positions) : any_valid));
-  const_i64_ptr po = reinterpret_cast<const_i64_ptr>(reinterpret_cast<uintptr_t>(r.offset ? static_cast<const void*>(r.offset) : any_valid));
-  const int64_t off_ld = po[0];
-  const int64_t off = r.offset ? off_ld : 0;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int64_t gi = g0 + j < rows ? g0 + j : rows - 1;
-    const int64_t ld = pp[r.positions ? gi : 0];
-    // two arrays: a lane picks row 2 i or 2 i + 1 by a select between them (of one array the compiler makes an
-    // indexed access, and the array then lives in scratch memory)
-    if (j & 1) pos_odd[j >> 1] = r.positions ? ld : off;
-    else pos_even[j >> 1] = r.positions ? ld : off;
-  }
 }
 
 // TABLE: cos / sin come from the caller's tables (two loads per value) instead of the YaRN parameters.
@@ -715,6 +688,17 @@ extern "C" int tllm_qkv_rope_prefill_bf16(const void* x, const void* W, const vo
     launch_qkv_generic(a, ra, fr, st);
     return check_launch("qkv_rope_prefill(generic)");
   }
+  const int heads = n_q_heads + 2 * n_kv_heads;
+  // Tile height by a cost model: a round of 128-token tiles over the 256 CUs takes ~57 us, a round of 256-token tiles ~105 us
+  // (both per 45 slices of K); whichever needs less in total. T = 2048 is one round of 128s; anything that would need a
+  // second round of 128s is one round of 256s instead, T = 8192 two rounds of 256s instead of four of 128s. Up to about
+  // 1500 rows (of 5120 columns) smaller tiles fill the machine in less than a round of these (tile_gemm.hip: 1536 rows 50.9
+  // against 57 us, 999 rows 39.8 against 49.1, 97 rows 16.1 against 51).
+  const int64_t tn = (heads + HPT - 1) / HPT;
+  const int64_t rounds128 = (((rows + 127) / 128) * tn + 255) / 256, rounds256 = (((rows + 255) / 256) * tn + 255) / 256;
+  const int BM = rounds256 * 105 < rounds128 * 57 ? 256 : 128;
+  const int64_t here_ns = (BM == 256 ? rounds256 * 105000 : rounds128 * 57000) * (hidden / BK) / 45;
+  if (tile_gemm_ns(rows, static_cast<int64_t>(heads) * 64, hidden) < here_ns) return launch_tile_gemm_qkv("qkv_rope_prefill", a, ra, fr, st);
   static bool attr_set = false;   // raising the dynamic-LDS limit is idempotent; a benign race at worst repeats it
   if (!attr_set) {
     const void* k128[] = {reinterpret_cast<const void*>(qkv_prefill_quads_kernel<false>), reinterpret_cast<const void*>(qkv_prefill_quads_kernel<true>)};
@@ -726,13 +710,6 @@ extern "C" int tllm_qkv_rope_prefill_bf16(const void* x, const void* W, const vo
     }
     attr_set = true;
   }
-  const int heads = n_q_heads + 2 * n_kv_heads;
-  // Tile height by a two-number cost model: a round of 128-token tiles over the 256 CUs takes ~62 us, a round of
-  // 256-token tiles ~105 us (3 : 5); whichever needs less in total. T = 2048 is one round of 128s; anything that would
-  // need a second round of 128s is one round of 256s instead, T = 8192 two rounds of 256s instead of four of 128s.
-  const int64_t tn = (heads + HPT - 1) / HPT;
-  const int64_t rounds128 = (((rows + 127) / 128) * tn + 255) / 256, rounds256 = (((rows + 255) / 256) * tn + 255) / 256;
-  const int BM = rounds256 * 5 < rounds128 * 3 ? 256 : 128;
   const int64_t tiles_m = (rows + BM - 1) / BM;
   const int tiles_n = (heads + HPT - 1) / HPT;
   const int64_t tiles = tiles_m * tiles_n;
