@@ -9,27 +9,44 @@ namespace tllm {
 // rows of one chunk land on the eight chunk positions, and rows r, r + 8 on positions that differ in bit 0.
 __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 
-// Unwrapped rotary positions of 16 consecutive rows starting at row g0 (the same in every lane; rows past the last one
-// repeat it), read through the scalar cache: positions and offset were written before this kernel started and nothing
-// writes them while it runs, and a scalar load does not involve the vector-memory counter the look-ahead loads are
-// waited for with. Without a positions tensor the result is offset[0] alone and the caller adds row % tokens_per_batch.
-__device__ __forceinline__ void rope_positions_16_uniform(const RopeArgs& r, const void* any_valid, int64_t g0, int64_t rows, int64_t (&pos_even)[8],
-                                                          int64_t (&pos_odd)[8]) {
+// Rotary positions of N consecutive rows starting at row g0 (the same in every lane; rows past the last one repeat it), as
+// they are when all of them lie in [0, max_ctx) -- which the return value says -- and no row belongs to a second sequence.
+// Otherwise (wrap-around, several sequences without a positions tensor) the caller fills its table with rope_position(), in
+// a rolled loop: the 64-bit divisions inlined per row were 32 KB of code to fetch, executed or not, at about 1 us per 8 KB.
+// Read through the scalar cache: positions and offset were written before this kernel started and nothing writes them while
+// it runs, and a scalar load does not involve the vector-memory counter the look-ahead loads are waited for with.
+template <int N>
+__device__ __forceinline__ bool rope_positions_uniform(const RopeArgs& r, const void* any_valid, int64_t g0, int64_t rows, int (&pos)[N]) {
   typedef const int64_t __attribute__((address_space(4))) * const_i64_ptr;
-  // branch-free (an absent tensor reads a valid dummy address), so that the sixteen values stay in scalar registers
+  // branch-free (an absent tensor reads a valid dummy address), so that the values stay in scalar registers
   const_i64_ptr pp = reinterpret_cast<const_i64_ptr>(reinterpret_cast<uintptr_t>(r.positions ? static_cast<const void*>(r.positions) : any_valid));
   const_i64_ptr po = reinterpret_cast<const_i64_ptr>(reinterpret_cast<uintptr_t>(r.offset ? static_cast<const void*>(r.offset) : any_valid));
   const int64_t off_ld = po[0];
   const int64_t off = r.offset ? off_ld : 0;
+  uint64_t most = 0;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
+  for (int j = 0; j < N; ++j) {
     const int64_t gi = g0 + j < rows ? g0 + j : rows - 1;
     const int64_t ld = pp[r.positions ? gi : 0];
-    // two arrays: a lane picks row 2 i or 2 i + 1 by a select between them (of one array the compiler makes an
-    // indexed access, and the array then lives in scratch memory)
-    if (j & 1) pos_odd[j >> 1] = r.positions ? ld : off;
-    else pos_even[j >> 1] = r.positions ? ld : off;
+    const uint64_t q = static_cast<uint64_t>(r.positions ? ld : off + gi);
+    pos[j] = static_cast<int>(q);
+    if (q > most) most = q;
   }
+  return most < static_cast<uint64_t>(r.max_ctx) && most < (1ull << 31) && (r.positions || rows <= r.tokens_per_batch);
+}
+
+// (cos, sin) of frequency f at position p in [0, max_ctx)
+template <bool TABLE>
+__device__ __forceinline__ float2 rope_cos_sin_at(const RopeArgs& r, const YarnFreqs& fr, int p, int f) {
+  float c, s;
+  if constexpr (TABLE) {
+    const int64_t at = p * r.table_row_stride + f;
+    c = r.cos_table[at];
+    s = r.sin_table[at];
+  } else {
+    yarn_cos_sin(p, fr.v[f], r.concentration, &c, &s);
+  }
+  return make_float2(c, s);
 }
 
 // Tiles of 64 x 32 .. 128 x 256 (tile_gemm.hip). QKV + bias + rotary: hidden % 64 == 0, head_dim 64, x and W 16-byte aligned,

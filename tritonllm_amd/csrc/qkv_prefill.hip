@@ -90,7 +90,7 @@ __device__ __forceinline__ void prefill_copy_out(const QkvArgs& a, const bf16* i
   const bool vec_ok = (reinterpret_cast<uintptr_t>(a.q) % 16 == 0) && (reinterpret_cast<uintptr_t>(a.k) % 16 == 0) &&
                       (reinterpret_cast<uintptr_t>(a.v) % 16 == 0) && a.q_rs % 8 == 0 && a.k_rs % 8 == 0 && a.v_rs % 8 == 0 &&
                       a.kv_slot_stride % 8 == 0;
-#pragma unroll 4
+#pragma unroll 2
   for (int ch = tid; ch < EROWS * (BN / 8); ch += NT) {
     const int r = ch / (BN / 8), cc = ch - r * (BN / 8);
     const int hl = cc >> 3, d8 = (cc & 7) * 8;
@@ -290,33 +290,15 @@ __global__ __launch_bounds__(512) void qkv_prefill_quads_kernel(QkvArgs a, RopeA
   constexpr int CSN = 8;
   static_assert(NW * 2 * CSN == EROWS && EROWS == BM, "eight wavefronts x two rows x eight rounds cover the tile");
   float2 csr[CSN];
-  if (TABLE || a.has_rope) {
-    const int f = lane & 31;
-    int64_t pos_even[CSN], pos_odd[CSN];
-    rope_positions_16_uniform(ra, a.W, row0 + 16 * wave, a.rows, pos_even, pos_odd);
-    // TABLE: the loads go out whether there is a rotation or not (without one they read the weight's first bytes), so
-    // that the waits below can count on them, and no branch surrounds a load.
-    const float* cos_t = a.has_rope ? ra.cos_table : reinterpret_cast<const float*>(a.W);
-    const float* sin_t = a.has_rope ? ra.sin_table : reinterpret_cast<const float*>(a.W);
+  const int64_t first_row = row0 + 16 * wave;
+  bool plain = true;
+  if (a.has_rope) {
+    int pos[2 * CSN];
+    plain = rope_positions_uniform<2 * CSN>(ra, a.W, first_row, a.rows, pos);
+    // TABLE: the youngest loads of the prologue: every wait below is for older loads and so at most stricter than it
+    // needs to be until these have landed, which they have by the loop's second slice.
 #pragma unroll
-    for (int j = 0; j < CSN; ++j) {
-      int64_t p = lane < 32 ? pos_even[j] : pos_odd[j];
-      if (!ra.positions) {                                  // uniform
-        int64_t grow = row0 + 16 * wave + 2 * j + (lane >> 5);
-        if (grow >= a.rows) grow = a.rows - 1;
-        p += grow < ra.tokens_per_batch ? grow : grow % ra.tokens_per_batch;
-      }
-      if constexpr (TABLE) {
-        const int64_t at = a.has_rope ? rope_wrap(p, ra.max_ctx) * ra.table_row_stride + f : f;
-        // The youngest loads of the prologue: every wait below is for older loads and so at most stricter than it
-        // needs to be until these have landed, which they have by the loop's second slice.
-        csr[j] = make_float2(cos_t[at], sin_t[at]);
-      } else {
-        float c, sn;
-        yarn_cos_sin(rope_wrap(p, ra.max_ctx), fr.v[f], ra.concentration, &c, &sn);
-        csr[j] = make_float2(c, sn);
-      }
-    }
+    for (int j = 0; j < CSN; ++j) csr[j] = rope_cos_sin_at<TABLE>(ra, fr, plain ? (lane < 32 ? pos[2 * j] : pos[2 * j + 1]) : 0, lane & 31);
   }
   // slice 0 has landed when only those are outstanding
   // (TABLE: the sixteen table loads are younger still and are not counted in, so this wait also takes some of the
@@ -352,8 +334,20 @@ __global__ __launch_bounds__(512) void qkv_prefill_quads_kernel(QkvArgs a, RopeA
   bf16* img = reinterpret_cast<bf16*>(smem);
   const int64_t slot_off = qkv_slot(a, ra) * a.kv_slot_stride;
   if (a.has_rope) {
+    float2* const mine = cs_tab + (16 * wave + (lane >> 5)) * CSROW + (lane & 31);
+    if (plain) {
 #pragma unroll
-    for (int j = 0; j < CSN; ++j) cs_tab[(16 * wave + 2 * j + (lane >> 5)) * CSROW + (lane & 31)] = csr[j];
+      for (int j = 0; j < CSN; ++j) mine[2 * j * CSROW] = csr[j];
+    } else {
+#pragma unroll 1
+      for (int j = 0; j < CSN; ++j) {
+        int64_t gi = first_row + 2 * j + (lane >> 5);
+        if (gi >= a.rows) gi = a.rows - 1;
+        float c, sn;
+        rope_cos_sin(ra, fr, rope_position(ra, gi), lane & 31, &c, &sn);
+        mine[2 * j * CSROW] = make_float2(c, sn);
+      }
+    }
   }
   if (tid < BN) bias_s[tid] = a.bias ? static_cast<float>(bias_raw) : 0.f;
   __syncthreads();
@@ -526,7 +520,7 @@ __global__ __launch_bounds__(512) void qkv_prefill_kernel256(QkvArgs a, RopeArgs
   constexpr int BIAS_OFF = ring_bytes(BM);
   float2* cs_tab = reinterpret_cast<float2*>(smem + CS_OFF);
   float* bias_s = reinterpret_cast<float*>(smem + BIAS_OFF);
-  int64_t* pos_s = reinterpret_cast<int64_t*>(smem + BIAS_OFF + BIAS_BYTES);
+  int64_t* pos_s = reinterpret_cast<int64_t*>(smem + BIAS_OFF + BIAS_BYTES);   // wrapped into [0, max_ctx) here, once
 #pragma unroll
   for (int j = 0; j < LPW; ++j) issue_load(-2, j);
   if (tid < BN) {
@@ -538,7 +532,7 @@ __global__ __launch_bounds__(512) void qkv_prefill_kernel256(QkvArgs a, RopeArgs
     for (int r = tid; r < BM; r += NT) {
       int64_t grow = row0 + r;
       if (grow >= a.rows) grow = a.rows - 1;
-      pos_s[r] = rope_position_raw(ra, grow);
+      pos_s[r] = rope_position(ra, grow);
     }
   }
 #pragma unroll
@@ -592,7 +586,7 @@ __global__ __launch_bounds__(512) void qkv_prefill_kernel256(QkvArgs a, RopeArgs
         float c[EROWS / 16], sn[EROWS / 16];                   // all sixteen loads out before the first is looked at
 #pragma unroll
         for (int j = 0; j < EROWS / 16; ++j) {
-          const int64_t at = rope_wrap(pos[j], ra.max_ctx) * ra.table_row_stride + f;
+          const int64_t at = pos[j] * ra.table_row_stride + f;
           c[j] = ra.cos_table[at];
           sn[j] = ra.sin_table[at];
         }
@@ -602,7 +596,7 @@ __global__ __launch_bounds__(512) void qkv_prefill_kernel256(QkvArgs a, RopeArgs
 #pragma unroll
         for (int j = 0; j < EROWS / 16; ++j) {
           float c, sn;
-          yarn_cos_sin(rope_wrap(pos[j], ra.max_ctx), fr.v[f], ra.concentration, &c, &sn);
+          yarn_cos_sin(static_cast<int>(pos[j]), fr.v[f], ra.concentration, &c, &sn);   // (max_ctx <= 2^24 with YaRN parameters)
           cs_tab[((tid >> 5) + 16 * j) * CSROW + f] = make_float2(c, sn);
         }
       }

@@ -217,25 +217,11 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
   const int f = lane & 31;
   float2 csr[CSN];
   bool plain = true;
-  if (MODE == kGemmYarn && a.has_rope) {
-    typedef const int64_t __attribute__((address_space(4))) * const_i64_ptr;
-    const_i64_ptr pp = reinterpret_cast<const_i64_ptr>(reinterpret_cast<uintptr_t>(ra.positions ? static_cast<const void*>(ra.positions) : a.W));
-    const_i64_ptr po = reinterpret_cast<const_i64_ptr>(reinterpret_cast<uintptr_t>(ra.offset ? static_cast<const void*>(ra.offset) : a.W));
-    const int64_t off_ld = po[0];
-    const int64_t off = ra.offset ? off_ld : 0;
+  if (MODE != kGemmLinear && a.has_rope) {
     int pos[RPW];
-    uint64_t most = 0;
+    plain = rope_positions_uniform<RPW>(ra, a.W, first_row, a.rows, pos);
 #pragma unroll
-    for (int j = 0; j < RPW; ++j) {
-      const int64_t gi = first_row + j < a.rows ? first_row + j : a.rows - 1;
-      const int64_t ld = pp[ra.positions ? gi : 0];
-      const uint64_t q = static_cast<uint64_t>(ra.positions ? ld : off + gi);   // (without positions: right for a single sequence)
-      pos[j] = static_cast<int>(q);
-      if (q > most) most = q;
-    }
-    plain = most < static_cast<uint64_t>(ra.max_ctx) && (ra.positions || a.rows <= ra.tokens_per_batch);   // (max_ctx <= 2^24 with YaRN parameters)
-#pragma unroll
-    for (int j = 0; j < CSN; ++j) yarn_cos_sin(lane < 32 ? pos[2 * j] : pos[2 * j + 1], fr.v[f], ra.concentration, &csr[j].x, &csr[j].y);
+    for (int j = 0; j < CSN; ++j) csr[j] = rope_cos_sin_at<MODE == kGemmTable>(ra, fr, plain ? (lane < 32 ? pos[2 * j] : pos[2 * j + 1]) : 0, f);
   }
   wait_slices_left<S - 1, LPW>(first - 1);
   asm volatile("s_barrier" ::: "memory");
@@ -287,7 +273,7 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
     __syncthreads();                                                 // the ring, or the pass before, is done with
     if (MODE != kGemmLinear && a.has_rope && pass == 0) {
       float2* const mine = cs_tab + (RPW * wave + (lane >> 5)) * CSROW + f;
-      if (MODE == kGemmYarn && plain) {
+      if (plain) {
 #pragma unroll
         for (int j = 0; j < CSN; ++j) mine[2 * j * CSROW] = csr[j];
       } else {
