@@ -6,10 +6,12 @@ entry point raises. Build it with ``python -m tritonllm_amd.build``.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "lib", "libtllm_hip.so")
+HOST_PATH = os.path.join(_PKG, "lib", "tllm_host.so")
 
 MAX_ROPE_FREQS = 128
 ABI_VERSION = 1
@@ -91,6 +93,23 @@ def lib() -> C.CDLL:
             raise RuntimeError(f"libtllm_hip.so has ABI version {got}, this package expects {ABI_VERSION}: rebuild it")
         _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The ops' host side in C++ (csrc/host_ops.cpp), loaded once; it launches through the same shared library."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: the extension is not built (python -m tritonllm_amd.build)")
+        spec = importlib.util.spec_from_file_location("tllm_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def require(cond, msg: str = "") -> None:

@@ -1,4 +1,4 @@
-"""Compile the HIP sources into ``tritonllm_amd/lib/libtllm_hip.so`` for gfx950.
+"""Compile the HIP sources into ``tritonllm_amd/lib/libtllm_hip.so`` for gfx950, and the host side of the ops next to it.
 
 ``hipcc`` cross-compiles without a GPU, so this runs anywhere the ROCm toolchain
 is installed. Usage: ``python -m tritonllm_amd.build``.
@@ -16,6 +16,7 @@ ROOT = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libtllm_hip.so")
+HOST_PATH = os.path.join(LIB_DIR, "tllm_host.so")
 INCLUDE = os.path.join(ROOT, "include")
 
 SOURCES = ["abi.hip", "rmsnorm.hip", "embedding.hip", "swiglu.hip", "rope.hip", "qkv_decode.hip", "qkv_decode_r8.hip", "qkv_decode_r32.hip", "qkv_decode_rows.hip", "qkv_prefill.hip", "tile_gemm.hip", "decode_general.hip", "out_decode.hip", "out_decode_r8.hip", "out_decode_r32.hip", "unembed.hip", "attn_decode.hip", "attn_prefill.hip", "mxfp4.hip"]
@@ -44,6 +45,24 @@ def _compile(src: str, obj_dir: str) -> str:
     return obj
 
 
+def _compile_host(out: str) -> None:
+    """The Python-side half (csrc/host_ops.cpp): plain C++ against torch's headers, linked to the kernels' library."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE, *(f"-I{d}" for d in include_paths()),
+           f"-I{os.path.join(rocm, 'include')}", f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, "host_ops.cpp"), "-o", out,
+           f"-L{LIB_DIR}", "-ltllm_hip", f"-L{torch_lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on host_ops.cpp:\n{r.stdout}\n{r.stderr}")
+
+
 def build_library(verbose: bool = False) -> str:
     obj_dir = os.path.join(PKG_DIR, "build")
     os.makedirs(obj_dir, exist_ok=True)
@@ -56,8 +75,11 @@ def build_library(verbose: bool = False) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB_PATH)
+    _compile_host(HOST_PATH + ".tmp")
+    os.replace(HOST_PATH + ".tmp", HOST_PATH)
     if verbose:
-        print(f"built {LIB_PATH} ({os.path.getsize(LIB_PATH)} bytes)")
+        for p in (LIB_PATH, HOST_PATH):
+            print(f"built {p} ({os.path.getsize(p)} bytes)")
     return LIB_PATH
 
 

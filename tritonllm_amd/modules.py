@@ -14,7 +14,7 @@ import os
 import torch
 
 from . import ops
-from ._lib import check, lib
+from ._lib import check, host, lib
 from ._lib import require as _require
 from .yarn import YarnParams
 
@@ -91,6 +91,9 @@ class OUT(torch.nn.Module):
         return self._weight_fp8, self._weight_scale
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        done = host().linear(x, self.weight, self.bias)
+        if done is not None:
+            return done
         if ops.linear_fits(x, self.weight, self.bias):
             return ops.linear_forward(x, self.weight, self.bias)
         return torch.nn.functional.linear(x, self.weight, self.bias)

@@ -6,6 +6,10 @@ hands them to ``libtllm_hip.so`` on the current PyTorch HIP stream. PyTorch is p
 here -- memory, streams, dtypes; all arithmetic happens in the HIP kernels. There is no
 CPU path: tensors must live on the GPU and the shared library must be built.
 
+The ops a model calls per layer first offer their arguments to the C++ side (``csrc/host_ops.cpp``), which checks and
+launches the ordinary case in a fraction of the host time; it answers ``None`` to anything else -- a strided operand, a
+wrong shape or type, a failed launch -- and the code here makes the copy or raises the error.
+
 Reference signatures (paths under ``tritonllm/gpt_oss/triton/``):
 
     rmsnorm_forward(x, scale, eps, out=None)                         triton_kernels.py:28
@@ -28,7 +32,7 @@ import math
 import torch
 
 from . import scratch_pool
-from ._lib import TllmRope, check, lib
+from ._lib import TllmRope, check, host, lib
 from ._lib import require as _require
 from .yarn import YarnParams
 
@@ -77,15 +81,21 @@ def _yarn_of(t) -> YarnParams | None:
     return getattr(t, "_tllm_yarn", None)
 
 
+def _yarn_or_tables(yarn, cos, sin) -> YarnParams | None:
+    """``yarn``, or the parameters that a pair of tables carries."""
+    if yarn is None and cos is not None:
+        yarn = _yarn_of(cos)
+        if yarn is not None and _yarn_of(sin) is not yarn:
+            yarn = None
+    return yarn
+
+
 def _rope_desc(cos, sin, yarn, positions, offset, tokens_per_batch, max_ctx, keep: list, rows: int) -> TllmRope:
     """Fill the C descriptor of where the rotary angles come from. ``keep`` collects
     objects that must stay alive until the launch call has returned. ``rows`` is the number of rows the kernel
     will rotate: it reads ``positions[row]`` for each of them, and only the host can check that they exist."""
     r = TllmRope()
-    if yarn is None and cos is not None:
-        yarn = _yarn_of(cos)
-        if yarn is not None and _yarn_of(sin) is not yarn:
-            yarn = None
+    yarn = _yarn_or_tables(yarn, cos, sin)
     if yarn is not None:
         r.yarn = yarn.c_pointer()
         keep.append(yarn)
@@ -123,6 +133,9 @@ def _rope_desc(cos, sin, yarn, positions, offset, tokens_per_batch, max_ctx, kee
 # --------------------------------------------------------------------------------------- RMSNorm
 def rmsnorm_forward(x: torch.Tensor, scale: torch.Tensor, eps: float, out: torch.Tensor | None = None) -> torch.Tensor:
     """``y = x * rsqrt(mean(x^2) + eps) * scale`` over the last dim; ``out`` may alias ``x``."""
+    done = host().rmsnorm(x, scale, eps, out)       # here and below: None means anything but the ordinary case, see below
+    if done is not None:
+        return done
     _on_gpu(x, scale, out)
     _require(x.dtype == _BF16, "rmsnorm_forward: x must be bfloat16")
     _require(scale.dtype in (torch.float32, _BF16), "rmsnorm_forward: scale must be float32 or bfloat16")
@@ -149,6 +162,9 @@ def embedding_forward(ids: torch.Tensor, table: torch.Tensor, out: torch.Tensor 
 
     An id outside ``[0, vocab)`` produces a zero row and sets ``oob_flag`` (int32 device
     scalar) to 1 when one is given -- never a device fault."""
+    done = host().embedding(ids, table, out, oob_flag)
+    if done is not None:
+        return done
     _on_gpu(ids, table, out, oob_flag)
     _require(table.dtype == _BF16 and table.ndim == 2 and table.is_contiguous())
     _require(ids.dtype in (torch.int32, torch.int64))
@@ -174,6 +190,9 @@ def embedding_rmsnorm_forward(ids: torch.Tensor, table: torch.Tensor, scale: tor
     Returns ``(x, normed)``, both ``[*ids.shape, hidden]``: ``x`` bit-exact like ``embedding_forward`` (a fresh tensor
     unless ``x_out`` is given), ``normed`` identical to ``rmsnorm_forward(x, scale, eps)`` (pooled unless ``out`` is given).
     Hidden sizes the fused kernel does not cover take the two separate calls."""
+    done = host().embedding_rmsnorm(ids, table, scale, eps, x_out, out, oob_flag)
+    if done is not None:
+        return done
     _on_gpu(ids, table, scale, x_out, out, oob_flag)
     _require(table.dtype == _BF16 and table.ndim == 2 and table.is_contiguous())
     _require(ids.dtype in (torch.int32, torch.int64))
@@ -208,6 +227,9 @@ def embedding_rmsnorm_forward(ids: torch.Tensor, table: torch.Tensor, scale: tor
 def swiglu(x: torch.Tensor, alpha: float = 1.702, limit: float | None = 7.0, interleaved: bool = True,
            out: torch.Tensor | None = None) -> torch.Tensor:
     """Clamped SwiGLU over the last dim: ``[..., 2n] -> [..., n]``."""
+    done = host().swiglu(x, alpha, limit, interleaved, out)
+    if done is not None:
+        return done
     _on_gpu(x, out)
     _require(x.dtype == _BF16, "swiglu: x must be bfloat16")
     _require(x.shape[-1] % 2 == 0)
@@ -343,6 +365,11 @@ def qkv_rope_forward(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
     outputs written to three dense tensors. ``mode``: "decode" (weight streaming),
     "prefill" (MFMA GEMM) or "auto" (by row count). No reference twin as a single call:
     it is F.linear + split + contiguous + rope_forward of model.py:506-522 in one launch."""
+    done = host().qkv_rope(x, weight, bias, num_q_heads, num_kv_heads, head_dim, _yarn_or_tables(yarn, cos, sin), positions, offset,
+                           tokens_per_batch, max_context_length, rotate, mode, out, norm_scale, norm_eps, weight_scale,
+                           norm_scale is not None and _norm_fusable("prefill" if mode == "prefill" else "decode", x.shape[0], x.shape[-1], head_dim))
+    if done is not None:
+        return done
     _on_gpu(x, weight, bias, positions, offset, cos, sin, norm_scale, weight_scale)
     _require(x.ndim == 2)
     _require((weight.dtype == _FP8) == (weight_scale is not None), "a float8 weight needs weight_scale, a bfloat16 one takes none")
@@ -480,6 +507,11 @@ def qkv_rope_cache_decode_forward(hidden, weight, bias, sin, cos, max_context_le
     (a borrowed pool buffer). ``offset`` is an int64 device tensor of shape (1,) and is read
     on the device, so the call can be replayed from a HIP graph. With ``norm_scale`` the
     block's input RMSNorm (model.py:476) runs inside the same kernel on the raw ``hidden``."""
+    done = host().qkv_rope_cache(hidden, weight, bias, _yarn_or_tables(yarn, cos, sin), max_context_length, cache_k, cache_v, offset,
+                                 num_q_heads, num_kv_heads, head_dim, weight_scale, positions, norm_scale, norm_eps,
+                                 norm_scale is not None and _norm_fusable("decode", hidden.shape[0], hidden.shape[-1], head_dim))
+    if done is not None:
+        return done
     _on_gpu(hidden, weight, bias, cache_k, cache_v, offset, positions, norm_scale, weight_scale)
     _require((weight.dtype == _FP8) == (weight_scale is not None), "a float8 weight needs weight_scale, a bfloat16 one takes none")
     batch, num_tokens, hidden_size = hidden.shape
@@ -563,6 +595,9 @@ def out_residual_decode_forward(hidden: torch.Tensor, weight: torch.Tensor, bias
     ``hidden [B,1,out_dim]``, ``weight [hidden_size, out_dim]`` (bf16, or float8_e4m3fn with ``weight_scale
     [hidden_size]``), ``bias [hidden_size]``, ``residual [B,1,hidden_size]``. Like the reference the result is
     written into ``residual``'s storage (when its last dimension is dense) and returned as ``[B,1,hidden_size]``."""
+    done = host().out_residual(hidden, weight, bias, residual, weight_scale)
+    if done is not None:
+        return done
     _on_gpu(hidden, weight, bias, residual, weight_scale)
     batch, num_tokens, out_dim_hidden = hidden.shape
     hidden_size, out_dim_weight = weight.shape
@@ -614,6 +649,9 @@ def _unembed_prep(hidden, weight, weight_scale):
 def unembedding_decode_forward(hidden: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor | None = None) -> torch.Tensor:
     """``hidden [B,1,H] @ weight[V,H].T -> logits [B,1,V]`` (a borrowed pool buffer), triton_kernels.py:163-197;
     with ``weight_scale`` the fp8 form :271-302."""
+    done = host().unembedding(hidden, weight, weight_scale)
+    if done is not None:
+        return done
     x2, weight, ws, batch, hidden_size, vocab_size = _unembed_prep(hidden, weight, weight_scale)
     logits = scratch_pool.get((batch, vocab_size), hidden.dtype, hidden.device)
     rc = lib().tllm_unembedding_decode_bf16(x2.data_ptr(), weight.data_ptr(), ws.data_ptr() if ws is not None else None,
@@ -690,6 +728,9 @@ def attention_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sinks: t
     only the splits the context at ``start_q`` needs. ``kv_len_hint`` (an extension; the host's idea of how many keys
     are visible, e.g. the decode loop's position + 1) plans the launch for that length instead, which is faster when
     the context is far shorter than the cache; the result never depends on it."""
+    done = host().attention_decode(q, k, v, sinks, sm_scale, bandwidth, start_q, kv_len_hint)
+    if done is not None:
+        return done
     _on_gpu(q, k, v, sinks, start_q)
     _require(len(start_q) == 1 and start_q.dtype in (torch.int32, torch.int64))
     bs, n_ctx, n_kv_heads, repeat_kv, head_dim_q = q.shape
@@ -740,6 +781,9 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sinks: torch.Te
 
     ``q`` may be a view into the fused QKV output and ``k`` / ``v`` views of the cache: the kernel takes batch and
     token strides, so none of the reference's transposed, padded copies (:180-191) is made."""
+    done = host().attention(q, k, v, sinks, sm_scale, bandwidth, start_q)
+    if done is not None:
+        return done
     _on_gpu(q, k, v, sinks, start_q)
     _require(len(start_q) == 1 and start_q.dtype in (torch.int32, torch.int64))
     bs, n_ctx, n_kv_heads, repeat_kv, head_dim_q = q.shape

@@ -8,6 +8,7 @@ same fp32 operation order as the reference's ``RotaryEmbedding._compute_concentr
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import math
 from dataclasses import dataclass, field
 
@@ -49,6 +50,11 @@ class YarnParams:
             s.n_freq = len(self.inv_freq)
             object.__setattr__(self, "_c", s)
         return s
+
+    @functools.cached_property
+    def _c_address(self) -> int:
+        """Address of ``c_struct()``, which this object keeps (read by the ops' C++ side)."""
+        return C.addressof(self.c_struct())
 
     def c_pointer(self):
         return C.pointer(self.c_struct())
