@@ -1120,6 +1120,31 @@ def test_unembedding_more_than_16_rows_one_pass_over_the_weight(gpu, rows, vocab
     _argmax_ok(T.unembedding_decode_fp8_argmax_forward(xg, w8, ws), want8)
 
 
+@pytest.mark.parametrize("rows,vocab,hidden", [(9, 40, 4096), (24, 3001, 4096), (33, 20, 2880), (48, 70003, 2880), (65, 40000, 2880), (96, 5001, 64),
+                                                (97, 33001, 2880), (128, 9000, 2880), (128, 3001, 128), (131, 5000, 2880), (300, 2050, 192)])
+def test_unembedding_logits_in_tiles(gpu, rows, vocab, hidden):
+    """More rows than the kernels that keep them in LDS take: tiles of the vocabulary with the activations streamed next to
+    the weight. One to four row blocks per wavefront, several chunks of rows, workgroups with no vocabulary, one unit, many
+    and a last tile narrower than the others, vocabularies that are no multiple of 16 (and odd: no 8-byte stores), K of one
+    slice up (fewer stages than the ring), and neighbouring rows of the output left alone."""
+    from tritonllm_amd._lib import lib
+    g = torch.Generator().manual_seed(1300 + rows + hidden)
+    x = torch.randn(rows, hidden, generator=g).bfloat16()
+    w = ((0.02 if hidden == 2880 else 0.05) * torch.randn(vocab, hidden, generator=g)).bfloat16()
+    xg = x.view(rows, 1, hidden).to(gpu)
+    close(T.unembedding_decode_forward(xg, w.to(gpu)).view(rows, vocab), O.linear_ref(x, w, None))
+    w8, ws = T.quantize_fp8_rows(w.to(gpu))
+    want8 = O.linear_ref(x, O.dequant_fp8_ref(w8.cpu(), ws.cpu()), None)
+    close(T.unembedding_decode_fp8_forward(xg, w8, ws).view(rows, vocab), want8)
+    ld = vocab + 5                                             # a row stride of its own: the gap between rows is not written
+    buf = torch.full((rows, ld), 7.0, dtype=torch.bfloat16, device=gpu)
+    rc = lib().tllm_unembedding_decode_bf16(xg.data_ptr(), w8.data_ptr(), ws.data_ptr(), buf.data_ptr(), ld, rows, hidden, vocab,
+                                            torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    close(buf[:, :vocab], want8)
+    assert (buf[:, vocab:] == 7.0).all()
+
+
 def test_unembedding_32_rows_full_vocabulary(gpu):
     """[201088, 2880] at 32 rows: three or four tiles per wavefront. Logits against the oracle on a sample of columns,
     argmax against planted winners."""

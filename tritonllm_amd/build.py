@@ -19,7 +19,7 @@ LIB_PATH = os.path.join(LIB_DIR, "libtllm_hip.so")
 HOST_PATH = os.path.join(LIB_DIR, "tllm_host.so")
 INCLUDE = os.path.join(ROOT, "include")
 
-SOURCES = ["abi.hip", "rmsnorm.hip", "embedding.hip", "swiglu.hip", "rope.hip", "qkv_decode.hip", "qkv_decode_r8.hip", "qkv_decode_r32.hip", "qkv_decode_rows.hip", "qkv_prefill.hip", "tile_gemm.hip", "decode_general.hip", "out_decode.hip", "out_decode_r8.hip", "out_decode_r32.hip", "unembed.hip", "attn_decode.hip", "attn_prefill.hip", "mxfp4.hip"]
+SOURCES = ["abi.hip", "rmsnorm.hip", "embedding.hip", "swiglu.hip", "rope.hip", "qkv_decode.hip", "qkv_decode_r8.hip", "qkv_decode_r32.hip", "qkv_decode_rows.hip", "qkv_prefill.hip", "tile_gemm.hip", "decode_general.hip", "out_decode.hip", "out_decode_r8.hip", "out_decode_r32.hip", "unembed.hip", "unembed_tiles.hip", "attn_decode.hip", "attn_prefill.hip", "mxfp4.hip"]
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_*_f32 from ordinary float code.
 HIPCC_FLAGS = [

@@ -25,22 +25,9 @@
 // weight is streamed as pairs of rows (SR, below), whose bytes are whole cache lines.
 #include <mutex>
 
-#include "common.h"
+#include "unembed_common.h"
 
 namespace tllm {
-
-struct UnembedArgs {
-  const bf16* x;          // [rows, hidden]
-  const void* W;          // [vocab, hidden] bf16, or fp8 bytes when w_scale != null
-  const float* w_scale;   // [vocab] or null
-  bf16* logits;           // [rows, vocab] with row stride ld (logits form)
-  int64_t ld;
-  float* part_max;        // [gridDim.y][gridDim.x * UNW][XR] (argmax form)
-  int* part_idx;
-  int64_t rows;
-  int hidden, vocab;
-  int pair_stores;        // the logits rows allow 4-byte stores at even columns
-};
 
 __host__ __device__ constexpr int unembed_patch(int ks) { return 32 * (ks * 2 + 16); }   // wavefront patch: 32 rows of KS bf16 + padding
 
@@ -572,8 +559,6 @@ __global__ __launch_bounds__(kArgmaxReduceThreads) void unembed_argmax_reduce_ke
 using namespace tllm;
 
 namespace {
-constexpr int kUnembedGrid = 256;      // one workgroup per CU
-
 int unembed_xr_most(int64_t rows) { return rows <= 8 ? 8 : 16; }
 
 // (wavefronts, K step, steps in flight), measured at B = 8 on the full vocabulary:
@@ -629,8 +614,15 @@ int unembed_check(const char* who, const void* x, const void* W, bool w8, int64_
   return TLLM_OK;
 }
 
+// Logits of more rows than one pass of the kernels above takes
+bool unembed_tiled(int64_t rows, bool w8, int64_t hidden, int64_t vocab) {
+  const int64_t one_pass = unembed_rows32(rows, w8, hidden, vocab, false) ? 32 : unembed_xr(rows, w8, hidden);
+  return rows > one_pass && unembed_tiles_fit(rows, w8, hidden, vocab);
+}
+
 template <bool ARGMAX>
 int unembed_launch(const char* who, const UnembedArgs& a, bool w8, hipStream_t st) {
+  if (!ARGMAX && unembed_tiled(a.rows, w8, a.hidden, a.vocab)) return launch_unembed_tiles(who, a, w8, st);
   if (unembed_rows32(a.rows, w8, a.hidden, a.vocab, ARGMAX)) {
     auto kern = w8 ? unembed_rows32_kernel<kRows32Waves, 64, 4, true, ARGMAX> : unembed_rows32_kernel<kRows32Waves, 64, 3, false, ARGMAX>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
