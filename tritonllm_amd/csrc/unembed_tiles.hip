@@ -6,14 +6,19 @@
 // What bounds it is the weight, 1.16 GB at gpt-oss's size, and the kernels for few rows read it once per chunk of 32 rows
 // (of 8, for a model too wide for 32 rows in the LDS). Here K is cut into slices of 64 instead, and a slice of the
 // activations travels with the weight's: one workgroup of eight wavefronts per CU owns a contiguous run of the vocabulary
-// for the whole launch and walks it in tiles of up to 128 vocabulary rows (the run divided evenly: 49 sixteen-row units per
-// CU are seven tiles of seven units, not six of eight and one of one), and the ring of S stages -- global memory straight
-// into LDS, 16-byte chunks XOR-swizzled by row -- runs on across tiles, so that 64-80 KB of the weight are in flight per CU
-// from the first instruction to the last. The activations (737 KB at 128 rows) come from the L2: a stage is 16 KB of weight
-// and 4-16 KB of them. Wavefronts: four over the vocabulary (two units each) x two over the batch rows, on
-// v_mfma_f32_16x16x32_bf16 with the vocabulary on M, so that a lane ends up with four consecutive logits of a row. One
-// barrier per stage. The LDS reads of a stage (12 KB per wavefront at 128 rows) take about half of the time that its bytes
-// take from HBM.
+// for the whole launch and walks it in tiles of up to 256 vocabulary rows (the run divided evenly: 49 sixteen-row units per
+// CU are four tiles of thirteen, not three of sixteen and one of one), and the ring of S stages -- global memory straight
+// into LDS, 16-byte chunks XOR-swizzled by row -- runs on across tiles, so that 64-96 KB of the weight are in flight per CU
+// from the first instruction to the last. The activations (737 KB at 128 rows) come from the L2, once per tile: a stage is
+// 32 KB of weight and 4-16 KB of them, and they take their share of the loads a CU can have in flight, which is what the
+// time grows with (tiles of 128: 49 rows 225 us against 219, 128 rows 280 against 261). Wavefronts: four over the
+// vocabulary (four units each) x two over the batch rows, on v_mfma_f32_16x16x32_bf16 with the vocabulary on M, so that a
+// lane ends up with four consecutive logits of a row. One barrier per stage.
+//
+// [rows, 2880] x [201088, 2880], us (before: chunks of 32 rows, of 8 where the width is 4096; a read of the weight alone: 174):
+//   bf16   33 rows 205 (377)   49 219 (382)   64 228 (386)   96 245 (586)   128 261 (782)   200 510 (1370)
+//   fp8    33 rows 138 (240)   49 145 (251)   64 149 (253)   96 179 (372)   128 209 (491)
+//   4096 wide, bf16: 9 rows 251 (520)   32 280 (1035)   64 307 (2065)   128 346 (4098)
 #include <atomic>
 
 #include "qkv_prefill.h"
@@ -22,7 +27,7 @@
 namespace tllm {
 
 namespace unembed_tiles {
-constexpr int BK = 64, NW = 8, UNITS = 8;      // K slice; wavefronts; sixteen-row units of a tile
+constexpr int BK = 64, NW = 8, UNITS = 16;      // K slice; wavefronts; sixteen-row units of a tile
 constexpr int MAX_RUN = 64;                    // units of a workgroup's run whose fp8 scales the LDS holds
 
 template <int MB, bool W8>                     // MB blocks of sixteen batch rows
@@ -33,10 +38,10 @@ struct Shape {
   static constexpr int TAIL = W8 ? MAX_RUN * 16 * 4 : 0;
   static constexpr int S_FIT = (160 * 1024 - TAIL) / STAGE, S = S_FIT > 8 ? 8 : S_FIT;
   static constexpr int SMEM = S * STAGE + TAIL;
-  static constexpr int LW = W8 ? 1 : 2;                      // loads of 1 KB per wavefront and stage: its unit of the weight ...
+  static constexpr int LW = (W8 ? 1 : 2) * UNITS / NW;                      // loads of 1 KB per wavefront and stage: its unit of the weight ...
   static constexpr int XR = MB * 2, LX = (XR + 7) / 8;       // ... and XR rows of the activations, eight to a load, the last one may be half
   static constexpr int LPW = LW + LX;
-  static_assert(S >= 4 && (S - 2) * LPW < 64, "the loads in flight are countable");
+  static_assert(S >= 3 && (S - 2) * LPW < 64, "the loads in flight are countable");
 };
 }  // namespace unembed_tiles
 
@@ -44,7 +49,7 @@ template <int MB, bool W8>
 __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int chunk_rows) {
   using namespace unembed_tiles;
   typedef Shape<MB, W8> C;
-  constexpr int S = C::S, STAGE = C::STAGE, WBYTES = C::WBYTES, WROW = C::WROW, XR = C::XR, LX = C::LX, LW = C::LW, LPW = C::LPW, TB = MB / 2;
+  constexpr int S = C::S, STAGE = C::STAGE, WBYTES = C::WBYTES, WROW = C::WROW, XR = C::XR, LX = C::LX, LW = C::LW, LPW = C::LPW, TB = MB / 2, UB = UNITS / 4;
   extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -78,10 +83,11 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
   const int run_rows = a.vocab - u0 * 16 < run * 16 ? a.vocab - u0 * 16 : run * 16;
   auto weight_offsets = [&](int tile) {
     const int left = run - tile * width, here = left < width ? left : width;
-    const int unit = tile * width + (wave < here ? wave : here - 1);
 #pragma unroll
     for (int j = 0; j < LW; ++j) {
-      const int r = W8 ? lane >> 2 : 8 * j + (lane >> 3);
+      constexpr int LU = W8 ? 1 : 2;                         // loads per unit
+      const int u = wave * (UNITS / NW) + j / LU, unit = tile * width + (u < here ? u : here - 1);
+      const int r = W8 ? lane >> 2 : 8 * (j % LU) + (lane >> 3);
       const unsigned c = (W8 ? static_cast<unsigned>((lane & 3) ^ (r >> 2)) : static_cast<unsigned>((lane & 7) ^ swz(r))) * 16u;
       const int row = unit * 16 + r < run_rows ? unit * 16 + r : run_rows - 1;
       woff[j] = static_cast<unsigned>(row) * wpitch + c;
@@ -97,7 +103,7 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
     const unsigned char* const xb = x_base + static_cast<int64_t>(l_k) * (BK * 2);
 #pragma unroll
     for (int j = 0; j < LW; ++j) {
-      const unsigned d = dst + wave * (16 * WROW) + j * 1024;
+      const unsigned d = dst + wave * (UNITS / NW * 16 * WROW) + j * 1024;
       // a slice of an fp8 row is half a line, so its line is needed again one stage on: no streaming hint
       if constexpr (W8) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(d), "v"(woff[j]), "s"(wb) : "memory", "m0");
       else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(d), "v"(woff[j]), "s"(wb) : "memory", "m0");
@@ -131,24 +137,24 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
   // ---- fragments: lane group g supplies chunk 4 kk + gc of both operands' rows (any assignment will do as long as the two
   // agree); under swz() the sixteen lanes that a 128-bit LDS read is served by (0-7 with 32-39, ...) are on different banks.
   const int gc = (g >> 1) | ((g & 1) << 1);
-  int fx_o[TB], fw_o[2];
+  int fx_o[TB], fw_o[UB];
 #pragma unroll
   for (int tb = 0; tb < TB; ++tb) {
     const int r = 16 * (TB * wm + tb) + m16;
     fx_o[tb] = WBYTES + r * 128 + ((gc ^ swz(r)) << 4);
   }
 #pragma unroll
-  for (int ub = 0; ub < 2; ++ub) {
-    if constexpr (W8) fw_o[ub] = (2 * wn + ub) * 1024 + m16 * 64 + (((gc >> 1) ^ (m16 >> 2)) << 4) + (gc & 1) * 8;
-    else fw_o[ub] = (2 * wn + ub) * 2048 + m16 * 128 + ((gc ^ swz(m16)) << 4);
+  for (int ub = 0; ub < UB; ++ub) {
+    if constexpr (W8) fw_o[ub] = (UB * wn + ub) * 1024 + m16 * 64 + (((gc >> 1) ^ (m16 >> 2)) << 4) + (gc & 1) * 8;
+    else fw_o[ub] = (UB * wn + ub) * 2048 + m16 * 128 + ((gc ^ swz(m16)) << 4);
   }
   const bool vec4 = reinterpret_cast<uintptr_t>(a.logits) % 8 == 0 && a.ld % 4 == 0;
 
   int c_slot = 0;
   for (int tile = 0; tile < ntiles; ++tile) {
-    f32x4 acc[2][TB];
+    f32x4 acc[UB][TB];
 #pragma unroll
-    for (int ub = 0; ub < 2; ++ub)
+    for (int ub = 0; ub < UB; ++ub)
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb) acc[ub][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
@@ -158,11 +164,11 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
       // read the slot that the next loads go into.
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * LPW) : "memory");
       const unsigned char* const st = smem + c_slot * STAGE;
-      bf16x8 fx[2][TB], fw[2][2];
+      bf16x8 fx[2][TB], fw[2][UB];
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
-        for (int ub = 0; ub < 2; ++ub) {
+        for (int ub = 0; ub < UB; ++ub) {
           if constexpr (W8) {
             typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u32x2;
             const u32x2 raw = *reinterpret_cast<const u32x2*>(st + (fw_o[ub] ^ (kk << 5)));
@@ -178,7 +184,7 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-        for (int ub = 0; ub < 2; ++ub)
+        for (int ub = 0; ub < UB; ++ub)
 #pragma unroll
           for (int tb = 0; tb < TB; ++tb) acc[ub][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[kk][ub], fx[kk][tb], acc[ub][tb], 0, 0, 0);
       c_slot = c_slot + 1 == S ? 0 : c_slot + 1;
@@ -186,8 +192,8 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
     // ---- the tile's logits: lane (batch row m16 of block tb) has vocabulary rows 4 g .. 4 g + 3 of a unit
     const int left = run - tile * width, here = left < width ? left : width;
 #pragma unroll
-    for (int ub = 0; ub < 2; ++ub) {
-      const int unit = 2 * wn + ub;
+    for (int ub = 0; ub < UB; ++ub) {
+      const int unit = UB * wn + ub;
       if (unit >= here) continue;                            // uniform
       const int lv = (tile * width + unit) * 16 + 4 * g;     // in the run
       f32x4 sc = {1.f, 1.f, 1.f, 1.f};
