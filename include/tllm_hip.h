@@ -285,7 +285,7 @@ int tllm_unembedding_argmax_noalloc_bf16(const void* x, const void* W, const flo
  * not depend on it, a hint that is too small only costs speed. Pass min(hint, n_kv_ctx) as n_kv_ctx to the three
  * planning helpers below when a hint is used. */
 int tllm_attention_decode_splits(int64_t batch, int n_kv_heads, int64_t n_kv_ctx, int window);
-/* Diagnostic: KV heads served by one workgroup for these arguments (8 or 4: one wavefront per head, contiguous
+/* Diagnostic: KV heads served by one workgroup for these arguments (8, 4 or 2: contiguous runs of
  * cache rows; 0: one KV head per workgroup). No counterpart in the reference. */
 int tllm_attention_decode_heads_per_workgroup(int64_t batch, int n_kv_heads, int64_t n_kv_ctx, int window);
 int64_t tllm_attention_decode_workspace_bytes(int64_t batch, int n_q_heads, int n_kv_heads, int64_t n_kv_ctx, int window);

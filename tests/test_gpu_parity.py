@@ -1281,6 +1281,26 @@ def test_attention_decode_row_workgroups(gpu, case):
     _attn_case(gpu, seed=11 + c["start_q"], **c)
 
 
+@pytest.mark.parametrize("batch_size,num_keys,start_q,hpw", [
+    (1, 129, 128, 0), (1, 512, 511, 0), (3, 200, 37, 0), (8, 800, 799, 0),          # eight wavefronts per KV head; less than a block each
+    (33, 256, 255, 2), (64, 1280, 1279, 2), (49, 1111, 1110, 2), (43, 4096, 30, 2),   # two heads, two wavefronts each: ragged, nearly empty
+    (8, 3000, 2999, 2), (16, 1111, 700, 2),                                           # ... with context splits
+    (65, 100, 99, 4), (97, 333, 332, 4), (111, 515, 31, 4), (128, 511, 0, 4),         # four heads, two wavefronts each
+])
+@pytest.mark.parametrize("kv", [dict(), dict(groups=5, with_sinks=False)], ids=["g8", "g5"])
+def test_attention_decode_wavefronts_per_head(gpu, batch_size, num_keys, start_q, hpw, kv):
+    """Workgroup shapes with several wavefronts per KV head, at the edges of the ranges that take them."""
+    from tritonllm_amd._lib import lib
+    assert lib().tllm_attention_decode_heads_per_workgroup(batch_size, 8, num_keys, 0) == hpw
+    _attn_case(gpu, batch_size, num_keys, None, start_q, seed=batch_size + num_keys, **kv)
+
+
+@pytest.mark.parametrize("batch_size,window", [(65, 128), (40, 300), (6, 200)])
+def test_attention_decode_window_wavefronts_per_head(gpu, batch_size, window):
+    """... and under a sliding window, whose first block is ragged too."""
+    _attn_case(gpu, batch_size, 700, window, 613, seed=window)
+
+
 @pytest.mark.parametrize("batch_size,num_keys", [(2, 600), (8, 8192)])
 def test_attention_decode_strided_cache_views(gpu, batch_size, num_keys):
     """K / V handed over as views of a larger allocation: more tokens and more heads per token than are used, so both

@@ -6,16 +6,16 @@
 //   out[h]   = sum_n exp(s[h, n] - m) v[n] / (sum_n exp(s[h, n] - m) + exp(sink[h] - m)),   m = max(sink[h], max_n s[h, n])
 //
 // The reference runs one program per query head, so the G heads of a group each read the same K and V; here a
-// wavefront serves all G heads of a KV head from one pass over K and V, in one of two workgroup shapes:
-//   * ROWS (large batch x context): a workgroup takes a (batch row, context split, group of eight or four adjacent
-//     KV heads) and has one wavefront per KV head, each walking the split's 32-key blocks in order. Together the
-//     wavefronts read whole (or half) cache rows -- all KV heads of a token are adjacent in memory -- so the workgroup
-//     streams long contiguous runs of K and of V; with nontemporal loads the whole-row pattern measures 6.8 TB/s on
-//     its own, where one-KV-head-per-workgroup streams stop at 5.2 TB/s (128-byte pieces at a 1 KB stride, the
-//     sibling heads arriving from other workgroups at other times);
-//   * HEAD (few batch rows): a workgroup takes a (batch row, KV head, context split); four wavefronts take the
-//     split's blocks in turn, each with its own running (max, sum, accumulator), and meet once at the end through
-//     LDS. This shape yields n_kv_heads times more workgroups, which is what fills the machine at batch 1;
+// wavefront serves all G heads of a KV head from one pass over K and V. A workgroup takes a (batch row, context split,
+// group of HPW adjacent KV heads) with KW wavefronts for each head, which take the split's 32-key blocks in turn, each
+// with its own running (max, sum, accumulator), and meet once at the end through LDS:
+//   * 8 x 1, 4 x 1 (HPW x KW, "ROWS": large batch x context): together the wavefronts read whole (or half) cache rows --
+//     all KV heads of a token are adjacent in memory -- so the workgroup streams long contiguous runs of K and of V; with
+//     nontemporal loads the whole-row pattern measures 6.8 TB/s on its own, where one-KV-head-per-workgroup streams
+//     stop at 5.2 TB/s (128-byte pieces at a 1 KB stride, the sibling heads arriving from other workgroups at other times);
+//   * 1 x 4 ("HEAD": few batch rows), 1 x 8: n_kv_heads times more workgroups, which is what fills the machine at batch 1;
+//   * 2 x 2, 4 x 2 in between: contiguous runs of 256 / 512 bytes at 6 - 6.5 TB/s, and short enough a walk for a context to
+//     need no splitting from 33 batch rows on (the rule and what each shape measured stand at attn_plan);
 //   * S^T = K . Q^T on v_mfma_f32_16x16x32_bf16 with the keys on M: K rows are K-contiguous in memory, so a lane
 //     loads its 16 bytes of a key row straight into operand layout; Q sits in registers as the B operand;
 //   * the accumulator layout of S^T (lane = head, registers = keys) IS the A-operand layout of P for O = P . V when
@@ -65,10 +65,9 @@ __host__ __device__ inline int attn_splits_for(int fill, int ctx, int keys_shift
 }
 
 namespace {
-constexpr int AW = 4;                 // wavefronts per workgroup, HEAD shape
-constexpr int RW = 8;                 // most wavefronts (= KV heads) per workgroup, ROWS shape
 constexpr int VROW = 128 + 16;        // V tile row in LDS: 64 bf16 + padding, bytes
 constexpr int VTILE = 32 * VROW;
+constexpr int AROW = 64 + 1;          // accumulator row of a head in LDS, floats
 constexpr float kNegBig = -1.0e30f;
 constexpr int PART = 66;              // floats per (split, row, head) in the workspace
 }  // namespace
@@ -90,12 +89,14 @@ __device__ __forceinline__ int attn_live_splits(const AttnArgs& a, int* lo_out, 
   return s < a.splits ? s : a.splits;
 }
 
-template <bool ROWS>
-__global__ __launch_bounds__((ROWS ? RW : AW) * 64) void attn_decode_kernel(AttnArgs a) {
-  __shared__ __align__(16) unsigned char vt[(ROWS ? RW : AW) * VTILE];
-  __shared__ __align__(16) unsigned char kt[(ROWS ? RW : AW) * VTILE];   // K tile, the same shape
-  __shared__ float s_m[ROWS ? 1 : AW][16], s_l[ROWS ? 1 : AW][16];
-  __shared__ float s_acc[ROWS ? 1 : AW][ROWS ? 1 : 16][64 + 1];
+// HPW adjacent KV heads per workgroup, KW wavefronts for each of them.
+template <int HPW, int KW>
+__global__ __launch_bounds__(HPW * KW * 64) void attn_decode_kernel(AttnArgs a) {
+  constexpr int NW = HPW * KW;
+  // A K and a V tile per wavefront; behind the last block a wavefront's K tile takes its accumulator on the way to the others.
+  __shared__ __align__(16) unsigned char vt[NW * VTILE], kt[NW * VTILE];
+  __shared__ float s_m[KW > 1 ? NW : 1][16], s_l[KW > 1 ? NW : 1][16];
+  static_assert(16 * AROW * 4 <= VTILE, "an accumulator fits a tile");
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r16 = lane & 15, g = lane >> 4;
@@ -125,8 +126,7 @@ __global__ __launch_bounds__((ROWS ? RW : AW) * 64) void attn_decode_kernel(Attn
     grp = r / live;
     split = r - grp * live;
   }
-  // ROWS: the group's KV heads sit on the workgroup's wavefronts
-  const int kvh = ROWS ? grp * static_cast<int>(blockDim.x >> 6) + wave : grp;
+  const int kvh = grp * HPW + wave % HPW;
   const int len = hi - lo;
   int chunk = (len + live - 1) / live;
   chunk = (chunk + 31) & ~31;                                 // whole 32-key blocks per split
@@ -154,10 +154,10 @@ __global__ __launch_bounds__((ROWS ? RW : AW) * 64) void attn_decode_kernel(Attn
   // Rows past the end of the split are clamped to its last key (finite values; their probabilities are zeroed).
   // Addressing is a block base (uniform) plus a 32-bit lane offset: row * token stride + a lane constant.
   const unsigned ts_b = static_cast<unsigned>(a.kv_ts) * 2u;   // token stride, bytes (a 32-key block spans < 4 GB)
-  // The ROWS stream is read once and is far larger than the caches: nontemporal. The HEAD shape serves short
+  // Several heads per workgroup: the stream is read once and is far larger than the caches, nontemporal. One head: short
   // contexts, where the cache lines of a token are shared with sibling workgroups and may still be cache-resident.
   auto ld = [](const unsigned char* p) {
-    return ROWS ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p)) : *reinterpret_cast<const bf16x8*>(p);
+    return HPW > 1 ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p)) : *reinterpret_cast<const bf16x8*>(p);
   };
   // K and V both arrive row-major, eight neighbouring lanes covering one 128-byte row piece; K's A-operand fragments
   // (lane = (key, k group)) are then read out of LDS. Loaded straight into operand layout, neighbouring lanes ask for
@@ -177,8 +177,8 @@ __global__ __launch_bounds__((ROWS ? RW : AW) * 64) void attn_decode_kernel(Attn
     }
   };
 
-  constexpr int STEP = ROWS ? 1 : AW;                          // ROWS: every wavefront walks all blocks (of its own KV head)
-  const int first = ROWS ? 0 : wave;
+  constexpr int STEP = KW;                                     // the wavefronts of a KV head take its blocks in turn
+  const int first = wave / HPW;
   if (first < nblk) load_block(s_lo + 32 * first);
   for (int blk = first; blk < nblk; blk += STEP) {
     const int k0 = s_lo + 32 * blk;
@@ -262,7 +262,7 @@ __global__ __launch_bounds__((ROWS ? RW : AW) * 64) void attn_decode_kernel(Attn
     __builtin_amdgcn_wave_barrier();
   }
 
-  if constexpr (ROWS) {
+  if constexpr (KW == 1) {
     // ---- each wavefront owns its heads outright: O sits in lane (d = 16 nb + r16), registers = heads 4 g + i; the
     // (max, sum) of head h sit in the lanes with r16 == h
     float* p = a.part + ((static_cast<int64_t>(split) * gridDim.y + b) * n_q_heads + static_cast<int64_t>(kvh) * G) * PART;
@@ -292,36 +292,39 @@ __global__ __launch_bounds__((ROWS ? RW : AW) * 64) void attn_decode_kernel(Attn
     return;
   }
 
-  // ---- HEAD: the four wavefronts meet: (max, sum) per head, accumulator per (head, d)
+  // ---- the KW wavefronts of a KV head meet: (max, sum) per head, accumulator per (head, d)
   if (g == 0) {
     s_m[wave][r16] = m_run;
     s_l[wave][r16] = l_run;
   }
+  float* const mine = reinterpret_cast<float*>(ktile);         // (this wavefront is past its last read of the tile)
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s_acc[wave][4 * g + i][16 * nb + r16] = acc[nb][i];
+    for (int i = 0; i < 4; ++i) mine[(4 * g + i) * AROW + 16 * nb + r16] = acc[nb][i];
   __syncthreads();
 
-  // thread -> (head = tid / 16 (< 16), four d: tid % 16 + 16 j)
-  const int eh = tid >> 4, ed = tid & 15;
+  // thread -> (KV head ej, query head eh (< 16), DPT of its 64 d: ed + TPH j)
+  constexpr int TPH = 4 * KW, DPT = 64 / TPH;
+  const int ej = tid / (64 * KW), eh = tid / TPH & 15, ed = tid % TPH;
   if (eh >= G) return;
   float m_all = kNegBig;
 #pragma unroll
-  for (int w = 0; w < AW; ++w) m_all = fmaxf(m_all, s_m[w][eh]);
-  float l_all = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int w = 0; w < KW; ++w) m_all = fmaxf(m_all, s_m[w * HPW + ej][eh]);
+  float l_all = 0.f, o[DPT] = {};
 #pragma unroll
-  for (int w = 0; w < AW; ++w) {
-    const float f = __expf(s_m[w][eh] - m_all);              // a wavefront without keys has sum 0 and accumulator 0
-    l_all += s_l[w][eh] * f;
+  for (int w = 0; w < KW; ++w) {
+    const float f = __expf(s_m[w * HPW + ej][eh] - m_all);   // a wavefront without keys has sum 0 and accumulator 0
+    l_all += s_l[w * HPW + ej][eh] * f;
+    const float* from = reinterpret_cast<const float*>(kt + (w * HPW + ej) * VTILE) + eh * AROW + ed;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] += s_acc[w][eh][ed + 16 * j] * f;
+    for (int j = 0; j < DPT; ++j) o[j] += from[TPH * j] * f;
   }
-  const int head = kvh * G + eh;
+  const int head = (grp * HPW + ej) * G + eh;
   if (a.splits > 1) {
     float* p = a.part + ((static_cast<int64_t>(split) * gridDim.y + b) * n_q_heads + head) * PART;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) p[ed + 16 * j] = o[j];
+    for (int j = 0; j < DPT; ++j) p[ed + TPH * j] = o[j];
     if (ed == 0) {
       p[64] = m_all;
       p[65] = l_all;
@@ -334,7 +337,7 @@ __global__ __launch_bounds__((ROWS ? RW : AW) * 64) void attn_decode_kernel(Attn
   const float z = l_all * f + __expf(sink - m_f);
   bf16* orow = a.out + b * a.out_rs + static_cast<int64_t>(head) * 64;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) orow[ed + 16 * j] = static_cast<bf16>(o[j] * f / z);
+  for (int j = 0; j < DPT; ++j) orow[ed + TPH * j] = static_cast<bf16>(o[j] * f / z);
 }
 
 // One wavefront per (batch row, head): fold the context splits and the sink. Lane s first fetches (max, sum) of
@@ -409,9 +412,27 @@ using namespace tllm;
 // B = 20 at 3K 29.9 -> 24.1; B = 24 at 2K 25.0 -> 20.6; B = 28 at 1280 keys 21.4 -> 17.6; B = 3 at 100K 106 -> 97;
 // unchanged (within 0.3 %) at the other 30 of 48 batch x context points tried.
 // A sliding window bounds the context.
-struct AttnPlan { int heads_per_wg; int splits; int fill; int keys_shift; };   // heads_per_wg 0: the HEAD shape
+//
+// With one split there is no second kernel, and about 3 us are saved; so shapes with two or more wavefronts per KV head,
+// which walk a whole context in half or a quarter of the steps, take over wherever their grid fills most of the CUs
+// without splitting (eight KV heads, us, what was launched before -> now):
+//   2 x 2   B = 33 .. 64, contexts of 256 - 4096 (up to 1280 below B = 43, where three splits of ROWS are ahead of it from
+//           there on): B = 40 at 700 20 -> 14.5, B = 49 at 1111 28.4 -> 21.8, at 2048 47.9 -> 35.0, B = 64 at 400 15.0 -> 12.6,
+//           at 2048 45.4 -> 41.8, at 4096 81.2 -> 79.5 (at 200 keys HEAD is ahead, B = 49 7.6 and 8.1, and at 5000 splits are,
+//           B = 47 78.5 and 81.7)
+//   4 x 2   B = 65 .. 111, and up to 128 below 512 keys; contexts up to 8192: B = 80 at 1111 42.7 -> 32.5, at 2048 66.6 -> 54.1, B = 85 at 8192 245 -> 214, B = 96 at 256
+//           15.8 -> 12.1, at 1111 50.9 -> 36.8, B = 128 at 256 19.6 -> 15.5; window of 128: B = 96 9.6 -> 8.9, B = 128 12.4 -> 10.6
+//           (from B = 112 and 512 keys on one wavefront per head fills the CUs as well and is ahead: 68.7 against 73 at 2048)
+//   1 x 8   up to 128 streams and 512 keys, 64 .. 128 streams and 800 keys: B = 1 at 256 6.0 -> 4.4, B = 5 at 400 7.0 -> 6.3,
+//           B = 8 at 700 8.5 -> 7.7, B = 12 at 256 7.5 -> 5.4, B = 16 at 512 8.9 -> 7.4 (beyond: two launches are ahead, B = 5 at 1111
+//           8.5 and 9.1, B = 14 at 900 11.5 and 12.2)
+// 2 x 2 with splits of 257 - 511 keys: its 256-byte pieces stream nearly as fast as ROWS' and it needs half as many splits:
+// B = 8 at 3000 16.1 -> 13.8, B = 16 at 1111 14.0 -> 12.5 (fewer than 64 streams: B = 5 at 4096 15.0 -> 13.4, but planned for
+// 4096 with 300 visible 7.1 -> 8.0; HEAD kept).
+struct AttnPlan { int hpw, kw; int splits; int fill; int keys_shift; };   // KV heads per workgroup, wavefronts for each
 
 constexpr int kRowsKeysShift = 12, kHeadKeysShift = 11;   // log2 of the keys per workgroup beyond which a context is split further
+constexpr int kUnsplitQuads = 8192, kUnsplitPairs = 4096; // longest contexts that 4 x 2 and 2 x 2 walk without splitting them
 // Splits for `units` streams: attn_splits_for's answer, unless one split fewer per unit-row of workgroups spreads the
 // work more evenly -- 24 units x 11 splits are 264 workgroups, eight CUs with two of them while the rest have one,
 // where 24 x 10 leave sixteen CUs idle and everybody done 1.8 times sooner. Compared by the keys the busiest CU walks.
@@ -427,34 +448,46 @@ static int attn_pick_splits(int64_t units, int ctx, int shift) {
     const int64_t keys = (((ctx + s - 1) / s) + 31) & ~31;
     return rounds * keys;
   };
-  return busiest(s1) < busiest(s0) ? s1 : s0;
+  return busiest(s1) <= busiest(s0) ? s1 : s0;                // a tie: fewer records to fold, or no second launch
 }
 
 static AttnPlan attn_plan(int64_t batch, int n_kv_heads, int64_t n_kv_ctx, int window) {
   const int64_t ctx = (window > 0 && window < n_kv_ctx) ? window : n_kv_ctx;
+  const int64_t streams = batch * n_kv_heads;
+  const int head_splits = attn_pick_splits(streams, static_cast<int>(ctx), kHeadKeysShift);
+  if (n_kv_heads % 4 == 0 && n_kv_heads <= 8) {     // one launch on most of the CUs
+    const int64_t quads = streams / 4, pairs = streams / 2;
+    if (ctx <= kUnsplitQuads && quads > 128 && (quads < 224 || (quads <= 256 && ctx < 512))) return {4, 2, 1, 1, kRowsKeysShift};
+    if (ctx >= 256 && ctx <= kUnsplitPairs && pairs > 128 && pairs <= 256 && (pairs > 168 || ctx <= 1280)) return {2, 2, 1, 1, kRowsKeysShift};
+  }
+  if (ctx > 128 && streams <= 128 && ctx <= (streams >= 64 ? 800 : 512)) return {1, 8, 1, 1, kHeadKeysShift};
   // eight or four KV heads per workgroup: whichever fills the machine with the longest splits (ties: the wider one)
-  AttnPlan best{0, 0, 0, 0};
+  AttnPlan best{0, 0, 0, 0, 0};
   int64_t best_keys = 0;
-  for (int hpw = RW; hpw >= 4; hpw >>= 1) {
+  for (int hpw = 8; hpw >= 4; hpw >>= 1) {
     if (n_kv_heads % hpw != 0) continue;
     const int64_t units = batch * (n_kv_heads / hpw);
     const int s = attn_pick_splits(units, static_cast<int>(ctx), kRowsKeysShift);
     const int64_t keys = ctx / s;
-    // splits of 256-511 keys too, when there are not too many of them and the HEAD shape would need its second launch as well
-    const bool head_splits_too = attn_splits_for(attn_fill(batch * n_kv_heads), static_cast<int>(ctx), kHeadKeysShift) > 1;
-    const bool long_enough = keys >= 512 || (head_splits_too && ((keys >= 256 && s <= 28) || (keys >= 320 && s <= 32)));
-    if (units * s >= 224 && long_enough && keys > best_keys) {
-      best = {hpw, s, s, kRowsKeysShift};                 // (the kernels' own evaluation starts from the chosen count)
+    // splits of 256-511 keys too, when there are not too many of them and the HEAD shape would need its second launch as
+    // well or is past what one launch of it is good for
+    const bool long_enough = keys >= 512 || ((head_splits > 1 || ctx >= 1400) && ((keys >= 256 && s <= 28) || (keys >= 320 && s <= 32)));
+    if (units * s >= (streams > 256 ? 208 : 224) && long_enough && keys > best_keys) {
+      best = {hpw, 1, s, s, kRowsKeysShift};              // (the kernels' own evaluation starts from the chosen count)
       best_keys = keys;
     }
   }
-  if (best.heads_per_wg) return best;
-  const int sh = attn_pick_splits(batch * n_kv_heads, static_cast<int>(ctx), kHeadKeysShift);
-  return {0, sh, sh, kHeadKeysShift};
+  if (best_keys < 512 && head_splits > 1 && streams >= 64 && n_kv_heads % 4 == 0 && n_kv_heads <= 8) {
+    const int s = attn_pick_splits(streams / 2, static_cast<int>(ctx), kRowsKeysShift);
+    if (s > 1 && streams / 2 * s >= 208 && ctx / s > 256 && ctx / s < 512) return {2, 2, s, s, kRowsKeysShift};
+  }
+  if (best.hpw) return best;
+  return {1, 4, head_splits, head_splits, kHeadKeysShift};
 }
 
 extern "C" int tllm_attention_decode_heads_per_workgroup(int64_t batch, int n_kv_heads, int64_t n_kv_ctx, int window) {
-  return attn_plan(batch, n_kv_heads, n_kv_ctx, window).heads_per_wg;
+  const int hpw = attn_plan(batch, n_kv_heads, n_kv_ctx, window).hpw;
+  return hpw > 1 ? hpw : 0;
 }
 
 extern "C" int tllm_attention_decode_splits(int64_t batch, int n_kv_heads, int64_t n_kv_ctx, int window) {
@@ -511,11 +544,16 @@ extern "C" int tllm_attention_decode_bf16(const void* q, const void* k, const vo
                (long long)workspace_bytes);
   a.part = static_cast<float*>(workspace);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (plan.heads_per_wg)
-    hipLaunchKernelGGL(attn_decode_kernel<true>, dim3((unsigned)(n_kv_heads / plan.heads_per_wg * a.splits), (unsigned)batch),
-                       dim3(plan.heads_per_wg * 64), 0, st, a);
-  else
-    hipLaunchKernelGGL(attn_decode_kernel<false>, dim3((unsigned)(n_kv_heads * a.splits), (unsigned)batch), dim3(AW * 64), 0, st, a);
+  const dim3 grid(static_cast<unsigned>(n_kv_heads / plan.hpw * a.splits), static_cast<unsigned>(batch)), block(plan.hpw * plan.kw * 64);
+#define TLLM_SHAPE(HPW, KW) \
+  if (plan.hpw == HPW && plan.kw == KW) hipLaunchKernelGGL((attn_decode_kernel<HPW, KW>), grid, block, 0, st, a)
+  TLLM_SHAPE(1, 4);
+  TLLM_SHAPE(1, 8);
+  TLLM_SHAPE(2, 2);
+  TLLM_SHAPE(4, 1);
+  TLLM_SHAPE(4, 2);
+  TLLM_SHAPE(8, 1);
+#undef TLLM_SHAPE
   int rc = check_launch("attention_decode");
   if (rc != TLLM_OK || a.splits == 1) return rc;
   hipLaunchKernelGGL(attn_decode_reduce_kernel, dim3((unsigned)(n_kv_heads * group), (unsigned)batch), dim3(64), 0, st, a, (int)batch);
