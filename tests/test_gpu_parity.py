@@ -1383,6 +1383,18 @@ def test_attention_prefill_shapes(gpu, case):
     _attn_prefill_case(gpu, seed=3 + case["num_queries"] + case["start_q"], **case)
 
 
+@pytest.mark.parametrize("batch_size,num_queries,num_keys,start_q,window", [
+    (1, 1, 193, 192, None), (1, 33, 260, 200, None), (1, 97, 1597, 1500, None), (2, 128, 448, 320, None), (4, 64, 700, 1, None),   # four key groups
+    (1, 97, 1597, 1500, 128), (1, 200, 1000, 800, 1), (2, 100, 800, 333, 300),
+    (1, 64, 192, 128, None), (1, 65, 65, 0, None), (1, 257, 300, 40, None), (8, 64, 100, 9, None), (3, 129, 1200, 1071, 200),      # two
+], ids=str)
+@pytest.mark.parametrize("kv", [dict(), dict(groups=3, kv_heads=4, with_sinks=False)], ids=["g8", "g3"])
+def test_attention_prefill_key_groups(gpu, batch_size, num_queries, num_keys, start_q, window, kv):
+    """Launches of at most two workgroups of 64 queries x 1 head per CU: the key blocks are shared out between wavefronts,
+    from fewer blocks than groups to many of them, the last round ragged, a group with nothing visible among them."""
+    _attn_prefill_case(gpu, batch_size, num_queries, num_keys, window, start_q, seed=num_queries + num_keys, **kv)
+
+
 def test_attention_prefill_views_of_the_qkv_buffer_and_the_cache(gpu):
     """q as a slice of the fused projection output, k / v as slices of a larger cache whose other slots hold NaN: the
     kernel reads them in place (batch and token strides) and never touches a key no query can see."""

@@ -12,8 +12,10 @@
 //
 //   * a workgroup takes 128 consecutive queries of NH query heads that share a KV head, four wavefronts of 32 queries;
 //     K / V blocks of 64 keys pass through four LDS stages filled by global_load_lds_dwordx4 (no staging registers, no
-//     LDS writes; three blocks in flight behind the one being computed, one hand-spelled wait + barrier per block)
-//     and serve all NH heads;
+//     LDS writes; two blocks in flight behind the two being computed, one hand-spelled wait + barrier per two blocks)
+//     and serve all NH heads; small launches take 64 queries, and the smallest share the key blocks of 64 queries x 1
+//     head out to two or four groups of two wavefronts, which meet in LDS at the end (what is bound there is the serial
+//     walk over the keys, ~1 us a block);
 //   * S^T = K . Q^T on v_mfma_f32_32x32x16_bf16 with the keys on M: a lane then owns ONE query (column) and 16 keys
 //     per 32-key block, so the running maximum, the running sum and the rescale factor of the online softmax are
 //     lane-local apart from one exchange between the two half-wavefronts;
@@ -50,7 +52,6 @@ constexpr int PBN = 64;               // keys per block
 constexpr int KT_BYTES = PBN * 128;   // K tile [key][64 d]
 constexpr int VT_BYTES = PBN * 128;   // V tile [key][64 d]
 constexpr int PSTAGE = KT_BYTES + VT_BYTES;
-constexpr int NSTG = 4;               // LDS stages: three blocks in flight behind the one being computed
 constexpr float kLog2e = 1.4426950408889634f;
 }  // namespace
 
@@ -69,14 +70,18 @@ __device__ __forceinline__ float other_half(float x, int high) {
 
 typedef __attribute__((__vector_size__(4 * sizeof(short)))) short i16x4;
 
-// NH: query heads (of one KV head) per wavefront. QG: groups of 32 queries per workgroup; the four wavefronts are QG
-// query groups x 4 / QG head sets, so a workgroup covers 32 * QG queries of NH * 4 / QG heads.
-template <int NH, int QG>
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a) {
+// NH: query heads (of one KV head) per wavefront. QG: groups of 32 queries per workgroup, KG: groups that share the key
+// blocks out. The NW wavefronts are QG query groups x KG key groups x HS head sets, so a workgroup covers 32 * QG queries of
+// NH * HS heads.
+template <int NH, int QG, int KG, int NW>
+__global__ __launch_bounds__(NW * 64, KG > 2 ? NW / 4 : NW / 2) void attn_prefill_kernel(AttnPrefillArgs a) {
   constexpr int PBM = 32 * QG;                    // queries per workgroup
-  constexpr int HS = 4 / QG;                      // head sets
-  constexpr int DPT = 4;                          // global->LDS load instructions per wavefront and block (1 KB each)
-  __shared__ __align__(16) unsigned char smem[NSTG * PSTAGE];
+  constexpr int HS = NW / (QG * KG);              // head sets
+  static_assert(HS * QG * KG == NW && (KG == 1 || (NH == 1 && HS == 1)), "wavefronts of a workgroup");
+  constexpr int STEP = KG == 1 ? 2 : KG;          // blocks between two barriers
+  constexpr int NSTG = 2 * STEP;                  // LDS stages: the step's blocks and the next one's
+  constexpr int DPT = KG == 1 ? 16 / NW : 16 * STEP / NW;   // global->LDS load instructions (1 KB each) per wavefront: of every block / of its block of a step
+  extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l31 = lane & 31, h = lane >> 5;
@@ -99,7 +104,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
   const int b = id % a.batch;
   id /= a.batch;
   const int tile = ntiles - 1 - static_cast<int>(id);
-  const int head0 = kvh * a.group + (sub * HS + wave / QG) * NH;
+  const int kgrp = KG == 1 ? 0 : wave / QG;       // the wavefront's key group (KG == 1: wave / QG is its head set)
+  const int head0 = kvh * a.group + (KG == 1 ? sub * HS + wave / QG : sub) * NH;
 
   // ---- Q fragments (B operand: lane = query, 8 d per half-wavefront and k16 step), requested before the start
   // position is read: their addresses do not depend on it, so they travel while that (dependent) load is on its way
@@ -125,6 +131,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
   kv_lo = kv_lo > 0 ? kv_lo : 0;
   kv_lo = kv_lo < kv_hi ? kv_lo : kv_hi;
   const int blk_lo = kv_lo / PBN, blk_hi = (kv_hi + PBN - 1) / PBN;
+  const int nblk = blk_hi - blk_lo;
   const int key_max = kv_hi - 1;           // rows beyond it are never visible and may hold anything: not loaded
 
   const bf16* kp = a.k + b * a.kv_bs + kvh * 64;
@@ -134,18 +141,19 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
   // 1 KB = 8 tile rows, the lanes' 16 bytes landing at M0 + 16 * lane; the swizzle is applied by choosing which chunk of
   // the row a lane fetches. A stage is the K tile followed by the V tile, so a wavefront's DPT instructions all belong
   // to one of the two.
-  const bool dma_v = wave * DPT >= 8;
-  const bf16* dma_src = dma_v ? vp : kp;
+  const int dma_first = wave * DPT & 15;          // the wavefront's first instruction of the block's sixteen: eight of K, eight of V
+  const int dma_block = KG == 1 ? 0 : wave * DPT >> 4;
   int dma_row[DPT], dma_col[DPT];
   const bf16* dma_ptr[DPT];                       // the lane's chunk of its row of key block 0
 #pragma unroll
   for (int j = 0; j < DPT; ++j) {
-    const int row = ((wave * DPT + j) & 7) * 8 + (lane >> 3);
+    const bool dma_v = dma_first + j >= 8;
+    const int row = ((dma_first + j) & 7) * 8 + (lane >> 3);
     dma_row[j] = row;
     dma_col[j] = ((lane & 7) ^ (dma_v ? v_swizzle(row) : ((row >> 1) & 7))) * 8;
-    dma_ptr[j] = dma_src + static_cast<int64_t>(row) * a.kv_ts + dma_col[j];
+    dma_ptr[j] = (dma_v ? vp : kp) + static_cast<int64_t>(row) * a.kv_ts + dma_col[j];
   }
-  const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem)) + wave * DPT * 1024;
+  const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem)) + dma_first * 1024;
   const int64_t blk_stride = static_cast<int64_t>(PBN) * a.kv_ts;
   auto issue_block = [&](int blk, int stage) {
     const bool whole = blk * PBN + PBN - 1 <= key_max;       // no row of the block lies beyond the last visible key
@@ -157,21 +165,24 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
       } else {
         int key = blk * PBN + dma_row[j];
         key = key < key_max ? key : key_max;
-        g = dma_src + static_cast<int64_t>(key) * a.kv_ts + dma_col[j];
+        g = (dma_first + j >= 8 ? vp : kp) + static_cast<int64_t>(key) * a.kv_ts + dma_col[j];
       }
       const unsigned m0v = lds0 + stage * PSTAGE + j * 1024;
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0v), "v"(g) : "memory", "m0");
     }
   };
-  // wait until all but the `behind` youngest blocks' loads of this wavefront have landed, then meet the others
-  auto wait_and_meet = [&](int behind) {
-    if (behind >= 2)
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * DPT) : "memory");
-    else if (behind == 1)
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(DPT) : "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  // the blocks of the step that starts at block i (counted from blk_lo) into their stages
+  auto issue_step = [&](int i) {
+    if constexpr (KG == 1) {
+#pragma unroll
+      for (int j = 0; j < STEP; ++j)
+        if (i + j < nblk) issue_block(blk_lo + i + j, (i + j) & (NSTG - 1));
+    } else {
+      if (i + dma_block < nblk) issue_block(blk_lo + i + dma_block, (i + dma_block) & (NSTG - 1));
+    }
   };
+  // wait until this wavefront's loads have landed, then meet the others
+  auto wait_and_meet = [] { asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); };
 
   // K fragment (A operand of S^T): lane = key l31 of a 32-key half, 16 bytes at d = kk*16 + h*8
   const int k_row = l31 * 128, k_sw = (l31 >> 1) & 7;
@@ -194,10 +205,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
       for (int r = 0; r < 16; ++r) o[hd][db][r] = 0.f;
   }
 
-  const int nblk = blk_hi - blk_lo;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    if (i < nblk) issue_block(blk_lo + i, i);
+  issue_step(0);
 
   {
     // The compiler does not see the direct-to-LDS loads in its count of outstanding loads; were the fragments first
@@ -209,7 +217,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
       for (int kk = 0; kk < 4; ++kk) asm volatile("" : "+v"(qf[hd][kk]));
   }
 
-  wait_and_meet(0);                              // blocks 0 and 1 have landed
+  wait_and_meet();                               // the first step's blocks have landed
 
   auto process = [&](int blk, int stage) __attribute__((always_inline)) {
     const int key0 = blk * PBN;
@@ -324,44 +332,85 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
     }
   };
 
-  // Two blocks per step: the step's loads refill the two stages the previous step read (every wavefront has left it),
-  // have two blocks of arithmetic to land behind, and are met with one wait + barrier.
-  for (int i = 0; i < nblk; i += 2) {
-#pragma unroll
-    for (int j = 2; j < 4; ++j)
-      if (i + j < nblk) issue_block(blk_lo + i + j, (i + j) & (NSTG - 1));
-    process(blk_lo + i, i & (NSTG - 1));
-    if (i + 1 < nblk) process(blk_lo + i + 1, (i + 1) & (NSTG - 1));
-    wait_and_meet(0);
+  // Two (KG) blocks per step: the step's loads refill the stages the previous step read (every wavefront has left them),
+  // have the step's arithmetic to land behind, and are met with one wait + barrier.
+  for (int i = 0; i < nblk; i += STEP) {
+    issue_step(i + STEP);
+    if constexpr (KG == 1) {
+      process(blk_lo + i, i & (NSTG - 1));
+      if (i + 1 < nblk) process(blk_lo + i + 1, (i + 1) & (NSTG - 1));
+    } else {
+      if (i + kgrp < nblk) process(blk_lo + i + kgrp, (i + kgrp) & (NSTG - 1));
+    }
+    wait_and_meet();
   }
 
   // ---- the sink joins the denominator; normalise. A lane holds 8-byte runs of ONE query's row, so storing from here
   // would be 64 scattered 8-byte writes per instruction (measured: ~3 us of a workgroup's life). The wavefront's
   // 32 x (NH x 64) tile goes through its own patch of the now idle stages instead and leaves as whole 128-byte rows.
   constexpr int OROW = NH * 128 + 16;            // patch row: the NH heads of a query + padding (2-way conflicts at most)
-  unsigned char* patch = smem + wave * (32 * OROW);
+  unsigned char* patch = smem + (KG == 1 ? wave : wave % QG) * (32 * OROW);
+  if constexpr (KG == 1) {
 #pragma unroll
-  for (int hd = 0; hd < NH; ++hd) {
-    const float l_tot = l_run[hd] + other_half(l_run[hd], h);
-    const float sk = a.sinks ? static_cast<float>(a.sinks[head0 + hd]) * kLog2e : 0.f;
-    const float m_f = fmaxf(m_run[hd], sk);
-    const float so = __builtin_amdgcn_exp2f(m_run[hd] - m_f);
-    const float inv = so / fmaf(l_tot, so, __builtin_amdgcn_exp2f(sk - m_f));
+    for (int hd = 0; hd < NH; ++hd) {
+      const float l_tot = l_run[hd] + other_half(l_run[hd], h);
+      const float sk = a.sinks ? static_cast<float>(a.sinks[head0 + hd]) * kLog2e : 0.f;
+      const float m_f = fmaxf(m_run[hd], sk);
+      const float so = __builtin_amdgcn_exp2f(m_run[hd] - m_f);
+      const float inv = so / fmaf(l_tot, so, __builtin_amdgcn_exp2f(sk - m_f));
 #pragma unroll
-    for (int db = 0; db < 2; ++db)
+      for (int db = 0; db < 2; ++db)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        bf16x4 w;
+        for (int j = 0; j < 4; ++j) {
+          bf16x4 w;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = static_cast<bf16>(o[hd][db][4 * j + i] * inv);
-        *reinterpret_cast<bf16x4*>(patch + l31 * OROW + hd * 128 + (db * 32 + 8 * j + 4 * h) * 2) = w;
-      }
+          for (int i = 0; i < 4; ++i) w[i] = static_cast<bf16>(o[hd][db][4 * j + i] * inv);
+          *reinterpret_cast<bf16x4*>(patch + l31 * OROW + hd * 128 + (db * 32 + 8 * j + 4 * h) * 2) = w;
+        }
+    }
+  } else {
+    // The key groups' shares of a query group meet in the idle stages: the accumulator as it is (32 values of 64 lanes), the
+    // running maximum and the sum. Wavefront kgrp adds 32 / KG of the 32 values up.
+    constexpr int SHARE = 34 * 64;                 // floats of a wavefront
+    constexpr int RPG = 32 / KG;
+    float* const shares = reinterpret_cast<float*>(smem + QG * 32 * OROW);
+    float* const mine = shares + wave * SHARE + lane;
+#pragma unroll
+    for (int r = 0; r < 32; ++r) mine[r * 64] = o[0][r >> 4][r & 15];
+    mine[32 * 64] = m_run[0];
+    mine[33 * 64] = l_run[0] + other_half(l_run[0], h);
+    __syncthreads();
+    const float* const from = shares + (wave % QG) * SHARE + lane;   // key group k: + k * QG * SHARE
+    const float sk = a.sinks ? static_cast<float>(a.sinks[head0]) * kLog2e : 0.f;
+    float m_f = sk;
+#pragma unroll
+    for (int k = 0; k < KG; ++k) m_f = fmaxf(m_f, from[k * QG * SHARE + 32 * 64]);
+    float den = __builtin_amdgcn_exp2f(sk - m_f);
+    float v[RPG] = {};
+#pragma unroll
+    for (int k = 0; k < KG; ++k) {
+      const float* const p = from + k * QG * SHARE;
+      const float f = __builtin_amdgcn_exp2f(p[32 * 64] - m_f);      // a group without a visible key: exp2(-inf) = 0
+      den = fmaf(p[33 * 64], f, den);
+#pragma unroll
+      for (int r = 0; r < RPG; ++r) v[r] = fmaf(p[(RPG * kgrp + r) * 64], f, v[r]);
+    }
+    const float inv = 1.f / den;
+#pragma unroll
+    for (int r = 0; r < RPG; r += 4) {
+      const int rr = RPG * kgrp + r, db = rr >> 4, j = rr >> 2 & 3;
+      bf16x4 w;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = static_cast<bf16>(v[r + i] * inv);
+      *reinterpret_cast<bf16x4*>(patch + l31 * OROW + (db * 32 + 8 * j + 4 * h) * 2) = w;
+    }
+    __syncthreads();
   }
   // 16-byte chunks in row-major order: eight lanes per 128-byte head row, NH x 8 per query
   bf16* ob = a.out + b * a.out_bs + head0 * 64;
 #pragma unroll
-  for (int it = 0; it < NH * 4; ++it) {
-    const int idx = it * 64 + lane;
+  for (int it = 0; it < NH * 4 / KG; ++it) {
+    const int idx = (it * KG + kgrp) * 64 + lane;
     const int row = idx / (NH * 8), ch = idx % (NH * 8);
     const bf16x8 w = *reinterpret_cast<const bf16x8*>(patch + row * OROW + ch * 16);
     if (qw0 + row < a.n_q) *reinterpret_cast<bf16x8*>(ob + static_cast<int64_t>(qw0 + row) * a.out_ts + ch * 8) = w;
@@ -371,6 +420,20 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
 }  // namespace tllm
 
 using namespace tllm;
+
+template <int NH, int QG, int KG, int NW>
+static int launch_prefill(const AttnPrefillArgs& a, hipStream_t st) {
+  constexpr int SMEM = 2 * (KG == 1 ? 2 : KG) * PSTAGE, HS = NW / (QG * KG);
+  static_assert(KG == 1 || QG * 32 * (128 + 16) + NW * 34 * 256 <= SMEM, "the key groups' shares fit the stages");
+  static_assert(KG > 1 || NW * 32 * (NH * 128 + 16) <= SMEM, "the output patches fit the stages");
+  static std::atomic<uint64_t> done{0};
+  const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(attn_prefill_kernel<NH, QG, KG, NW>), SMEM, done);
+  TLLM_REQUIRE(e == hipSuccess, TLLM_E_LAUNCH, "attention_prefill: cannot raise LDS limit: %s", hipGetErrorString(e));
+  const int64_t wgs = static_cast<int64_t>((a.n_q + 32 * QG - 1) / (32 * QG)) * a.batch * a.n_kv_heads * (a.group / (NH * HS));
+  TLLM_REQUIRE(wgs < (1ll << 31), TLLM_E_SHAPE, "attention_prefill: %lld workgroups are too many for one launch", (long long)wgs);
+  hipLaunchKernelGGL((attn_prefill_kernel<NH, QG, KG, NW>), dim3((unsigned)wgs), dim3(NW * 64), SMEM, st, a);
+  return check_launch("attention_prefill");
+}
 
 extern "C" int tllm_attention_prefill_bf16(const void* q, const void* k, const void* v, const void* sinks, void* out, int64_t q_batch_stride,
                                            int64_t q_token_stride, int64_t out_batch_stride, int64_t out_token_stride,
@@ -416,21 +479,23 @@ extern "C" int tllm_attention_prefill_bf16(const void* q, const void* k, const v
   a.group = group;
   a.window = window;
   a.sm_scale = sm_scale;
-  // Workgroup shape: 128 queries x 2 heads (two heads per wavefront) as soon as that gives every CU two workgroups;
-  // below that 64 queries x 2 heads with one head per wavefront: twice the workgroups, and the longest of them -- it
-  // sets the time of so small a launch -- takes about half as long per key block (one prompt of 1024 tokens: 28.8 ->
-  // 21.4 us; at 2048 tokens, 512 workgroups of the large shape, the two are level). Odd group sizes: 128 x 1.
+  // Workgroup shape, by how many workgroups the launch has. 128 queries x 2 heads (two heads per wavefront) as soon as
+  // that gives every CU two of them; below that 64 queries x 2 heads with one head per wavefront: twice the workgroups, and the
+  // longest of them -- it sets the time of so small a launch -- takes about half as long per key block. When even 64
+  // queries x 1 head are at most two per CU, the wavefronts share the key blocks out as well: two groups of two
+  // wavefronts, or four (one workgroup of eight wavefronts per CU), us before -> now:
+  //   97 queries behind 1500 keys 27.0 -> 16.1 (two groups 18.3), with a window of 128 9.3 -> 6.9; 16 behind 4000 58.3 -> 29.9;
+  //   256 behind 2000 37.4 -> 20.3 (23.8); 400 queries 11.3 -> 9.7; 500 behind 1000 27.4 -> 21.3; 512 behind 4000 67.9 -> 56.1
+  //   (from three workgroups per CU on the longer walk is hidden by the others: 777 queries 17.8, shared out 19.1).
+  // Odd group sizes: 128 x 1.
   const int nh = group % 2 == 0 ? 2 : 1;
-  const int64_t wgs128 = (n_q + 127) / 128 * batch * n_kv_heads * (group / nh);
-  const bool small = nh == 2 && wgs128 < 512;
-  const int64_t wgs = small ? (n_q + 63) / 64 * batch * n_kv_heads * (group / 2) : wgs128;
-  TLLM_REQUIRE(batch < (1ll << 24) && wgs < (1ll << 31), TLLM_E_SHAPE, "attention_prefill: %lld workgroups are too many for one launch", (long long)wgs);
+  const int64_t wgs64 = (n_q + 63) / 64 * batch * n_heads, wgs128 = (n_q + 127) / 128 * batch * n_kv_heads * (group / nh);
+  const int64_t span = window > 0 && window < n_kv_ctx - n_q ? n_q + window : n_kv_ctx;     // most keys there can be to visit
+  TLLM_REQUIRE(batch < (1ll << 24) && wgs128 < (1ll << 31), TLLM_E_SHAPE, "attention_prefill: %lld workgroups are too many for one launch", (long long)wgs128);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (small)
-    hipLaunchKernelGGL((attn_prefill_kernel<1, 2>), dim3((unsigned)wgs), dim3(256), 0, st, a);
-  else if (nh == 2)
-    hipLaunchKernelGGL((attn_prefill_kernel<2, 4>), dim3((unsigned)wgs), dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL((attn_prefill_kernel<1, 4>), dim3((unsigned)wgs), dim3(256), 0, st, a);
-  return check_launch("attention_prefill");
+  if (wgs64 <= 256 && span > 192) return launch_prefill<1, 2, 4, 8>(a, st);
+  if (wgs64 <= 512) return launch_prefill<1, 2, 2, 4>(a, st);
+  if (nh == 2 && wgs128 < 512) return launch_prefill<1, 2, 1, 4>(a, st);
+  if (nh == 2) return launch_prefill<2, 4, 1, 4>(a, st);
+  return launch_prefill<1, 4, 1, 4>(a, st);
 }
