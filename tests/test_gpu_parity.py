@@ -1093,6 +1093,35 @@ def test_unembedding_other_hidden_sizes(gpu, rows, hidden):
     _argmax_ok(T.unembedding_decode_fp8_argmax_forward(xg, w8, ws), want8)
 
 
+@pytest.mark.parametrize("hidden", [2048, 4096, 6144, 8192])
+def test_rows_of_a_power_of_two_pitch(gpu, hidden):
+    """Weights whose rows begin on the same memory channels: every workgroup begins its walk over K somewhere else -- logits
+    (tiles for some wavefronts only, several each, a ragged last one; fp8 in pairs of rows and one by one) and projections."""
+    g = torch.Generator().manual_seed(hidden)
+    for rows, vocab in ((1, 3001), (8, 100002 if hidden == 2048 else 9001)) if hidden <= 4096 else ():   # (wider: not built for logits)
+        x = torch.randn(rows, hidden, generator=g).bfloat16()
+        w = (0.02 * torch.randn(vocab, hidden, generator=g)).bfloat16()
+        w[vocab // 3], w[5] = w[vocab - 1], w[vocab - 1]       # equal rows: the argmax of a tie is the lowest
+        x[0] = w[5] * 50
+        xg = x.view(rows, 1, hidden).to(gpu)
+        want = O.linear_ref(x, w, None)
+        close(T.unembedding_decode_forward(xg, w.to(gpu)).view(rows, vocab), want)
+        ids = T.unembedding_decode_argmax_forward(xg, w.to(gpu))
+        assert int(ids[0]) == 5
+        _argmax_ok(ids, want)
+        w8, ws = T.quantize_fp8_rows(w.to(gpu))
+        close(T.unembedding_decode_fp8_forward(xg, w8, ws).view(rows, vocab), O.linear_ref(x, O.dequant_fp8_ref(w8.cpu(), ws.cpu()), None))
+    for rows in (1, 7, 16, 19):
+        x = torch.randn(rows, 1, hidden, generator=g).bfloat16()
+        w, b = (0.02 * torch.randn(1040, hidden, generator=g)).bfloat16(), torch.randn(1040, generator=g).bfloat16()
+        def zero():
+            return torch.zeros(rows, 1, 1040, dtype=torch.bfloat16, device=gpu)
+
+        close(T.out_residual_decode_forward(x.to(gpu), w.to(gpu), b.to(gpu), zero()).view(rows, 1040), O.linear_ref(x[:, 0], w, b))
+        w8, ws = T.quantize_fp8_rows(w.to(gpu))
+        close(T.out_residual_decode_forward(x.to(gpu), w8, b.to(gpu), zero(), ws).view(rows, 1040), O.linear_ref(x[:, 0], O.dequant_fp8_ref(w8.cpu(), ws.cpu()), b))
+
+
 @pytest.mark.parametrize("rows,vocab,hidden", [(17, 3001, 2880), (32, 140000, 2880), (33, 70001, 2880), (50, 4096, 2880), (64, 9000, 2880),
                                                 (24, 5000, 128), (32, 5000, 192), (29, 5000, 1024), (20, 270000, 128)])
 def test_unembedding_more_than_16_rows_one_pass_over_the_weight(gpu, rows, vocab, hidden):

@@ -6,7 +6,7 @@
 //                              is generic over both, triton_kernels.py:1127-1158, 927-940)
 //   out_decode_general_kernel  out-projection + bias + residual, any in_dim % 32 == 0 (triton_kernels.py:1340-1467)
 //
-// HBM-bound: 8 rows, [4096, 4096] weight 8.0 us = 4.2 TB/s, of which 1.6 us are the launch (a wavefront per dot product:
+// HBM-bound: 8 rows, [4096, 4096] weight 7.1 us = 4.7 TB/s, of which 1.6 us are the launch (a wavefront per dot product:
 // 89.7 us); QKV at hidden 4096, 80 heads of 64 11.0 us = 3.8 TB/s (14.7 before), fp8 weight 8.0 (13.5). Above 8 rows the
 // sixteen-row form: its activations are half of what a workgroup reads, from the L2s.
 #include "decode_general_stream.h"

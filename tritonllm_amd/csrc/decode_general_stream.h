@@ -68,8 +68,14 @@ struct DecodeGeneralStream {
       xchunk[j] = static_cast<unsigned>((lane % XPOS) ^ r) * 16u;
       xrow_off[j] = static_cast<unsigned>(r < nvalid ? r : nvalid - 1) * xpitch;
     }
+    // Rows whose pitch is a multiple of 4 KB all begin on the same memory channels: the workgroups of an XCD start in different
+    // phases and go round (such a K has no ragged phase). [4096, 4096] at 8 rows 7.95 -> 7.1 us, fp8 6.3 -> 5.8,
+    // [4096, 8192] 15.5 -> 12.5; at K = 3072, whose rows spread by themselves, it makes no difference.
+    const int rot = wpitch % 4096 == 0 && nph > 0 ? static_cast<int>(blockIdx.x >> 3) % nph : 0;
+    auto phase = [&](int pp) { return pp + rot < nph ? pp + rot : pp + rot - nph; };
     auto lds_addr = [](const void* p) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>(p)); };
-    auto issue = [&](int p, int slot) {
+    auto issue = [&](int pp, int slot) {
+      const int p = phase(pp);
       unsigned char* reg = my + slot * REGION;
       const unsigned wk = static_cast<unsigned>(p * NS + wave) * 256u, xk = static_cast<unsigned>(p * NS + wave) * XROW;
       // a chunk behind the row's end re-reads the row's last one (its products are masked)
@@ -116,8 +122,8 @@ struct DecodeGeneralStream {
       // the region is free once its fragments are in registers
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (p + D < nph) issue(p + D, slot);
-      if (ragged && behind == 0) {
-        const int left = (K - (p * NS + wave) * KPH) >> 3;  // k8 groups that exist
+      if (ragged && phase(p) == nph - 1) {
+        const int left = (K - (phase(p) * NS + wave) * KPH) >> 3;  // k8 groups that exist
 #pragma unroll
         for (int st = 0; st < PST; ++st)
           if (k8_of(st, g) >= left) {

@@ -80,6 +80,13 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
   const int my_tiles = full_rounds + (tile_of(full_rounds) < ntiles ? 1 : 0);
   const int gw = wave * nwg + wg;                             // this wavefront's number (its slot in the argmax workspace)
   const int total = my_tiles * nsteps;                        // steps of the whole stream
+  // The step of a tile with which this workgroup's wavefronts begin; they go round from there. Rows whose pitch is a multiple of
+  // 4 KB all begin on the same memory channels, and workgroups that walk K in step ask for the same few of them at a time: 8 rows
+  // of width 4096 282 -> 249 us, 2048 146 -> 128 (a start of its own for every wavefront 252 and 131). Other pitches spread by
+  // themselves (2880 176.8 and 174.6, 5120 304 and 309): in step. So is the argmax form, whose rule for ties wants equal
+  // rows to have equal sums.
+  const int pitch = SR || !W8 ? 2 * a.hidden : a.hidden;
+  const int rot = !ARGMAX && pitch % 4096 == 0 ? ((wg >> 3) * 2) % nsteps : 0;
 
   // One load instruction moves 1 KB; the 32 x (KS elements) block of a step is dealt to the lanes as 16-byte
   // chunks in row-major order, so consecutive lanes cover consecutive bytes of a row (KS = 64: eight lanes per
@@ -97,7 +104,7 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
 
   bf16x8 buf[UD][LPS];
   const bf16x8* lp[LPS];                                      // load cursor: row bases of the tile being requested
-  int l_round = 0, l_tile = tile_of(0), l_step = 0, l_count = 0;
+  int l_round = 0, l_tile = tile_of(0), l_step = rot, l_count = 0;
 #pragma unroll
   for (int i = 0; i < LPS; ++i) lp[i] = row_base(my_tiles > 0 ? l_tile : 0, i);
   // Unconditional on purpose (a load under a branch makes the compiler wait for it where the paths join): past
@@ -112,8 +119,8 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
     }
     if (l_count + 1 < total) {
       ++l_count;
-      if (++l_step == nsteps) {
-        l_step = 0;
+      if (++l_step == nsteps) l_step = 0;
+      if (l_step == rot) {
         l_tile = tile_of(++l_round);
 #pragma unroll
         for (int i = 0; i < LPS; ++i) lp[i] = row_base(l_tile < ntiles ? l_tile : ntiles - 1, i);
@@ -147,7 +154,7 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
 
   const unsigned char* xfrag = xs + (m & (XR - 1)) * xrow_b + h * 16;   // activations on M: tile rows >= XR repeat, never stored
   const unsigned char* wfrag = patch + m * UPROW + h * 16;              // vocabulary rows on N
-  int c_round = 0, c_tile = tile_of(0), c_step = 0;
+  int c_round = 0, c_tile = tile_of(0), c_step = rot;
   for (int g0 = 0; g0 < total; g0 += UD) {
 #pragma unroll
     for (int d = 0; d < UD; ++d) {
@@ -208,7 +215,8 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        if (SR && ++c_step == nsteps) {                       // tile finished: lane owns vocabulary rows 2 p and 2 p + 1, p = c_tile*32 + m
+        if (++c_step == nsteps) c_step = 0;
+        if (SR && c_step == rot) {                            // tile finished: lane owns vocabulary rows 2 p and 2 p + 1, p = c_tile*32 + m
           const int v0 = 2 * (c_tile * 32 + m), v1 = v0 + 1;  // the vocabulary is even here: both are inside it, or neither
           const float sc0 = a.w_scale[v0 < a.vocab ? v0 : a.vocab - 2], sc1 = a.w_scale[v1 < a.vocab ? v1 : a.vocab - 1];
 #pragma unroll
@@ -239,10 +247,9 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
           }
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[r] = acc2[r] = 0.f;
-          c_step = 0;
           c_tile = tile_of(++c_round);
         }
-        if (!SR && ++c_step == nsteps) {                      // tile finished: lane owns vocabulary row c_tile*32 + m
+        if (!SR && c_step == rot) {                           // tile finished: lane owns vocabulary row c_tile*32 + m
           const int v = c_tile * 32 + m;
           float sc = 1.f;
           if constexpr (W8) sc = a.w_scale[v < a.vocab ? v : a.vocab - 1];
@@ -261,7 +268,6 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
           }
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-          c_step = 0;
           c_tile = tile_of(++c_round);
         }
       }
