@@ -1,7 +1,9 @@
 """CPU-side checks of the C-ABI boundary: the library loads, exports every symbol the
 header declares, and rejects bad arguments on the host before anything is launched."""
+import copy
 import ctypes as C
 import os
+import pickle
 import re
 
 import pytest
@@ -32,6 +34,15 @@ def test_library_exports_every_declared_symbol():
 def test_struct_layout_matches_header():
     assert C.sizeof(_lib.TllmYarn) == 128 * 4 + 4 + 4
     assert C.sizeof(_lib.TllmRope) == 8 * 8
+
+
+def test_yarn_address_is_the_objects_own():
+    """Copies of a YarnParams whose C struct has been used hand out their own struct's address."""
+    y = gpt_oss_yarn()
+    assert y._c_address == C.addressof(y.c_struct())
+    for z in (copy.deepcopy(y), pickle.loads(pickle.dumps(y))):
+        assert z._c_address == C.addressof(z.c_struct())
+        assert bytes(_lib.TllmYarn.from_address(z._c_address)) == bytes(y.c_struct())
 
 
 def _err():

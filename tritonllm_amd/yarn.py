@@ -8,7 +8,6 @@ same fp32 operation order as the reference's ``RotaryEmbedding._compute_concentr
 from __future__ import annotations
 
 import ctypes as C
-import functools
 import math
 from dataclasses import dataclass, field
 
@@ -51,9 +50,10 @@ class YarnParams:
             object.__setattr__(self, "_c", s)
         return s
 
-    @functools.cached_property
+    @property
     def _c_address(self) -> int:
-        """Address of ``c_struct()``, which this object keeps (read by the ops' C++ side)."""
+        """Address of ``c_struct()``, which this object keeps (read by the ops' C++ side). Not cached: a copied or
+        unpickled object carries the attributes of the original, and its struct lies elsewhere."""
         return C.addressof(self.c_struct())
 
     def c_pointer(self):
