@@ -10,6 +10,7 @@ import torch
 import tritonllm_amd as T
 from oracle import layers as O
 from tritonllm_amd import ops, scratch_pool
+from tritonllm_amd._lib import host
 
 pytestmark = pytest.mark.gpu
 
@@ -759,16 +760,60 @@ def test_linear_tile_gemm(gpu, rows, k, n):
     mod.weight.copy_((0.05 * torch.randn(n, k, generator=g)).bfloat16())
     mod.bias.copy_((0.05 * torch.randn(n, generator=g)).bfloat16())
     want = O.linear_ref(x[0], mod.weight.cpu(), mod.bias.cpu())
-    assert ops.linear_fits(x.to(gpu), mod.weight, mod.bias)
+    assert host().linear(x.to(gpu), mod.weight, mod.bias) is not None
     out = mod(x.to(gpu))
     assert out.shape == (1, rows, n)
     close(out[0], want)
-    assert not ops.linear_fits(torch.empty(128 * 256 + 1, k, dtype=torch.bfloat16, device=gpu), mod.weight, mod.bias)
+    assert host().linear(torch.empty(128 * 256 + 1, k, dtype=torch.bfloat16, device=gpu), mod.weight, mod.bias) is None
     mod.weight.requires_grad_(True)
-    assert not ops.linear_fits(x.to(gpu), mod.weight, mod.bias)
+    assert host().linear(x.to(gpu), mod.weight, mod.bias) is None
     y = mod(x.to(gpu))
     assert y.requires_grad
     close(y.detach()[0], want)
+
+
+def test_linear_leaves_torch_its_hooks(gpu):
+    """OUT.forward under what F.linear takes part in: vmap, forward-mode derivatives, autocast, tracing, symbolic tracing, a
+    dispatch mode, a tensor subclass; a strided operand and one that is not 16-byte aligned."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    g = torch.Generator().manual_seed(77)
+    x, dx = (torch.randn(3, 40, 128, generator=g).bfloat16().to(gpu) for _ in range(2))
+    mod = T.OUT(128, 48, device=gpu).requires_grad_(False)
+    mod.weight.copy_((0.05 * torch.randn(48, 128, generator=g)).bfloat16())
+    mod.bias.copy_((0.05 * torch.randn(48, generator=g)).bfloat16())
+    w, b = mod.weight, mod.bias
+    want = O.linear_ref(x.cpu().view(120, 128), w.cpu(), b.cpu()).view(3, 40, 48)
+    close(mod(x), want)
+    close(torch.vmap(mod)(x), want)
+    y, dy = torch.func.jvp(mod, (x,), (dx,))
+    close(y, want)
+    close(dy, O.linear_ref(dx.cpu().view(120, 128), w.cpu(), torch.zeros(48)).view(3, 40, 48))
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert mod(x).dtype == torch.float16
+    traced = torch.jit.trace(mod, (x,))
+    close(traced(dx), mod(dx).cpu())
+    close(torch.fx.symbolic_trace(mod)(x), want)
+
+    class Seen(TorchDispatchMode):
+        ops = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops += 1
+            return func(*args, **(kwargs or {}))
+
+    with Seen() as seen:
+        close(mod(x), want)
+    assert seen.ops > 0
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert type(mod(x.as_subclass(Sub))) is Sub
+    close(mod(x.transpose(0, 1)), want.transpose(0, 1))
+    flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=gpu)[1:].view(x.shape)
+    flat.copy_(x)
+    close(mod(flat), want)
 
 
 def test_qkv_generic_shapes(gpu):

@@ -72,7 +72,7 @@ class QKV(torch.nn.Module):
 class OUT(torch.nn.Module):
     """Attention out-projection (model.py:170-216): ``weight [hidden_size, out_dim]``, ``bias [hidden_size]``.
     ``decode_residual`` is the decode kernel; ``forward`` is ``F.linear``: the HIP tile GEMM for prompts of up to a few
-    thousand rows, the library's beyond that, for other types and where gradients are wanted."""
+    thousand rows, the library's beyond that, for other types and wherever torch has more to do than the product (gradients, autocast, vmap, tracing)."""
 
     def __init__(self, out_dim: int, hidden_size: int, device: torch.device | None = None):
         super().__init__()
@@ -91,11 +91,10 @@ class OUT(torch.nn.Module):
         return self._weight_fp8, self._weight_scale
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        done = host().linear(x, self.weight, self.bias)
-        if done is not None:
-            return done
-        if ops.linear_fits(x, self.weight, self.bias):
-            return ops.linear_forward(x, self.weight, self.bias)
+        if not torch.compiler.is_compiling():
+            done = host().linear(x, self.weight, self.bias)
+            if done is not None:
+                return done
         return torch.nn.functional.linear(x, self.weight, self.bias)
 
     def decode_residual(self, x: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:

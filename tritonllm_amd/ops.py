@@ -557,37 +557,6 @@ def linear_qkv_forward(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor
     return out
 
 
-# --------------------------------------------------------------------------------------- plain projection (prompts)
-def linear_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
-    """Whether ``linear_forward`` takes these operands and is the faster form: bf16 on the GPU, K a multiple of 64, outputs
-    of 16, no gradient wanted, and the largest tile (128 x 256) covering the result in one round of the 256 CUs. Beyond
-    that the library's GEMM is ahead ([2880, 4096] weight: 2688 rows 64.6 against 63.5 us, 4096 rows 103 against 83;
-    below, 97 rows 13.9 against 15.4, 192 rows 18.8 against 32, 999 rows 33.9 against 36.6)."""
-    n, k = weight.shape
-    if not (x.is_cuda and weight.is_cuda and x.dtype == weight.dtype == _BF16 and (bias is None or (bias.is_cuda and bias.dtype == _BF16))):
-        return False
-    if k % 64 or n % 16 or n * k >= 2 ** 31 or x.shape[-1] != k or x.numel() == 0:
-        return False
-    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):
-        return False
-    rows = x.numel() // k
-    return -(-rows // 128) * -(-n // 256) <= 256
-
-
-def linear_forward(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
-    """``F.linear(x, weight, bias)`` as one launch (OUT.forward of a prompt, model.py:196-197): ``[..., K] -> [..., N]``, a fresh
-    tensor. ``linear_fits`` says for which operands."""
-    _on_gpu(x, weight, bias)
-    n, k = weight.shape
-    _require(x.shape[-1] == k and weight.dtype == _BF16 and (bias is None or bias.shape == (n,)))
-    x2, weight, bias = _prep_linear(x.reshape(-1, k), weight, bias)
-    out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
-    rc = lib().tllm_linear_bf16(x2.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(), n,
-                                x2.shape[0], k, n, _stream())
-    check(rc, "linear_forward")
-    return out
-
-
 # --------------------------------------------------------------------------------------- out-projection (decode)
 def out_residual_decode_forward(hidden: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, residual: torch.Tensor,
                                 weight_scale: torch.Tensor | None = None) -> torch.Tensor:
