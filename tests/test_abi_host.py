@@ -6,10 +6,11 @@ import os
 import pickle
 import re
 
+import numpy as np
 import pytest
 import torch
 
-from tritonllm_amd import _lib
+from tritonllm_amd import _lib, scratch_pool
 from tritonllm_amd.yarn import YarnParams, gpt_oss_yarn
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -43,6 +44,11 @@ def test_yarn_address_is_the_objects_own():
     for z in (copy.deepcopy(y), pickle.loads(pickle.dumps(y))):
         assert z._c_address == C.addressof(z.c_struct())
         assert bytes(_lib.TllmYarn.from_address(z._c_address)) == bytes(y.c_struct())
+
+
+def test_scratch_pool_takes_any_integers():
+    a = scratch_pool.get((np.int64(3), 5), torch.float32, "cpu")
+    assert a.shape == (3, 5) and scratch_pool.get(torch.Size((3, 5)), torch.float32, torch.device("cpu")).data_ptr() == a.data_ptr()
 
 
 def _err():

@@ -8,6 +8,7 @@ The pool itself lives in ``csrc/host_ops.cpp``, where the ops take their outputs
 """
 from __future__ import annotations
 
+from operator import index
 from typing import Any
 
 import torch
@@ -16,7 +17,7 @@ from ._lib import host
 
 
 def get(shape: tuple, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
-    return host().pool_get(tuple(shape), dtype, torch.device(device))
+    return host().pool_get(tuple(map(index, shape)), dtype, torch.device(device))
 
 
 def clear() -> None:
