@@ -441,10 +441,10 @@ bool plain_operand(PyObject* o, c10::DeviceIndex device) {
          !(c10::GradMode::is_enabled() && t.requires_grad()) && !t._fw_grad(0).defined();
 }
 
-// linear(x, weight, bias): F.linear for plain bf16 tensors, K a multiple of 64 and outputs of 16, as long as the largest tile
-// (128 x 256) covers the result in one round of the 256 CUs. Beyond that the library's GEMM is ahead ([2880, 4096] weight: 2688
-// rows 64.6 against 63.5 us, 4096 rows 103 against 83; below, 97 rows 13.9 against 15.4, 192 rows 18.8 against 32, 999 rows 33.9
-// against 36.6).
+// linear(x, weight, bias): F.linear for plain bf16 tensors, K a multiple of 64 and outputs of 16, as long as tiles of
+// 128 x 224 cover the result in one round of the 256 CUs. Beyond that the library's GEMM is ahead ([2880, 4096] weight: 2500
+// rows 57.4 against 55.9 us, 2700 67.8 against 58.2, 4096 103 against 83; below, 97 rows 13.9 against 15.4, 192 rows 18.8 against
+// 32, 999 rows 33.9 against 36.6, 2400 rows 53.0 against 54.8).
 PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 3 || !only_eager() || !THPVariable_CheckExact(a[0]) || !tensor(a[0]).is_cuda()) return none();
   const c10::DeviceIndex device = c10::hip::current_device();
@@ -456,7 +456,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!bf16(x) || x.dim() < 1 || x.size(-1) != k || x.numel() == 0 || !bias_ok(a[2], out) || k % 64 || out % 16 || out * k >= (1ll << 31))
     return none();
   const int64_t rows = x.numel() / k;
-  if (((rows + 127) / 128) * ((out + 255) / 256) > 256) return none();
+  if (((rows + 127) / 128) * ((out + 223) / 224) > 256) return none();
   at::DimVector shape(x.sizes().begin(), x.sizes().end());
   shape.back() = out;
   const Tensor xc = x.contiguous(), y = at::empty(shape, xc.options());

@@ -691,7 +691,9 @@ extern "C" int tllm_qkv_rope_prefill_bf16(const void* x, const void* W, const vo
   const int64_t tn = (heads + HPT - 1) / HPT;
   const int64_t rounds128 = (((rows + 127) / 128) * tn + 255) / 256, rounds256 = (((rows + 255) / 256) * tn + 255) / 256;
   const int BM = rounds256 * 105 < rounds128 * 57 ? 256 : 128;
-  const int64_t here_ns = (BM == 256 ? rounds256 * 105000 : rounds128 * 57000) * (hidden / BK) / 45;
+  // (a single round of 256s rarely fills the CUs and takes 83 - 92 us then: 2900 rows 86.5, where two rounds of 128 x 256 take
+  // 91.3; up to 2816 rows two rounds of 128 x 224 are ahead, 2600 rows 82.3 against 84.6)
+  const int64_t here_ns = (BM == 128 ? rounds128 * 57000 : rounds256 == 1 ? 90000 : rounds256 * 105000) * (hidden / BK) / 45;
   if (tile_gemm_ns(rows, static_cast<int64_t>(heads) * 64, hidden) < here_ns) return launch_tile_gemm_qkv("qkv_rope_prefill", a, ra, fr, st);
   static bool attr_set = false;   // raising the dynamic-LDS limit is idempotent; a benign race at worst repeats it
   if (!attr_set) {
