@@ -9,7 +9,7 @@ import torch
 
 import tritonllm_amd as T
 from oracle import layers as O
-from tritonllm_amd import ops, scratch_pool
+from tritonllm_amd import _lib, ops, scratch_pool
 from tritonllm_amd._lib import host
 
 pytestmark = pytest.mark.gpu
@@ -814,6 +814,27 @@ def test_linear_leaves_torch_its_hooks(gpu):
     flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=gpu)[1:].view(x.shape)
     flat.copy_(x)
     close(mod(flat), want)
+
+
+def test_a_launch_error_is_raised_and_the_op_not_repeated(gpu):
+    """The runtime reports the error an earlier call has left at the next launch, which has gone out by then: the op raises
+    it, and the residual, updated in place, has the projection added once."""
+    g = torch.Generator().manual_seed(90)
+    h, w, b, res = (torch.randn(*s, generator=g).bfloat16().to(gpu) for s in ((3, 1, 128), (64, 128), (64,), (3, 1, 64)))
+    scale = torch.ones(128, device=gpu)
+    once = T.out_residual_decode_forward(h, w, b, res.clone())
+    calls = [lambda r: T.out_residual_decode_forward(h, w, b, r), lambda r: T.rmsnorm_forward(h, scale, 1e-5),
+             lambda r: T.swiglu(h), lambda r: T.qkv_rope_forward(h.view(3, 128), w, b, 2, 1, 16, rotate=False)]
+    for i, call in enumerate(calls):
+        r = res.clone()
+        call(res.clone())
+        assert _lib.lib().hipSetDevice(1 << 20) != 0            # an error that nothing has looked at yet
+        with pytest.raises(RuntimeError, match="launch failed"):
+            call(r)
+        torch.cuda.synchronize()
+        call(res.clone())                                       # it has been reported: the next call is an ordinary one
+        if i == 0:
+            assert torch.equal(r, once)
 
 
 def test_qkv_generic_shapes(gpu):

@@ -4,8 +4,9 @@
 // attribute at a time and converting twenty arguments through ctypes took 9-13 us more per call -- a decode step issued call
 // by call (24 layers, ~122 launches) spent 1690 us on the host for 670 us of GPU work. Each function here takes the
 // arguments of its namesake in ops.py, does the same checks and the same launch, and returns None as soon as anything is not
-// the ordinary case (another dtype, a strided operand, a wrong shape, a CPU tensor, an error from the launch): ops.py then
-// runs its own checks, which make the copy or raise the error. Nothing is remembered between calls but the scratch pool.
+// the ordinary case (another dtype, a strided operand, a wrong shape, a CPU tensor, arguments that the entry point refuses):
+// ops.py then runs its own checks, which make the copy or raise the error. Only a call that has launched nothing is answered
+// so; what the runtime reports at a launch is raised here. Nothing is remembered between calls but the scratch pool.
 #include <Python.h>
 
 #include <c10/core/GradMode.h>
@@ -19,6 +20,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/autocast_mode.h>
 
+#include <stdexcept>
 #include <string>
 #include <unordered_map>
 
@@ -79,6 +81,16 @@ inline bool to_f64(PyObject* o, double* v) {
 
 inline void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
 PyObject* none() { Py_RETURN_NONE; }
+
+// Calls an entry point: true behind a launch, false where it refused its arguments and launched nothing. An error of the
+// runtime's is raised and the call not made again: the kernel may be on its way (the error that an earlier call left is
+// reported by the next launch), and an op that writes in place would be applied twice.
+template <class F>
+bool launch(const char* what, F entry_point) {
+  const int rc = entry_point();
+  if (rc == TLLM_E_LAUNCH) throw std::runtime_error(std::string(what) + " failed (code " + std::to_string(rc) + "): " + tllm_last_error());
+  return rc == TLLM_OK;
+}
 inline PyObject* wrap(const Tensor& t) { return THPVariable_Wrap(t); }
 
 // ---- scratch pool -----------------------------------------------------------------------------------------------------------
@@ -186,8 +198,10 @@ bool rope_of(PyObject* yarn, PyObject* positions, PyObject* offset, int64_t rows
 // ---- ops ----------------------------------------------------------------------------------------------------------------------
 bool rmsnorm_into(const Tensor& x, const Tensor& scale, double eps, const Tensor& out) {
   const int64_t hidden = x.size(-1);
-  return tllm_rmsnorm_bf16(x.const_data_ptr(), scale.const_data_ptr(), bf16(scale), mut(out), hidden ? x.numel() / hidden : 0, hidden,
-                           static_cast<float>(eps), stream()) == TLLM_OK;
+  return launch("rmsnorm_forward", [&] {
+    return tllm_rmsnorm_bf16(x.const_data_ptr(), scale.const_data_ptr(), bf16(scale), mut(out), hidden ? x.numel() / hidden : 0, hidden,
+                             static_cast<float>(eps), stream());
+  });
 }
 
 // rmsnorm(x, scale, eps, out)
@@ -233,9 +247,11 @@ PyObject* embedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
     out = tensor(a[2]);
     if (!bf16(out) || out.sizes() != at::IntArrayRef(shape) || !out.is_contiguous()) return none();
   }
-  if (tllm_embedding_bf16(table.const_data_ptr(), ids.const_data_ptr(), ids.scalar_type() == at::kLong, mut(out), ids.numel(), table.size(1),
-                          table.size(0), flag(a[3]), stream()) != TLLM_OK)
-    return none();
+  const bool done = launch("embedding_forward", [&] {
+    return tllm_embedding_bf16(table.const_data_ptr(), ids.const_data_ptr(), ids.scalar_type() == at::kLong, mut(out), ids.numel(), table.size(1),
+                          table.size(0), flag(a[3]), stream());
+  });
+  if (!done) return none();
   return wrap(out);
 }
 
@@ -259,9 +275,11 @@ PyObject* embedding_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
   }
   if (got[0].const_data_ptr() == got[1].const_data_ptr()) return none();
-  if (tllm_embed_rmsnorm_bf16(table.const_data_ptr(), ids.const_data_ptr(), ids.scalar_type() == at::kLong, mut(got[0]), scale.const_data_ptr(),
-                              bf16(scale), mut(got[1]), ids.numel(), hidden, table.size(0), static_cast<float>(eps), flag(a[6]), stream()) != TLLM_OK)
-    return none();
+  const bool done = launch("embedding_rmsnorm_forward", [&] {
+    return tllm_embed_rmsnorm_bf16(table.const_data_ptr(), ids.const_data_ptr(), ids.scalar_type() == at::kLong, mut(got[0]), scale.const_data_ptr(),
+                              bf16(scale), mut(got[1]), ids.numel(), hidden, table.size(0), static_cast<float>(eps), flag(a[6]), stream());
+  });
+  if (!done) return none();
   PyObject *x = wrap(got[0]), *y = wrap(got[1]);
   PyObject* r = PyTuple_Pack(2, x, y);
   Py_XDECREF(x);
@@ -286,9 +304,11 @@ PyObject* swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
     out = tensor(a[4]);
     if (!bf16(out) || out.sizes() != at::IntArrayRef(shape) || !out.is_contiguous()) return none();
   }
-  if (tllm_swiglu_bf16(x.const_data_ptr(), mut(out), x.numel() / (2 * n_out), n_out, 2 * n_out, static_cast<float>(alpha), static_cast<float>(limit),
-                       !is_none(a[2]), a[3] == Py_True, stream()) != TLLM_OK)
-    return none();
+  const bool done = launch("swiglu", [&] {
+    return tllm_swiglu_bf16(x.const_data_ptr(), mut(out), x.numel() / (2 * n_out), n_out, 2 * n_out, static_cast<float>(alpha), static_cast<float>(limit),
+                       !is_none(a[2]), a[3] == Py_True, stream());
+  });
+  if (!done) return none();
   return wrap(out);
 }
 
@@ -310,21 +330,23 @@ bool launch_qkv(bool decode, const Tensor& x_in, const Tensor& w, PyObject* bias
       x = t;
     }
   }
-  void* st = stream();
   const float e = static_cast<float>(eps);
-  int rc;
   if (ws != nullptr) {
     if (!decode || hidden % 32 != 0 || hd % 16 != 0) return false;
-    rc = tllm_qkv_rope_decode_w8_bf16(x.const_data_ptr(), ns, ns_bf16, e, w.const_data_ptr(), static_cast<const float*>(ws), ptr(bias), q, k, v, q_rs,
-                                      k_rs, v_rs, kv_slot, rows, hidden, nq, nkv, hd, rope, st);
-  } else if (ns != nullptr) {
-    rc = tllm_norm_qkv_rope_decode_bf16(x.const_data_ptr(), ns, ns_bf16, e, w.const_data_ptr(), ptr(bias), q, k, v, q_rs, k_rs, v_rs, kv_slot, rows,
-                                        hidden, nq, nkv, hd, rope, st);
-  } else {
-    rc = (decode ? tllm_qkv_rope_decode_bf16 : tllm_qkv_rope_prefill_bf16)(x.const_data_ptr(), w.const_data_ptr(), ptr(bias), q, k, v, q_rs, k_rs,
-                                                                          v_rs, kv_slot, rows, hidden, nq, nkv, hd, rope, st);
+    return launch("qkv_rope_decode_w8", [&] {
+      return tllm_qkv_rope_decode_w8_bf16(x.const_data_ptr(), ns, ns_bf16, e, w.const_data_ptr(), static_cast<const float*>(ws), ptr(bias), q, k, v,
+                                          q_rs, k_rs, v_rs, kv_slot, rows, hidden, nq, nkv, hd, rope, stream());
+    });
   }
-  return rc == TLLM_OK;
+  if (ns != nullptr)
+    return launch("norm_qkv_rope_decode", [&] {
+      return tllm_norm_qkv_rope_decode_bf16(x.const_data_ptr(), ns, ns_bf16, e, w.const_data_ptr(), ptr(bias), q, k, v, q_rs, k_rs, v_rs, kv_slot,
+                                            rows, hidden, nq, nkv, hd, rope, stream());
+    });
+  return launch(decode ? "qkv_rope_decode" : "qkv_rope_prefill", [&] {
+    return (decode ? tllm_qkv_rope_decode_bf16 : tllm_qkv_rope_prefill_bf16)(x.const_data_ptr(), w.const_data_ptr(), ptr(bias), q, k, v, q_rs, k_rs, v_rs,
+                                                                            kv_slot, rows, hidden, nq, nkv, hd, rope, stream());
+  });
 }
 
 bool heads_of(PyObject* const* a, int64_t total_out, int* nq, int* nkv, int* hd) {
@@ -460,7 +482,10 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::DimVector shape(x.sizes().begin(), x.sizes().end());
   shape.back() = out;
   const Tensor xc = x.contiguous(), y = at::empty(shape, xc.options());
-  if (tllm_linear_bf16(xc.const_data_ptr(), w.const_data_ptr(), ptr(a[2]), mut(y), out, rows, k, out, stream()) != TLLM_OK) return none();
+  const bool done = launch("linear", [&] {
+    return tllm_linear_bf16(xc.const_data_ptr(), w.const_data_ptr(), ptr(a[2]), mut(y), out, rows, k, out, stream());
+  });
+  if (!done) return none();
   return wrap(y);
 }
 
@@ -472,9 +497,11 @@ PyObject* out_residual(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!bf16(h) || h.dim() != 3 || h.size(1) != 1 || h.size(2) != in || !h.is_contiguous() || !bias_ok(a[2], out)) return none();
   const int64_t batch = h.size(0);
   if (!bf16(res) || res.dim() != 3 || res.size(0) != batch || res.size(1) != 1 || res.size(2) != out || !res.is_contiguous()) return none();
-  if (tllm_out_residual_decode_bf16(h.const_data_ptr(), w.const_data_ptr(), static_cast<const float*>(ptr(a[4])), ptr(a[2]), mut(res), mut(res), out, out,
-                                    batch, in, out, stream()) != TLLM_OK)
-    return none();
+  const bool done = launch("out_residual_decode_forward", [&] {
+    return tllm_out_residual_decode_bf16(h.const_data_ptr(), w.const_data_ptr(), static_cast<const float*>(ptr(a[4])), ptr(a[2]), mut(res), mut(res), out, out,
+                                    batch, in, out, stream());
+  });
+  if (!done) return none();
   return wrap(res.view({batch, 1, out}));
 }
 
@@ -484,9 +511,11 @@ PyObject* unembedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor &h = tensor(a[0]), &w = tensor(a[1]);
   if (!bf16(h) || h.dim() != 3 || h.size(1) != 1 || h.size(2) != w.size(1) || !h.is_contiguous()) return none();
   const Tensor logits = pool_get({h.size(0), w.size(0)}, at::kBFloat16, h.device());
-  if (tllm_unembedding_decode_bf16(h.const_data_ptr(), w.const_data_ptr(), static_cast<const float*>(ptr(a[2])), mut(logits), w.size(0), h.size(0),
-                                   w.size(1), w.size(0), stream()) != TLLM_OK)
-    return none();
+  const bool done = launch("unembedding_decode_forward", [&] {
+    return tllm_unembedding_decode_bf16(h.const_data_ptr(), w.const_data_ptr(), static_cast<const float*>(ptr(a[2])), mut(logits), w.size(0), h.size(0),
+                                   w.size(1), w.size(0), stream());
+  });
+  if (!done) return none();
   return wrap(logits.unsqueeze(1));
 }
 
@@ -545,10 +574,12 @@ PyObject* attention_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor o = pool_get({t.bs, width}, at::kBFloat16, t.q->device());
   Tensor work;
   if (bytes) work = pool_get({bytes / 4 > 1 ? bytes / 4 : 1}, at::kFloat, t.q->device());
-  if (tllm_attention_decode_bf16(t.q->const_data_ptr(), t.k->const_data_ptr(), t.v->const_data_ptr(), t.sinks, mut(o), width, width, t.k->stride(0),
+  const bool done = launch("attention_decode", [&] {
+    return tllm_attention_decode_bf16(t.q->const_data_ptr(), t.k->const_data_ptr(), t.v->const_data_ptr(), t.sinks, mut(o), width, width, t.k->stride(0),
                                  t.k->stride(1), t.bs, t.n_kv_ctx, t.nkv, t.group, 64, t.scale, static_cast<int>(t.window), t.start,
-                                 static_cast<int>(t.start_is_i64), hint, bytes ? mut(work) : nullptr, bytes, stream()) != TLLM_OK)
-    return none();
+                                 static_cast<int>(t.start_is_i64), hint, bytes ? mut(work) : nullptr, bytes, stream());
+  });
+  if (!done) return none();
   return wrap(o.view({t.bs, 1, width}));
 }
 
@@ -563,10 +594,12 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   const int64_t width = static_cast<int64_t>(t.nkv) * t.group * 64;
   const Tensor o = pool_get({t.bs, t.n_ctx, width}, at::kBFloat16, q.device());
-  if (tllm_attention_prefill_bf16(q.const_data_ptr(), t.k->const_data_ptr(), t.v->const_data_ptr(), t.sinks, mut(o), q.stride(0), q.stride(1),
+  const bool done = launch("attention", [&] {
+    return tllm_attention_prefill_bf16(q.const_data_ptr(), t.k->const_data_ptr(), t.v->const_data_ptr(), t.sinks, mut(o), q.stride(0), q.stride(1),
                                   o.stride(0), o.stride(1), t.k->stride(0), t.k->stride(1), t.bs, t.n_ctx, t.n_kv_ctx, t.nkv, t.group, 64, t.scale,
-                                  static_cast<int>(t.window), t.start, static_cast<int>(t.start_is_i64), stream()) != TLLM_OK)
-    return none();
+                                  static_cast<int>(t.window), t.start, static_cast<int>(t.start_is_i64), stream());
+  });
+  if (!done) return none();
   return wrap(o);
 }
 

@@ -8,7 +8,7 @@ CPU path: tensors must live on the GPU and the shared library must be built.
 
 The ops a model calls per layer first offer their arguments to the C++ side (``csrc/host_ops.cpp``), which checks and
 launches the ordinary case in a fraction of the host time; it answers ``None`` to anything else -- a strided operand, a
-wrong shape or type, a failed launch -- and the code here makes the copy or raises the error.
+wrong shape or type -- and the code here makes the copy or raises the error.
 
 Reference signatures (paths under ``tritonllm/gpt_oss/triton/``):
 
