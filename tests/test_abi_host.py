@@ -5,6 +5,8 @@ import ctypes as C
 import os
 import pickle
 import re
+import threading
+from itertools import chain, starmap
 
 import numpy as np
 import pytest
@@ -49,6 +51,29 @@ def test_yarn_address_is_the_objects_own():
 def test_scratch_pool_takes_any_integers():
     a = scratch_pool.get((np.int64(3), 5), torch.float32, "cpu")
     assert a.shape == (3, 5) and scratch_pool.get(torch.Size((3, 5)), torch.float32, torch.device("cpu")).data_ptr() == a.data_ptr()
+
+
+def test_allocation_gives_up_the_interpreter_lock():
+    """Another thread runs while the host side allocates (here: while the new buffer is filled). list() draws all three values
+    without going back to the interpreter, so nothing else can let the thread in between them."""
+    n, stop = [0], threading.Event()
+
+    def count():
+        while not stop.is_set():
+            n[0] += 1
+
+    thread = threading.Thread(target=count)
+    torch.use_deterministic_algorithms(True)
+    thread.start()
+    try:
+        args = ((1 << 27,), torch.float32, torch.device("cpu"))
+        before, _, after = list(chain(map(n.__getitem__, [0]), starmap(_lib.host().pool_get, [args]), map(n.__getitem__, [0])))
+    finally:
+        stop.set()
+        thread.join()
+        torch.use_deterministic_algorithms(False)
+        scratch_pool.clear()
+    assert after > before
 
 
 def _err():

@@ -4,6 +4,10 @@ Bar: bit-exact for the embedding gather; rtol 1.6e-2 / atol 1e-2 against the fp3
 oracle for every bf16 output. Inputs are the seeded synthetic tensors of the benchmark
 configurations plus edge cases (ragged rows, wrap-around positions, clamps, odd sizes).
 """
+import sys
+import threading
+from itertools import chain, repeat, starmap
+
 import pytest
 import torch
 
@@ -835,6 +839,73 @@ def test_a_launch_error_is_raised_and_the_op_not_repeated(gpu):
         call(res.clone())                                       # it has been reported: the next call is an ordinary one
         if i == 0:
             assert torch.equal(r, once)
+
+
+def test_launches_give_up_the_interpreter_lock(gpu):
+    """(as test_allocation_gives_up_the_interpreter_lock)"""
+    n, stop = [0], threading.Event()
+
+    def count():
+        while not stop.is_set():
+            n[0] += 1
+
+    x, s, w, b = (torch.randn(*shape, device=gpu).bfloat16() for shape in ((4, 128), (128,), (64, 128), (64,)))
+    out = torch.empty_like(x)
+    calls = {"rmsnorm": (x, s, 1e-5, out), "swiglu": (x, 1.7, 7.0, True, out[:, :64].contiguous()), "linear": (x, w, b),
+             "out_residual": (x.view(4, 1, 128), w, b, torch.zeros(4, 1, 64, device=gpu).bfloat16(), None)}
+    interval, thread = sys.getswitchinterval(), threading.Thread(target=count)
+    sys.setswitchinterval(1e-6)                      # the waiting thread asks for the lock at once
+    thread.start()
+    try:
+        seen = {}
+        for name, args in calls.items():
+            op = getattr(host(), name)
+            assert op(*args) is not None
+            got = list(chain(map(n.__getitem__, [0]), starmap(op, repeat(args, 200)), map(n.__getitem__, [0])))
+            seen[name] = got[-1] - got[0]
+    finally:
+        stop.set()
+        thread.join()
+        sys.setswitchinterval(interval)
+    assert all(d > 0 for d in seen.values()), seen
+
+
+def test_two_threads_on_two_streams(gpu):
+    g = torch.Generator().manual_seed(91)
+    sets = []
+    for rows in (5, 37):
+        x, s, w, b, r = (torch.randn(*shape, generator=g).bfloat16().to(gpu) for shape in ((rows, 256), (256,), (256, 256), (256,), (rows, 1, 256)))
+        mod = T.OUT(256, 256, device=gpu).requires_grad_(False)
+        mod.weight.copy_(w)
+        mod.bias.copy_(b)
+        sets.append((x, s.float(), mod, r))
+
+    def step(x, s, mod, r):
+        t = T.rmsnorm_forward(x, s, 1e-5, out=torch.empty_like(x))
+        y = mod(t)
+        y = T.out_residual_decode_forward(y.view(-1, 1, 256), mod.weight, mod.bias, r.clone())
+        return T.swiglu(y.view(-1, 256))
+
+    want = [step(*s) for s in sets]
+    torch.cuda.synchronize()
+    got, errors = [[], []], []
+
+    def run(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(200):
+                    got[i].append(step(*sets[i]))
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    assert all(torch.equal(y, want[i]) for i in range(2) for y in got[i])
 
 
 def test_qkv_generic_shapes(gpu):

@@ -82,20 +82,34 @@ inline bool to_f64(PyObject* o, double* v) {
 inline void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
 PyObject* none() { Py_RETURN_NONE; }
 
+// Ahead of a launch and of an allocation the interpreter lock is given up, as ctypes and torch's own bindings do: both may wait
+// (a full queue, a kernel's first load, memory that has to be freed first), and what they wait for may need the lock.
+struct Unlocked {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+Tensor empty(at::IntArrayRef shape, const at::TensorOptions& options) {
+  Unlocked u;
+  return at::empty(shape, options);
+}
+
 // Calls an entry point: true behind a launch, false where it refused its arguments and launched nothing. An error of the
 // runtime's is raised and the call not made again: the kernel may be on its way (the error that an earlier call left is
 // reported by the next launch), and an op that writes in place would be applied twice.
 template <class F>
 bool launch(const char* what, F entry_point) {
-  const int rc = entry_point();
+  const int rc = [&] {
+    Unlocked u;
+    return entry_point();
+  }();
   if (rc == TLLM_E_LAUNCH) throw std::runtime_error(std::string(what) + " failed (code " + std::to_string(rc) + "): " + tllm_last_error());
   return rc == TLLM_OK;
 }
 inline PyObject* wrap(const Tensor& t) { return THPVariable_Wrap(t); }
 
 // ---- scratch pool -----------------------------------------------------------------------------------------------------------
-// One buffer per (shape, dtype, device), kept until clear() (scratch_pool.py:17-22 of the reference); the interpreter lock
-// is what makes it safe to share between threads.
+// One buffer per (shape, dtype, device), kept until clear() (scratch_pool.py:17-22 of the reference); it is touched under the
+// interpreter lock only, which makes it safe to share between threads.
 std::unordered_map<std::string, Tensor>& pool() {
   static auto* p = new std::unordered_map<std::string, Tensor>();   // never destroyed: tensors outlive the interpreter otherwise
   return *p;
@@ -112,13 +126,12 @@ Tensor pool_get(at::IntArrayRef shape, at::ScalarType dtype, at::Device device) 
     buf[n++] = static_cast<char>(device.index());
     key.assign(buf, n);
   } else {
-    return at::empty(shape, at::TensorOptions().dtype(dtype).device(device));
+    return empty(shape, at::TensorOptions().dtype(dtype).device(device));
   }
   auto it = pool().find(key);
   if (it != pool().end()) return it->second;
-  Tensor t = at::empty(shape, at::TensorOptions().dtype(dtype).device(device));
-  pool().emplace(std::move(key), t);
-  return t;
+  const Tensor t = empty(shape, at::TensorOptions().dtype(dtype).device(device));
+  return pool().emplace(std::move(key), t).first->second;   // (another thread's, if it was first)
 }
 
 // An output the kernel writes while other workgroups still read `in`: not a pool buffer that is that very memory.
@@ -126,7 +139,7 @@ Tensor pooled_output(at::IntArrayRef shape, const Tensor& in) {
   Tensor t = pool_get(shape, at::kBFloat16, in.device());
   const char *a = static_cast<const char*>(t.const_data_ptr()), *b = static_cast<const char*>(in.const_data_ptr());
   if (t.numel() && in.numel() && a < b + in.numel() * in.element_size() && b < a + t.numel() * t.element_size())
-    return at::empty(shape, in.options().dtype(at::kBFloat16));
+    return empty(shape, in.options().dtype(at::kBFloat16));
   return t;
 }
 
@@ -241,7 +254,7 @@ PyObject* embedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const auto shape = with_last(ids, table.size(1));
   Tensor out;
   if (is_none(a[2])) {
-    out = at::empty(shape, table.options());
+    out = empty(shape, table.options());
   } else {
     if (!gpu_tensor(a[2])) return none();
     out = tensor(a[2]);
@@ -267,7 +280,7 @@ PyObject* embedding_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor got[2];
   for (int i = 0; i < 2; ++i) {
     if (is_none(a[4 + i])) {
-      got[i] = i == 0 ? at::empty(shape, table.options()) : pool_get(shape, at::kBFloat16, table.device());
+      got[i] = i == 0 ? empty(shape, table.options()) : pool_get(shape, at::kBFloat16, table.device());
     } else {
       if (!gpu_tensor(a[4 + i])) return none();
       got[i] = tensor(a[4 + i]);
@@ -298,7 +311,7 @@ PyObject* swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
   shape.back() = n_out;
   Tensor out;
   if (is_none(a[4])) {
-    out = at::empty(shape, x.options());
+    out = empty(shape, x.options());
   } else {
     if (!gpu_tensor(a[4])) return none();
     out = tensor(a[4]);
@@ -481,7 +494,11 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (((rows + 127) / 128) * ((out + 223) / 224) > 256) return none();
   at::DimVector shape(x.sizes().begin(), x.sizes().end());
   shape.back() = out;
-  const Tensor xc = x.contiguous(), y = at::empty(shape, xc.options());
+  const Tensor xc = x.is_contiguous() ? x : [&] {
+    Unlocked u;
+    return x.contiguous();
+  }();
+  const Tensor y = empty(shape, xc.options());
   const bool done = launch("linear", [&] {
     return tllm_linear_bf16(xc.const_data_ptr(), w.const_data_ptr(), ptr(a[2]), mut(y), out, rows, k, out, stream());
   });
