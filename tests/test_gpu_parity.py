@@ -908,6 +908,20 @@ def test_two_threads_on_two_streams(gpu):
     assert all(torch.equal(y, want[i]) for i in range(2) for y in got[i])
 
 
+@pytest.mark.parametrize("rotate", [True, False])
+@pytest.mark.parametrize("name", ["cos", "sin", "positions", "offset"])
+def test_qkv_rope_refuses_tensors_that_are_not_on_the_gpu(gpu, name, rotate):
+    rope = T.RotaryEmbedding(64, 150000, torch.float32, initial_context_length=4096, scaling_factor=32.0, device=gpu)   # (its tables carry their parameters)
+    x, w, b = (torch.zeros(*s, dtype=torch.bfloat16, device=gpu) for s in ((4, 64), (192, 64), (192,)))
+    kw = dict(cos=rope.cos, sin=rope.sin, positions=torch.arange(4, device=gpu), offset=torch.zeros(1, dtype=torch.int64, device=gpu), rotate=rotate)
+    T.qkv_rope_forward(x, w, b, 1, 1, 64, **kw)
+    away = kw[name].cpu()
+    if hasattr(kw[name], "_tllm_yarn"):
+        away._tllm_yarn = kw[name]._tllm_yarn
+    with pytest.raises(RuntimeError, match="GPU only"):
+        T.qkv_rope_forward(x, w, b, 1, 1, 64, **{**kw, name: away})
+
+
 def test_qkv_generic_shapes(gpu):
     g = torch.Generator().manual_seed(23)
     hidden, nq, nkv, hd = 100, 3, 1, 32                     # hidden % 32 != 0, head_dim != 64 -> generic kernel

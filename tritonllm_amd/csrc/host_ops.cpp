@@ -374,12 +374,15 @@ bool heads_of(PyObject* const* a, int64_t total_out, int* nq, int* nkv, int* hd)
 }
 
 // qkv_rope(x, weight, bias, num_q_heads, num_kv_heads, head_dim, yarn, positions, offset, tokens_per_batch, max_context_length,
-//          rotate, mode, out, norm_scale, norm_eps, weight_scale, fuse_norm)
+//          rotate, mode, out, norm_scale, norm_eps, weight_scale, fuse_norm, cos, sin)
+// (the tables are looked at for their device alone: yarn are the parameters that they carry)
 PyObject* qkv_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int nq, nkv, hd;
   int64_t tpb, max_ctx;
   double eps;
-  if (n != 18 || !PyBool_Check(a[17]) || !gpu_tensor(a[0]) || !weight_ok(a[1], a[16]) || !to_i64(a[10], &max_ctx) || !to_f64(a[15], &eps) || !PyBool_Check(a[11])) return none();
+  if (n != 20 || !PyBool_Check(a[17]) || !gpu_tensor(a[0]) || !weight_ok(a[1], a[16]) || !to_i64(a[10], &max_ctx) || !to_f64(a[15], &eps) || !PyBool_Check(a[11])) return none();
+  for (int i : {7, 8, 18, 19})                     // used or not: a tensor of another device is the caller's mistake
+    if (!is_none(a[i]) && !gpu_tensor(a[i])) return none();
   const Tensor &x = tensor(a[0]), &w = tensor(a[1]);
   if (!bf16(x) || x.dim() != 2 || !x.is_contiguous() || x.size(1) != w.size(1) || x.size(0) == 0 || !bias_ok(a[2], w.size(0)) ||
       !heads_of(a + 3, w.size(0), &nq, &nkv, &hd))

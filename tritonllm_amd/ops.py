@@ -367,7 +367,7 @@ def qkv_rope_forward(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
     it is F.linear + split + contiguous + rope_forward of model.py:506-522 in one launch."""
     done = host().qkv_rope(x, weight, bias, num_q_heads, num_kv_heads, head_dim, _yarn_or_tables(yarn, cos, sin), positions, offset,
                            tokens_per_batch, max_context_length, rotate, mode, out, norm_scale, norm_eps, weight_scale,
-                           norm_scale is not None and _norm_fusable("prefill" if mode == "prefill" else "decode", x.shape[0], x.shape[-1], head_dim))
+                           norm_scale is not None and _norm_fusable("prefill" if mode == "prefill" else "decode", x.shape[0], x.shape[-1], head_dim), cos, sin)
     if done is not None:
         return done
     _on_gpu(x, weight, bias, positions, offset, cos, sin, norm_scale, weight_scale)
