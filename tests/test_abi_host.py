@@ -5,6 +5,8 @@ import ctypes as C
 import os
 import pickle
 import re
+import subprocess
+import sys
 import threading
 from itertools import chain, starmap
 
@@ -74,6 +76,22 @@ def test_allocation_gives_up_the_interpreter_lock():
         torch.use_deterministic_algorithms(False)
         scratch_pool.clear()
     assert after > before
+
+
+def test_cpu_buffers_need_no_library():
+    """The scratch pool of other devices is torch alone: no library is loaded for it, and any shape that torch has is one."""
+    code = '''if True:
+        import torch
+        from tritonllm_amd import _lib, scratch_pool
+        _lib.LIB_PATH = _lib.HOST_PATH = "/nowhere.so"
+        a = scratch_pool.get((2, 3), torch.float32, "cpu")
+        assert scratch_pool.get((2, 3), torch.float32, torch.device("cpu")) is a
+        assert scratch_pool.get((1,) * 17, torch.float32, "cpu").dim() == 17
+        assert scratch_pool.stats() == {"num_buffers": 2, "total_bytes": 28}
+        scratch_pool.clear()
+        assert scratch_pool.stats() == {"num_buffers": 0, "total_bytes": 0}
+        '''
+    subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True)
 
 
 def _err():

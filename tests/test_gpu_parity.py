@@ -922,6 +922,13 @@ def test_qkv_rope_refuses_tensors_that_are_not_on_the_gpu(gpu, name, rotate):
         T.qkv_rope_forward(x, w, b, 1, 1, 64, **{**kw, name: away})
 
 
+def test_scratch_pool_shapes_on_the_gpu(gpu):
+    deep = (1,) * 17 + (2,)
+    assert scratch_pool.get(deep, torch.float32, gpu).data_ptr() == scratch_pool.get(deep, torch.float32, gpu).data_ptr()
+    with pytest.raises((TypeError, OverflowError)):              # torch's own error: no such size
+        scratch_pool.get((1 << 70,), torch.float32, gpu)
+
+
 def test_qkv_generic_shapes(gpu):
     g = torch.Generator().manual_seed(23)
     hidden, nq, nkv, hd = 100, 3, 1, 32                     # hidden % 32 != 0, head_dim != 64 -> generic kernel

@@ -116,18 +116,8 @@ std::unordered_map<std::string, Tensor>& pool() {
 }
 
 Tensor pool_get(at::IntArrayRef shape, at::ScalarType dtype, at::Device device) {
-  char buf[16 * 8 + 8];
-  std::string key;
-  if (shape.size() <= 16) {
-    memcpy(buf, shape.data(), shape.size() * 8);
-    size_t n = shape.size() * 8;
-    buf[n++] = static_cast<char>(dtype);
-    buf[n++] = static_cast<char>(device.type());
-    buf[n++] = static_cast<char>(device.index());
-    key.assign(buf, n);
-  } else {
-    return empty(shape, at::TensorOptions().dtype(dtype).device(device));
-  }
+  std::string key(reinterpret_cast<const char*>(shape.data()), shape.size() * 8);
+  for (int v : {static_cast<int>(dtype), static_cast<int>(device.type()), static_cast<int>(device.index())}) key.push_back(static_cast<char>(v));
   auto it = pool().find(key);
   if (it != pool().end()) return it->second;
   const Tensor t = empty(shape, at::TensorOptions().dtype(dtype).device(device));
@@ -143,22 +133,14 @@ Tensor pooled_output(at::IntArrayRef shape, const Tensor& in) {
   return t;
 }
 
+// pool_get(shape tuple, dtype, device)
 PyObject* py_pool_get(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 3 || !PyTuple_Check(a[0]) || !THPDtype_Check(a[1]) || !THPDevice_Check(a[2])) {
-    PyErr_SetString(PyExc_TypeError, "scratch pool: (shape tuple, dtype, device)");
-    return nullptr;
-  }
-  int64_t dims[16];
-  const Py_ssize_t nd = PyTuple_GET_SIZE(a[0]);
-  for (Py_ssize_t i = 0; i < nd; ++i) {
-    if (i >= 16 || !PyLong_Check(PyTuple_GET_ITEM(a[0], i))) {
-      PyErr_SetString(PyExc_TypeError, "scratch pool: a shape is up to 16 integers");
-      return nullptr;
-    }
-    dims[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(a[0], i));
-  }
+  if (n != 3 || !PyTuple_Check(a[0]) || !THPDtype_Check(a[1]) || !THPDevice_Check(a[2])) return none();
+  at::DimVector dims(PyTuple_GET_SIZE(a[0]));
+  for (size_t i = 0; i < dims.size(); ++i)
+    if (!to_i64(PyTuple_GET_ITEM(a[0], i), &dims[i])) return none();
   try {
-    return wrap(pool_get(at::IntArrayRef(dims, nd), reinterpret_cast<THPDtype*>(a[1])->scalar_type, reinterpret_cast<THPDevice*>(a[2])->device));
+    return wrap(pool_get(dims, reinterpret_cast<THPDtype*>(a[1])->scalar_type, reinterpret_cast<THPDevice*>(a[2])->device));
   } catch (const std::exception& e) {
     PyErr_SetString(PyExc_RuntimeError, e.what());
     return nullptr;
