@@ -925,6 +925,8 @@ def test_qkv_rope_refuses_tensors_that_are_not_on_the_gpu(gpu, name, rotate):
 def test_scratch_pool_shapes_on_the_gpu(gpu):
     deep = (1,) * 17 + (2,)
     assert scratch_pool.get(deep, torch.float32, gpu).data_ptr() == scratch_pool.get(deep, torch.float32, gpu).data_ptr()
+    with pytest.raises(torch.OutOfMemoryError):                  # what a caller that frees memory and tries again looks for
+        scratch_pool.get((1 << 45,), torch.float32, gpu)
     with pytest.raises((TypeError, OverflowError)):              # torch's own error: no such size
         scratch_pool.get((1 << 70,), torch.float32, gpu)
 

@@ -134,17 +134,12 @@ Tensor pooled_output(at::IntArrayRef shape, const Tensor& in) {
 }
 
 // pool_get(shape tuple, dtype, device)
-PyObject* py_pool_get(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* pool_buffer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 3 || !PyTuple_Check(a[0]) || !THPDtype_Check(a[1]) || !THPDevice_Check(a[2])) return none();
   at::DimVector dims(PyTuple_GET_SIZE(a[0]));
   for (size_t i = 0; i < dims.size(); ++i)
     if (!to_i64(PyTuple_GET_ITEM(a[0], i), &dims[i])) return none();
-  try {
-    return wrap(pool_get(dims, reinterpret_cast<THPDtype*>(a[1])->scalar_type, reinterpret_cast<THPDevice*>(a[2])->device));
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
-  }
+  return wrap(pool_get(dims, reinterpret_cast<THPDtype*>(a[1])->scalar_type, reinterpret_cast<THPDevice*>(a[2])->device));
 }
 
 PyObject* py_pool_clear(PyObject*, PyObject*) {
@@ -626,7 +621,7 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef kMethods[] = {
     TLLM_OP(rmsnorm), TLLM_OP(embedding), TLLM_OP(embedding_rmsnorm), TLLM_OP(swiglu), TLLM_OP(qkv_rope), TLLM_OP(qkv_rope_cache), TLLM_OP(linear),
     TLLM_OP(out_residual), TLLM_OP(unembedding), TLLM_OP(attention_decode), TLLM_OP(attention),
-    {"pool_get", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_pool_get)), METH_FASTCALL, nullptr},
+    {"pool_get", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<pool_buffer>)), METH_FASTCALL, nullptr},
     {"pool_clear", py_pool_clear, METH_NOARGS, nullptr},
     {"pool_stats", py_pool_stats, METH_NOARGS, nullptr},
     {nullptr, nullptr, 0, nullptr},
