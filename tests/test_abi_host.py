@@ -79,10 +79,11 @@ def test_allocation_gives_up_the_interpreter_lock():
 
 
 def test_cpu_buffers_need_no_library():
-    """The scratch pool of other devices is torch alone: no library is loaded for it, and any shape that torch has is one."""
+    """The scratch pool of other devices is torch alone: no library is loaded for it, and any shape that torch has is one. So is
+    the out-projection of a prompt, F.linear, under torch's tracers as well."""
     code = '''if True:
         import torch
-        from tritonllm_amd import _lib, scratch_pool
+        from tritonllm_amd import OUT, _lib, scratch_pool
         _lib.LIB_PATH = _lib.HOST_PATH = "/nowhere.so"
         a = scratch_pool.get((2, 3), torch.float32, "cpu")
         assert scratch_pool.get((2, 3), torch.float32, torch.device("cpu")) is a
@@ -90,6 +91,13 @@ def test_cpu_buffers_need_no_library():
         assert scratch_pool.stats() == {"num_buffers": 2, "total_bytes": 28}
         scratch_pool.clear()
         assert scratch_pool.stats() == {"num_buffers": 0, "total_bytes": 0}
+        out = OUT(64, 32, device="cpu").requires_grad_(False)
+        out.weight.normal_()
+        out.bias.normal_()
+        x = torch.randn(3, 64).bfloat16()
+        want = torch.nn.functional.linear(x, out.weight, out.bias)
+        for form in (out, torch.fx.symbolic_trace(out), torch.jit.trace(out, (x,))):
+            assert torch.equal(form(x), want)
         '''
     subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True)
 

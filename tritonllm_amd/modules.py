@@ -91,7 +91,7 @@ class OUT(torch.nn.Module):
         return self._weight_fp8, self._weight_scale
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if not torch.compiler.is_compiling():
+        if not torch.compiler.is_compiling() and isinstance(x, torch.Tensor) and x.is_cuda:
             done = host().linear(x, self.weight, self.bias)
             if done is not None:
                 return done
