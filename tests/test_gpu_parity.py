@@ -1282,6 +1282,22 @@ def test_rows_of_a_power_of_two_pitch(gpu, hidden):
         close(T.out_residual_decode_forward(x.to(gpu), w8, b.to(gpu), zero(), ws).view(rows, 1040), O.linear_ref(x[:, 0], O.dequant_fp8_ref(w8.cpu(), ws.cpu()), b))
 
 
+@pytest.mark.parametrize("hidden,rows,vocab,fp8", [(4096, 8, 32000, False), (2048, 1, 200000, False), (2048, 8, 32000, True),
+                                                   (4096, 8, 32000, True), (4096, 12, 32000, False), (2880, 8, 32000, False)])
+def test_equal_rows_have_equal_logits(gpu, hidden, rows, vocab, fp8):
+    """Two equal rows of the weight give the same number whichever workgroups they fall to (a pitch of a multiple of 4 KB: where
+    the walk over K does not begin at 0 everywhere), so that a caller's argmax over the logits sees a tie, as the argmax op does."""
+    g = torch.Generator(device=gpu).manual_seed(hidden + rows)
+    x = torch.randn(rows, 1, hidden, device=gpu, generator=g).bfloat16()
+    w = (0.02 * torch.randn(vocab // 2, hidden, device=gpu, generator=g)).bfloat16()
+    w, ws = ops.quantize_fp8_rows(w) if fp8 else (w, None)
+    w = torch.cat((w.view(torch.uint8), w.view(torch.uint8))).view(w.dtype)
+    ws = torch.cat((ws, ws)) if fp8 else None
+    logits = T.unembedding_decode_forward(x, w, ws)[:, 0]
+    assert torch.equal(logits[:, :vocab // 2], logits[:, vocab // 2:])
+    assert (T.unembedding_decode_argmax_forward(x, w, ws) < vocab // 2).all()
+
+
 @pytest.mark.parametrize("rows,vocab,hidden", [(17, 3001, 2880), (32, 140000, 2880), (33, 70001, 2880), (50, 4096, 2880), (64, 9000, 2880),
                                                 (24, 5000, 128), (32, 5000, 192), (29, 5000, 1024), (20, 270000, 128)])
 def test_unembedding_more_than_16_rows_one_pass_over_the_weight(gpu, rows, vocab, hidden):

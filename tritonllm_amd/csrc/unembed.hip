@@ -41,9 +41,17 @@ __host__ __device__ constexpr int unembed_xrow(int hidden) { return hidden * 2 +
 // the pair's first row while they lie below `hidden` and to its second row from there on -- two accumulator tiles, the
 // K offset into the activations chosen per MFMA. A lane ends up with the logits of rows 2p and 2p + 1: one 4-byte store,
 // whole 128-byte lines per wavefront. (A bare read in this pattern: 86 us for the 580 MB; in 192-byte row pieces: 96-98.)
-template <int XR, int UNW, int KS, int UD, bool W8, bool ARGMAX, bool SR = false>
+// PIECES: rows whose pitch is a multiple of 4 KB all begin on the same memory channels, and workgroups that walk K in step
+// ask for the same half of them at a time. There, half of the workgroups begin a tile 2 KB into its rows and come back for
+// those at its end (us, in step -> so; in brackets a start of its own for every few workgroups: 8 rows, 4096 wide 285 -> 252 (247),
+// 2048 148 -> 132 (128), fp8 155 -> 134 (131) and 83 -> 69 (72); dealt by another bit of the workgroup's number 252 - 300, 1 KB into
+// the rows 264, 4 KB 279). The two pieces of K are summed apart and added last, in either order the same number: equal rows
+// of the weight have equal logits whichever workgroup they fall to, so that a caller's argmax sees ties as ties. Other
+// pitches spread by themselves (2880 176.8 and 174.6, 5120 304 and 309).
+template <int XR, int UNW, int KS, int UD, bool W8, bool ARGMAX, bool SR = false, bool PIECES = false>
 __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
   static_assert(!SR || (W8 && KS == 128), "pairs of rows: fp8 weight, 128 bytes per pair and step");
+  static_assert(!PIECES || !ARGMAX, "the argmax form walks K in step");
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m = lane & 31, h = lane >> 5;
@@ -80,13 +88,10 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
   const int my_tiles = full_rounds + (tile_of(full_rounds) < ntiles ? 1 : 0);
   const int gw = wave * nwg + wg;                             // this wavefront's number (its slot in the argmax workspace)
   const int total = my_tiles * nsteps;                        // steps of the whole stream
-  // The step of a tile with which this workgroup's wavefronts begin; they go round from there. Rows whose pitch is a multiple of
-  // 4 KB all begin on the same memory channels, and workgroups that walk K in step ask for the same few of them at a time: 8 rows
-  // of width 4096 282 -> 249 us, 2048 146 -> 128 (a start of its own for every wavefront 252 and 131). Other pitches spread by
-  // themselves (2880 176.8 and 174.6, 5120 304 and 309): in step. So is the argmax form, whose rule for ties wants equal
-  // rows to have equal sums.
-  const int pitch = SR || !W8 ? 2 * a.hidden : a.hidden;
-  const int rot = !ARGMAX && pitch % 4096 == 0 ? ((wg >> 3) * 2) % nsteps : 0;
+  // The steps of a tile, [k0, k1) first; PIECES: [k2, k3) after them.
+  constexpr int PIECE = 2048 / (SR || W8 ? KS : 2 * KS);
+  const bool late = PIECES && (wg & 64);
+  const int k0 = late ? PIECE : 0, k1 = PIECES && !late ? PIECE : nsteps, k2 = late ? 0 : PIECE, k3 = late ? PIECE : nsteps;
 
   // One load instruction moves 1 KB; the 32 x (KS elements) block of a step is dealt to the lanes as 16-byte
   // chunks in row-major order, so consecutive lanes cover consecutive bytes of a row (KS = 64: eight lanes per
@@ -104,7 +109,7 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
 
   bf16x8 buf[UD][LPS];
   const bf16x8* lp[LPS];                                      // load cursor: row bases of the tile being requested
-  int l_round = 0, l_tile = tile_of(0), l_step = rot, l_count = 0;
+  int l_round = 0, l_tile = tile_of(0), l_step = k0, l_end = k1, l_count = 0;
 #pragma unroll
   for (int i = 0; i < LPS; ++i) lp[i] = row_base(my_tiles > 0 ? l_tile : 0, i);
   // Unconditional on purpose (a load under a branch makes the compiler wait for it where the paths join): past
@@ -119,8 +124,14 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
     }
     if (l_count + 1 < total) {
       ++l_count;
-      if (++l_step == nsteps) l_step = 0;
-      if (l_step == rot) {
+      if (++l_step == l_end) {
+        if (PIECES && l_end == k1) {
+          l_step = k2;
+          l_end = k3;
+          return;
+        }
+        l_step = k0;
+        l_end = k1;
         l_tile = tile_of(++l_round);
 #pragma unroll
         for (int i = 0; i < LPS; ++i) lp[i] = row_base(l_tile < ntiles ? l_tile : ntiles - 1, i);
@@ -144,17 +155,18 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = acc2[v] = 0.f;
   constexpr int NB = XR / 2;                                  // accumulator registers that carry batch rows: row(v) = 8*(v>>2) + 4*h + (v&3)
-  float best[NB];
+  float best[NB], piece[NB];                                  // piece: sums over the tile's first piece of K
   int best_i[NB];
 #pragma unroll
   for (int v = 0; v < NB; ++v) {
     best[v] = -3.0e38f;
     best_i[v] = 0x7fffffff;
+    piece[v] = 0.f;
   }
 
   const unsigned char* xfrag = xs + (m & (XR - 1)) * xrow_b + h * 16;   // activations on M: tile rows >= XR repeat, never stored
   const unsigned char* wfrag = patch + m * UPROW + h * 16;              // vocabulary rows on N
-  int c_round = 0, c_tile = tile_of(0), c_step = rot;
+  int c_round = 0, c_tile = tile_of(0), c_step = k0, c_end = k1;
   for (int g0 = 0; g0 < total; g0 += UD) {
 #pragma unroll
     for (int d = 0; d < UD; ++d) {
@@ -215,8 +227,22 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        if (++c_step == nsteps) c_step = 0;
-        if (SR && c_step == rot) {                            // tile finished: lane owns vocabulary rows 2 p and 2 p + 1, p = c_tile*32 + m
+        bool finished = ++c_step == c_end;
+        if (PIECES && finished) {                             // uniform: a piece
+          finished = c_end == k3;
+          c_step = finished ? k0 : k2;
+          c_end = finished ? k1 : k3;
+#pragma unroll
+          for (int r = 0; r < NB; ++r) {
+            acc[r] += piece[r];
+            piece[r] = finished ? 0.f : acc[r];
+          }
+          if (!finished) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+          }
+        }
+        if (SR && finished) {                            // tile finished: lane owns vocabulary rows 2 p and 2 p + 1, p = c_tile*32 + m
           const int v0 = 2 * (c_tile * 32 + m), v1 = v0 + 1;  // the vocabulary is even here: both are inside it, or neither
           const float sc0 = a.w_scale[v0 < a.vocab ? v0 : a.vocab - 2], sc1 = a.w_scale[v1 < a.vocab ? v1 : a.vocab - 1];
 #pragma unroll
@@ -247,9 +273,10 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
           }
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[r] = acc2[r] = 0.f;
+          if (!PIECES) c_step = 0;
           c_tile = tile_of(++c_round);
         }
-        if (!SR && c_step == rot) {                           // tile finished: lane owns vocabulary row c_tile*32 + m
+        if (!SR && finished) {                                // tile finished: lane owns vocabulary row c_tile*32 + m
           const int v = c_tile * 32 + m;
           float sc = 1.f;
           if constexpr (W8) sc = a.w_scale[v < a.vocab ? v : a.vocab - 1];
@@ -268,6 +295,7 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
           }
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+          if (!PIECES) c_step = 0;
           c_tile = tile_of(++c_round);
         }
       }
@@ -645,20 +673,23 @@ int unembed_launch(const char* who, const UnembedArgs& a, bool w8, hipStream_t s
   const bool pairs16 = unembed_pairs16(a.rows, w8, a.hidden, a.vocab);
   const size_t smem = pairs ? smem_pairs : (pairs16 ? smem_pairs16 : unembed_smem(xr, w8, a.hidden));
   const dim3 grid(kUnembedGrid, (unsigned)((a.rows + xr - 1) / xr));
-#define TLLM_UNEMBED(XR, NW, KS, UD, W8F, ...)                                                                              \
+  const bool pieces = !ARGMAX && (a.hidden * (w8 && !pairs && !pairs16 ? 1 : 2)) % 4096 == 0;   // (such a width is no multiple of 192 that fits the LDS)
+#define TLLM_UNEMBED(XR, NW, KS, UD, W8F, SR)                                                                               \
   do {                                                                                                                      \
-    auto kern = unembed_kernel<XR, NW, KS, UD, W8F, ARGMAX, ##__VA_ARGS__>;                                                 \
+    auto kern = unembed_kernel<XR, NW, KS, UD, W8F, ARGMAX, SR>;                                                            \
+    if constexpr (!ARGMAX && KS != 192)                                                                                     \
+      if (pieces) kern = unembed_kernel<XR, NW, KS, UD, W8F, false, SR, true>;                                              \
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
     TLLM_REQUIRE(e == hipSuccess, TLLM_E_LAUNCH, "%s: cannot raise LDS limit: %s", who, hipGetErrorString(e));              \
     hipLaunchKernelGGL(kern, grid, dim3(NW * 64), smem, st, a);                                                             \
   } while (0)
   if (pairs16) TLLM_UNEMBED(16, 6, 128, 2, true, true);
   else if (pairs) TLLM_UNEMBED(8, 8, 128, 2, true, true);          // steps in flight 1 / 2 / 3 / 4: 122 / 99 / 105 / 107 us; 12 wavefronts x 3: 103, 10 x 2: 103, 6 x 2: 115
-  else if (xr == 8 && !w8) TLLM_UNEMBED(8, 10, 64, 3, false);
-  else if (xr == 8 && unembed_ks(8, true, a.hidden) == 192) TLLM_UNEMBED(8, 8, 192, 2, true);
-  else if (xr == 8) TLLM_UNEMBED(8, 8, 64, 4, true);
-  else if (w8) TLLM_UNEMBED(16, 8, 64, 4, true);
-  else TLLM_UNEMBED(16, 8, 64, 3, false);
+  else if (xr == 8 && !w8) TLLM_UNEMBED(8, 10, 64, 3, false, false);
+  else if (xr == 8 && unembed_ks(8, true, a.hidden) == 192) TLLM_UNEMBED(8, 8, 192, 2, true, false);
+  else if (xr == 8) TLLM_UNEMBED(8, 8, 64, 4, true, false);
+  else if (w8) TLLM_UNEMBED(16, 8, 64, 4, true, false);
+  else TLLM_UNEMBED(16, 8, 64, 3, false, false);
 #undef TLLM_UNEMBED
   return check_launch(who);
 }
