@@ -264,6 +264,9 @@ def test_attention_decode_shape_planning():
     assert hpw(2, 8, 16384, 0) == 0
     assert hpw(1, 8, 131072, 0) == 0
     assert hpw(64, 8, 131072, 128) == 0 and splits(64, 8, 131072, 128) == 1      # a sliding window bounds the context
+    # more than eight KV heads: where one split fewer is as good but leaves CUs without a workgroup, the splits stay
+    assert [(hpw(b, n, c, 0), splits(b, n, c, 0)) for b, n, c in ((33, 16, 2048), (49, 16, 4096), (24, 32, 2048), (33, 24, 3000))] == [(4, 2)] * 4
+    assert (hpw(38, 16, 3000, 0), splits(38, 16, 3000, 0)) == (8, 3)
     for b in (1, 3, 8, 100):
         for ctx in (1, 127, 128, 129, 5000, 131072):
             s = splits(b, 8, ctx, 0)

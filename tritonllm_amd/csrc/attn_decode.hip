@@ -436,7 +436,8 @@ constexpr int kUnsplitQuads = 8192, kUnsplitPairs = 4096; // longest contexts th
 // Splits for `units` streams: attn_splits_for's answer, unless one split fewer per unit-row of workgroups spreads the
 // work more evenly -- 24 units x 11 splits are 264 workgroups, eight CUs with two of them while the rest have one,
 // where 24 x 10 leave sixteen CUs idle and everybody done 1.8 times sooner. Compared by the keys the busiest CU walks.
-static int attn_pick_splits(int64_t units, int ctx, int shift) {
+// `need`: on a tie, the fewest workgroups that one split fewer may leave.
+static int attn_pick_splits(int64_t units, int ctx, int shift, int64_t need = 0) {
   const int s0 = attn_splits_for(attn_fill(units), ctx, shift);
   const int by_work = ((ctx - 1) >> shift) + 1;
   int s1 = static_cast<int>(256 / (units > 0 ? units : 1));
@@ -448,7 +449,8 @@ static int attn_pick_splits(int64_t units, int ctx, int shift) {
     const int64_t keys = (((ctx + s - 1) / s) + 31) & ~31;
     return rounds * keys;
   };
-  return busiest(s1) <= busiest(s0) ? s1 : s0;                // a tie: fewer records to fold, or no second launch
+  if (busiest(s1) == busiest(s0)) return units * s1 >= need ? s1 : s0;   // a tie: fewer records to fold, or no second launch
+  return busiest(s1) < busiest(s0) ? s1 : s0;
 }
 
 static AttnPlan attn_plan(int64_t batch, int n_kv_heads, int64_t n_kv_ctx, int window) {
@@ -461,22 +463,26 @@ static AttnPlan attn_plan(int64_t batch, int n_kv_heads, int64_t n_kv_ctx, int w
     if (ctx >= 256 && ctx <= kUnsplitPairs && pairs > 128 && pairs <= 256 && (pairs > 168 || ctx <= 1280)) return {2, 2, 1, 1, kRowsKeysShift};
   }
   if (ctx > 128 && streams <= 128 && ctx <= (streams >= 64 ? 800 : 512)) return {1, 8, 1, 1, kHeadKeysShift};
-  // eight or four KV heads per workgroup: whichever fills the machine with the longest splits (ties: the wider one)
+  // eight or four KV heads per workgroup: whichever fills the machine with the longest splits (ties: the wider one). If neither
+  // does, and that is because one split fewer was as good (more than eight KV heads), with the splits that it had: 16 heads, B = 49
+  // at 2048 HEAD 97 us, so 70; 24 heads, B = 33 at 4096 179 and 137; 12 heads, B = 44 at 1400 as good either way
+  const int64_t need = streams > 256 ? 208 : 224;
   AttnPlan best{0, 0, 0, 0, 0};
   int64_t best_keys = 0;
-  for (int hpw = 8; hpw >= 4; hpw >>= 1) {
-    if (n_kv_heads % hpw != 0) continue;
-    const int64_t units = batch * (n_kv_heads / hpw);
-    const int s = attn_pick_splits(units, static_cast<int>(ctx), kRowsKeysShift);
-    const int64_t keys = ctx / s;
-    // splits of 256-511 keys too, when there are not too many of them and the HEAD shape would need its second launch as
-    // well or is past what one launch of it is good for
-    const bool long_enough = keys >= 512 || ((head_splits > 1 || ctx >= 1400) && ((keys >= 256 && s <= 28) || (keys >= 320 && s <= 32)));
-    if (units * s >= (streams > 256 ? 208 : 224) && long_enough && keys > best_keys) {
-      best = {hpw, 1, s, s, kRowsKeysShift};              // (the kernels' own evaluation starts from the chosen count)
-      best_keys = keys;
+  for (int keep = 0; keep < 2 && !best.hpw; ++keep)
+    for (int hpw = 8; hpw >= 4; hpw >>= 1) {
+      if (n_kv_heads % hpw != 0) continue;
+      const int64_t units = batch * (n_kv_heads / hpw);
+      const int s = attn_pick_splits(units, static_cast<int>(ctx), kRowsKeysShift, keep ? need : 0);
+      const int64_t keys = ctx / s;
+      // splits of 256-511 keys too, when there are not too many of them and the HEAD shape would need its second launch as
+      // well or is past what one launch of it is good for
+      const bool long_enough = keys >= 512 || ((head_splits > 1 || ctx >= 1400) && ((keys >= 256 && s <= 28) || (keys >= 320 && s <= 32)));
+      if (units * s >= need && long_enough && keys > best_keys) {
+        best = {hpw, 1, s, s, kRowsKeysShift};            // (the kernels' own evaluation starts from the chosen count)
+        best_keys = keys;
+      }
     }
-  }
   if (best_keys < 512 && head_splits > 1 && streams >= 64 && n_kv_heads % 4 == 0 && n_kv_heads <= 8) {
     const int s = attn_pick_splits(streams / 2, static_cast<int>(ctx), kRowsKeysShift);
     if (s > 1 && streams / 2 * s >= 208 && ctx / s > 256 && ctx / s < 512) return {2, 2, s, s, kRowsKeysShift};
