@@ -271,3 +271,15 @@ def test_attention_decode_shape_planning():
         for ctx in (1, 127, 128, 129, 5000, 131072):
             s = splits(b, 8, ctx, 0)
             assert 1 <= s <= 64 and (s == 1 or ctx >= 128 * (s - 1))
+
+
+def test_attention_prefill_shape_planning():
+    """Key blocks are shared out between wavefronts where the launch is small and the walk long enough to pay for the meeting."""
+    groups = _lib.lib().tllm_attention_prefill_key_groups
+    assert [groups(1, n, n, 8, 8, 0) for n in (1, 16, 64)] == [1, 1, 1]              # one block: nothing to share
+    assert [groups(b, 64, 64, 8, 8, w) for b in (4, 8) for w in (0, 128)] == [1] * 4
+    assert groups(1, 97, 97, 8, 8, 0) == 2 and groups(4, 128, 128, 8, 8, 0) == 1     # two blocks: at one workgroup per CU
+    assert [groups(1, n, n, 8, 8, 128) for n in (400, 512)] == [1, 1]                # a window's three blocks at two per CU
+    assert [groups(1, n, n, 8, 8, 0) for n in (300, 400, 512)] == [2, 2, 2]
+    assert [groups(1, 97, 1597, 8, 8, w) for w in (0, 128)] == [4, 4]
+    assert groups(1, 777, 777, 8, 8, 0) == 1

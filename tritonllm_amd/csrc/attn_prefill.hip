@@ -435,6 +435,27 @@ static int launch_prefill(const AttnPrefillArgs& a, hipStream_t st) {
   return check_launch("attention_prefill");
 }
 
+// Workgroup shape, by how many workgroups the launch has. 128 queries x 2 heads (two heads per wavefront) as soon as that
+// gives every CU two of them; below that 64 queries x 2 heads with one head per wavefront: twice the workgroups, and the
+// longest of them -- it sets the time of so small a launch -- takes about half as long per key block. When even 64
+// queries x 1 head are at most two per CU, the wavefronts share the key blocks out as well: two groups of two
+// wavefronts, or four (one workgroup of eight wavefronts per CU), us before -> now:
+//   97 queries behind 1500 keys 27.0 -> 16.1 (two groups 18.3), with a window of 128 9.3 -> 6.9; 16 behind 4000 58.3 -> 29.9;
+//   256 behind 2000 37.4 -> 20.3 (23.8); 400 queries 11.3 -> 9.7; 500 behind 1000 27.4 -> 21.3; 512 behind 4000 67.9 -> 56.1
+//   (from three workgroups per CU on the longer walk is hidden by the others: 777 queries 17.8, shared out 19.1).
+// A walk has to be long enough to pay for the meeting at its end: more than one block (16 or 64 queries alone 5.5 us, shared
+// out 6.1; two blocks, 97 queries, 6.6 and 6.3), and at two workgroups per CU more than three (eight prompts of 64 6.2 and
+// 7.5, four of 128 6.9 and 7.6, window of 128: 400 queries 8.2 and 9.4, 512 8.3 and 9.5; five blocks, 300 queries, 9.4 and 8.9).
+// Odd group sizes: 128 x 1.
+extern "C" int tllm_attention_prefill_key_groups(int64_t batch, int64_t n_q, int64_t n_kv_ctx, int n_kv_heads, int group, int window) {
+  const int64_t wgs64 = (n_q + 63) / 64 * batch * n_kv_heads * group;
+  const int64_t span = window > 0 && window < n_kv_ctx - n_q ? n_q + window : n_kv_ctx;     // most keys there can be to visit
+  int64_t walk = (n_kv_ctx + PBN - 1) / PBN;                                                // blocks of a workgroup of 64 queries
+  if (window > 0 && (static_cast<int64_t>(window) + 126) / PBN < walk) walk = (static_cast<int64_t>(window) + 126) / PBN;
+  if (wgs64 <= 256 && span > 192) return 4;
+  return wgs64 <= 512 && walk > (wgs64 <= 256 ? 1 : 3) ? 2 : 1;
+}
+
 extern "C" int tllm_attention_prefill_bf16(const void* q, const void* k, const void* v, const void* sinks, void* out, int64_t q_batch_stride,
                                            int64_t q_token_stride, int64_t out_batch_stride, int64_t out_token_stride,
                                            int64_t kv_batch_stride, int64_t kv_token_stride, int64_t batch, int64_t n_q, int64_t n_kv_ctx,
@@ -479,22 +500,13 @@ extern "C" int tllm_attention_prefill_bf16(const void* q, const void* k, const v
   a.group = group;
   a.window = window;
   a.sm_scale = sm_scale;
-  // Workgroup shape, by how many workgroups the launch has. 128 queries x 2 heads (two heads per wavefront) as soon as
-  // that gives every CU two of them; below that 64 queries x 2 heads with one head per wavefront: twice the workgroups, and the
-  // longest of them -- it sets the time of so small a launch -- takes about half as long per key block. When even 64
-  // queries x 1 head are at most two per CU, the wavefronts share the key blocks out as well: two groups of two
-  // wavefronts, or four (one workgroup of eight wavefronts per CU), us before -> now:
-  //   97 queries behind 1500 keys 27.0 -> 16.1 (two groups 18.3), with a window of 128 9.3 -> 6.9; 16 behind 4000 58.3 -> 29.9;
-  //   256 behind 2000 37.4 -> 20.3 (23.8); 400 queries 11.3 -> 9.7; 500 behind 1000 27.4 -> 21.3; 512 behind 4000 67.9 -> 56.1
-  //   (from three workgroups per CU on the longer walk is hidden by the others: 777 queries 17.8, shared out 19.1).
-  // Odd group sizes: 128 x 1.
   const int nh = group % 2 == 0 ? 2 : 1;
-  const int64_t wgs64 = (n_q + 63) / 64 * batch * n_heads, wgs128 = (n_q + 127) / 128 * batch * n_kv_heads * (group / nh);
-  const int64_t span = window > 0 && window < n_kv_ctx - n_q ? n_q + window : n_kv_ctx;     // most keys there can be to visit
+  const int64_t wgs128 = (n_q + 127) / 128 * batch * n_kv_heads * (group / nh);
   TLLM_REQUIRE(batch < (1ll << 24) && wgs128 < (1ll << 31), TLLM_E_SHAPE, "attention_prefill: %lld workgroups are too many for one launch", (long long)wgs128);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (wgs64 <= 256 && span > 192) return launch_prefill<1, 2, 4, 8>(a, st);
-  if (wgs64 <= 512) return launch_prefill<1, 2, 2, 4>(a, st);
+  const int key_groups = tllm_attention_prefill_key_groups(batch, n_q, n_kv_ctx, n_kv_heads, group, window);
+  if (key_groups == 4) return launch_prefill<1, 2, 4, 8>(a, st);
+  if (key_groups == 2) return launch_prefill<1, 2, 2, 4>(a, st);
   if (nh == 2 && wgs128 < 512) return launch_prefill<1, 2, 1, 4>(a, st);
   if (nh == 2) return launch_prefill<2, 4, 1, 4>(a, st);
   return launch_prefill<1, 4, 1, 4>(a, st);
