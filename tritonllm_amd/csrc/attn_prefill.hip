@@ -143,15 +143,16 @@ __global__ __launch_bounds__(NW * 64, KG > 2 ? NW / 4 : NW / 2) void attn_prefil
   // to one of the two.
   const int dma_first = wave * DPT & 15;          // the wavefront's first instruction of the block's sixteen: eight of K, eight of V
   const int dma_block = KG == 1 ? 0 : wave * DPT >> 4;
+  const bool dma_v = dma_first >= 8;              // they all belong to one of the two tiles
+  const bf16* const dma_src = dma_v ? vp : kp;
   int dma_row[DPT], dma_col[DPT];
   const bf16* dma_ptr[DPT];                       // the lane's chunk of its row of key block 0
 #pragma unroll
   for (int j = 0; j < DPT; ++j) {
-    const bool dma_v = dma_first + j >= 8;
     const int row = ((dma_first + j) & 7) * 8 + (lane >> 3);
     dma_row[j] = row;
     dma_col[j] = ((lane & 7) ^ (dma_v ? v_swizzle(row) : ((row >> 1) & 7))) * 8;
-    dma_ptr[j] = (dma_v ? vp : kp) + static_cast<int64_t>(row) * a.kv_ts + dma_col[j];
+    dma_ptr[j] = dma_src + static_cast<int64_t>(row) * a.kv_ts + dma_col[j];
   }
   const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem)) + dma_first * 1024;
   const int64_t blk_stride = static_cast<int64_t>(PBN) * a.kv_ts;
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(NW * 64, KG > 2 ? NW / 4 : NW / 2) void attn_prefil
       } else {
         int key = blk * PBN + dma_row[j];
         key = key < key_max ? key : key_max;
-        g = (dma_first + j >= 8 ? vp : kp) + static_cast<int64_t>(key) * a.kv_ts + dma_col[j];
+        g = dma_src + static_cast<int64_t>(key) * a.kv_ts + dma_col[j];
       }
       const unsigned m0v = lds0 + stage * PSTAGE + j * 1024;
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0v), "v"(g) : "memory", "m0");
