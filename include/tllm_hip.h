@@ -211,6 +211,12 @@ int tllm_qkv_rope_prefill_bf16(const void* x, const void* W, const void* b,
                                int64_t rows, int64_t hidden, int n_q_heads, int n_kv_heads, int head_dim,
                                const TllmRope* rope, void* stream);
 
+/* Diagnostics: the GEMM tile (rows << 16 | columns) that tllm_qkv_rope_prefill_bf16 (prefill != 0) or
+ * tllm_qkv_rope_decode_bf16 takes for aligned operands of these sizes, 0 where it is another kernel's; and
+ * the one that tllm_linear_bf16 takes. No counterpart in the reference. */
+int tllm_qkv_gemm_tile(int prefill, int64_t rows, int64_t hidden, int n_q_heads, int n_kv_heads, int head_dim);
+int tllm_linear_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim);
+
 /* out[r, n] = sum_k x[r, k] * W[n, k] + b[n] for a prompt's rows (bf16 in, fp32 accumulate, one RNE to bf16): what OUT.forward
  * is, model.py:196-197. x [rows, in_dim], W [out_dim, in_dim] dense and 16-byte aligned, b [out_dim] or NULL, out with
  * out_row_stride elements between rows. in_dim a multiple of 64, out_dim of 16. */

@@ -114,6 +114,16 @@ void launch_qkv_generic(const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& f
   hipLaunchKernelGGL(qkv_generic_kernel, dim3((unsigned)heads, gy), dim3(256), 0, st, a, ra, fr);
 }
 
+bool qkv_decode_tiles(int64_t rows, int64_t hidden, int heads, int head_dim) {
+  const int64_t cols = static_cast<int64_t>(heads) * 64;
+  if (rows <= 32 || head_dim != 64 || hidden % 64 != 0 || cols * hidden * 2 >= (1ll << 32)) return false;
+  // the rows kernel takes 6.4 us and 1.4 per block of 16 rows (97 rows 15.9, 128 rows 17.5, 256 rows 26.6): from about a
+  // hundred rows a GEMM tile is ahead of it (97 rows 16.1, 128 rows 16.2, 256 rows 21.2)
+  if (hidden == 2880) return tile_gemm_ns(rows, cols, hidden) < 6400 + 1400 * ((rows + 15) / 16);
+  // Beyond 32 rows the general kernel reads the weight a third time (hidden 4096: 40 rows 22.7 us).
+  return true;
+}
+
 }  // namespace tllm
 
 using namespace tllm;
@@ -131,12 +141,9 @@ static int launch_decode_2880(const char* what, QkvArgs& a, const RopeArgs& ra, 
   // that keeps the weight and streams the rows past it, so that the weight is read once whatever the row count
   const unsigned col_groups = (unsigned)((heads * 32 + 9) / 10);
   const bool use_rows = rows > 32;                        // (at 17..32 rows the 32-row kernel is 0.7-1.6 us faster: it overlaps the two streams)
-  // the rows kernel takes 6.4 us and 1.4 per block of 16 rows (97 rows 15.9, 128 rows 17.5, 256 rows 26.6): from about a
-  // hundred rows a GEMM tile is ahead of it (97 rows 16.1, 128 rows 16.2, 256 rows 21.2)
-  const int64_t rows_ns = 6400 + 1400 * ((rows + 15) / 16);
   if (rows <= 8) launch_qkv_decode_r8(8, norm, emb, w8, dim3(col_groups, 1), st, a, ra, fr);
   else if (rows <= 16 && (norm != 0 || emb)) launch_qkv_decode_r8(16, norm, emb, w8, dim3(col_groups, 1), st, a, ra, fr);
-  else if (use_rows && !w8 && tile_gemm_ns(rows, static_cast<int64_t>(heads) * 64, 2880) < rows_ns) return launch_tile_gemm_qkv(what, a, ra, fr, st);
+  else if (use_rows && !w8 && qkv_decode_tiles(rows, 2880, heads, 64)) return launch_tile_gemm_qkv(what, a, ra, fr, st);
   else if (use_rows) launch_qkv_decode_rows(w8, dim3(col_groups, 1), st, a, ra, fr);
   else {
     const int64_t chunks = (rows + 31) / 32;
@@ -277,8 +284,7 @@ extern "C" int tllm_qkv_rope_decode_bf16(const void* x, const void* W, const voi
   const bool out4 = (reinterpret_cast<uintptr_t>(q) % 4 == 0) && (reinterpret_cast<uintptr_t>(k) % 4 == 0) &&
                     (reinterpret_cast<uintptr_t>(v) % 4 == 0) && q_row_stride % 2 == 0 && k_row_stride % 2 == 0 &&
                     v_row_stride % 2 == 0 && kv_slot_stride % 2 == 0;
-  // Beyond 32 rows the general kernel reads the weight a third time (hidden 4096: 40 rows 22.7 us).
-  if (rows > 32 && head_dim == 64 && hidden % 64 == 0 && aligned16(x) && aligned16(W) && static_cast<int64_t>(heads) * 64 * hidden * 2 < (1ll << 32))
+  if (aligned16(x) && aligned16(W) && qkv_decode_tiles(rows, hidden, heads, head_dim))
     return launch_tile_gemm_qkv("qkv_rope_decode", a, ra, fr, st);
   // (the general kernel addresses a head's rows of the weight with 32-bit byte offsets)
   if (mfma_ok && out4 && static_cast<int64_t>(head_dim) * hidden * 2 < (1ll << 31))

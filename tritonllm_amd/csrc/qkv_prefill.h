@@ -52,7 +52,15 @@ __device__ __forceinline__ float2 rope_cos_sin_at(const RopeArgs& r, const YarnF
 // Tiles of 64 x 32 .. 128 x 256 (tile_gemm.hip). QKV + bias + rotary: hidden % 64 == 0, head_dim 64, x and W 16-byte aligned,
 // weight below 4 GiB.
 int launch_tile_gemm_qkv(const char* what, const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& fr, hipStream_t st);
-// What the host expects such a launch to take for `rows` rows, `cols` output columns and K = k, in ns.
+struct TileSize {
+  int bm, bn;
+};
+// The tile that such a launch takes for `rows` rows, `cols` output columns and K = k, and what the host expects it to take, in ns.
+TileSize tile_gemm_pick(int64_t rows, int64_t cols, int64_t k, int64_t* ns);
 int64_t tile_gemm_ns(int64_t rows, int64_t cols, int64_t k);
+
+// Whether tllm_qkv_rope_decode_bf16 and tllm_qkv_rope_prefill_bf16 take GEMM tiles for aligned operands of these sizes.
+bool qkv_decode_tiles(int64_t rows, int64_t hidden, int heads, int head_dim);
+bool qkv_prefill_tiles(int64_t rows, int64_t hidden, int heads, int head_dim);
 
 }  // namespace tllm

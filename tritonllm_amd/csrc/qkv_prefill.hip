@@ -658,6 +658,36 @@ __global__ __launch_bounds__(512) void qkv_prefill_kernel256(QkvArgs a, RopeArgs
   }
 }
 
+namespace {
+// the kernels address a tile's rows and the weight with 32-bit byte offsets
+bool prefill_fits(int64_t hidden, int heads, int head_dim) {
+  return head_dim == 64 && hidden % BK == 0 && static_cast<int64_t>(heads) * 64 * hidden * 2 < (1ll << 32) && 256 * hidden * 2 < (1ll << 32);
+}
+
+// Tile height by a cost model: a round of 128-token tiles over the 256 CUs takes ~57 us, a round of 256-token tiles ~105 us
+// (both per 45 slices of K); whichever needs less in total. T = 2048 is one round of 128s; anything that would need a
+// second round of 128s is one round of 256s instead, T = 8192 two rounds of 256s instead of four of 128s.
+int prefill_tile_height(int64_t rows, int heads, int64_t* rounds128, int64_t* rounds256) {
+  const int64_t tn = (heads + HPT - 1) / HPT;
+  const int64_t r128 = (((rows + 127) / 128) * tn + 255) / 256, r256 = (((rows + 255) / 256) * tn + 255) / 256;
+  if (rounds128) *rounds128 = r128;
+  if (rounds256) *rounds256 = r256;
+  return r256 * 105 < r128 * 57 ? 256 : 128;
+}
+}  // namespace
+
+// Up to about 1500 rows (of 5120 columns) smaller tiles fill the machine in less than a round of these (tile_gemm.hip: 1536
+// rows 50.9 against 57 us, 999 rows 39.8 against 49.1, 97 rows 16.1 against 51).
+bool qkv_prefill_tiles(int64_t rows, int64_t hidden, int heads, int head_dim) {
+  if (!prefill_fits(hidden, heads, head_dim)) return false;
+  int64_t rounds128, rounds256;
+  const int BM = prefill_tile_height(rows, heads, &rounds128, &rounds256);
+  // (a single round of 256s rarely fills the CUs and takes 83 - 92 us then: 2900 rows 86.5, where two rounds of 128 x 256 take
+  // 91.3; up to 2816 rows two rounds of 128 x 224 are ahead, 2600 rows 82.3 against 84.6)
+  const int64_t here_ns = (BM == 128 ? rounds128 * 57000 : rounds256 == 1 ? 90000 : rounds256 * 105000) * (hidden / BK) / 45;
+  return tile_gemm_ns(rows, static_cast<int64_t>(heads) * 64, hidden) < here_ns;
+}
+
 }  // namespace tllm
 
 using namespace tllm;
@@ -675,26 +705,13 @@ extern "C" int tllm_qkv_rope_prefill_bf16(const void* x, const void* W, const vo
   a.bias = (const bf16*)b;
   if (rows == 0) return TLLM_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // the kernels address a tile's rows and the weight with 32-bit byte offsets
-  const bool fast = head_dim == 64 && hidden % BK == 0 && aligned16(x) && aligned16(W) &&
-                    static_cast<int64_t>(n_q_heads + 2 * n_kv_heads) * 64 * hidden * 2 < (1ll << 32) && 256 * hidden * 2 < (1ll << 32);
-  if (!fast) {
+  const int heads = n_q_heads + 2 * n_kv_heads;
+  if (!prefill_fits(hidden, heads, head_dim) || !aligned16(x) || !aligned16(W)) {
     launch_qkv_generic(a, ra, fr, st);
     return check_launch("qkv_rope_prefill(generic)");
   }
-  const int heads = n_q_heads + 2 * n_kv_heads;
-  // Tile height by a cost model: a round of 128-token tiles over the 256 CUs takes ~57 us, a round of 256-token tiles ~105 us
-  // (both per 45 slices of K); whichever needs less in total. T = 2048 is one round of 128s; anything that would need a
-  // second round of 128s is one round of 256s instead, T = 8192 two rounds of 256s instead of four of 128s. Up to about
-  // 1500 rows (of 5120 columns) smaller tiles fill the machine in less than a round of these (tile_gemm.hip: 1536 rows 50.9
-  // against 57 us, 999 rows 39.8 against 49.1, 97 rows 16.1 against 51).
-  const int64_t tn = (heads + HPT - 1) / HPT;
-  const int64_t rounds128 = (((rows + 127) / 128) * tn + 255) / 256, rounds256 = (((rows + 255) / 256) * tn + 255) / 256;
-  const int BM = rounds256 * 105 < rounds128 * 57 ? 256 : 128;
-  // (a single round of 256s rarely fills the CUs and takes 83 - 92 us then: 2900 rows 86.5, where two rounds of 128 x 256 take
-  // 91.3; up to 2816 rows two rounds of 128 x 224 are ahead, 2600 rows 82.3 against 84.6)
-  const int64_t here_ns = (BM == 128 ? rounds128 * 57000 : rounds256 == 1 ? 90000 : rounds256 * 105000) * (hidden / BK) / 45;
-  if (tile_gemm_ns(rows, static_cast<int64_t>(heads) * 64, hidden) < here_ns) return launch_tile_gemm_qkv("qkv_rope_prefill", a, ra, fr, st);
+  if (qkv_prefill_tiles(rows, hidden, heads, head_dim)) return launch_tile_gemm_qkv("qkv_rope_prefill", a, ra, fr, st);
+  const int BM = prefill_tile_height(rows, heads, nullptr, nullptr);
   static bool attr_set = false;   // raising the dynamic-LDS limit is idempotent; a benign race at worst repeats it
   if (!attr_set) {
     const void* k128[] = {reinterpret_cast<const void*>(qkv_prefill_quads_kernel<false>), reinterpret_cast<const void*>(qkv_prefill_quads_kernel<true>)};

@@ -6,7 +6,7 @@
 // At these sizes the machine is short of tiles, not of matrix cores: 128 x 320 tiles -- right for T = 2048, one per CU --
 // are 128 workgroups at 1000 rows and 16 at 100, and a launch takes 50 us however few there are. So the tile comes in
 // sizes from 64 x 32 to 128 x 256, and the host takes the one whose grid fills the 256 CUs in the fewest, cheapest rounds
-// (pick_tile below). What bounds a tile is the bytes its CU pulls in, (BM + BN) x K x 2: a CU has about 64 KB of loads in
+// (tile_gemm_pick below). What bounds a tile is the bytes its CU pulls in, (BM + BN) x K x 2: a CU has about 64 KB of loads in
 // flight whatever the LDS would hold, and a line that no CU of the XCD has asked for yet is about a microsecond away -- 60
 // GB/s, where lines that are in the L2 arrive at 100 (measured with the MFMAs and the LDS reads taken out: 0.58 us per
 // slice of a 128 x 160 tile, 0.37 with the weight L2-resident; the MFMAs alone 0.34).
@@ -377,9 +377,6 @@ int launch_one(const char* what, const QkvArgs& a, const RopeArgs& ra, const Yar
 //   97 rows   64 x 48 16.1   64 x 64 17.2   64 x 32 24.5        256 rows  64 x 80 21.2    64 x 64 34.2    64 x 128 25.3
 //   333 rows  64 x 128 23.2  64 x 160 27.1  64 x 96 36.3        512 rows  64 x 160 29.6   128 x 128 33.7  64 x 128 47.5
 //   777 rows  128 x 160 33.9 128 x 192 36.3 64 x 160 52.2       999 rows  128 x 160 39.8  128 x 192 41.1  128 x 128 64.2
-struct TileSize {
-  int bm, bn;
-};
 constexpr TileSize kTiles[] = {{64, 32}, {64, 48}, {64, 64}, {64, 80}, {64, 96}, {64, 128}, {64, 160}, {64, 192}, {128, 96}, {128, 128}, {128, 160}, {128, 192}, {128, 224}, {128, 256}};
 
 int64_t tile_ns(int64_t rows, int64_t cols, int64_t k, TileSize t) {
@@ -387,7 +384,9 @@ int64_t tile_ns(int64_t rows, int64_t cols, int64_t k, TileSize t) {
   return 1600 + rounds * (1700 + 20 * (t.bm + t.bn) + (k / 64) * (t.bm + t.bn) * 215 / 100);
 }
 
-TileSize pick_tile(int64_t rows, int64_t cols, int64_t k, int64_t* ns) {
+}  // namespace
+
+TileSize tile_gemm_pick(int64_t rows, int64_t cols, int64_t k, int64_t* ns) {
   TileSize best = kTiles[0];
   *ns = tile_ns(rows, cols, k, best);
   for (const TileSize& t : kTiles) {
@@ -400,10 +399,11 @@ TileSize pick_tile(int64_t rows, int64_t cols, int64_t k, int64_t* ns) {
   return best;
 }
 
+namespace {
 template <int MODE>
 int launch_mode(const char* what, const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& fr, int n_blocks, hipStream_t st) {
   int64_t ns;
-  TileSize t = pick_tile(a.rows, static_cast<int64_t>(n_blocks) * 16, a.hidden, &ns);
+  TileSize t = tile_gemm_pick(a.rows, static_cast<int64_t>(n_blocks) * 16, a.hidden, &ns);
 #define TLLM_TILE(...)                                   \
   if (typedef tile_gemm::Tile<__VA_ARGS__> C; t.bm == C::BM && t.bn == C::BN) return launch_one<C, MODE>(what, a, ra, fr, n_blocks, st)
   TLLM_TILE(2, 2, 2, 1, 4);
@@ -428,7 +428,7 @@ int launch_mode(const char* what, const QkvArgs& a, const RopeArgs& ra, const Ya
 
 int64_t tile_gemm_ns(int64_t rows, int64_t cols, int64_t k) {
   int64_t ns;
-  pick_tile(rows, cols, k, &ns);
+  tile_gemm_pick(rows, cols, k, &ns);
   return ns;
 }
 
@@ -440,6 +440,20 @@ int launch_tile_gemm_qkv(const char* what, const QkvArgs& a, const RopeArgs& ra,
 }  // namespace tllm
 
 using namespace tllm;
+
+extern "C" int tllm_qkv_gemm_tile(int prefill, int64_t rows, int64_t hidden, int n_q_heads, int n_kv_heads, int head_dim) {
+  const int heads = n_q_heads + 2 * n_kv_heads;
+  if (rows < 1 || hidden < 1 || heads < 1 || !(prefill ? qkv_prefill_tiles : qkv_decode_tiles)(rows, hidden, heads, head_dim)) return 0;
+  int64_t ns;
+  const TileSize t = tile_gemm_pick(rows, static_cast<int64_t>(heads) * 64, hidden, &ns);
+  return t.bm << 16 | t.bn;
+}
+
+extern "C" int tllm_linear_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim) {
+  int64_t ns;
+  const TileSize t = tile_gemm_pick(rows, out_dim, in_dim, &ns);
+  return t.bm << 16 | t.bn;
+}
 
 extern "C" int tllm_linear_bf16(const void* x, const void* W, const void* b, void* out, int64_t out_row_stride, int64_t rows, int64_t in_dim,
                                 int64_t out_dim, void* stream) {
