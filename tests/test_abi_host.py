@@ -283,3 +283,13 @@ def test_attention_prefill_shape_planning():
     assert [groups(1, n, n, 8, 8, 0) for n in (300, 400, 512)] == [2, 2, 2]
     assert [groups(1, 97, 1597, 8, 8, w) for w in (0, 128)] == [4, 4]
     assert groups(1, 777, 777, 8, 8, 0) == 1
+
+
+def test_qkv_decode_tiles_or_the_general_kernel():
+    """Decode batches of more than 32 rows at widths other than 2880: GEMM tiles only where the general kernel's passes over the
+    weight cost more than a tile's fixed time."""
+    tile = _lib.lib().tllm_qkv_gemm_tile
+    assert [tile(0, rows, hidden, nq, nkv, 64) for rows, hidden, nq, nkv in ((33, 256, 4, 2), (64, 512, 8, 2), (48, 1024, 12, 4), (64, 4096, 4, 2),
+                                                                          (256, 1024, 4, 2), (128, 512, 12, 4))] == [0] * 6
+    assert all(tile(0, rows, hidden, nq, nkv, 64) for rows, hidden, nq, nkv in ((40, 4096, 64, 8), (64, 1024, 64, 8), (448, 512, 12, 4), (128, 8192, 64, 8)))
+    assert [tile(0, rows, 4096, 64, 8, hd) for rows, hd in ((32, 64), (40, 128))] == [0, 0]

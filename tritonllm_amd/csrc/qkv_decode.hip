@@ -114,14 +114,23 @@ void launch_qkv_generic(const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& f
   hipLaunchKernelGGL(qkv_generic_kernel, dim3((unsigned)heads, gy), dim3(256), 0, st, a, ra, fr);
 }
 
+static bool qkv_tiles_fit(int64_t rows, int64_t hidden, int heads, int head_dim) {
+  return rows > 32 && head_dim == 64 && hidden % 64 == 0 && static_cast<int64_t>(heads) * 64 * hidden * 2 < (1ll << 32);
+}
+
 bool qkv_decode_tiles(int64_t rows, int64_t hidden, int heads, int head_dim) {
+  if (!qkv_tiles_fit(rows, hidden, heads, head_dim)) return false;
   const int64_t cols = static_cast<int64_t>(heads) * 64;
-  if (rows <= 32 || head_dim != 64 || hidden % 64 != 0 || cols * hidden * 2 >= (1ll << 32)) return false;
   // the rows kernel takes 6.4 us and 1.4 per block of 16 rows (97 rows 15.9, 128 rows 17.5, 256 rows 26.6): from about a
   // hundred rows a GEMM tile is ahead of it (97 rows 16.1, 128 rows 16.2, 256 rows 21.2)
   if (hidden == 2880) return tile_gemm_ns(rows, cols, hidden) < 6400 + 1400 * ((rows + 15) / 16);
-  // Beyond 32 rows the general kernel reads the weight a third time (hidden 4096: 40 rows 22.7 us).
-  return true;
+  // Beyond 32 rows the general kernel reads the weight a third time, which costs little while its workgroups -- sixteen weight
+  // rows x sixteen rows -- share the CUs in a round or two. Its time over widths of 128 - 8192, 1 - 144 heads and 33 - 448 rows:
+  // 3.0 us, and for every 256 workgroups (fewer count as 256) 0.3 and 1.9 ns per element of K. Chosen so, 596 of 600 points are within
+  // 3 % of the better of the two; us, general and tiles: hidden 512, 8 + 4 heads, 64 rows 3.8 and 6.2, 1024, 20 heads, 48 rows 4.3 and
+  // 7.4, 1024, 80 heads, 64 rows 12.4 and 7.9; 4096, 80 heads, 40 rows 22.7 and 16.9, 8 heads, 64 rows 6.6 and 12.5
+  const int64_t workgroups = static_cast<int64_t>(heads) * 4 * ((rows + 15) / 16);
+  return tile_gemm_ns(rows, cols, hidden) <= 3000 + (workgroups > 256 ? workgroups : 256) * (300 + hidden * 19 / 10) / 256;
 }
 
 }  // namespace tllm
@@ -284,7 +293,7 @@ extern "C" int tllm_qkv_rope_decode_bf16(const void* x, const void* W, const voi
   const bool out4 = (reinterpret_cast<uintptr_t>(q) % 4 == 0) && (reinterpret_cast<uintptr_t>(k) % 4 == 0) &&
                     (reinterpret_cast<uintptr_t>(v) % 4 == 0) && q_row_stride % 2 == 0 && k_row_stride % 2 == 0 &&
                     v_row_stride % 2 == 0 && kv_slot_stride % 2 == 0;
-  if (aligned16(x) && aligned16(W) && qkv_decode_tiles(rows, hidden, heads, head_dim))
+  if (aligned16(x) && aligned16(W) && (qkv_decode_tiles(rows, hidden, heads, head_dim) || (!out4 && qkv_tiles_fit(rows, hidden, heads, head_dim))))
     return launch_tile_gemm_qkv("qkv_rope_decode", a, ra, fr, st);
   // (the general kernel addresses a head's rows of the weight with 32-bit byte offsets)
   if (mfma_ok && out4 && static_cast<int64_t>(head_dim) * hidden * 2 < (1ll << 31))
