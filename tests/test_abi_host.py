@@ -293,3 +293,14 @@ def test_qkv_decode_tiles_or_the_general_kernel():
                                                                           (256, 1024, 4, 2), (128, 512, 12, 4))] == [0] * 6
     assert all(tile(0, rows, hidden, nq, nkv, 64) for rows, hidden, nq, nkv in ((40, 4096, 64, 8), (64, 1024, 64, 8), (448, 512, 12, 4), (128, 8192, 64, 8)))
     assert [tile(0, rows, 4096, 64, 8, hd) for rows, hd in ((32, 64), (40, 128))] == [0, 0]
+
+
+def test_qkv_prefill_tiles_at_other_widths():
+    """A prompt's route at K other than 2880: the fixed part of a launch counts once, whatever K is."""
+    tile = _lib.lib().tllm_qkv_gemm_tile
+    assert [tile(1, rows, 8192, 64, 8, 64) for rows in (2048, 4096, 8192)] == [0, 0, 0]
+    assert tile(1, 2900, 4096, 64, 8, 64) == 0
+    assert all(tile(1, rows, hidden, 64, 8, 64) for rows in (1, 97, 999) for hidden in (64, 512, 2880, 8192))
+    # 2880 wide: smaller tiles up to 1536 rows and where a launch of the larger ones would need a round for little
+    assert [bool(tile(1, rows, 2880, 64, 8, 64)) for rows in (97, 1536, 1537, 2048, 2049, 2816, 2817, 4096, 4097, 8192)] == \
+        [True, True, False, False, True, True, False, False, True, False]

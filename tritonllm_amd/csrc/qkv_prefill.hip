@@ -665,7 +665,7 @@ bool prefill_fits(int64_t hidden, int heads, int head_dim) {
 }
 
 // Tile height by a cost model: a round of 128-token tiles over the 256 CUs takes ~57 us, a round of 256-token tiles ~105 us
-// (both per 45 slices of K); whichever needs less in total. T = 2048 is one round of 128s; anything that would need a
+// (at 45 slices of K, 2880); whichever needs less in total. T = 2048 is one round of 128s; anything that would need a
 // second round of 128s is one round of 256s instead, T = 8192 two rounds of 256s instead of four of 128s.
 int prefill_tile_height(int64_t rows, int heads, int64_t* rounds128, int64_t* rounds256) {
   const int64_t tn = (heads + HPT - 1) / HPT;
@@ -682,9 +682,13 @@ bool qkv_prefill_tiles(int64_t rows, int64_t hidden, int heads, int head_dim) {
   if (!prefill_fits(hidden, heads, head_dim)) return false;
   int64_t rounds128, rounds256;
   const int BM = prefill_tile_height(rows, heads, &rounds128, &rounds256);
-  // (a single round of 256s rarely fills the CUs and takes 83 - 92 us then: 2900 rows 86.5, where two rounds of 128 x 256 take
-  // 91.3; up to 2816 rows two rounds of 128 x 224 are ahead, 2600 rows 82.3 against 84.6)
-  const int64_t here_ns = (BM == 128 ? rounds128 * 57000 : rounds256 == 1 ? 90000 : rounds256 * 105000) * (hidden / BK) / 45;
+  // What a round takes that does not depend on K -- launch, first slices, epilogue -- and per slice of it, measured from
+  // K = 256 to 8192: 128-token tiles 13 us at 4 slices, 23 at 16, 55 at 45, 74 at 64, 134 at 128; 256-token tiles 103, 138 and 258 at
+  // 45, 64 and 128. (a single round of 256s rarely fills the CUs and takes 83 - 92 us at 45 slices, 119 at 64 and 222 at 128: 2900
+  // rows of 2880 86.5, where two rounds of 128 x 256 take 91.3; up to 2816 rows two rounds of 128 x 224 are ahead, 2600 rows
+  // 82.3 against 84.6)
+  const int64_t slices = hidden / BK;
+  const int64_t here_ns = BM == 128 ? rounds128 * (11000 + 1022 * slices) : rounds256 == 1 ? 16000 + 1645 * slices : rounds256 * (16000 + 1978 * slices);
   return tile_gemm_ns(rows, static_cast<int64_t>(heads) * 64, hidden) < here_ns;
 }
 
