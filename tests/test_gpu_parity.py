@@ -776,6 +776,15 @@ def test_linear_tile_gemm(gpu, rows, k, n):
     close(y.detach()[0], want)
 
 
+@pytest.mark.parametrize("k,n,tiles,library", [(4096, 2880, (1, 24, 65, 97, 640, 2048, 2432), (32, 64, 2600)), (2048, 512, (), (1, 16, 48, 128)),
+                                               (8192, 1024, (), (1, 48, 128, 2048)), (5120, 2880, (200,), (8, 64)), (1024, 1024, (1, 32, 128, 2048), (2, 24, 3000)),
+                                               (128, 2880, (1, 24, 64, 2000), (3000,))])
+def test_linear_hands_over_to_the_library_where_that_is_ahead(gpu, k, n, tiles, library):
+    w, b = torch.zeros(n, k, dtype=torch.bfloat16, device=gpu), torch.zeros(n, dtype=torch.bfloat16, device=gpu)
+    took = lambda rows: host().linear(torch.zeros(rows, k, dtype=torch.bfloat16, device=gpu), w, b) is not None
+    assert [took(rows) for rows in tiles] == [True] * len(tiles) and [took(rows) for rows in library] == [False] * len(library)
+
+
 def test_linear_leaves_torch_its_hooks(gpu):
     """OUT.forward under what F.linear takes part in: vmap, forward-mode derivatives, autocast, tracing, symbolic tracing, a
     dispatch mode, a tensor subclass; a strided operand and one that is not 16-byte aligned."""

@@ -456,10 +456,24 @@ bool plain_operand(PyObject* o, c10::DeviceIndex device) {
          !(c10::GradMode::is_enabled() && t.requires_grad()) && !t._fw_grad(0).defined();
 }
 
-// linear(x, weight, bias): F.linear for plain bf16 tensors, K a multiple of 64 and outputs of 16, as long as tiles of
-// 128 x 224 cover the result in one round of the 256 CUs. Beyond that the library's GEMM is ahead ([2880, 4096] weight: 2500
-// rows 57.4 against 55.9 us, 2700 67.8 against 58.2, 4096 103 against 83; below, 97 rows 13.9 against 15.4, 192 rows 18.8 against
-// 32, 999 rows 33.9 against 36.6, 2400 rows 53.0 against 54.8).
+// Whether a GEMM tile is ahead of the library's GEMM. Up to tiles of 128 x 224 covering the result in one round of the 256 CUs
+// and about 2500 rows it mostly is ([2880, 4096] weight, us: 97 rows 13.9 and 15.4, 192 rows 18.8 and 32, 999 rows 33.9 and 36.6,
+// 2400 rows 53.0 and 54.8; behind that 2500 rows 57.4 and 55.9, 2700 67.8 and 58.2, 4096 103 and 83; other weights 3000 rows
+// 0.84 - 0.92 of the library's rate). Where the tiles are few and K is long the library shares K out between workgroups: from a K of
+// 50 per tile on (32 above 4096) it is ahead ([512, 2048] 48 rows 5.7 and 7.4, [1024, 8192] 48 rows 11.9 and 17.2, [2880, 5120]
+// 8 rows 10.5 and 15.5), with 25 - 64 rows of a K of 2900 and more from 30 on ([2880, 4096] 48 rows 13.1 and 14.9). And it has
+// a kernel for a few rows of a small weight ([512, 512] 16 rows 4.1 and 4.7, [1024, 1024] 4.6 and 5.8). Of 1600 calls of a K of
+// 64 .. 8192 and 128 .. 8192 outputs measured, 85 are 3 % slower so than with the library, 353 without the latter three.
+bool linear_in_tiles(int64_t rows, int64_t k, int64_t out) {
+  if (rows > 2560 || ((rows + 127) / 128) * ((out + 223) / 224) > 256) return false;
+  const int tile = tllm_linear_gemm_tile(rows, k, out);
+  const int64_t bm = tile >> 16, bn = tile & 0xffff, tiles = ((rows + bm - 1) / bm) * ((out + bn - 1) / bn);
+  if (k >= 1024 && k >= (k > 4096 ? 32 : 50) * tiles) return false;
+  if (rows > 24 && rows <= 64 && k >= 2900 && k >= 30 * tiles) return false;
+  return !(rows > 1 && rows <= 24 && k >= 512 && k < 2048 && out <= 2048);
+}
+
+// linear(x, weight, bias): F.linear for plain bf16 tensors, K a multiple of 64 and outputs of 16, where a tile is ahead
 PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 3 || !only_eager() || !THPVariable_CheckExact(a[0]) || !tensor(a[0]).is_cuda()) return none();
   const c10::DeviceIndex device = c10::hip::current_device();
@@ -471,7 +485,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!bf16(x) || x.dim() < 1 || x.size(-1) != k || x.numel() == 0 || !bias_ok(a[2], out) || k % 64 || out % 16 || out * k >= (1ll << 31))
     return none();
   const int64_t rows = x.numel() / k;
-  if (((rows + 127) / 128) * ((out + 223) / 224) > 256) return none();
+  if (!linear_in_tiles(rows, k, out)) return none();
   at::DimVector shape(x.sizes().begin(), x.sizes().end());
   shape.back() = out;
   const Tensor xc = x.is_contiguous() ? x : [&] {
