@@ -304,3 +304,12 @@ def test_qkv_prefill_tiles_at_other_widths():
     # 2880 wide: smaller tiles up to 1536 rows and where a launch of the larger ones would need a round for little
     assert [bool(tile(1, rows, 2880, 64, 8, 64)) for rows in (97, 1536, 1537, 2048, 2049, 2816, 2817, 4096, 4097, 8192)] == \
         [True, True, False, False, True, True, False, False, True, False]
+
+
+def test_logits_of_a_small_vocabulary_stay_in_passes():
+    tiled = _lib.lib().tllm_unembedding_decode_tiled
+    assert [tiled(rows, 0, hidden, vocab) for rows, hidden, vocab in ((9, 4096, 1000), (16, 4096, 4000), (33, 2880, 1000), (64, 2880, 4096))] == [0] * 4
+    assert [tiled(rows, 0, hidden, vocab) for rows, hidden, vocab in ((17, 4096, 1000), (65, 2880, 1000), (9, 4096, 8000), (33, 2880, 8000),
+                                                                      (33, 2880, 201088))] == [1] * 5
+    assert [tiled(16, 1, 4096, 1000), tiled(33, 1, 2880, 1000), tiled(40, 0, 1024, 1000)] == [1, 0, 1]
+    assert [tiled(rows, 0, 2880, 201088) for rows in (8, 32)] == [0, 0]

@@ -648,10 +648,16 @@ int unembed_check(const char* who, const void* x, const void* W, bool w8, int64_
   return TLLM_OK;
 }
 
-// Logits of more rows than one pass of the kernels above takes
+// Logits of more rows than one pass of the kernels above takes -- two, for a wide model's vocabulary that gives a CU's run less
+// than a sixteen-row unit: the passes' few workgroups are on the machine together then, and a tile is sixteen units, one of them
+// real (us, two passes and tiles: 4096 wide, 16 rows, vocabulary 1000 25.5 and 35.0, 4096 26.5 and 37.1, 4200 40.9 and 37.0; 2880
+// wide, 40 rows 30.8 and 31.6, 30.6 and 32.9, 42.2 and 32.9; three passes 24 rows 45 and 37; 1024 wide 16.3 and 12.2; the
+// eight-row passes of an fp8 weight 41 and 29).
 bool unembed_tiled(int64_t rows, bool w8, int64_t hidden, int64_t vocab) {
-  const int64_t one_pass = unembed_rows32(rows, w8, hidden, vocab, false) ? 32 : unembed_xr(rows, w8, hidden);
-  return rows > one_pass && unembed_tiles_fit(rows, w8, hidden, vocab);
+  const bool rows32 = unembed_rows32(rows, w8, hidden, vocab, false);
+  const int64_t one_pass = rows32 ? 32 : unembed_xr(rows, w8, hidden);
+  const int64_t passes = vocab <= 16 * kUnembedGrid && hidden >= 2560 && (rows32 || !w8) ? 2 : 1;
+  return rows > passes * one_pass && unembed_tiles_fit(rows, w8, hidden, vocab);
 }
 
 template <bool ARGMAX>
@@ -694,6 +700,8 @@ int unembed_launch(const char* who, const UnembedArgs& a, bool w8, hipStream_t s
   return check_launch(who);
 }
 }  // namespace
+
+extern "C" int tllm_unembedding_decode_tiled(int64_t rows, int fp8, int64_t hidden, int64_t vocab) { return unembed_tiled(rows, fp8 != 0, hidden, vocab); }
 
 extern "C" int tllm_unembedding_decode_bf16(const void* x, const void* W, const float* w_scale, void* logits, int64_t logits_row_stride,
                                             int64_t rows, int64_t hidden, int64_t vocab, void* stream) {
