@@ -609,7 +609,7 @@ def test_qkv_rope_prefill_long_context(gpu, yarn):
     _check_qkv(gpu, yarn, 8192, "prefill", seed=4, prefill_positions=True)
 
 
-@pytest.mark.parametrize("rows", [2049, 2304, 3841, 4000, 4096, 5000])
+@pytest.mark.parametrize("rows", [2049, 2304, 2817, 3333, 3841, 4000, 4096, 5000])
 def test_qkv_rope_prefill_256_token_tiles(gpu, yarn, rows):
     """Row counts that would need a second round of 128-token tiles run on 256-token tiles instead (two-pass epilogue,
     table built after the K loop; 8192 rows in the long-context test too): ragged last tiles, the XCD-swizzled and the
@@ -617,7 +617,7 @@ def test_qkv_rope_prefill_256_token_tiles(gpu, yarn, rows):
     _check_qkv(gpu, yarn, rows, "prefill", seed=rows, prefill_positions=rows % 2 == 0, max_pos=131072)
 
 
-@pytest.mark.parametrize("rows", [300, 2304])
+@pytest.mark.parametrize("rows", [300, 2304, 2000, 3000])
 def test_qkv_rope_prefill_cos_sin_tables(gpu, rows):
     """The prefill kernels' table variants (cos / sin loaded, as the reference passes them, triton_kernels.py:90) at both
     tile heights, arbitrary positions, against the oracle; plain tensors, which the host side cannot trace back to YaRN
@@ -720,10 +720,10 @@ def test_qkv_decode_fp8_weight_other_shapes(gpu, hd, nq, nkv, rows):
                                                 (1100, 576, 64, 8), (1400, 512, 64, 8), (1500, 1024, 64, 8)])
 @pytest.mark.parametrize("how", ["positions", "offset", "wrap", "table", "plain"])
 def test_qkv_tile_gemm(gpu, rows, hidden, nq, nkv, how):
-    """The GEMM tiles at sizes that take each of them (64 x 32 .. 128 x 256): fewer K slices than ring stages, odd and even
-    slice counts (tiles that split a stage's two slices between their wavefronts), ragged last row and column tiles, and
-    every source of the rotary positions: a tensor, one sequence behind an offset, several sequences with wrap-around, a
-    cos / sin table, no rotation."""
+    """GEMM tiles at widths up to 2880: fewer K slices than ring stages and more, odd and even slice counts (tiles that split a
+    stage's two slices between their wavefronts), ragged last row and column tiles, and every source of the rotary
+    positions: a tensor, one sequence behind an offset, several sequences with wrap-around, a cos / sin table, no rotation."""
+    assert _lib.lib().tllm_qkv_gemm_tile(1, rows, hidden, nq, nkv, 64) != 0
     g = torch.Generator().manual_seed(40 + rows)
     x = torch.randn(rows, hidden, generator=g).bfloat16()
     w = (0.05 * torch.randn((nq + 2 * nkv) * 64, hidden, generator=g)).bfloat16()
@@ -751,6 +751,100 @@ def test_qkv_tile_gemm(gpu, rows, hidden, nq, nkv, how):
     close(q, qr)
     close(k, kr)
     close(v, vr)
+
+
+def _qkv_position_sources(gpu, rows, g):
+    """(name, arguments, positions): every source of the rotary positions; two of them wrap around and hold several sequences."""
+    pos, seqs = torch.randint(0, 8192, (rows,), generator=g), (90 + torch.arange(rows) % 100) % 150
+    cos, sin = (t.to(gpu) for t in O.yarn_cos_sin(torch.arange(8192)))
+    wrap = dict(offset=torch.tensor([90], device=gpu), tokens_per_batch=100, max_context_length=150)
+    return [("positions", dict(yarn=T.gpt_oss_yarn(), positions=pos.to(gpu)), pos),
+            ("offset", dict(yarn=T.gpt_oss_yarn(), offset=torch.tensor([37], device=gpu)), 37 + torch.arange(rows)),
+            ("wrap", dict(yarn=T.gpt_oss_yarn(), **wrap), seqs),
+            ("table", dict(cos=cos, sin=sin, positions=pos.to(gpu), max_context_length=8192), pos),
+            ("table, wrap", dict(cos=cos, sin=sin, **wrap), seqs),
+            ("plain", dict(rotate=False), None)]
+
+
+def _check_qkv_position_sources(gpu, rows, hidden, nq, nkv, mode, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(rows, hidden, generator=g).bfloat16()
+    w = (0.05 * torch.randn((nq + 2 * nkv) * 64, hidden, generator=g)).bfloat16()
+    b = (0.05 * torch.randn((nq + 2 * nkv) * 64, generator=g)).bfloat16()
+    plain = O.linear_ref(x, w, b)
+    xg, wg, bg = x.to(gpu), w.to(gpu), b.to(gpu)
+    for name, kw, pos in _qkv_position_sources(gpu, rows, g):
+        want = plain.clone()
+        if pos is not None:
+            n = (nq + nkv) * 64
+            want[:, :n] = O.rope_rotate_ref(plain[:, :n].reshape(rows, nq + nkv, 64), *O.yarn_cos_sin(pos)).reshape(rows, n)
+        got = T.qkv_rope_forward(xg, wg, bg, nq, nkv, 64, mode=mode, **kw)
+        try:
+            for have, part in zip(got, torch.split(want, (nq * 64, nkv * 64, nkv * 64), dim=1)):
+                close(have, part)
+        except AssertionError as e:
+            raise AssertionError(f"{name}: {e}") from None
+
+
+@pytest.mark.parametrize("bm,bn,rows,nq,nkv", [(64, 32, 33, 1, 1), (64, 48, 67, 64, 8), (64, 64, 131, 64, 8), (64, 80, 771, 10, 5), (64, 96, 2307, 6, 1),
+                                              (64, 128, 1155, 10, 5), (64, 160, 701, 32, 8), (64, 192, 515, 64, 8), (128, 96, 771, 32, 8),
+                                              (128, 128, 2307, 10, 5), (128, 160, 771, 64, 8), (128, 192, 1411, 40, 8), (128, 224, 1155, 64, 8),
+                                              (128, 256, 2307, 32, 8)])
+@pytest.mark.parametrize("hidden", [64, 192])
+def test_qkv_every_gemm_tile(gpu, bm, bn, rows, nq, nkv, hidden):
+    """Each tile that is compiled, with every source of the rotary positions: a K of one slice and of three (tiles that take
+    two slices to a stage: the last stage is half empty), ragged last row tiles."""
+    assert _lib.lib().tllm_qkv_gemm_tile(1, rows, hidden, nq, nkv, 64) == bm << 16 | bn
+    _check_qkv_position_sources(gpu, rows, hidden, nq, nkv, "prefill", seed=bm + bn + hidden)
+
+
+@pytest.mark.parametrize("rows", [2011, 4000])
+def test_qkv_large_tiles_every_position_source(gpu, rows):
+    """The 128- and 256-token tiles of long prompts."""
+    assert _lib.lib().tllm_qkv_gemm_tile(1, rows, 2880, 64, 8, 64) == 0
+    _check_qkv_position_sources(gpu, rows, 2880, 64, 8, "prefill", seed=rows)
+
+
+@pytest.mark.parametrize("batch,hidden,nq,nkv,tiles", [(100, 2880, 64, 8, False), (131, 2880, 64, 8, True), (41, 4096, 64, 8, True), (40, 512, 8, 2, False)])
+@pytest.mark.parametrize("how", ["offset", "positions"])
+def test_qkv_cache_form_of_large_batches(gpu, batch, hidden, nq, nkv, tiles, how):
+    """Batches above 32 rows write k and v into their slot of the cache and touch no other, by the kernel that streams the rows,
+    by GEMM tiles and by the general kernel; all rows at the slot's position, or each at its own."""
+    assert bool(_lib.lib().tllm_qkv_gemm_tile(0, batch, hidden, nq, nkv, 64)) == tiles
+    g = torch.Generator().manual_seed(batch + hidden)
+    x = torch.randn(batch, hidden, generator=g).bfloat16()
+    w = (0.05 * torch.randn((nq + 2 * nkv) * 64, hidden, generator=g)).bfloat16()
+    b = (0.05 * torch.randn((nq + 2 * nkv) * 64, generator=g)).bfloat16()
+    scale = 1 + 0.1 * torch.randn(hidden, generator=g)
+    slots, slot = 7, 5
+    ck, cv = (torch.full((batch, slots, nkv, 64), 3.0, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    pos = torch.randint(0, 8192, (batch,), generator=g) if how == "positions" else torch.full((batch,), slot)
+    q = T.qkv_rope_cache_decode_forward(x.view(batch, 1, hidden).to(gpu), w.to(gpu), b.to(gpu), None, None, 131072, ck, cv,
+                                        torch.tensor([slot], device=gpu), nq, nkv, 64, yarn=T.gpt_oss_yarn(),
+                                        positions=pos.to(gpu) if how == "positions" else None, norm_scale=scale.to(gpu), norm_eps=1e-5)
+    qr, kr, vr = O.qkv_rope_ref(O.rmsnorm_ref(x, scale, 1e-5).bfloat16(), w, b, pos, nq, nkv, 64)
+    close(q.view(batch, -1), qr)
+    close(ck[:, slot].reshape(batch, -1), kr)
+    close(cv[:, slot].reshape(batch, -1), vr)
+    others = [s for s in range(slots) if s != slot]
+    assert (ck[:, others] == 3.0).all() and (cv[:, others] == 3.0).all()
+
+
+@pytest.mark.parametrize("bm,bn,rows,n", [(64, 32, 1, 16), (64, 48, 67, 5120), (64, 64, 131, 4096), (64, 80, 2307, 400), (64, 96, 2307, 512), (64, 128, 333, 4096),
+                                         (64, 160, 2051, 1024), (64, 192, 515, 5120), (128, 96, 2307, 1024), (128, 128, 1501, 2048), (128, 160, 771, 5120),
+                                         (128, 192, 1155, 4096), (128, 224, 1411, 4096), (128, 256, 1411, 5120)])
+@pytest.mark.parametrize("k", [64, 192])
+def test_linear_every_gemm_tile(gpu, bm, bn, rows, n, k):
+    """Each tile that is compiled, through the entry point: the columns behind the last row's end are left alone."""
+    L = _lib.lib()
+    assert L.tllm_linear_gemm_tile(rows, k, n) == bm << 16 | bn
+    g = torch.Generator().manual_seed(rows + n + k)
+    x, w, b = torch.randn(rows, k, generator=g).bfloat16(), (0.05 * torch.randn(n, k, generator=g)).bfloat16(), (0.05 * torch.randn(n, generator=g)).bfloat16()
+    xg, wg, bg, out = x.to(gpu), w.to(gpu), b.to(gpu), torch.full((rows, n + 8), 7.0, dtype=torch.bfloat16, device=gpu)
+    rc = L.tllm_linear_bf16(xg.data_ptr(), wg.data_ptr(), bg.data_ptr(), out.data_ptr(), n + 8, rows, k, n, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, L.tllm_last_error()
+    close(out[:, :n], O.linear_ref(x, w, b))
+    assert (out[:, n:] == 7.0).all()
 
 
 @pytest.mark.parametrize("rows,k,n", [(1, 64, 16), (3, 4096, 2880), (97, 4096, 2880), (200, 448, 2880), (333, 576, 2880), (512, 640, 2880),
@@ -1608,6 +1702,20 @@ def test_attention_prefill_key_groups(gpu, batch_size, num_queries, num_keys, st
     """Launches of at most two workgroups of 64 queries x 1 head per CU: the key blocks are shared out between wavefronts,
     from fewer blocks than groups to many of them, the last round ragged, a group with nothing visible among them."""
     _attn_prefill_case(gpu, batch_size, num_queries, num_keys, window, start_q, seed=num_queries + num_keys, **kv)
+
+
+@pytest.mark.parametrize("window", [None, 128])
+def test_attention_prefill_odd_group_large_launch(gpu, window):
+    """Three query heads per KV head, more than two workgroups of 64 queries x 1 head per CU: 128 queries of one head each."""
+    assert _lib.lib().tllm_attention_prefill_key_groups(1, 1500, 1500, 8, 3, window or 0) == 1
+    _attn_prefill_case(gpu, 1, 1500, 1500, window, 0, groups=3, seed=15)
+
+
+@pytest.mark.parametrize("batch_size,num_keys,kv_heads,plan", [(33, 1400, 16, (4, 2)), (19, 1400, 32, (8, 3))])
+def test_attention_decode_more_than_eight_kv_heads(gpu, batch_size, num_keys, kv_heads, plan):
+    L = _lib.lib()
+    assert (L.tllm_attention_decode_heads_per_workgroup(batch_size, kv_heads, num_keys, 0), L.tllm_attention_decode_splits(batch_size, kv_heads, num_keys, 0)) == plan
+    _attn_case(gpu, batch_size, num_keys, None, num_keys - 1, groups=2, kv_heads=kv_heads, seed=batch_size)
 
 
 def test_attention_prefill_views_of_the_qkv_buffer_and_the_cache(gpu):
