@@ -273,6 +273,17 @@ def test_qkv_rope_auto_mode_either_side_of_the_row_threshold(gpu, yarn, rows):
     _check_qkv(gpu, yarn, rows, "auto", seed=40 + rows)
 
 
+def test_qkv_rope_auto_mode_follows_the_row_threshold(gpu, yarn, monkeypatch):
+    """One place holds the number of rows: an fp8 weight has decode kernels only, so its refusal shows the mode that was chosen."""
+    d = O.make_inputs(8, seed=41)
+    w8, ws = T.quantize_fp8_rows(d["w"].to(gpu))
+    args, kw = (d["x"].to(gpu), w8, d["b"].to(gpu), 64, 8, 64), dict(yarn=yarn, positions=d["positions"].to(gpu), weight_scale=ws)
+    T.qkv_rope_forward(*args, **kw)
+    monkeypatch.setattr(ops, "DECODE_MAX_ROWS_2880", 7)
+    with pytest.raises(NotImplementedError):
+        T.qkv_rope_forward(*args, **kw)
+
+
 @pytest.mark.parametrize("rows", [1, 100, 128, 200, 2048])
 def test_qkv_rope_prefill_parity(gpu, yarn, rows):
     _check_qkv(gpu, yarn, rows, "prefill", seed=100 + rows, prefill_positions=rows >= 128)

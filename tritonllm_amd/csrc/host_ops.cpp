@@ -351,7 +351,7 @@ bool heads_of(PyObject* const* a, int64_t total_out, int* nq, int* nkv, int* hd)
 }
 
 // qkv_rope(x, weight, bias, num_q_heads, num_kv_heads, head_dim, yarn, positions, offset, tokens_per_batch, max_context_length,
-//          rotate, mode, out, norm_scale, norm_eps, weight_scale, fuse_norm, cos, sin)
+//          rotate, kind, out, norm_scale, norm_eps, weight_scale, fuse_norm, cos, sin)
 // (the tables are looked at for their device alone: yarn are the parameters that they carry)
 PyObject* qkv_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int nq, nkv, hd;
@@ -371,8 +371,7 @@ PyObject* qkv_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (tpb == 0) tpb = rows;
   bool decode;
   if (!PyUnicode_Check(a[12])) return none();
-  if (PyUnicode_CompareWithASCIIString(a[12], "auto") == 0) decode = rows <= (x.size(1) == 2880 && hd == 64 ? 448 : 64);   // ops._decode_max_rows
-  else if (PyUnicode_CompareWithASCIIString(a[12], "decode") == 0) decode = true;
+  if (PyUnicode_CompareWithASCIIString(a[12], "decode") == 0) decode = true;
   else if (PyUnicode_CompareWithASCIIString(a[12], "prefill") == 0) decode = false;
   else return none();
   TllmRope r;

@@ -365,9 +365,11 @@ def qkv_rope_forward(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
     outputs written to three dense tensors. ``mode``: "decode" (weight streaming),
     "prefill" (MFMA GEMM) or "auto" (by row count). No reference twin as a single call:
     it is F.linear + split + contiguous + rope_forward of model.py:506-522 in one launch."""
+    if mode == "auto" and x.ndim == 2:
+        mode = "decode" if x.shape[0] <= _decode_max_rows(x.shape[1], head_dim) else "prefill"
     done = host().qkv_rope(x, weight, bias, num_q_heads, num_kv_heads, head_dim, _yarn_or_tables(yarn, cos, sin), positions, offset,
                            tokens_per_batch, max_context_length, rotate, mode, out, norm_scale, norm_eps, weight_scale,
-                           norm_scale is not None and _norm_fusable("prefill" if mode == "prefill" else "decode", x.shape[0], x.shape[-1], head_dim), cos, sin)
+                           norm_scale is not None and x.ndim == 2 and _norm_fusable(mode, *x.shape, head_dim), cos, sin)
     if done is not None:
         return done
     _on_gpu(x, weight, bias, positions, offset, cos, sin, norm_scale, weight_scale)
@@ -394,8 +396,6 @@ def qkv_rope_forward(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
     if rotate:
         desc = _rope_desc(cos, sin, yarn, positions, offset, tokens_per_batch if tokens_per_batch else max(rows, 1),
                           max_context_length, keep, rows)
-    if mode == "auto":
-        mode = "decode" if rows <= _decode_max_rows(x.shape[-1], head_dim) else "prefill"
     _require(mode in ("decode", "prefill"))
     _launch_qkv(mode, x, weight, bias, q, k, v, q.stride(0), k.stride(0), v.stride(0), 0, num_q_heads, num_kv_heads, head_dim, desc,
                 norm=None if norm_scale is None else (norm_scale, norm_eps),
@@ -509,7 +509,7 @@ def qkv_rope_cache_decode_forward(hidden, weight, bias, sin, cos, max_context_le
     block's input RMSNorm (model.py:476) runs inside the same kernel on the raw ``hidden``."""
     done = host().qkv_rope_cache(hidden, weight, bias, _yarn_or_tables(yarn, cos, sin), max_context_length, cache_k, cache_v, offset,
                                  num_q_heads, num_kv_heads, head_dim, weight_scale, positions, norm_scale, norm_eps,
-                                 norm_scale is not None and _norm_fusable("decode", hidden.shape[0], hidden.shape[-1], head_dim))
+                                 norm_scale is not None and hidden.ndim == 3 and _norm_fusable("decode", hidden.shape[0], hidden.shape[2], head_dim))
     if done is not None:
         return done
     _on_gpu(hidden, weight, bias, cache_k, cache_v, offset, positions, norm_scale, weight_scale)
