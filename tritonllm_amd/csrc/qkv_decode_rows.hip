@@ -1,5 +1,5 @@
 // Decode-size fused QKV projection + bias + rotary for hidden == 2880 and any number of activation rows, with ONE pass
-// over the weight: the kernel for the batches between the 32-row streaming kernel and the prefill GEMM.
+// over the weight: the kernel for the batches between the 32-row streaming kernel and the GEMM tiles (fp8 weights: for every one above).
 //
 // Same division of the output as the other streaming kernels: 256 workgroups of ten rotation pairs (20 weight rows, two
 // 16-row MFMA tiles with the quad layout [lo(2i), lo(2i+1), hi(2i), hi(2i+1)]), six streaming wavefronts that each own
@@ -14,7 +14,7 @@
 // rounding, stores) while the next block is multiplied.
 // Per CU: 115 KB of weight from HBM once, and rows x 5760 bytes of activations from the L2s. A block of 16 rows costs
 // ~1.4 us, most of it the streaming wavefronts' own chain (wait, fragment reads, dependent MFMAs, barrier) rather than
-// the bytes; the prefill GEMM, whose tiles share activations between fewer CUs, takes over at a few hundred rows.
+// the bytes; the GEMM tiles, which share activations between fewer CUs, take over at 113 rows.
 // W8: the weight is fp8 (OCP e4m3) with one fp32 scale per output row (triton_kernels.py:261-268, 927-965): the
 // fragments are widened to bf16 (exact) once, on their way into the registers; the row scale multiplies the finished sum.
 #include "qkv_decode_stream.h"

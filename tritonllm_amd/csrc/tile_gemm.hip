@@ -1,5 +1,8 @@
-// GEMM tiles for prompts of up to about 1500 rows and decode batches of more than a hundred: the QKV projection with bias +
-// rotary (qkv_prefill.hip does it for longer prompts) and the plain projection with bias.
+// GEMM tiles for short prompts and large decode batches: the QKV projection with bias + rotary and the plain projection
+// with bias. At 80 heads of 64 and a width of 2880 that is prompts of up to 1536 rows, those for which the larger tiles of
+// qkv_prefill.hip would need one more round for little (2049 - 2816, 4097 - 4864, 6145 - 6528, ... rows; qkv_prefill_tiles), and
+// decode batches from 113 rows on (qkv_decode_tiles); the plain projection where it is ahead of the library's GEMM, up to
+// 2432 rows of [2880, 4096] (linear_in_tiles in host_ops.cpp).
 //
 //   D[rows, n] = X[rows, K] . W[n, K]^T      (both operands K-contiguous, K a multiple of 64)
 //

@@ -71,8 +71,9 @@ class QKV(torch.nn.Module):
 
 class OUT(torch.nn.Module):
     """Attention out-projection (model.py:170-216): ``weight [hidden_size, out_dim]``, ``bias [hidden_size]``.
-    ``decode_residual`` is the decode kernel; ``forward`` is ``F.linear``: the HIP tile GEMM for prompts of up to a few
-    thousand rows, the library's beyond that, for other types and wherever torch has more to do than the product (gradients, autocast, vmap, tracing)."""
+    ``decode_residual`` is the decode kernel; ``forward`` is ``F.linear``: the HIP tile GEMM on the GPU where it is ahead of
+    the library's (prompts of up to about 2500 rows, K not too long for the number of tiles), the library's otherwise, for other
+    types and wherever torch has more to do than the product (gradients, autocast, vmap, tracing)."""
 
     def __init__(self, out_dim: int, hidden_size: int, device: torch.device | None = None):
         super().__init__()

@@ -38,11 +38,11 @@ from .yarn import YarnParams
 
 _BF16 = torch.bfloat16
 
-# rows at or below this use the weight-streaming decode kernel, above it the MFMA GEMM
+# rows at or below this use the decode entry point, above it the prefill one
 DECODE_MAX_ROWS = 64
-# At the gpt-oss shape the weight is read once whatever the row count (above 32 rows a kernel holds its share of the
-# weight and streams the rows past it: ~6.5 us + 0.09 us per row -- 96 rows 16 us, 192 rows 24 us, 384 rows 38-42 us),
-# where the GEMM's one round of tiles costs 50-56 us however few rows there are: they meet near 500 rows.
+# The entry points choose their kernels by size. At the gpt-oss shape decode holds the weight and streams the rows past it up
+# to 112 rows (64 rows 12.7 us, where prefill's GEMM tile takes 15.8); from there on both take the same tiles (128 rows 16 us,
+# 448 rows 29), so that for a bf16 weight nothing changes at this number. An fp8 weight has decode kernels only.
 DECODE_MAX_ROWS_2880 = 448
 
 
@@ -362,20 +362,20 @@ def qkv_rope_forward(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
     With ``weight_scale`` the weight is float8_e4m3fn with per-row scales (see ``quantize_fp8_rows``).
 
     One fused kernel: projection, bias, rotary on q/k (fp32 accumulator, one rounding),
-    outputs written to three dense tensors. ``mode``: "decode" (weight streaming),
-    "prefill" (MFMA GEMM) or "auto" (by row count). No reference twin as a single call:
+    outputs written to three dense tensors. ``mode``: "decode" (weight streaming; GEMM tiles for large
+    batches), "prefill" (MFMA GEMM) or "auto" (by row count). No reference twin as a single call:
     it is F.linear + split + contiguous + rope_forward of model.py:506-522 in one launch."""
-    if mode == "auto" and x.ndim == 2:
-        mode = "decode" if x.shape[0] <= _decode_max_rows(x.shape[1], head_dim) else "prefill"
+    rows, hidden = x.shape if x.ndim == 2 else (0, 0)       # (refused below)
+    if mode == "auto":
+        mode = "decode" if rows <= _decode_max_rows(hidden, head_dim) else "prefill"
     done = host().qkv_rope(x, weight, bias, num_q_heads, num_kv_heads, head_dim, _yarn_or_tables(yarn, cos, sin), positions, offset,
                            tokens_per_batch, max_context_length, rotate, mode, out, norm_scale, norm_eps, weight_scale,
-                           norm_scale is not None and x.ndim == 2 and _norm_fusable(mode, *x.shape, head_dim), cos, sin)
+                           norm_scale is not None and _norm_fusable(mode, rows, hidden, head_dim), cos, sin)
     if done is not None:
         return done
     _on_gpu(x, weight, bias, positions, offset, cos, sin, norm_scale, weight_scale)
     _require(x.ndim == 2)
     _require((weight.dtype == _FP8) == (weight_scale is not None), "a float8 weight needs weight_scale, a bfloat16 one takes none")
-    rows, hidden = x.shape
     total_out, hidden_w = weight.shape
     _require(hidden == hidden_w)
     _require(total_out == (num_q_heads + 2 * num_kv_heads) * head_dim)
