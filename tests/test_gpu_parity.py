@@ -624,7 +624,8 @@ def test_qkv_rope_prefill_long_context(gpu, yarn):
 def test_qkv_rope_prefill_256_token_tiles(gpu, yarn, rows):
     """Row counts that would need a second round of 128-token tiles run on 256-token tiles instead (two-pass epilogue,
     table built after the K loop; 8192 rows in the long-context test too): ragged last tiles, the XCD-swizzled and the
-    plain tile order, arbitrary positions. 5000 rows fall back on 128-token tiles in three rounds."""
+    plain tile order, arbitrary positions. 5000 rows fall back on 128-token tiles in three rounds, and 2049 and 2304, a little
+    more than one round of those, on the smaller GEMM tiles."""
     _check_qkv(gpu, yarn, rows, "prefill", seed=rows, prefill_positions=rows % 2 == 0, max_pos=131072)
 
 

@@ -2,11 +2,12 @@
 //
 // A launch takes ~4 us of host time, but checking a dozen tensors, reading their shapes, strides and addresses one
 // attribute at a time and converting twenty arguments through ctypes took 9-13 us more per call -- a decode step issued call
-// by call (24 layers, ~122 launches) spent 1690 us on the host for 670 us of GPU work. Each function here takes the
+// by call (24 layers, 123 calls) spent 1690 us on the host for 670 us of GPU work. Each function here takes the
 // arguments of its namesake in ops.py, does the same checks and the same launch, and returns None as soon as anything is not
 // the ordinary case (another dtype, a strided operand, a wrong shape, a CPU tensor, arguments that the entry point refuses):
 // ops.py then runs its own checks, which make the copy or raise the error. Only a call that has launched nothing is answered
-// so; what the runtime reports at a launch is raised here. Nothing is remembered between calls but the scratch pool.
+// so (the norm ahead of a QKV projection that is then refused aside: it fills a pool buffer, and ops.py fills it again); what the
+// runtime reports at a launch is raised here. Nothing is remembered between calls but the scratch pool.
 #include <Python.h>
 
 #include <c10/core/GradMode.h>
