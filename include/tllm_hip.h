@@ -216,6 +216,8 @@ int tllm_qkv_rope_prefill_bf16(const void* x, const void* W, const void* b,
  * the one that tllm_linear_bf16 takes. No counterpart in the reference. */
 int tllm_qkv_gemm_tile(int prefill, int64_t rows, int64_t hidden, int n_q_heads, int n_kv_heads, int head_dim);
 int tllm_linear_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim);
+/* Diagnostic: wavefronts that stream the weight in a workgroup of the general-shape decode projections (4, 2 or 1). */
+int tllm_decode_general_streams(int64_t rows, int64_t in_dim, int64_t out_dim, int fp8);
 
 /* out[r, n] = sum_k x[r, k] * W[n, k] + b[n] for a prompt's rows (bf16 in, fp32 accumulate, one RNE to bf16): what OUT.forward
  * is, model.py:196-197. x [rows, in_dim], W [out_dim, in_dim] dense and 16-byte aligned, b [out_dim] or NULL, out with

@@ -295,6 +295,16 @@ def test_qkv_decode_tiles_or_the_general_kernel():
     assert [tile(0, rows, 4096, 64, 8, hd) for rows, hd in ((32, 64), (40, 128))] == [0, 0]
 
 
+def test_decode_general_streaming_wavefronts_follow_the_grid():
+    """Four wavefronts stream a workgroup's weight rows while all workgroups are on the machine together, fewer, with less LDS,
+    beyond that (fp8, 1536 wide, 400 rows 78 us with four, 37 with one); never more than K has phases for."""
+    streams = _lib.lib().tllm_decode_general_streams
+    assert [streams(rows, 1536, 5120, 1) for rows in (1, 8, 12, 32, 64, 400)] == [4, 4, 2, 2, 1, 1]
+    assert [streams(rows, 1536, 5120, 0) for rows in (1, 8, 12, 32, 64)] == [4, 4, 4, 1, 1]
+    assert [streams(rows, 4096, 2048, 1) for rows in (16, 32, 64, 150)] == [4, 4, 2, 1]
+    assert [streams(8, k, 5120, fp8) for fp8 in (0, 1) for k in (128, 256, 512, 1024)] == [1, 2, 4, 4, 1, 1, 2, 4]
+
+
 def test_qkv_prefill_tiles_at_other_widths():
     """A prompt's route at K other than 2880: the fixed part of a launch counts once, whatever K is."""
     tile = _lib.lib().tllm_qkv_gemm_tile

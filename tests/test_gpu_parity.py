@@ -727,6 +727,29 @@ def test_qkv_decode_fp8_weight_other_shapes(gpu, hd, nq, nkv, rows):
     close(v, vr)
 
 
+@pytest.mark.parametrize("fp8,rows,k,nq,nkv,streams", [
+    (True, 5, 96, 6, 2, 1), (True, 9, 288, 6, 2, 2), (True, 20, 544, 6, 2, 4), (True, 20, 1312, 6, 2, 4),                      # by K
+    (True, 45, 1056, 40, 5, 2), (True, 45, 4096, 40, 5, 2), (True, 200, 608, 64, 8, 1), (True, 200, 4096, 64, 8, 1), (True, 200, 256, 64, 8, 1),   # by workgroups
+    (False, 5, 96, 6, 2, 1), (False, 9, 160, 6, 2, 2), (False, 20, 288, 6, 2, 4), (False, 40, 1056, 52, 6, 2), (False, 40, 2048, 52, 6, 2),
+    (False, 200, 416, 64, 8, 1), (False, 200, 2048, 64, 8, 1)])
+def test_decode_general_streaming_wavefronts(gpu, fp8, rows, k, nq, nkv, streams):
+    """One, two and four wavefronts that stream the weight of a general-shape decode projection, as K and the number of
+    workgroups have it: one phase each and several, a last phase that is cut short or missing, rows of a pitch of 4 KB."""
+    n = (nq + 2 * nkv) * 32
+    assert _lib.lib().tllm_decode_general_streams(rows, k, n, fp8) == _lib.lib().tllm_decode_general_streams(rows, k, n - 3, fp8) == streams
+    g = torch.Generator().manual_seed(rows + k)
+    x, w, b, r = (f * torch.randn(*s, generator=g) for f, s in ((1, (rows, k)), (0.05, (n, k)), (0.05, (n,)), (1, (rows, n))))
+    x, w, b, r = x.bfloat16(), w.bfloat16(), b.bfloat16(), r.bfloat16()
+    wg, ws = T.quantize_fp8_rows(w.to(gpu)) if fp8 else (w.to(gpu), None)
+    want = O.linear_ref(x, O.dequant_fp8_ref(wg.cpu(), ws.cpu()) if fp8 else w, b)
+    got = T.qkv_rope_forward(x.to(gpu), wg, b.to(gpu), nq, nkv, 32, rotate=False, mode="decode", weight_scale=ws)
+    for have, part in zip(got, torch.split(want, (nq * 32, nkv * 32, nkv * 32), dim=1)):
+        close(have, part)
+    m = n - 3
+    y = T.out_residual_decode_forward(x.view(rows, 1, k).to(gpu), wg[:m], b[:m].to(gpu), r[:, :m].contiguous().view(rows, 1, m).to(gpu), None if ws is None else ws[:m])
+    close(y.view(rows, m), want[:, :m] + r[:, :m].float())
+
+
 @pytest.mark.parametrize("rows,hidden,nq,nkv", [(1, 64, 3, 1), (65, 128, 2, 1), (97, 2880, 64, 8), (130, 192, 40, 8), (200, 320, 64, 8),
                                                 (333, 640, 64, 8), (450, 2880, 64, 8), (600, 704, 64, 8), (999, 448, 64, 8),
                                                 (1100, 576, 64, 8), (1400, 512, 64, 8), (1500, 1024, 64, 8)])

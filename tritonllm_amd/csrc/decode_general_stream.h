@@ -2,11 +2,11 @@
 // activation rows over any K that is a multiple of 32, on v_mfma_f32_16x16x32_bf16 with the weight rows on M.
 //
 // What bounds it is how many bytes of the weight are in flight: each CU's share of HBM is ~28 GB/s, two microseconds
-// away. Four streaming wavefronts deal K by phase -- in phase p wavefront w takes the 128 K (fp8 weight: 256 K) behind
-// (4 p + w) * 128, so a workgroup asks for 1 KB contiguous of every row at a time -- and every operand goes from global
+// away. NS = 4, 2 or 1 streaming wavefronts deal K by phase -- in phase p wavefront w takes the 128 K (fp8 weight: 256 K) behind
+// (NS p + w) * 128, so that four ask for 1 KB contiguous of every row at a time -- and every operand goes from global
 // memory straight into LDS (global_load_lds_dwordx4) through a ring of two phases that belongs to the wavefront alone: no
-// barrier, no staging registers, and no wavefront waits for another one's loads. Two phases per wavefront are 48 KB (fp8
-// weight or sixteen rows: 64-96), so that two or three workgroups share a CU and a grid that does not divide by 256 (4096
+// barrier, no staging registers, and no wavefront waits for another one's loads. Two phases for each of four wavefronts are 48
+// KB (fp8 weight or sixteen rows: 64-96), so that two or three workgroups share a CU and a grid that does not divide by 256 (4096
 // wide with 80 heads: 320 workgroups) leaves no CU idle early. Measured at hidden 4096, 80 heads of 64, 8 rows: four
 // wavefronts with two phases 11.0 us, three 11.1, four (one workgroup per CU) 13.0; eight wavefronts 12.3. The kernel
 // before -- a wavefront per workgroup, loads through registers and an LDS patch -- took 14.7.
@@ -19,7 +19,7 @@ namespace tllm {
 
 template <int XR, bool W8>
 struct DecodeGeneralStream {
-  static constexpr int NS = 4;                              // streaming wavefronts
+  static constexpr int NS = 4;                              // most streaming wavefronts; 1 << ns_log2 are launched
   static constexpr int KPH = W8 ? 256 : 128;                // K of a wavefront's phase (both: 256 bytes of a weight row)
   static constexpr int PST = KPH / 32;                      // k32 steps of it
   static constexpr int XROW = KPH * 2;                      // bytes of an activation row's piece
@@ -29,8 +29,8 @@ struct DecodeGeneralStream {
   static constexpr int LPP = WL + XL;                       // load instructions per phase
   static constexpr int D = 2;                               // phases resident per wavefront
   static constexpr int REGION = WBYTES + XBYTES;
-  static constexpr int WAVE_LDS = D * REGION;
-  static constexpr int LDS = NS * WAVE_LDS;
+  // LDS of a wavefront; one that has a single phase needs no second one
+  static __host__ __device__ __forceinline__ int wave_lds(int K, int ns_log2) { return (K > (KPH << ns_log2) ? D : 1) * REGION; }
 
   // k8 group (eight consecutive K) that lane group g = lane / 16 supplies in step st of a phase. Any assignment will do
   // as long as both operands agree; this one is made for the LDS: a 128-bit read is served 16 lanes at a time, lanes 0-7
@@ -39,18 +39,18 @@ struct DecodeGeneralStream {
   // 2 i and 2 i + 1.
   static __device__ __forceinline__ int k8_of(int st, int g) { return 16 * (st >> 2) + 8 * (g >> 1) + 2 * (st & 3) + (g & 1); }
 
-  // The wavefront's share of the sixteen dot products, left as a f32x4 per lane at smem + wave * WAVE_LDS + lane * 16
+  // The wavefront's share of the sixteen dot products, left as a f32x4 per lane at smem + wave * wave_lds() + lane * 16
   // (lane: activation row lane % 16, tile rows 4 (lane / 16) .. + 3). wbase: first byte of the rows' common base,
   // wrow(i): tile row i's row index behind it (any valid row for rows past the last one).
   template <class WRow>
   static __device__ __forceinline__ void run(unsigned char* smem, int wave, int lane, const unsigned char* xbase, int nvalid,
-                                             const unsigned char* wbase, WRow wrow, int K) {
+                                             const unsigned char* wbase, WRow wrow, int K, int ns_log2) {
     const int m = lane & 15, g = lane >> 4, mx = m & (XR - 1);
     const unsigned wpitch = static_cast<unsigned>(K) * (W8 ? 1 : 2), xpitch = static_cast<unsigned>(K) * 2;
-    unsigned char* my = smem + wave * WAVE_LDS;
-    const int k0 = wave * KPH;
-    const int nph = K > k0 ? (K - k0 + NS * KPH - 1) / (NS * KPH) : 0;
-    const bool ragged = (K - k0) % (NS * KPH) != 0 && (K - k0) % (NS * KPH) < KPH;   // the last phase is cut short
+    unsigned char* my = smem + wave * wave_lds(K, ns_log2);
+    const int k0 = wave * KPH, turn = KPH << ns_log2;       // K of a phase of all wavefronts
+    const int nph = K > k0 ? (K - k0 + turn - 1) / turn : 0;
+    const bool ragged = (K - k0) % turn != 0 && (K - k0) % turn < KPH;   // the last phase is cut short
 
     // Load j of the weight: rows 4 j + lane / 16, 16-byte position lane % 16 <- chunk position ^ row. Of the
     // activations: a KB is 1024 / XROW rows, position <- chunk position ^ row likewise.
@@ -77,7 +77,7 @@ struct DecodeGeneralStream {
     auto issue = [&](int pp, int slot) {
       const int p = phase(pp);
       unsigned char* reg = my + slot * REGION;
-      const unsigned wk = static_cast<unsigned>(p * NS + wave) * 256u, xk = static_cast<unsigned>(p * NS + wave) * XROW;
+      const unsigned at_phase = static_cast<unsigned>((p << ns_log2) + wave), wk = at_phase * 256u, xk = at_phase * XROW;
       // a chunk behind the row's end re-reads the row's last one (its products are masked)
 #pragma unroll
       for (int j = 0; j < XL; ++j) {
@@ -123,7 +123,7 @@ struct DecodeGeneralStream {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (p + D < nph) issue(p + D, slot);
       if (ragged && phase(p) == nph - 1) {
-        const int left = (K - (phase(p) * NS + wave) * KPH) >> 3;  // k8 groups that exist
+        const int left = (K - ((phase(p) << ns_log2) + wave) * KPH) >> 3;  // k8 groups that exist
 #pragma unroll
         for (int st = 0; st < PST; ++st)
           if (k8_of(st, g) >= left) {
@@ -139,12 +139,12 @@ struct DecodeGeneralStream {
     *reinterpret_cast<f32x4*>(my + lane * 16) = acc;
   }
 
-  // Behind the barrier that follows run(): the four partial tiles added in a fixed order.
-  static __device__ __forceinline__ f32x4 sum(const unsigned char* smem, int lane) {
-    f32x4 t[NS];
-#pragma unroll
-    for (int w = 0; w < NS; ++w) t[w] = *reinterpret_cast<const f32x4*>(smem + w * WAVE_LDS + lane * 16);
-    return (t[0] + t[1]) + (t[2] + t[3]);
+  // Behind the barrier that follows run(): the partial tiles added in a fixed order.
+  static __device__ __forceinline__ f32x4 sum(const unsigned char* smem, int lane, int K, int ns_log2) {
+    const int stride = wave_lds(K, ns_log2);
+    auto part = [&](int w) { return *reinterpret_cast<const f32x4*>(smem + w * stride + lane * 16); };
+    if (ns_log2 == 2) return (part(0) + part(1)) + (part(2) + part(3));
+    return ns_log2 == 1 ? part(0) + part(1) : part(0);
   }
 };
 
