@@ -155,13 +155,14 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = acc2[v] = 0.f;
   constexpr int NB = XR / 2;                                  // accumulator registers that carry batch rows: row(v) = 8*(v>>2) + 4*h + (v&3)
-  float best[NB], piece[NB];                                  // piece: sums over the tile's first piece of K
+  float best[NB], piece[NB], piece2[SR ? NB : 1];             // piece: sums over the tile's first piece of K (piece2: a pair's second row)
   int best_i[NB];
 #pragma unroll
   for (int v = 0; v < NB; ++v) {
     best[v] = -3.0e38f;
     best_i[v] = 0x7fffffff;
     piece[v] = 0.f;
+    piece2[SR ? v : 0] = 0.f;
   }
 
   const unsigned char* xfrag = xs + (m & (XR - 1)) * xrow_b + h * 16;   // activations on M: tile rows >= XR repeat, never stored
@@ -241,6 +242,11 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[r] = 0.f;
           }
+        } else if (PIECES && SR && c_step == nsteps / 2 + PIECE) {   // the second row of a pair is summed in the same two pieces
+#pragma unroll
+          for (int r = 0; r < NB; ++r) piece2[SR ? r : 0] = acc2[r];
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc2[r] = 0.f;
         }
         if (SR && finished) {                            // tile finished: lane owns vocabulary rows 2 p and 2 p + 1, p = c_tile*32 + m
           const int v0 = 2 * (c_tile * 32 + m), v1 = v0 + 1;  // the vocabulary is even here: both are inside it, or neither
@@ -248,6 +254,10 @@ __global__ __launch_bounds__(UNW * 64) void unembed_kernel(UnembedArgs a) {
 #pragma unroll
           for (int r = 0; r < NB; ++r) {
             const int brow = 8 * (r >> 2) + 4 * h + (r & 3);
+            if (PIECES) {
+              acc2[r] += piece2[SR ? r : 0];
+              piece2[SR ? r : 0] = 0.f;
+            }
             const float val0 = acc[r] * sc0, val1 = acc2[r] * sc1;
             if constexpr (ARGMAX) {
               if (v0 < a.vocab && val0 > best[r]) {           // ascending order: '>' keeps the lowest index
