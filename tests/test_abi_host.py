@@ -321,5 +321,5 @@ def test_logits_of_a_small_vocabulary_stay_in_passes():
     assert [tiled(rows, 0, hidden, vocab) for rows, hidden, vocab in ((9, 4096, 1000), (16, 4096, 4000), (33, 2880, 1000), (64, 2880, 4096))] == [0] * 4
     assert [tiled(rows, 0, hidden, vocab) for rows, hidden, vocab in ((17, 4096, 1000), (65, 2880, 1000), (9, 4096, 8000), (33, 2880, 8000),
                                                                       (33, 2880, 201088))] == [1] * 5
-    assert [tiled(16, 1, 4096, 1000), tiled(33, 1, 2880, 1000), tiled(40, 0, 1024, 1000)] == [1, 0, 1]
+    assert [tiled(16, 1, 4096, 1000), tiled(16, 1, 4096, 1001), tiled(33, 1, 2880, 1000), tiled(40, 0, 1024, 1000)] == [1, 0, 0, 1]
     assert [tiled(rows, 0, 2880, 201088) for rows in (8, 32)] == [0, 0]

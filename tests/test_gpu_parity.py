@@ -1422,10 +1422,12 @@ def test_rows_of_a_power_of_two_pitch(gpu, hidden):
 
 @pytest.mark.parametrize("hidden,rows,vocab,fp8", [(4096, 8, 32000, False), (2048, 1, 200000, False), (2048, 8, 32000, True),
                                                    (4096, 8, 32000, True), (4096, 12, 32000, False), (2880, 8, 32000, False),
-                                                   (4096, 7, 30002, True), (2048, 8, 30002, True), (2048, 12, 30002, True)])
+                                                   (4096, 7, 60002, True), (2048, 8, 60002, True), (2048, 12, 60002, True), (4096, 7, 49152, True), (4096, 7, 49154, True),
+                                                   (4096, 8, 12288, False), (4096, 8, 12290, False)])
 def test_equal_rows_have_equal_logits(gpu, hidden, rows, vocab, fp8):
     """Two equal rows of the weight give the same number whichever workgroups they fall to (a pitch of a multiple of 4 KB: where
-    the walk over K does not begin at 0 everywhere) and whether they are the first or the second of a pair (fp8), so that a caller's argmax over the logits sees a tie, as the argmax op does."""
+    the walk over K does not begin at 0 everywhere, from a vocabulary of about 12000, 24000 or 49000 on) and whether they are the
+    first or the second of a pair (fp8), so that a caller's argmax over the logits sees a tie, as the argmax op does."""
     g = torch.Generator(device=gpu).manual_seed(hidden + rows)
     x = torch.randn(rows, 1, hidden, device=gpu, generator=g).bfloat16()
     w = (0.02 * torch.randn(vocab // 2, hidden, device=gpu, generator=g)).bfloat16()

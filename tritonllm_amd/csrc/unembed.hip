@@ -662,11 +662,11 @@ int unembed_check(const char* who, const void* x, const void* W, bool w8, int64_
 // than a sixteen-row unit: the passes' few workgroups are on the machine together then, and a tile is sixteen units, one of them
 // real (us, two passes and tiles: 4096 wide, 16 rows, vocabulary 1000 25.5 and 35.0, 4096 26.5 and 37.1, 4200 40.9 and 37.0; 2880
 // wide, 40 rows 30.8 and 31.6, 30.6 and 32.9, 42.2 and 32.9; three passes 24 rows 45 and 37; 1024 wide 16.3 and 12.2; the
-// eight-row passes of an fp8 weight 41 and 29).
+// eight-row passes of an fp8 weight 41 and 29, where its rows do not go in pairs 25.8 and 28.5).
 bool unembed_tiled(int64_t rows, bool w8, int64_t hidden, int64_t vocab) {
   const bool rows32 = unembed_rows32(rows, w8, hidden, vocab, false);
   const int64_t one_pass = rows32 ? 32 : unembed_xr(rows, w8, hidden);
-  const int64_t passes = vocab <= 16 * kUnembedGrid && hidden >= 2560 && (rows32 || !w8) ? 2 : 1;
+  const int64_t passes = vocab <= 16 * kUnembedGrid && hidden >= 2560 && (rows32 || !w8 || vocab % 2) ? 2 : 1;
   return rows > passes * one_pass && unembed_tiles_fit(rows, w8, hidden, vocab);
 }
 
@@ -689,7 +689,12 @@ int unembed_launch(const char* who, const UnembedArgs& a, bool w8, hipStream_t s
   const bool pairs16 = unembed_pairs16(a.rows, w8, a.hidden, a.vocab);
   const size_t smem = pairs ? smem_pairs : (pairs16 ? smem_pairs16 : unembed_smem(xr, w8, a.hidden));
   const dim3 grid(kUnembedGrid, (unsigned)((a.rows + xr - 1) / xr));
-  const bool pieces = !ARGMAX && (a.hidden * (w8 && !pairs && !pairs16 ? 1 : 2)) % 4096 == 0;   // (such a width is no multiple of 192 that fits the LDS)
+  // PIECES from a vocabulary on that keeps the channels busy: below, the pieces' additions are 1 - 3 us at its end and nothing is gained
+  // (us, in step and in pieces; 4096 wide, 500 rows 21.1 and 22.1, 8000 23.3 and 23.2, 14001 27.8 and 25.4; fp8 14001 23.5 and 24.4,
+  // 28003 32.2 and 28.8; pairs of rows 500 36.8 and 40.0, 32000 42.5 and 43.2, 50002 50.0 and 47.9, 64002 59.8 and 51.4; 2048 wide, pairs,
+  // 40002 24.3 and 26.8, 64002 33.7 and 28.7). (Such a width is no multiple of 192 that fits the LDS.)
+  const bool in_pairs = pairs || pairs16;
+  const bool pieces = !ARGMAX && (a.hidden * (w8 && !in_pairs ? 1 : 2)) % 4096 == 0 && a.vocab > (in_pairs ? 49152 : w8 ? 24576 : 12288);
 #define TLLM_UNEMBED(XR, NW, KS, UD, W8F, SR)                                                                               \
   do {                                                                                                                      \
     auto kern = unembed_kernel<XR, NW, KS, UD, W8F, ARGMAX, SR>;                                                            \
