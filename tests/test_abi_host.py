@@ -267,6 +267,9 @@ def test_attention_decode_shape_planning():
     # more than eight KV heads: where one split fewer is as good but leaves CUs without a workgroup, the splits stay
     assert [(hpw(b, n, c, 0), splits(b, n, c, 0)) for b, n, c in ((33, 16, 2048), (49, 16, 4096), (24, 32, 2048), (33, 24, 3000))] == [(4, 2)] * 4
     assert (hpw(38, 16, 3000, 0), splits(38, 16, 3000, 0)) == (8, 3)
+    # one launch of eight wavefronts per KV head, as long as its few workgroups are not what takes longest
+    assert [splits(b, 8, c, 0) for b, c in ((1, 512), (7, 512), (8, 640), (11, 640), (12, 800), (16, 800))] == [1] * 6
+    assert all(splits(b, 8, c, 0) > 1 for b, c in ((8, 700), (8, 800), (9, 700), (10, 700), (11, 641)))
     for b in (1, 3, 8, 100):
         for ctx in (1, 127, 128, 129, 5000, 131072):
             s = splits(b, 8, ctx, 0)

@@ -1631,7 +1631,7 @@ def test_attention_decode_row_workgroups(gpu, case):
 
 
 @pytest.mark.parametrize("batch_size,num_keys,start_q,hpw", [
-    (1, 129, 128, 0), (1, 512, 511, 0), (3, 200, 37, 0), (8, 800, 799, 0),          # eight wavefronts per KV head; less than a block each
+    (1, 129, 128, 0), (1, 512, 511, 0), (3, 200, 37, 0), (8, 640, 639, 0), (8, 800, 799, 0), (12, 800, 799, 0),        # eight wavefronts per KV head; less than a block each
     (33, 256, 255, 2), (64, 1280, 1279, 2), (49, 1111, 1110, 2), (43, 4096, 30, 2),   # two heads, two wavefronts each: ragged, nearly empty
     (8, 3000, 2999, 2), (16, 1111, 700, 2),                                           # ... with context splits
     (65, 100, 99, 4), (97, 333, 332, 4), (111, 515, 31, 4), (128, 511, 0, 4),         # four heads, two wavefronts each

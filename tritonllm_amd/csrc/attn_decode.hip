@@ -423,9 +423,10 @@ using namespace tllm;
 //   4 x 2   B = 65 .. 111, and up to 128 below 512 keys; contexts up to 8192: B = 80 at 1111 42.7 -> 32.5, at 2048 66.6 -> 54.1, B = 85 at 8192 245 -> 214, B = 96 at 256
 //           15.8 -> 12.1, at 1111 50.9 -> 36.8, B = 128 at 256 19.6 -> 15.5; window of 128: B = 96 9.6 -> 8.9, B = 128 12.4 -> 10.6
 //           (from B = 112 and 512 keys on one wavefront per head fills the CUs as well and is ahead: 68.7 against 73 at 2048)
-//   1 x 8   up to 128 streams and 512 keys, 64 .. 128 streams and 800 keys: B = 1 at 256 6.0 -> 4.4, B = 5 at 400 7.0 -> 6.3,
-//           B = 8 at 700 8.5 -> 7.7, B = 12 at 256 7.5 -> 5.4, B = 16 at 512 8.9 -> 7.4 (beyond: two launches are ahead, B = 5 at 1111
-//           8.5 and 9.1, B = 14 at 900 11.5 and 12.2)
+//   1 x 8   up to 128 streams and 512 keys, from 64 streams on 640, from 96 on 800: B = 1 at 256 6.0 -> 4.4, B = 5 at 400 7.0 -> 6.3,
+//           B = 12 at 256 7.5 -> 5.4, B = 16 at 512 8.9 -> 7.4 (beyond: two launches are ahead, B = 5 at 1111 8.5 and 9.1, B = 14 at 900
+//           11.5 and 12.2; with the keys in no cache B = 8 at 700 8.9 and 9.6, at 800 9.4 and 10.9, B = 10 at 700 9.5 and 10.3, B = 12 at 800
+//           11.4 and 11.2)
 // 2 x 2 with splits of 257 - 511 keys: its 256-byte pieces stream nearly as fast as ROWS' and it needs half as many splits:
 // B = 8 at 3000 16.1 -> 13.8, B = 16 at 1111 14.0 -> 12.5 (fewer than 64 streams: B = 5 at 4096 15.0 -> 13.4, but planned for
 // 4096 with 300 visible 7.1 -> 8.0; HEAD kept).
@@ -462,7 +463,7 @@ static AttnPlan attn_plan(int64_t batch, int n_kv_heads, int64_t n_kv_ctx, int w
     if (ctx <= kUnsplitQuads && quads > 128 && (quads < 224 || (quads <= 256 && ctx < 512))) return {4, 2, 1, 1, kRowsKeysShift};
     if (ctx >= 256 && ctx <= kUnsplitPairs && pairs > 128 && pairs <= 256 && (pairs > 168 || ctx <= 1280)) return {2, 2, 1, 1, kRowsKeysShift};
   }
-  if (ctx > 128 && streams <= 128 && ctx <= (streams >= 64 ? 800 : 512)) return {1, 8, 1, 1, kHeadKeysShift};
+  if (ctx > 128 && streams <= 128 && ctx <= (streams >= 96 ? 800 : streams >= 64 ? 640 : 512)) return {1, 8, 1, 1, kHeadKeysShift};
   // eight or four KV heads per workgroup: whichever fills the machine with the longest splits (ties: the wider one). If neither
   // does, and that is because one split fewer was as good (more than eight KV heads), with the splits that it had: 16 heads, B = 49
   // at 2048 HEAD 97 us, so 70; 24 heads, B = 33 at 4096 179 and 137; 12 heads, B = 44 at 1400 as good either way
