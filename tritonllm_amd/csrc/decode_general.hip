@@ -9,7 +9,7 @@
 // HBM-bound: 8 rows, [4096, 4096] weight 7.1 us = 4.7 TB/s, of which 1.6 us are the launch (a wavefront per dot product:
 // 89.7 us); QKV at hidden 4096, 80 heads of 64 11.0 us = 3.8 TB/s (14.7 before), fp8 weight 8.0 (13.5). Above 8 rows the
 // sixteen-row form: its activations are half of what a workgroup reads, from the L2s, and there are as many workgroups per
-// weight row as chunks of rows (streams_log2 below).
+// weight row as chunks of rows (streams below).
 #include "decode_general_stream.h"
 #include "out_common.h"
 #include "qkv_common.h"
@@ -18,9 +18,9 @@ namespace tllm {
 
 // Rows [8 piece, 8 piece + 8) of a head and their rotation partners half = head_dim / 2 further on; tile row 4 qd + i is
 // dim 8 piece + 2 qd + (i & 1), plus half when i >= 2, so that a lane's four sums are two complete (lo, hi) pairs.
-template <int XR, bool W8>
-__global__ __launch_bounds__(320) void qkv_decode_general_kernel(QkvArgs a, RopeArgs ra, YarnFreqs fr, int ns_log2) {
-  using S = DecodeGeneralStream<XR, W8>;
+template <int XR, bool W8, int NS>
+__global__ __launch_bounds__(64 * (NS + 1)) void qkv_decode_general_kernel(QkvArgs a, RopeArgs ra, YarnFreqs fr) {
+  using S = DecodeGeneralStream<XR, W8, NS>;
   extern __shared__ __align__(1024) unsigned char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
@@ -28,10 +28,10 @@ __global__ __launch_bounds__(320) void qkv_decode_general_kernel(QkvArgs a, Rope
   const int head = blockIdx.x / pieces, piece = blockIdx.x - head * pieces;
   const int64_t row0 = static_cast<int64_t>(blockIdx.y) * XR;
   const int nvalid = static_cast<int>(a.rows - row0 < XR ? a.rows - row0 : XR);
-  if (wave < 1 << ns_log2) {
+  if (wave < NS) {
     const unsigned char* wbase = reinterpret_cast<const unsigned char*>(a.W) + static_cast<int64_t>(head) * a.head_dim * a.hidden * (W8 ? 1 : 2);
     S::run(smem, wave, lane, reinterpret_cast<const unsigned char*>(a.x + row0 * a.hidden), nvalid, wbase,
-           [&](int i) { return 8 * piece + 2 * (i >> 2) + (i & 1) + ((i & 2) ? half : 0); }, a.hidden, ns_log2);
+           [&](int i) { return 8 * piece + 2 * (i >> 2) + (i & 1) + ((i & 2) ? half : 0); }, a.hidden);
     __syncthreads();
     return;
   }
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(320) void qkv_decode_general_kernel(QkvArgs a, Rope
   asm volatile("" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(c0), "+v"(s0), "+v"(c1), "+v"(s1), "+v"(out));
   if constexpr (W8) asm volatile("" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]));
   __syncthreads();
-  const f32x4 t = S::sum(smem, lane, a.hidden, ns_log2);
+  const f32x4 t = S::sum(smem, lane, a.hidden);
   if (m >= nvalid) return;
   const float lo0 = t[0] * s[0] + b[0], lo1 = t[1] * s[1] + b[1], hi0 = t[2] * s[2] + b[2], hi1 = t[3] * s[3] + b[3];
   bf16x2 lo, hi;
@@ -68,20 +68,20 @@ __global__ __launch_bounds__(320) void qkv_decode_general_kernel(QkvArgs a, Rope
   *reinterpret_cast<bf16x2*>(out + half) = hi;
 }
 
-template <int XR, bool W8>
-__global__ __launch_bounds__(320) void out_decode_general_kernel(OutArgs a, int vec8, int ns_log2) {
-  using S = DecodeGeneralStream<XR, W8>;
+template <int XR, bool W8, int NS>
+__global__ __launch_bounds__(64 * (NS + 1)) void out_decode_general_kernel(OutArgs a, int vec8) {
+  using S = DecodeGeneralStream<XR, W8, NS>;
   extern __shared__ __align__(1024) unsigned char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   const int n0 = blockIdx.x * 16;
   const int64_t row0 = static_cast<int64_t>(blockIdx.y) * XR;
   const int nvalid = static_cast<int>(a.rows - row0 < XR ? a.rows - row0 : XR);
-  if (wave < 1 << ns_log2) {
+  if (wave < NS) {
     const unsigned char* wbase = reinterpret_cast<const unsigned char*>(a.W) + static_cast<int64_t>(n0) * a.in_dim * (W8 ? 1 : 2);
     const int last = a.out_dim - 1 - n0;
     S::run(smem, wave, lane, reinterpret_cast<const unsigned char*>(a.x + row0 * a.in_dim), nvalid, wbase,
-           [&](int i) { return i < last ? i : last; }, a.in_dim, ns_log2);
+           [&](int i) { return i < last ? i : last; }, a.in_dim);
     __syncthreads();
     return;
   }
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(320) void out_decode_general_kernel(OutArgs a, int 
   }
   asm volatile("" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]));
   __syncthreads();
-  const f32x4 t = S::sum(smem, lane, a.in_dim, ns_log2);
+  const f32x4 t = S::sum(smem, lane, a.in_dim);
   if (m >= nvalid || nfeat <= 0) return;
   bf16* out = a.out + row * a.out_rs + feat;
   bf16x4 o;
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(320) void out_decode_general_kernel(OutArgs a, int 
 }
 
 namespace {
-// Streaming wavefronts of a workgroup, as a power of two: no more than K has phases for, and four as long as all workgroups are on
+// Streaming wavefronts of a workgroup: no more than K has phases for, and four as long as all workgroups are on
 // the machine with them. Beyond that fewer, whose LDS lets more workgroups onto a CU (24 KB per wavefront with an fp8 weight:
 // one of 96 KB, three of 48, six): a workgroup's fixed time is then somebody else's stream. us, a wavefront per workgroup (the kernel
 // before this one), four, two, one; fp8, 80 heads of 64:
@@ -143,36 +143,43 @@ namespace {
 // and four wavefronts' LDS where K is one phase (fp8, 256 wide, 400 rows 28.7 before, 57.2, now 14.7). Up to eight rows there are as
 // many workgroups as the weight has sixteen rows: four.
 template <int XR, bool W8>
-int streams_log2(int K, int64_t workgroups) {
-  constexpr int KPH = DecodeGeneralStream<XR, W8>::KPH;
-  const int most = K > 2 * KPH ? 2 : K > KPH ? 1 : 0;
+int streams(int K, int64_t workgroups) {
+  constexpr int KPH = DecodeGeneralStream<XR, W8, 1>::KPH;
+  const int most = K > 2 * KPH ? 4 : K > KPH ? 2 : 1;
   if (XR == 8) return most;
-  const int fill = workgroups <= (W8 ? 256 : 352) ? 2 : workgroups <= (W8 ? 768 : 512) ? 1 : 0;
+  const int fill = workgroups <= (W8 ? 256 : 352) ? 4 : workgroups <= (W8 ? 768 : 512) ? 2 : 1;
   return fill < most ? fill : most;
 }
 
-template <int XR, bool W8, auto kernel, class... Args>
+template <class S, auto kernel, int NS, class... Args>
 int launch(const char* what, int K, unsigned gx, int64_t gy, hipStream_t st, const Args&... args) {
-  typedef DecodeGeneralStream<XR, W8> S;
   TLLM_REQUIRE(gy <= 65535, TLLM_E_SHAPE, "%s: too many rows for the decode kernel", what);
-  const int ns_log2 = streams_log2<XR, W8>(K, static_cast<int64_t>(gx) * gy), lds = S::wave_lds(K, ns_log2) << ns_log2;
+  const int lds = NS * S::wave_lds(K);
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> done{0};
-    hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kernel), S::NS * S::D * S::REGION, done);
+    hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds, done);   // (the larger of the kernel's two sizes)
     TLLM_REQUIRE(e == hipSuccess, TLLM_E_LAUNCH, "%s: cannot raise LDS limit: %s", what, hipGetErrorString(e));
   }
-  hipLaunchKernelGGL(kernel, dim3(gx, (unsigned)gy), dim3(64 * ((1 << ns_log2) + 1)), (size_t)lds, st, args..., ns_log2);
+  hipLaunchKernelGGL(kernel, dim3(gx, (unsigned)gy), dim3(64 * (NS + 1)), (size_t)lds, st, args...);
   return check_launch(what);
 }
 
 template <int XR, bool W8>
 int launch_qkv(const char* what, unsigned gx, int64_t gy, hipStream_t st, const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& fr) {
-  return launch<XR, W8, qkv_decode_general_kernel<XR, W8>>(what, a.hidden, gx, gy, st, a, ra, fr);
+  switch (streams<XR, W8>(a.hidden, gx * gy)) {
+    case 4: return launch<DecodeGeneralStream<XR, W8, 4>, qkv_decode_general_kernel<XR, W8, 4>, 4>(what, a.hidden, gx, gy, st, a, ra, fr);
+    case 2: return launch<DecodeGeneralStream<XR, W8, 2>, qkv_decode_general_kernel<XR, W8, 2>, 2>(what, a.hidden, gx, gy, st, a, ra, fr);
+    default: return launch<DecodeGeneralStream<XR, W8, 1>, qkv_decode_general_kernel<XR, W8, 1>, 1>(what, a.hidden, gx, gy, st, a, ra, fr);
+  }
 }
 
 template <int XR, bool W8>
 int launch_out(const char* what, unsigned gx, int64_t gy, hipStream_t st, const OutArgs& a, int vec8) {
-  return launch<XR, W8, out_decode_general_kernel<XR, W8>>(what, static_cast<int>(a.in_dim), gx, gy, st, a, vec8);
+  switch (streams<XR, W8>(a.in_dim, gx * gy)) {
+    case 4: return launch<DecodeGeneralStream<XR, W8, 4>, out_decode_general_kernel<XR, W8, 4>, 4>(what, a.in_dim, gx, gy, st, a, vec8);
+    case 2: return launch<DecodeGeneralStream<XR, W8, 2>, out_decode_general_kernel<XR, W8, 2>, 2>(what, a.in_dim, gx, gy, st, a, vec8);
+    default: return launch<DecodeGeneralStream<XR, W8, 1>, out_decode_general_kernel<XR, W8, 1>, 1>(what, a.in_dim, gx, gy, st, a, vec8);
+  }
 }
 
 int64_t chunks_of(int64_t rows) { return rows <= 8 ? 1 : (rows + 15) / 16; }
@@ -203,6 +210,6 @@ extern "C" int tllm_decode_general_streams(int64_t rows, int64_t in_dim, int64_t
   if (rows < 1 || in_dim < 1 || in_dim > INT32_MAX || out_dim < 1) return 0;
   const int K = static_cast<int>(in_dim);
   const int64_t workgroups = (out_dim + 15) / 16 * chunks_of(rows);
-  if (rows <= 8) return 1 << (fp8 ? streams_log2<8, true>(K, workgroups) : streams_log2<8, false>(K, workgroups));
-  return 1 << (fp8 ? streams_log2<16, true>(K, workgroups) : streams_log2<16, false>(K, workgroups));
+  if (rows <= 8) return fp8 ? streams<8, true>(K, workgroups) : streams<8, false>(K, workgroups);
+  return fp8 ? streams<16, true>(K, workgroups) : streams<16, false>(K, workgroups);
 }

@@ -17,9 +17,9 @@
 
 namespace tllm {
 
-template <int XR, bool W8>
+// NS: streaming wavefronts of a workgroup (4, 2 or 1)
+template <int XR, bool W8, int NS>
 struct DecodeGeneralStream {
-  static constexpr int NS = 4;                              // most streaming wavefronts; 1 << ns_log2 are launched
   static constexpr int KPH = W8 ? 256 : 128;                // K of a wavefront's phase (both: 256 bytes of a weight row)
   static constexpr int PST = KPH / 32;                      // k32 steps of it
   static constexpr int XROW = KPH * 2;                      // bytes of an activation row's piece
@@ -30,7 +30,7 @@ struct DecodeGeneralStream {
   static constexpr int D = 2;                               // phases resident per wavefront
   static constexpr int REGION = WBYTES + XBYTES;
   // LDS of a wavefront; one that has a single phase needs no second one
-  static __host__ __device__ __forceinline__ int wave_lds(int K, int ns_log2) { return (K > (KPH << ns_log2) ? D : 1) * REGION; }
+  static __host__ __device__ __forceinline__ int wave_lds(int K) { return (K > NS * KPH ? D : 1) * REGION; }
 
   // k8 group (eight consecutive K) that lane group g = lane / 16 supplies in step st of a phase. Any assignment will do
   // as long as both operands agree; this one is made for the LDS: a 128-bit read is served 16 lanes at a time, lanes 0-7
@@ -44,13 +44,13 @@ struct DecodeGeneralStream {
   // wrow(i): tile row i's row index behind it (any valid row for rows past the last one).
   template <class WRow>
   static __device__ __forceinline__ void run(unsigned char* smem, int wave, int lane, const unsigned char* xbase, int nvalid,
-                                             const unsigned char* wbase, WRow wrow, int K, int ns_log2) {
+                                             const unsigned char* wbase, WRow wrow, int K) {
     const int m = lane & 15, g = lane >> 4, mx = m & (XR - 1);
     const unsigned wpitch = static_cast<unsigned>(K) * (W8 ? 1 : 2), xpitch = static_cast<unsigned>(K) * 2;
-    unsigned char* my = smem + wave * wave_lds(K, ns_log2);
-    const int k0 = wave * KPH, turn = KPH << ns_log2;       // K of a phase of all wavefronts
-    const int nph = K > k0 ? (K - k0 + turn - 1) / turn : 0;
-    const bool ragged = (K - k0) % turn != 0 && (K - k0) % turn < KPH;   // the last phase is cut short
+    unsigned char* my = smem + wave * wave_lds(K);
+    const int k0 = wave * KPH;
+    const int nph = K > k0 ? (K - k0 + NS * KPH - 1) / (NS * KPH) : 0;
+    const bool ragged = (K - k0) % (NS * KPH) != 0 && (K - k0) % (NS * KPH) < KPH;   // the last phase is cut short
 
     // Load j of the weight: rows 4 j + lane / 16, 16-byte position lane % 16 <- chunk position ^ row. Of the
     // activations: a KB is 1024 / XROW rows, position <- chunk position ^ row likewise.
@@ -77,7 +77,7 @@ struct DecodeGeneralStream {
     auto issue = [&](int pp, int slot) {
       const int p = phase(pp);
       unsigned char* reg = my + slot * REGION;
-      const unsigned at_phase = static_cast<unsigned>((p << ns_log2) + wave), wk = at_phase * 256u, xk = at_phase * XROW;
+      const unsigned wk = static_cast<unsigned>(p * NS + wave) * 256u, xk = static_cast<unsigned>(p * NS + wave) * XROW;
       // a chunk behind the row's end re-reads the row's last one (its products are masked)
 #pragma unroll
       for (int j = 0; j < XL; ++j) {
@@ -123,7 +123,7 @@ struct DecodeGeneralStream {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (p + D < nph) issue(p + D, slot);
       if (ragged && phase(p) == nph - 1) {
-        const int left = (K - ((phase(p) << ns_log2) + wave) * KPH) >> 3;  // k8 groups that exist
+        const int left = (K - (phase(p) * NS + wave) * KPH) >> 3;  // k8 groups that exist
 #pragma unroll
         for (int st = 0; st < PST; ++st)
           if (k8_of(st, g) >= left) {
@@ -140,11 +140,13 @@ struct DecodeGeneralStream {
   }
 
   // Behind the barrier that follows run(): the partial tiles added in a fixed order.
-  static __device__ __forceinline__ f32x4 sum(const unsigned char* smem, int lane, int K, int ns_log2) {
-    const int stride = wave_lds(K, ns_log2);
-    auto part = [&](int w) { return *reinterpret_cast<const f32x4*>(smem + w * stride + lane * 16); };
-    if (ns_log2 == 2) return (part(0) + part(1)) + (part(2) + part(3));
-    return ns_log2 == 1 ? part(0) + part(1) : part(0);
+  static __device__ __forceinline__ f32x4 sum(const unsigned char* smem, int lane, int K) {
+    f32x4 t[NS];
+#pragma unroll
+    for (int w = 0; w < NS; ++w) t[w] = *reinterpret_cast<const f32x4*>(smem + w * wave_lds(K) + lane * 16);
+    if constexpr (NS == 4) return (t[0] + t[1]) + (t[2] + t[3]);
+    else if constexpr (NS == 2) return t[0] + t[1];
+    else return t[0];
   }
 };
 
