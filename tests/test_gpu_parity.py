@@ -1792,6 +1792,38 @@ def test_attention_prefill_large_launch_ragged(gpu, sliding_window):
     _attn_prefill_case(gpu, 4, 600, 700, sliding_window, 77, start_dtype=torch.int64, seed=41)
 
 
+@pytest.mark.parametrize("batch_size,num_queries,num_keys,start_q,window,kv", [
+    (1, 777, 777, 0, None, dict()),                                            # 64 queries x 2 heads, one per wavefront
+    (1, 833, 1200, 310, 257, dict()),                                          # the window's edge inside blocks; keys beyond the last query
+    (1, 600, 448, 0, None, dict(with_sinks=False)),                            # as short as walks in chunks get; queries past the keys
+    (4, 600, 700, 77, 400, dict()),                                            # 64 queries x 4 heads, two per wavefront
+    (3, 449, 640, 191, 321, dict(groups=4, kv_heads=16)),
+    (8, 650, 700, 49, None, dict(groups=2)), (6, 700, 777, 40, 350, dict(groups=6, kv_heads=4)),      # 128 queries x 2 heads
+    (2, 1000, 1100, 100, 300, dict(groups=5)),                                 # 128 queries x 1 head
+], ids=str)
+def test_attention_prefill_chunks(gpu, batch_size, num_queries, num_keys, start_q, window, kv):
+    """Walks of more than six key blocks, which run in chunks of 32 keys x one head."""
+    assert _lib.lib().tllm_attention_prefill_key_groups(batch_size, num_queries, num_keys, kv.get("kv_heads", 8), kv.get("groups", 8), window or 0) == 1
+    _attn_prefill_case(gpu, batch_size, num_queries, num_keys, window, start_q, seed=num_queries + num_keys, **kv)
+
+
+@pytest.mark.parametrize("batch_size,num_queries", [(1, 777), (4, 600)])
+def test_attention_prefill_growing_logits(gpu, batch_size, num_queries):
+    """Keys that grow along the context, so that block after block tops what the weights are taken relative to by far more than
+    2^8; and one query of nan, which stays alone."""
+    g = torch.Generator().manual_seed(77)
+    q = torch.randn(batch_size, num_queries, 8, 8, 64, generator=g).bfloat16()
+    k = (torch.randn(batch_size, num_queries, 8, 64, generator=g) * torch.linspace(0.1, 60.0, num_queries)[None, :, None, None]).bfloat16()
+    v = torch.randn(batch_size, num_queries, 8, 64, generator=g).bfloat16()
+    sinks = torch.randn(64, generator=g).bfloat16()
+    q[0, 40] = float("nan")
+    o1 = T.attention(q.to(gpu), k.to(gpu), v.to(gpu), sinks.to(gpu), 0.125, None, torch.tensor([0], device=gpu)).float().cpu()
+    o2 = O.attention_ref(q, k, v, sinks, 0.125, None, 0).float()
+    assert o1[0, 40].isnan().all()
+    o1[0, 40] = o2[0, 40] = 0.0
+    close(o1, o2)
+
+
 def test_attention_graph_replay_follows_device_start(gpu):
     """Both attention kernels read start_q on the device: a graph captured once follows the tensor's new value on every
     replay (decode: the growing context; prefill: the next chunk of a prompt), with eager work between the replays."""
