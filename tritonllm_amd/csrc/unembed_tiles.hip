@@ -6,19 +6,21 @@
 // What bounds it is the weight, 1.16 GB at gpt-oss's size, and the kernels for few rows read it once per chunk of 32 rows
 // (of 8, for a model too wide for 32 rows in the LDS). Here K is cut into slices of 64 instead, and a slice of the
 // activations travels with the weight's: one workgroup of eight wavefronts per CU owns a contiguous run of the vocabulary
-// for the whole launch and walks it in tiles of up to 256 vocabulary rows (the run divided evenly: 49 sixteen-row units per
-// CU are four tiles of thirteen, not three of sixteen and one of one), and the ring of S stages -- global memory straight
-// into LDS, 16-byte chunks XOR-swizzled by row -- runs on across tiles, so that 64-96 KB of the weight are in flight per CU
-// from the first instruction to the last. The activations (737 KB at 128 rows) come from the L2, once per tile: a stage is
-// 32 KB of weight and 4-16 KB of them, and they take their share of the loads a CU can have in flight, which is what the
-// time grows with (tiles of 128: 49 rows 225 us against 219, 128 rows 280 against 261). Wavefronts: four over the
-// vocabulary (four units each) x two over the batch rows, on v_mfma_f32_16x16x32_bf16 with the vocabulary on M, so that a
-// lane ends up with four consecutive logits of a row. One barrier per stage.
+// for the whole launch and walks it in tiles of up to 20 (bf16) or 28 (fp8) units of sixteen vocabulary rows (the run divided
+// evenly: 50 units per CU are three tiles of seventeen, not two of twenty and one of ten), and the ring of S stages -- global
+// memory straight into LDS, 16-byte chunks XOR-swizzled by row -- runs on across tiles, so that 64-96 KB of the weight are in
+// flight per CU from the first instruction to the last. The activations (737 KB at 128 rows) come from the L2, once per tile.
+// A CU takes in 33-35 GB/s of this stream, whatever mixture of the two it is (its loads come back in order, the weight's from
+// memory among them), so what counts is bytes: few tall tiles, no row of either operand that is not needed, the loads of a
+// stage dealt to the wavefronts one by one. Wavefronts: four over the vocabulary x two over the batch rows, on
+// v_mfma_f32_16x16x32_bf16 with the vocabulary on M, so that a lane ends up with four consecutive logits of a row. One barrier
+// per stage.
 //
-// [rows, 2880] x [201088, 2880], us (before: chunks of 32 rows, of 8 where the width is 4096; a read of the weight alone: 174):
-//   bf16   33 rows 205 (377)   49 219 (382)   64 228 (386)   96 245 (586)   128 261 (782)   200 510 (1370)
-//   fp8    33 rows 138 (240)   49 145 (251)   64 149 (253)   96 179 (372)   128 209 (491)
-//   4096 wide, bf16: 9 rows 251 (520)   32 280 (1035)   64 307 (2065)   128 346 (4098)
+// [rows, 2880] x [201088, 2880], us (in brackets four tiles of thirteen units whose stages had room and loads for sixteen; in
+// chunks of 32 rows, of 8 where the width is 4096; a read of the weight alone: 174):
+//   bf16   33 rows 198 (205, 377)   49 200 (218, 382)   64 205 (228, 386)   96 219 (245, 586)   128 240 (262, 782)   200 465 (510, 1370)
+//   fp8    33 rows 133 (143, 240)   49 139 (148, 251)   64 144 (153, 253)   96 157 (177, 372)   128 178 (205, 491)
+//   4096 wide, bf16: 9 rows 262 (257, 520; on another GPU 283 and 288)   32 275 (285, 1035)   49 273 (294)   128 313 (344, 4098)
 #include <atomic>
 
 #include "qkv_prefill.h"
@@ -27,106 +29,123 @@
 namespace tllm {
 
 namespace unembed_tiles {
-constexpr int BK = 64, NW = 8, UNITS = 16;      // K slice; wavefronts; sixteen-row units of a tile
-constexpr int MAX_RUN = 64;                    // units of a workgroup's run whose fp8 scales the LDS holds
+constexpr int BK = 64, NW = 8;                 // K slice; wavefronts
+constexpr int MAX_RUN = 64;                    // units (sixteen vocabulary rows) of a workgroup's run whose fp8 scales the LDS holds
+constexpr int LDS = 160 * 1024;
 
-template <int MB, bool W8>                     // MB blocks of sixteen batch rows
+template <int MB, bool W8, int UB>             // MB blocks of sixteen batch rows, up to UB units for each of the four wavefronts over the vocabulary
 struct Shape {
   static_assert(MB % 2 == 0 && MB >= 2 && MB <= 8, "two wavefronts over the batch rows");
-  static constexpr int WROW = W8 ? 64 : 128;                 // LDS bytes of a weight row's slice
-  static constexpr int WBYTES = UNITS * 16 * WROW, XBYTES = MB * 16 * 128, STAGE = WBYTES + XBYTES;
-  static constexpr int TAIL = W8 ? MAX_RUN * 16 * 4 : 0;
-  static constexpr int S_FIT = (160 * 1024 - TAIL) / STAGE, S = S_FIT > 8 ? 8 : S_FIT;
-  static constexpr int SMEM = S * STAGE + TAIL;
-  static constexpr int LW = (W8 ? 1 : 2) * UNITS / NW;                      // loads of 1 KB per wavefront and stage: its unit of the weight ...
-  static constexpr int XR = MB * 2, LX = (XR + 7) / 8;       // ... and XR rows of the activations, eight to a load, the last one may be half
-  static constexpr int LPW = LW + LX;
-  static_assert(S >= 3 && (S - 2) * LPW < 64, "the loads in flight are countable");
+  static constexpr int WROW = W8 ? 64 : 128, UBYTES = 16 * WROW;   // LDS bytes of a weight row's slice, of a unit's
+  static constexpr int XBYTES = MB * 16 * 128, TAIL = W8 ? MAX_RUN * 16 * 4 : 0;
+  static constexpr int LU = W8 ? 1 : 2;                      // loads of 1 KB per unit and stage
+  static constexpr int LMAX = (4 * UB * LU + MB * 2 + NW - 1) / NW;         // most loads of a wavefront per stage
+  static constexpr int most(int stages) {                    // units of the widest tile of which so many stages fit
+    const int fit = ((LDS - TAIL) / stages - XBYTES) / UBYTES;
+    return fit < 4 * UB ? fit : 4 * UB;
+  }
 };
 }  // namespace unembed_tiles
 
-template <int MB, bool W8>
-__global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int chunk_rows) {
+// Wait until at most the loads of `STAGES` stages of `cnt` (<= N) loads each are in flight.
+template <int N, int STAGES>
+__device__ __forceinline__ void wait_stages(int cnt) {
+  if constexpr (N == 0) {
+    (void)cnt;                                               // (a wavefront without loads)
+  } else {
+    if (cnt == N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N * STAGES) : "memory");
+    else wait_stages<N - 1, STAGES>(cnt);
+  }
+}
+
+// S stages in the ring; `slots`: units that a stage has room for, the widest tile of the launch.
+template <int MB, bool W8, int UB, int S>
+__global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int chunk_rows, int slots) {
   using namespace unembed_tiles;
-  typedef Shape<MB, W8> C;
-  constexpr int S = C::S, STAGE = C::STAGE, WBYTES = C::WBYTES, WROW = C::WROW, XR = C::XR, LX = C::LX, LW = C::LW, LPW = C::LPW, TB = MB / 2, UB = UNITS / 4;
+  typedef Shape<MB, W8, UB> C;
+  constexpr int UBYTES = C::UBYTES, LU = C::LU, LMAX = C::LMAX, TB = MB / 2;
+  static_assert((S - 2) * LMAX < 64, "the loads in flight are countable");
   extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = wave & 3, wm = wave >> 2, m16 = lane & 15, g = lane >> 4;
+  const int wbytes = slots * UBYTES, stage_bytes = wbytes + C::XBYTES;
 
   // ---- this workgroup's run of the vocabulary and its tiles
   const int units = (a.vocab + 15) >> 4, nwg = static_cast<int>(gridDim.x), wg = static_cast<int>(blockIdx.x);
   const int u0 = static_cast<int>(static_cast<int64_t>(wg) * units / nwg), u1 = static_cast<int>(static_cast<int64_t>(wg + 1) * units / nwg);
   const int run = u1 - u0;
   if (run == 0) return;                                      // the whole workgroup
-  const int ntiles = (run + UNITS - 1) / UNITS, width = (run + ntiles - 1) / ntiles;   // units per tile (the last one may be narrower)
-  const int nk = a.hidden / BK, total = ntiles * nk;         // stages of the stream
+  const int ntiles = (run + slots - 1) / slots, width = (run + ntiles - 1) / ntiles;   // units per tile (the last one may be narrower)
+  const int nk = a.hidden / BK;
   const int64_t row0 = static_cast<int64_t>(blockIdx.y) * chunk_rows;
   const int nrows = static_cast<int>(a.rows - row0 < chunk_rows ? a.rows - row0 : chunk_rows);
   const unsigned wpitch = static_cast<unsigned>(a.hidden) * (W8 ? 1 : 2), xpitch = static_cast<unsigned>(a.hidden) * 2;
   const unsigned char* const x_base = reinterpret_cast<const unsigned char*>(a.x) + row0 * a.hidden * 2;
   const unsigned char* const w_base = reinterpret_cast<const unsigned char*>(a.W) + static_cast<int64_t>(u0) * 16 * wpitch;
 
-  // ---- loads. Wavefront w fetches unit w of the tile (one past the tile's width repeats the last one: lines that are on
-  // their way already) and rows w * XR .. of the activations (rows past the last one repeat it; never stored). bf16: eight
-  // rows of 128 bytes per load, chunk position L % 8 holds chunk (L % 8) ^ swz(row). fp8: sixteen rows of 64 bytes, position
-  // L % 4 holds chunk (L % 4) ^ (row / 4).
-  unsigned xoff[LX], woff[LW];
-#pragma unroll
-  for (int j = 0; j < LX; ++j) {
-    int r = wave * XR + 8 * j + (lane >> 3);
-    const unsigned c = static_cast<unsigned>((lane & 7) ^ swz(r)) * 16u;
-    r = r < nrows ? r : nrows - 1;
-    xoff[j] = static_cast<unsigned>(r) * xpitch + c;
-  }
+  // ---- loads of a stage, dealt to the wavefronts in turn: the units of the tile (in the last, narrower tile the last unit again
+  // behind it: lines that are on their way already), then the activations, eight rows to a load (rows past the last one of an
+  // eight repeat it; never stored). bf16: eight rows of 128 bytes per load, chunk position L % 8 holds chunk (L % 8) ^ swz(row).
+  // fp8: sixteen rows of 64 bytes, position L % 4 holds chunk (L % 4) ^ (row / 4).
+  const int w_loads = width * LU, loads = w_loads + (nrows + 7) / 8;
+  const int mine = wave < loads ? (loads - wave + NW - 1) / NW : 0;         // this wavefront's
   const int run_rows = a.vocab - u0 * 16 < run * 16 ? a.vocab - u0 * 16 : run * 16;
-  auto weight_offsets = [&](int tile) {
+  unsigned off[LMAX];
+  auto offsets = [&](int tile) {
     const int left = run - tile * width, here = left < width ? left : width;
 #pragma unroll
-    for (int j = 0; j < LW; ++j) {
-      constexpr int LU = W8 ? 1 : 2;                         // loads per unit
-      const int u = wave * (UNITS / NW) + j / LU, unit = tile * width + (u < here ? u : here - 1);
-      const int r = W8 ? lane >> 2 : 8 * (j % LU) + (lane >> 3);
-      const unsigned c = (W8 ? static_cast<unsigned>((lane & 3) ^ (r >> 2)) : static_cast<unsigned>((lane & 7) ^ swz(r))) * 16u;
-      const int row = unit * 16 + r < run_rows ? unit * 16 + r : run_rows - 1;
-      woff[j] = static_cast<unsigned>(row) * wpitch + c;
+    for (int j = 0; j < LMAX; ++j) {
+      const int t = wave + NW * j;
+      if (t < w_loads) {
+        const int u = t / LU, unit = tile * width + (u < here ? u : here - 1);
+        const int r = W8 ? lane >> 2 : 8 * (t % LU) + (lane >> 3);
+        const unsigned c = (W8 ? static_cast<unsigned>((lane & 3) ^ (r >> 2)) : static_cast<unsigned>((lane & 7) ^ swz(r))) * 16u;
+        const int row = unit * 16 + r < run_rows ? unit * 16 + r : run_rows - 1;
+        off[j] = static_cast<unsigned>(row) * wpitch + c;
+      } else {
+        int r = 8 * (t - w_loads) + (lane >> 3);
+        const unsigned c = static_cast<unsigned>((lane & 7) ^ swz(r)) * 16u;
+        r = r < nrows ? r : nrows - 1;
+        off[j] = static_cast<unsigned>(r) * xpitch + c;
+      }
     }
   };
   int l_tile = 0, l_k = 0, l_slot = 0;                       // load cursor
-  weight_offsets(0);
+  offsets(0);
   const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem));
   // The next stage of the stream into the next slot. Always the same number of loads: past the end the last stage comes again.
+  // (The choices sit inside the assembly, so that the schedule around the loads stays one basic block.)
   auto issue = [&]() {
-    const unsigned dst = lds0 + l_slot * STAGE;
+    const unsigned dst = lds0 + l_slot * stage_bytes;
     const unsigned char* const wb = w_base + static_cast<int64_t>(l_k) * (W8 ? BK : BK * 2);
     const unsigned char* const xb = x_base + static_cast<int64_t>(l_k) * (BK * 2);
 #pragma unroll
-    for (int j = 0; j < LW; ++j) {
-      const unsigned d = dst + wave * (UNITS / NW * 16 * WROW) + j * 1024;
+    for (int j = 0; j < LMAX; ++j) {
+      const int t = wave + NW * j;
+      const unsigned d = dst + t * 1024 + (t < w_loads ? 0 : wbytes - w_loads * 1024);
       // a slice of an fp8 row is half a line, so its line is needed again one stage on: no streaming hint
-      if constexpr (W8) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(d), "v"(woff[j]), "s"(wb) : "memory", "m0");
-      else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(d), "v"(woff[j]), "s"(wb) : "memory", "m0");
-    }
-#pragma unroll
-    for (int j = 0; j < LX; ++j) {
-      const unsigned d = dst + WBYTES + (wave * XR + 8 * j) * 128;
-      if (8 * j + 8 > XR)                                    // known at compile time; every lane is active here, before and after
-        asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_hi, 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 exec_hi, -1" ::"s"(d), "v"(xoff[j]), "s"(xb)
-                     : "memory", "m0");
-      else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(d), "v"(xoff[j]), "s"(xb) : "memory", "m0");
+      if constexpr (W8) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_cmp_lt_i32 %3, %4\n\ts_cbranch_scc0 .Lskip%=\n\tglobal_load_lds_dwordx4 %1, %2\n.Lskip%=:" ::"s"(d), "v"(off[j]),
+                     "s"(t < w_loads ? wb : xb), "s"(t), "s"(loads)
+                     : "memory", "m0", "scc");
+      } else {
+        asm volatile("s_mov_b32 m0, %0\n\ts_cmp_lt_i32 %4, %5\n\ts_cbranch_scc0 .Lx%=\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_branch .Lskip%=\n.Lx%=:\n\t"
+                     "s_cmp_lt_i32 %4, %6\n\ts_cbranch_scc0 .Lskip%=\n\tglobal_load_lds_dwordx4 %1, %3\n.Lskip%=:" ::"s"(d), "v"(off[j]), "s"(wb), "s"(xb), "s"(t),
+                     "s"(w_loads), "s"(loads)
+                     : "memory", "m0", "scc");
+      }
     }
     l_slot = l_slot + 1 == S ? 0 : l_slot + 1;
     if (l_k + 1 < nk) {
       ++l_k;
     } else if (l_tile + 1 < ntiles) {
       l_k = 0;
-      weight_offsets(++l_tile);
+      offsets(++l_tile);
     }
   };
 
-  float* const scales = reinterpret_cast<float*>(smem + S * STAGE);
+  float* const scales = reinterpret_cast<float*>(smem + S * stage_bytes);
   if constexpr (W8) {                                        // the run's scales: loaded (and waited for) ahead of the stream
     for (int i = tid; i < run_rows; i += 512) scales[i] = a.w_scale[u0 * 16 + i];
     __syncthreads();
@@ -141,12 +160,13 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
 #pragma unroll
   for (int tb = 0; tb < TB; ++tb) {
     const int r = 16 * (TB * wm + tb) + m16;
-    fx_o[tb] = WBYTES + r * 128 + ((gc ^ swz(r)) << 4);
+    fx_o[tb] = wbytes + r * 128 + ((gc ^ swz(r)) << 4);
   }
 #pragma unroll
   for (int ub = 0; ub < UB; ++ub) {
-    if constexpr (W8) fw_o[ub] = (UB * wn + ub) * 1024 + m16 * 64 + (((gc >> 1) ^ (m16 >> 2)) << 4) + (gc & 1) * 8;
-    else fw_o[ub] = (UB * wn + ub) * 2048 + m16 * 128 + ((gc ^ swz(m16)) << 4);
+    const int unit = 4 * ub + wn < width ? 4 * ub + wn : width - 1;          // (past the tile's width: not stored)
+    if constexpr (W8) fw_o[ub] = unit * UBYTES + m16 * 64 + (((gc >> 1) ^ (m16 >> 2)) << 4) + (gc & 1) * 8;
+    else fw_o[ub] = unit * UBYTES + m16 * 128 + ((gc ^ swz(m16)) << 4);
   }
   const bool vec4 = reinterpret_cast<uintptr_t>(a.logits) % 8 == 0 && a.ld % 4 == 0;
 
@@ -162,8 +182,9 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
       // This wavefront's share of the stage has landed (the S - 2 stages behind it may be in flight; stores of the tile
       // before are younger than all of them, which makes the wait longer, never shorter), then everyone's; and everyone has
       // read the slot that the next loads go into.
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * LPW) : "memory");
-      const unsigned char* const st = smem + c_slot * STAGE;
+      wait_stages<LMAX, S - 2>(mine);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      const unsigned char* const st = smem + c_slot * stage_bytes;
       bf16x8 fx[2][TB], fw[2][UB];
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
@@ -193,7 +214,7 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
     const int left = run - tile * width, here = left < width ? left : width;
 #pragma unroll
     for (int ub = 0; ub < UB; ++ub) {
-      const int unit = UB * wn + ub;
+      const int unit = 4 * ub + wn;
       if (unit >= here) continue;                            // uniform
       const int lv = (tile * width + unit) * 16 + 4 * g;     // in the run
       f32x4 sc = {1.f, 1.f, 1.f, 1.f};
@@ -220,14 +241,34 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
 }
 
 namespace {
-template <int MB, bool W8>
-int launch_one(const char* who, const UnembedArgs& a, int chunk_rows, int chunks, hipStream_t st) {
-  typedef unembed_tiles::Shape<MB, W8> C;
+template <int MB, bool W8, int UB, int S>
+int launch_one(const char* who, const UnembedArgs& a, int chunk_rows, int chunks, int slots, hipStream_t st) {
+  typedef unembed_tiles::Shape<MB, W8, UB> C;
   static std::atomic<uint64_t> done{0};
-  const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(unembed_tiles_kernel<MB, W8>), C::SMEM, done);
+  const int smem = S * (slots * C::UBYTES + C::XBYTES) + C::TAIL;
+  const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(unembed_tiles_kernel<MB, W8, UB, S>), unembed_tiles::LDS, done);
   TLLM_REQUIRE(e == hipSuccess, TLLM_E_LAUNCH, "%s: cannot raise LDS limit: %s", who, hipGetErrorString(e));
-  hipLaunchKernelGGL((unembed_tiles_kernel<MB, W8>), dim3(kUnembedGrid, (unsigned)chunks), dim3(512), C::SMEM, st, a, chunk_rows);
+  hipLaunchKernelGGL((unembed_tiles_kernel<MB, W8, UB, S>), dim3(kUnembedGrid, (unsigned)chunks), dim3(512), smem, st, a, chunk_rows, slots);
   return check_launch(who);
+}
+
+// As few tiles as possible, since each reads the activations once: of up to 20 units (bf16) or 28 (fp8), and of no more than three
+// stages fit the LDS. [rows, 2880] x [201088, 2880], 49 / 128 rows, us: four tiles of thirteen units 206 / 253, three of seventeen
+// 200 / 240; fp8 147 / 208 and 143 / 234, two of twenty-five 139 / 178. A kernel for each quarter of those widths, as many stages
+// as fit it: units past the tile's width are multiplied as well, and a CU that holds a third of a tile wants more stages on
+// their way ([rows, 2880] x [8192, 2880], two units per CU, 49 / 128 rows 34 / 47 -> 20 / 30; 2048 wide, 32000 34 / 41 -> 31 / 35).
+template <int MB, bool W8>
+int launch_shape(const char* who, const UnembedArgs& a, int chunk_rows, int chunks, hipStream_t st) {
+  using unembed_tiles::Shape;
+  const int run = ((a.vocab + 15) / 16 + kUnembedGrid - 1) / kUnembedGrid;
+  constexpr int BIG = W8 ? 7 : 5;
+  constexpr int widest = Shape<MB, W8, BIG>::most(3);
+  const int tiles = (run + widest - 1) / widest, slots = (run + tiles - 1) / tiles;
+  if (slots <= 8) return launch_one<MB, W8, 2, MB <= 4 ? 6 : 5>(who, a, chunk_rows, chunks, slots, st);
+  if (slots <= 16) return launch_one<MB, W8, 4, W8 ? (MB == 2 ? 7 : MB == 4 ? 6 : MB == 6 ? 5 : 4) : MB <= 4 ? 4 : 3>(who, a, chunk_rows, chunks, slots, st);
+  if (W8 && slots <= Shape<MB, W8, 5>::most(5)) return launch_one<MB, W8, 5, 5>(who, a, chunk_rows, chunks, slots, st);
+  if (slots <= Shape<MB, W8, BIG>::most(4)) return launch_one<MB, W8, BIG, 4>(who, a, chunk_rows, chunks, slots, st);
+  return launch_one<MB, W8, BIG, 3>(who, a, chunk_rows, chunks, slots, st);
 }
 }  // namespace
 
@@ -242,7 +283,7 @@ int launch_unembed_tiles(const char* who, const UnembedArgs& a, bool w8, hipStre
   const int chunk_rows = static_cast<int>((a.rows + chunks - 1) / chunks);
   const int mb = (chunk_rows + 31) / 32 * 2;
 #define TLLM_TILES(MB) \
-  if (mb == MB) return w8 ? launch_one<MB, true>(who, a, chunk_rows, chunks, st) : launch_one<MB, false>(who, a, chunk_rows, chunks, st)
+  if (mb == MB) return w8 ? launch_shape<MB, true>(who, a, chunk_rows, chunks, st) : launch_shape<MB, false>(who, a, chunk_rows, chunks, st)
   TLLM_TILES(2);
   TLLM_TILES(4);
   TLLM_TILES(6);
