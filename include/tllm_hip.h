@@ -216,6 +216,8 @@ int tllm_qkv_rope_prefill_bf16(const void* x, const void* W, const void* b,
  * the one that tllm_linear_bf16 takes. No counterpart in the reference. */
 int tllm_qkv_gemm_tile(int prefill, int64_t rows, int64_t hidden, int n_q_heads, int n_kv_heads, int head_dim);
 int tllm_linear_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim);
+/* Diagnostic: whether that tile's launch (or the QKV projection's, out_dim = 64 x heads) spreads its row tiles' walks over K. */
+int tllm_gemm_tile_spread(int64_t rows, int64_t in_dim, int64_t out_dim);
 /* Diagnostic: wavefronts that stream the weight in a workgroup of the general-shape decode projections (4, 2 or 1). */
 int tllm_decode_general_streams(int64_t rows, int64_t in_dim, int64_t out_dim, int fp8);
 

@@ -882,6 +882,29 @@ def test_linear_every_gemm_tile(gpu, bm, bn, rows, n, k):
     assert (out[:, n:] == 7.0).all()
 
 
+@pytest.mark.parametrize("bm,bn,rows,n,k", [(64, 32, 113, 2880, 4096), (64, 32, 128, 2880, 4160), (64, 48, 128, 5120, 2880), (64, 64, 152, 5120, 2880),
+                                            (64, 80, 193, 5120, 2880), (64, 96, 450, 2880, 4096), (64, 128, 300, 5120, 2880), (64, 160, 500, 5120, 2880),
+                                            (64, 192, 513, 5120, 2880), (128, 96, 600, 4096, 2880), (128, 128, 595, 5120, 2880)])
+def test_linear_walks_spread_over_k(gpu, bm, bn, rows, n, k):
+    """Tiles whose row tiles begin at different places in K: an odd number of slices where a stage has two, so that the stage without
+    a second one is met in the middle of a walk, and what is infinite in the last slice stays infinite."""
+    L = _lib.lib()
+    assert L.tllm_linear_gemm_tile(rows, k, n) == bm << 16 | bn and L.tllm_gemm_tile_spread(rows, k, n) == 1
+    g = torch.Generator().manual_seed(rows + n + k)
+    x, w, b = torch.randn(rows, k, generator=g).bfloat16(), (0.02 * torch.randn(n, k, generator=g)).bfloat16(), (0.05 * torch.randn(n, generator=g)).bfloat16()
+    x[rows - 1, k - 1] = float("inf")
+    xg, wg, bg, out = x.to(gpu), w.to(gpu), b.to(gpu), torch.empty(rows, n, dtype=torch.bfloat16, device=gpu)
+    assert L.tllm_linear_bf16(xg.data_ptr(), wg.data_ptr(), bg.data_ptr(), out.data_ptr(), n, rows, k, n, torch.cuda.current_stream().cuda_stream) == 0
+    close(out[:rows - 1], O.linear_ref(x[:rows - 1], w, b))
+    assert torch.equal(out[rows - 1].float().cpu()[w[:, k - 1] != 0], (w[:, k - 1].float() * float("inf"))[w[:, k - 1] != 0])
+
+
+@pytest.mark.parametrize("rows", [128, 192, 333, 513, 640])
+def test_qkv_walks_spread_over_k(gpu, rows):
+    assert _lib.lib().tllm_gemm_tile_spread(rows, 2880, 5120) == 1
+    _check_qkv_position_sources(gpu, rows, 2880, 64, 8, "prefill", seed=rows)
+
+
 @pytest.mark.parametrize("rows,k,n", [(1, 64, 16), (3, 4096, 2880), (97, 4096, 2880), (200, 448, 2880), (333, 576, 2880), (512, 640, 2880),
                                       (999, 320, 2880), (1400, 256, 2880), (2048, 192, 2880), (70, 128, 48)])
 def test_linear_tile_gemm(gpu, rows, k, n):

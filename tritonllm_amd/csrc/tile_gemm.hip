@@ -29,10 +29,10 @@
 // multiple of sixteen columns will do as a tile.
 //
 // [rows, 2880] x [2880, 5120] + bias + rotary, us (before: the many-row decode kernel up to 448 rows, 128 x 320 tiles above):
-//   128 rows 16.2 (17.5)   192 19.0 (22.1)   256 21.2 (26.6)   333 23.2 (32.3)   512 29.6 (54.0)   777 33.9 (50.9)
-//   999 39.8 (49.1)   1100 41.4 (55.0)   1400 47.4 (57.1)   1536 50.9 (57)
+//   128 rows 15.9 (17.5)   192 16.1 (22.1)   256 18.4 (26.6)   333 21.0 (32.3)   512 25.9 (54.0)   777 32.5 (50.9)
+//   999 38.6 (49.1)   1100 40.4 (55.0)   1400 45.7 (57.1)   1536 49.9 (57)
 // [rows, 4096] x [4096, 2880] + bias (before: the library's GEMM):
-//   97 rows 13.8 (15.5)   192 18.8 (32.4)   333 20.4 (30.3)   512 24.9 (25.2)   999 33.5 (36.5)   2048 49.9 (53.4)
+//   97 rows 13.6 (15.5)   192 15.5 (32.4)   333 17.9 (30.3)   512 20.7 (25.2)   999 32.4 (36.5)   2048 49.9 (53.4)
 #include "qkv_prefill.h"
 
 namespace tllm {
@@ -73,7 +73,8 @@ __device__ __forceinline__ void wait_slices_left(int left) {     // at most `lef
   }
 }
 
-template <class C, int MODE>
+// TURN: the row tiles begin their walks over K at different places (tile_gemm_spread).
+template <class C, int MODE, bool TURN>
 __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, YarnFreqs fr, int tiles_m, int n_blocks) {
   using namespace tile_gemm;
   constexpr int TB = C::TB, RB = C::RB, KG = C::KG, KS = C::KS, BM = C::BM, BN = C::BN, S = C::S, STAGE = C::STAGE, SLICE = C::SLICE, WSLICE = C::WSLICE;
@@ -94,6 +95,9 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
   const int block0 = tile_n * NB;
   const int n_slices = a.hidden / BK, n_iter = (n_slices + KS - 1) / KS;
   const unsigned pitch = static_cast<unsigned>(a.hidden) * 2;
+
+  // Where in K the walk begins, in stages
+  const int rot = TURN ? tile_m * n_iter / tiles_m : 0;
 
   // weight row of tile row i (a block past the last one repeats it; its columns are never stored)
   auto weight_row = [&](int i) {
@@ -124,11 +128,11 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
       soff[j] = static_cast<unsigned>(weight_row(r)) * pitch + c;
     }
   }
-  // Stage number `st` goes into ring place `place`. Nothing is requested behind the last stage: the test sits inside the
-  // assembly so that the schedule around the load stays one basic block.
-  auto issue_load = [&](int st, int place, int j) {
+  // The walk's stage number `st`, which is stage `at` of K, goes into ring place `place`. Nothing is requested behind the last one:
+  // the test sits inside the assembly so that the schedule around the load stays one basic block.
+  auto issue_load = [&](int st, int at, int place, int j) {
     const bool is_x = j < LX;
-    int slice = KS * st + ls;
+    int slice = KS * at + ls;
     if (KS == 2 && slice >= n_slices) slice = n_slices - 1; // an odd number of slices: the last stage's second one is not used
     const unsigned dst = static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem)) + place * STAGE + ls * SLICE +
                          (is_x ? WSLICE + (lw * XR + 8 * j) * LROW : (lw * WR + 8 * (j - LX)) * LROW);
@@ -171,7 +175,7 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
   };
   // One k32 step on the fragments in buffer `cur`. Behind its first MFMAs go the reads of the next step's fragments (k32
   // step nkk of the slice at nsl); loads [l0, l1) of the stage handed on spread over all of them.
-  auto step = [&](auto cur_c, const unsigned char* nsl, int nkk, auto l0_c, auto l1_c, int stage_it, int stage) {
+  auto step = [&](auto cur_c, const unsigned char* nsl, int nkk, auto l0_c, auto l1_c, int stage_it, int stage_at, int stage) {
     constexpr int cur = decltype(cur_c)::value, l0 = decltype(l0_c)::value, l1 = decltype(l1_c)::value;
     constexpr int RPM = (NRD + NMF - 1) / NMF > 1 ? (NRD + NMF - 1) / NMF : 1;   // fragment reads behind an MFMA
 #pragma unroll
@@ -188,7 +192,7 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
 #pragma unroll
       for (int i = l0; i < l1; ++i) {
         if ((i - l0) * NMF / (l1 - l0) != m) continue;
-        issue_load(stage_it, stage, i);
+        issue_load(stage_it, stage_at, stage, i);
         __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);           // a VMEM read
       }
     }
@@ -204,10 +208,13 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
     bias_raw = bp[weight_row(tid < BN ? tid : BN - 1)];
   }
   const int first = n_iter < S ? n_iter : S;
+  int ahead = rot;                                                  // the stage of K that is loaded next
+  auto turn = [&](int next) { ahead = TURN ? (ahead + 1 == n_iter ? 0 : ahead + 1) : next; };
 #pragma unroll 1
   for (int s = 0; s < first; ++s) {
 #pragma unroll
-    for (int j = 0; j < LPW; ++j) issue_load(s, s, j);
+    for (int j = 0; j < LPW; ++j) issue_load(s, ahead, s, j);
+    turn(s + 1);
   }
   // cos / sin of (row, frequency), computed while the first slices arrive and kept in registers. Wavefront w: rows BM / 8 w
   // .. of the tile; lane: frequency lane % 32, rows 2 j + lane / 32 of those. The rows' positions come through the scalar
@@ -247,16 +254,30 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
   };
   auto next = [](int c) { return c + 1 == S ? 0 : c + 1; };
   int c = 0;
-  // (KG == 4, an odd number of slices: the last stage has no second one, half of the wavefronts sit it out)
-  const int live = KG == 4 && n_slices % 2 && kg >= 2 ? n_iter - 1 : n_iter;
+  // KG == 4, an odd number of slices: the last stage of K has no second one. Half of the wavefronts sit it out, or, where it is met in
+  // the middle of the walk, multiply zeros.
+  const bool lacks = KG == 4 && n_slices % 2 && kg >= 2;
+  const int live = !TURN && lacks ? n_iter - 1 : n_iter, none_at = TURN && lacks ? n_iter - 1 - rot : -1;
+  auto no_second_slice = [&](auto buf_c) {
+    constexpr int buf = decltype(buf_c)::value;
+    const bf16x8 zero = {};
+#pragma unroll
+    for (int i = 0; i < TB; ++i) fx[buf][i] = zero;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) fw[buf][i] = zero;
+  };
   for (int it = 0; it < n_iter; it += 2) {                           // the fragment buffers alternate, so stages go in pairs
     int n = next(c);
     stage_barrier(it);
-    if (it < live) step(I0{}, slice_at(n), kk0, I0{}, IL{}, it + S, c);   // (behind the last stage its reads are not used)
+    if (TURN && it == none_at) no_second_slice(I0{});
+    if (it < live) step(I0{}, slice_at(n), kk0, I0{}, IL{}, it + S, TURN ? ahead : it + S, c);   // (behind the last stage its reads are not used)
+    turn(it + S + 1);
     c = n;
     n = next(c);
     stage_barrier(it + 1);
-    if (it + 1 < live) step(I1{}, slice_at(n), kk0, I0{}, IL{}, it + 1 + S, c);
+    if (TURN && it + 1 == none_at) no_second_slice(I1{});
+    if (it + 1 < live) step(I1{}, slice_at(n), kk0, I0{}, IL{}, it + 1 + S, TURN ? ahead : it + 1 + S, c);
+    turn(it + S + 2);
     c = n;
   }
   float* const bias_s = reinterpret_cast<float*>(smem + S * STAGE);
@@ -362,14 +383,14 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
 }
 
 namespace {
-template <class C, int MODE>
+template <class C, int MODE, bool TURN>
 int launch_one(const char* what, const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& fr, int n_blocks, hipStream_t st) {
   static std::atomic<uint64_t> done{0};
-  const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(tile_gemm_kernel<C, MODE>), C::SMEM, done);
+  const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(tile_gemm_kernel<C, MODE, TURN>), C::SMEM, done);
   TLLM_REQUIRE(e == hipSuccess, TLLM_E_LAUNCH, "%s: cannot raise LDS limit: %s", what, hipGetErrorString(e));
   const int64_t tiles_m = (a.rows + C::BM - 1) / C::BM, tiles_n = (n_blocks * 16 + C::BN - 1) / C::BN;
   TLLM_REQUIRE(tiles_m * tiles_n < (1ll << 31), TLLM_E_SHAPE, "%s: too many tiles", what);
-  hipLaunchKernelGGL((tile_gemm_kernel<C, MODE>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), C::SMEM, st, a, ra, fr, (int)tiles_m, n_blocks);
+  hipLaunchKernelGGL((tile_gemm_kernel<C, MODE, TURN>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), C::SMEM, st, a, ra, fr, (int)tiles_m, n_blocks);
   return check_launch(what);
 }
 
@@ -403,26 +424,47 @@ TileSize tile_gemm_pick(int64_t rows, int64_t cols, int64_t k, int64_t* ns) {
 }
 
 namespace {
+// Whether the row tiles of a launch begin their walks over K at places spread over it (tile m of M at m / M). In step, the
+// workgroups that share weight columns all wait for the same lines from memory; spread, each finds most of K in its XCD's L2, where
+// another one has been. It pays while an XCD's share of the weight stays in its 4 MB (weights of 8 - 16 M elements) and costs beyond,
+// and with rows 4 or 8 KB apart below 10 M; us, in step and spread: [rows, 4096] x [4096, 2880] 128 rows 16.2 / 14.6, 256 18.3 / 15.7, 500
+// 24.4 / 20.3, 1000 33.7 / 32.4; [rows, 2880] x [2880, 5120] 192 16.2 / 14.4, 512 28.9 / 25.9; 6144 x 2048 640 rows 34.7 / 29.1; and
+// 4096 x 5120 256 rows 23.4 / 29.0, 2048 x 4096 230 rows 10.6 / 11.1, 1024 x 1024 as long either way.
+// In step, a last row tile that is mostly empty is ahead of the others and fetches for them, so that spreading wants one that is
+// filled: two row tiles, 97 rows (33 in the last) 13.8 / 14.4, 113 (49) 15.1 / 14.5; three, 160 (32) 16.6 / 15.6; from four on any
+// (230 16.8 / 15.5). 128-row tiles up to 128 columns: 5 tiles of 2880 x 5120 640 rows 29.9 / 27.2, six of them (720) 28.8 / 29.4,
+// 2880 x 4096 720 rows 27.5 / 25.0; 1300 rows (20 in the last) 35.5 / 38.
+bool tile_gemm_spread(int64_t rows, int64_t cols, int64_t k, TileSize t) {
+  const int64_t last = (rows - 1) % t.bm + 1, tiles_m = (rows + t.bm - 1) / t.bm, weight = cols * k;
+  if (tiles_m < 2 || weight < 8000000 || weight > 16000000 || (weight < 10000000 && k % 2048 == 0)) return false;
+  if (t.bm == 64) return tiles_m >= 4 || last >= (tiles_m == 3 ? 24 : 48);
+  return t.bn <= 128 && last >= 80 && (tiles_m <= 5 || weight <= 12000000);
+}
+
 template <int MODE>
 int launch_mode(const char* what, const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& fr, int n_blocks, hipStream_t st) {
   int64_t ns;
   TileSize t = tile_gemm_pick(a.rows, static_cast<int64_t>(n_blocks) * 16, a.hidden, &ns);
-#define TLLM_TILE(...)                                   \
-  if (typedef tile_gemm::Tile<__VA_ARGS__> C; t.bm == C::BM && t.bn == C::BN) return launch_one<C, MODE>(what, a, ra, fr, n_blocks, st)
-  TLLM_TILE(2, 2, 2, 1, 4);
-  TLLM_TILE(2, 3, 2, 1, 4);
-  TLLM_TILE(4, 2, 1, 2, 4);
-  TLLM_TILE(2, 5, 2, 1, 4);
-  TLLM_TILE(4, 3, 1, 2, 4);
-  TLLM_TILE(2, 4, 2, 2, 2);
-  TLLM_TILE(2, 5, 2, 2, 2);
-  TLLM_TILE(2, 6, 2, 2, 2);
-  TLLM_TILE(4, 3, 2, 2, 2);
-  TLLM_TILE(4, 4, 2, 2, 2);
-  TLLM_TILE(4, 5, 2, 2, 2);
-  TLLM_TILE(4, 6, 2, 2, 2);
-  TLLM_TILE(4, 7, 2, 2, 2);
-  TLLM_TILE(4, 8, 2, 2, 2);
+  const bool spread = tile_gemm_spread(a.rows, static_cast<int64_t>(n_blocks) * 16, a.hidden, t);
+#define TLLM_TILE(...)                                                                                                  \
+  if (typedef tile_gemm::Tile<__VA_ARGS__> C; t.bm == C::BM && t.bn == C::BN) {                          \
+    constexpr bool CAN = C::BM == 64 || C::BN <= 128;   /* (one kernel for both costs 1 - 4 % in step) */          \
+    return CAN && spread ? launch_one<C, MODE, CAN>(what, a, ra, fr, n_blocks, st) : launch_one<C, MODE, false>(what, a, ra, fr, n_blocks, st); \
+  }
+  TLLM_TILE(2, 2, 2, 1, 4)
+  TLLM_TILE(2, 3, 2, 1, 4)
+  TLLM_TILE(4, 2, 1, 2, 4)
+  TLLM_TILE(2, 5, 2, 1, 4)
+  TLLM_TILE(4, 3, 1, 2, 4)
+  TLLM_TILE(2, 4, 2, 2, 2)
+  TLLM_TILE(2, 5, 2, 2, 2)
+  TLLM_TILE(2, 6, 2, 2, 2)
+  TLLM_TILE(4, 3, 2, 2, 2)
+  TLLM_TILE(4, 4, 2, 2, 2)
+  TLLM_TILE(4, 5, 2, 2, 2)
+  TLLM_TILE(4, 6, 2, 2, 2)
+  TLLM_TILE(4, 7, 2, 2, 2)
+  TLLM_TILE(4, 8, 2, 2, 2)
 #undef TLLM_TILE
   set_error("%s: no kernel for a tile of %d x %d", what, t.bm, t.bn);
   return TLLM_E_SHAPE;
@@ -456,6 +498,11 @@ extern "C" int tllm_linear_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_d
   int64_t ns;
   const TileSize t = tile_gemm_pick(rows, out_dim, in_dim, &ns);
   return t.bm << 16 | t.bn;
+}
+
+extern "C" int tllm_gemm_tile_spread(int64_t rows, int64_t in_dim, int64_t out_dim) {
+  int64_t ns;
+  return tile_gemm_spread(rows, out_dim, in_dim, tile_gemm_pick(rows, out_dim, in_dim, &ns));
 }
 
 extern "C" int tllm_linear_bf16(const void* x, const void* W, const void* b, void* out, int64_t out_row_stride, int64_t rows, int64_t in_dim,
