@@ -21,7 +21,7 @@
 // W8: fp8 (OCP e4m3) weight with one fp32 scale per output row (the reference's ATTN_FP8 option,
 // triton_kernels.py:1385-1408): a weight row of a phase is 128 bytes (two loads of eight rows), fragments are widened
 // to bf16 (exact) between the LDS read and the MFMA, the row scale multiplies the finished sum.
-// More than 32 rows: a workgroup takes up to four chunks of 32 rows one after the other against the same resident
+// More than 32 rows: a workgroup takes up to four chunks of up to 32 rows one after the other against the same resident
 // weight (only the first chunk requests it), so the weight is read once for up to 128 rows; between chunks the
 // partial tiles pass through the first activation region behind two barriers (33 rows 13.3 -> 10.5 us, 64 rows
 // 14.0 -> 11.2, where every chunk was a workgroup of its own with its own pass over the weight).
@@ -32,7 +32,6 @@
 namespace tllm {
 
 namespace r32o {
-constexpr int XR = 32;            // activation rows per workgroup
 constexpr int NS = 4;             // streaming wavefronts = K slices
 constexpr int NE = 2;             // epilogue wavefronts = column blocks
 constexpr int RW = 12;            // weight rows (output features) per workgroup
@@ -66,10 +65,11 @@ __device__ __forceinline__ void wait_vmcnt() {
 }
 }  // namespace r32o
 
-template <int XB, bool W8>
-__global__ __launch_bounds__(384) void out_decode_r32_kernel(OutArgs a, int vec8, int cpw) {
+template <int XB, bool W8, bool SPREAD>
+__global__ __launch_bounds__(384) void out_decode_r32_kernel(OutArgs a, int vec8, int cpw, int chunks) {
   using namespace r32o;
   constexpr int LW = W8 ? 2 : 3;                            // weight load instructions per phase
+  constexpr int XR = 4 * XB;                                // activation rows of a chunk
   constexpr int XRING = 2;                                  // phases of activations resident per wavefront
   constexpr int WPH = 3 * 1024;                             // weight of one phase: 12 rows x four k32 steps (fp8: 2 KB of it)
   static_assert(XRING * XPH + WRING * WPH <= WAVE_LDS, "a wavefront's rings fit its share of the LDS");
@@ -78,10 +78,10 @@ __global__ __launch_bounds__(384) void out_decode_r32_kernel(OutArgs a, int vec8
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.x * RW;
-  // A workgroup takes up to `cpw` consecutive chunks of 32 rows, one after the other, against the weight it requested
+  // A workgroup takes up to `cpw` consecutive ones of the `chunks` chunks of XR rows, one after the other, against the weight it requested
   // for the first: every phase of the weight has a place of its own in LDS and stays there.
   const int64_t chunk0 = static_cast<int64_t>(blockIdx.y) * cpw;
-  const int64_t chunks_left = (a.rows + XR - 1) / XR - chunk0;
+  const int64_t chunks_left = chunks - chunk0;
   const int my_chunks = static_cast<int>(chunks_left < cpw ? chunks_left : cpw);   // >= 1 by the grid
 
   if (wave >= NS) {
@@ -189,8 +189,11 @@ __global__ __launch_bounds__(384) void out_decode_r32_kernel(OutArgs a, int vec8
   auto lds_addr = [](const void* p) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>(p)); };
   auto x_region = [&](int p) { return myring + (p % XRING) * XPH; };
   auto w_region = [&](int p) { return myring + XRING * XPH + (p % WRING) * WPH; };
+  // SPREAD: the workgroups that share an XCD's L2 begin their walks over K at different phases
+  const int rot = static_cast<int>(blockIdx.x >> 3) & (NPH - 1);
+  auto turned = [&](int p) { return SPREAD ? (p + rot) & (NPH - 1) : p; };
   auto issue_x = [&](int p) {
-    const unsigned char* xb = xbase + p * 1024;
+    const unsigned char* xb = xbase + turned(p) * 1024;
 #pragma unroll
     for (int j = 0; j < XB; ++j) {
       const unsigned dst = lds_addr(x_region(p) + j * 1024);
@@ -198,7 +201,7 @@ __global__ __launch_bounds__(384) void out_decode_r32_kernel(OutArgs a, int vec8
     }
   };
   auto issue_w = [&](int p) {
-    const unsigned char* wb = wbase + p * (W8 ? 512 : 1024);
+    const unsigned char* wb = wbase + turned(p) * (W8 ? 512 : 1024);
 #pragma unroll
     for (int j = 0; j < LW; ++j) {
       const unsigned dst = lds_addr(w_region(p) + j * 1024);
@@ -297,24 +300,38 @@ __global__ __launch_bounds__(384) void out_decode_r32_kernel(OutArgs a, int vec8
 void launch_out_decode_r32(dim3 grid, hipStream_t st, const OutArgs& a) {
   auto al8 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 8 == 0; };
   const int vec8 = al8(a.out) && a.out_rs % 4 == 0 && (a.res == nullptr || (al8(a.res) && a.res_rs % 4 == 0)) && (a.bias == nullptr || al8(a.bias));
-  const int rows = static_cast<int>(a.rows < 32 ? a.rows : 32);          // of the fullest chunk
-  // up to four chunks of 32 rows per workgroup: the weight is then read once for up to 128 rows
-  const int cpw = grid.y < 4 ? static_cast<int>(grid.y) : 4;
-  const dim3 g2(grid.x, (grid.y + cpw - 1) / cpw);
-#define TLLM_OUT32(XB)                                                                                        \
-  do {                                                                                                        \
-    if (a.w_scale) hipLaunchKernelGGL((out_decode_r32_kernel<XB, true>), g2, dim3(384), 0, st, a, vec8, cpw);   \
-    else hipLaunchKernelGGL((out_decode_r32_kernel<XB, false>), g2, dim3(384), 0, st, a, vec8, cpw);            \
+  // As few chunks as will do, of as few rows as will do, a multiple of four: a chunk of XB four-row blocks loads all of them, real rows or
+  // not (in chunks of 32 / so, us: 33 rows 10.9 / 9.6, 49 11.1 / 10.7, 65 14.5 / 12.7, 97 18.5 / 16.2, fp8 33 rows 9.5 / 8.2).
+  const int64_t fewest = (a.rows + 31) / 32;
+  const int xb = static_cast<int>(((a.rows + fewest - 1) / fewest + 3) / 4);
+  const unsigned chunks = static_cast<unsigned>((a.rows + 4 * xb - 1) / (4 * xb));
+  // up to four chunks per workgroup: the weight is then read once for up to 128 rows
+  const int cpw = chunks < 4 ? static_cast<int>(chunks) : 4;
+  const dim3 g2(grid.x, (chunks + cpw - 1) / cpw);
+  // Where the activations are most of what a CU takes in, its neighbours do not ask their L2 for the same lines of them at the same time
+  // (64 rows 12.0 -> 11.8 us, 96 16.1 -> 14.9, 128 19.7 -> 17.8; fp8 64 10.4 -> 9.8, 128 18.1 -> 16.0). With fewer rows what counts is that
+  // all ask memory for the same part of their weight rows at a time (9 rows 6.6, spread 7.1; 49 rows 11.1 and 11.4).
+  const bool spread = a.rows > (a.w_scale ? 52 : 56);
+#define TLLM_OUT32(XB, SPREAD)                                                                                                   \
+  do {                                                                                                                           \
+    if (a.w_scale) hipLaunchKernelGGL((out_decode_r32_kernel<XB, true, SPREAD>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks);   \
+    else hipLaunchKernelGGL((out_decode_r32_kernel<XB, false, SPREAD>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks);            \
   } while (0)
-  switch ((rows + 3) / 4) {
-    case 1: TLLM_OUT32(1); break;
-    case 2: TLLM_OUT32(2); break;
-    case 3: TLLM_OUT32(3); break;
-    case 4: TLLM_OUT32(4); break;
-    case 5: TLLM_OUT32(5); break;
-    case 6: TLLM_OUT32(6); break;
-    case 7: TLLM_OUT32(7); break;
-    default: TLLM_OUT32(8); break;
+  if (spread) {                                             // (more than 52 rows: chunks of 22 and more)
+    if (xb <= 6) TLLM_OUT32(6, true);
+    else if (xb == 7) TLLM_OUT32(7, true);
+    else TLLM_OUT32(8, true);
+    return;
+  }
+  switch (xb) {
+    case 1: TLLM_OUT32(1, false); break;
+    case 2: TLLM_OUT32(2, false); break;
+    case 3: TLLM_OUT32(3, false); break;
+    case 4: TLLM_OUT32(4, false); break;
+    case 5: TLLM_OUT32(5, false); break;
+    case 6: TLLM_OUT32(6, false); break;
+    case 7: TLLM_OUT32(7, false); break;
+    default: TLLM_OUT32(8, false); break;
   }
 #undef TLLM_OUT32
 }
