@@ -213,9 +213,10 @@ int tllm_qkv_rope_prefill_bf16(const void* x, const void* W, const void* b,
 
 /* Diagnostics: the GEMM tile (rows << 16 | columns) that tllm_qkv_rope_prefill_bf16 (prefill != 0) or
  * tllm_qkv_rope_decode_bf16 takes for aligned operands of these sizes, 0 where it is another kernel's; and
- * the one that tllm_linear_bf16 takes. No counterpart in the reference. */
+ * the ones that tllm_linear_bf16 and tllm_out_residual_decode_bf16 (bf16 weight) take. No counterpart in the reference. */
 int tllm_qkv_gemm_tile(int prefill, int64_t rows, int64_t hidden, int n_q_heads, int n_kv_heads, int head_dim);
 int tllm_linear_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim);
+int tllm_out_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim);
 /* Diagnostic: whether that tile's launch (or the QKV projection's, out_dim = 64 x heads) spreads its row tiles' walks over K. */
 int tllm_gemm_tile_spread(int64_t rows, int64_t in_dim, int64_t out_dim);
 /* Diagnostic: wavefronts that stream the weight in a workgroup of the general-shape decode projections (4, 2 or 1). */

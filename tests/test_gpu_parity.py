@@ -1285,6 +1285,36 @@ def test_out_residual_general_stream(gpu, in_dim, out_dim, rows, fp8):
     close(out.view(rows, out_dim), O.out_residual_ref(d["x"], ref, d["b"], d["r"]))
 
 
+@pytest.mark.parametrize("bm,bn,spread,rows,in_dim,out_dim", [
+    (64, 32, 0, 129, 4096, 48), (64, 32, 1, 113, 2880, 2880), (64, 48, 0, 113, 192, 5120), (64, 48, 1, 113, 2048, 5120), (64, 64, 0, 129, 192, 5120),
+    (64, 64, 1, 113, 1088, 8192), (64, 80, 0, 2307, 192, 400), (64, 80, 1, 193, 2048, 5120), (64, 96, 0, 1411, 64, 1024), (64, 96, 1, 257, 2112, 4096),
+    (64, 128, 0, 193, 64, 8192), (64, 128, 1, 153, 1088, 8192), (64, 160, 0, 515, 64, 4032), (64, 160, 1, 515, 2112, 4032), (64, 192, 0, 257, 64, 8192),
+    (64, 192, 1, 257, 1088, 8192), (128, 96, 0, 2307, 64, 1024), (128, 96, 1, 640, 2112, 4032), (128, 128, 0, 333, 64, 8192), (128, 128, 1, 640, 2048, 5120),
+    (128, 160, 0, 771, 64, 5120), (128, 192, 0, 515, 64, 8192), (128, 224, 0, 1411, 64, 4096), (128, 256, 0, 771, 64, 8192), (64, 32, 0, 81, 4096, 2880),
+    (64, 32, 1, 128, 4096, 2880), (64, 32, 0, 33, 4096, 4032)])
+def test_out_residual_in_gemm_tiles(gpu, bm, bn, spread, rows, in_dim, out_dim):
+    """Every tile the projection takes for many rows, walks in step and spread: in place with strides that allow 16-byte accesses; a
+    residual and an output of their own, two bytes off and with odd strides; no bias; no residual. Padding columns stay untouched."""
+    L = _lib.lib()
+    assert L.tllm_out_gemm_tile(rows, in_dim, out_dim) == bm << 16 | bn
+    assert L.tllm_gemm_tile_spread(rows, in_dim, out_dim) == spread
+    d = _out_inputs(rows, 7300 + in_dim + rows, in_dim=in_dim, out_dim=out_dim)
+    x, w, b = d["x"].to(gpu), d["w"].to(gpu), d["b"].to(gpu)
+    product = d["x"].float() @ d["w"].float().T
+    for pad, shift, with_bias, with_res in ((8, 0, True, True), (3, 1, False, True), (0, 0, True, False)):
+        stride = out_dim + pad
+        buf = torch.full((rows * stride + 8,), 7.0, dtype=torch.bfloat16, device=gpu)
+        out = buf[shift:shift + rows * stride].view(rows, stride)
+        res = out if with_res and not shift else torch.zeros(rows * stride + 8, dtype=torch.bfloat16, device=gpu)[shift:shift + rows * stride].view(rows, stride)
+        if with_res:
+            res[:, :out_dim] = d["r"].to(gpu)
+        rc = L.tllm_out_residual_decode_bf16(x.data_ptr(), w.data_ptr(), None, b.data_ptr() if with_bias else None, res.data_ptr() if with_res else None,
+                                             out.data_ptr(), stride, stride, rows, in_dim, out_dim, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, L.tllm_last_error()
+        close(out[:, :out_dim], product + (d["b"].float() if with_bias else 0) + (d["r"].float() if with_res else 0))
+        assert (out[:, out_dim:] == 7.0).all() and (buf[:shift] == 7.0).all() and (buf[shift + rows * stride:] == 7.0).all()
+
+
 def test_out_residual_other_shapes_module_and_errors(gpu, monkeypatch):
     # a shape the streaming kernel does not serve (in_dim != 4096): the plain kernel, bf16 and fp8
     d = _out_inputs(5, 61, in_dim=320, out_dim=100)

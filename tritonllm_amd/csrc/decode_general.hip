@@ -185,6 +185,12 @@ int launch_out(const char* what, unsigned gx, int64_t gy, hipStream_t st, const 
 int64_t chunks_of(int64_t rows) { return rows <= 8 ? 1 : (rows + 15) / 16; }
 }  // namespace
 
+// Up to 256 and 512 workgroups 3.3 us and 1.1 / 1.86 ns per element of K, beyond 3.05 us and for each of them 0.41 ns and 0.0045 per
+// element: fitted to widths of 64 - 8192, 1 - 144 heads of 64 and 33 - 448 rows.
+int64_t decode_general_ns(int64_t workgroups, int64_t K) {
+  return workgroups > 512 ? 3050 + workgroups * 41 / 100 + workgroups * K * 45 / 10000 : 3300 + K * (workgroups > 256 ? 186 : 110) / 100;
+}
+
 int launch_qkv_decode_general(const char* what, const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& fr, hipStream_t st) {
   const unsigned gx = (unsigned)((a.n_q_heads + 2 * a.n_kv_heads) * (a.head_dim / 16));
   const bool few = a.rows <= 8;

@@ -1,4 +1,4 @@
-// Argument block shared by the decode out-projection kernels (out_decode.hip, out_decode_r8.hip, out_decode_r32.hip, decode_general.hip).
+// Argument block shared by the decode out-projection kernels (out_decode.hip, out_decode_r8.hip, out_decode_r32.hip, decode_general.hip, tile_gemm.hip).
 #pragma once
 #include "common.h"
 
@@ -25,5 +25,12 @@ void launch_out_decode_r32(dim3 grid, hipStream_t st, const OutArgs& a);
 
 // any in_dim % 32 == 0 and out_dim, bf16 or fp8 weight, any rows in chunks of 8 or 16; x and W 16-byte aligned
 int launch_out_decode_general(const char* what, const OutArgs& a, hipStream_t st);
+
+// GEMM tiles (tile_gemm.hip), bf16 weight: whether they take these operands, and the launch
+bool linear_fits_tiles(const void* x, const void* W, int64_t rows, int64_t in_dim, int64_t out_dim);
+int launch_tile_gemm_out(const char* what, const OutArgs& a, hipStream_t st);
+
+// Whether tllm_out_residual_decode_bf16 takes them for aligned operands of these sizes and a bf16 weight (out_decode.hip)
+bool out_decode_tiles(int64_t rows, int64_t in_dim, int64_t out_dim);
 
 }  // namespace tllm

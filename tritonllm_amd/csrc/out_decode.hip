@@ -6,12 +6,14 @@
 //   out_decode_r32_kernel   (out_decode_r32.hip) the same shape, more rows in chunks of 32
 //                           both: bf16 or fp8 weight, weight-streaming through LDS, twelve output features per workgroup
 //   out_decode_general_kernel  (decode_general.hip)  any other in_dim % 32 == 0
+//   tile_gemm_kernel        (tile_gemm.hip) a bf16 weight and more rows than out_decode_tiles says
 //   out_generic_kernel      anything else: one wavefront per (row, feature) dot product.
 //
 // W8: fp8 (OCP e4m3) weight with one fp32 scale per output row, as the reference's ATTN_FP8 option
 // (triton_kernels.py:1385-1408); the values are widened to bf16 (exact) on their way into LDS and the row scale
 // multiplies the finished sum.
 #include "out_common.h"
+#include "qkv_prefill.h"
 
 namespace tllm {
 
@@ -42,9 +44,32 @@ __global__ __launch_bounds__(256) void out_generic_kernel(OutArgs a) {
   a.out[r * a.out_rs + n] = static_cast<bf16>(s);
 }
 
+// From where on GEMM tiles are ahead, us, decode kernel / tiles. The kernel for 4096 wide inputs reads its weight once for up to 128 rows in
+// chunks that follow each other, which is what it takes: [4096, 2880] 72 rows 12.8 / 13.2, 80 13.5 / 13.2, 96 14.9 / 13.8, 128 17.9 / 15.0, 192
+// 26.8 / 16.0, 400 51.2 / 19.5. Narrower outputs leave it as many CUs as it has workgroups of twelve columns, and each its own share of the
+// memory: 1536 columns 96 rows 12.3 / 13.2, 128 15.1 / 15.4, 144 15.1 / 12.8; 2304 columns 96 rows 13.4 / 13.5, 144 17.5 / 13.1. More than 256
+// workgroups take two rounds: 4032 columns 40 rows 16.0 / 14.5, 96 rows 25.0 / 14.1.
+// Any other width, as in qkv_decode_tiles: of 420 points at widths of 512 - 6144, 512 - 5120 columns and 16 - 400 rows 397 within 3 % of the
+// better one and none slower than before: [4096, 4096] 64 rows 17.9 / 17.0, 128 rows 34.8 / 16.5, 6144 x 5120 128 rows 93 / 30, 2048 x 2048 128
+// rows 10.2 / 9.6, and by the general kernel 1024 x 2880 64 rows 6.3 / 7.2, 2048 x 1024 192 rows 8.6 / 9.7.
+bool out_decode_tiles(int64_t rows, int64_t in_dim, int64_t out_dim) {
+  if (out_dim % 16 || in_dim % 64 || rows <= 32) return false;
+  if (in_dim == 4096 && out_dim % 12 == 0) return rows > (out_dim > 12 * 256 ? 32 : out_dim > 2560 ? 80 : 128);
+  const int64_t chunks = (rows + 15) / 16;
+  return tile_gemm_ns(rows, out_dim, in_dim) <= decode_general_ns(out_dim / 16 * chunks, in_dim);
+}
+
 }  // namespace tllm
 
 using namespace tllm;
+
+extern "C" int tllm_out_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim) {
+  if (rows < 1 || in_dim < 1 || out_dim < 1 || !out_decode_tiles(rows, in_dim, out_dim)) return 0;
+  int64_t ns;
+  const TileSize t = tile_gemm_pick(rows, out_dim, in_dim, &ns);
+  return t.bm << 16 | t.bn;
+}
+
 
 extern "C" int tllm_out_residual_decode_bf16(const void* x, const void* W, const float* w_scale, const void* bias, const void* residual,
                                              void* out, int64_t res_row_stride, int64_t out_row_stride, int64_t rows, int64_t in_dim,
@@ -71,7 +96,11 @@ extern "C" int tllm_out_residual_decode_bf16(const void* x, const void* W, const
   a.in_dim = (int)in_dim;
   a.out_dim = (int)out_dim;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (in_dim == 4096 && out_dim % 12 == 0 && aligned16(x) && aligned16(W) && out_dim * in_dim < (1ll << 31)) {
+  // (in as many rows as the decode kernels take)
+  const bool wide = in_dim == 4096 && out_dim % 12 == 0 && out_dim * in_dim < (1ll << 31);
+  if (!w_scale && rows <= (wide ? 32ll : 16ll) * 65535 && out_decode_tiles(rows, in_dim, out_dim) && linear_fits_tiles(x, W, rows, in_dim, out_dim))
+    return launch_tile_gemm_out("out_residual_decode", a, st);
+  if (wide && aligned16(x) && aligned16(W)) {
     const int64_t chunks = (rows + 31) / 32;
     TLLM_REQUIRE(chunks <= 65535, TLLM_E_SHAPE, "out_residual_decode: rows %lld too many for the decode kernel", (long long)rows);
     const dim3 grid((unsigned)(out_dim / 12), (unsigned)chunks);

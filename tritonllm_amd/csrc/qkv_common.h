@@ -58,6 +58,10 @@ void launch_qkv_decode_r32(bool w8, dim3 grid, hipStream_t st, const QkvArgs& a,
 // ... and for any number of rows in one pass over the weight, activations already normalised (qkv_decode_rows.hip).
 void launch_qkv_decode_rows(bool w8, dim3 grid, hipStream_t st, const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& fr);
 
+// What the general decode kernels (decode_general.hip) take beyond 32 rows with a bf16 weight, in ns: `workgroups` of sixteen weight rows x
+// sixteen rows, K of each.
+int64_t decode_general_ns(int64_t workgroups, int64_t K);
+
 // Any hidden % 32 == 0 and head_dim % 16 == 0, bf16 or (a.w_scale != null) fp8 weight, any rows in chunks of 8 or 16; x and W
 // 16-byte aligned, q / k / v 4-byte aligned with even strides (decode_general.hip).
 int launch_qkv_decode_general(const char* what, const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& fr, hipStream_t st);

@@ -125,13 +125,11 @@ bool qkv_decode_tiles(int64_t rows, int64_t hidden, int heads, int head_dim) {
   // hundred rows a GEMM tile is ahead of it (97 rows 16.1, 128 rows 16.2, 256 rows 21.2)
   if (hidden == 2880) return tile_gemm_ns(rows, cols, hidden) < 6400 + 1400 * ((rows + 15) / 16);
   // Beyond 32 rows the general kernel reads the weight a third time, which costs little while its workgroups -- sixteen weight
-  // rows x sixteen rows -- are on the machine together. Its time over widths of 64 - 8192, 1 - 144 heads and 33 - 448 rows, ns: up to
-  // 256 and 512 workgroups 3300 and 1.1 / 1.86 per element of K, beyond 3050 and 0.41 and 0.0045 per element for each of them.
-  // Chosen so, 848 of 864 points are within 3 % of the better of the two; us, general and tiles: hidden 512, 12 heads, 64 rows 3.7
+  // rows x sixteen rows -- are on the machine together (decode_general_ns).
+  // Over widths of 64 - 8192, 1 - 144 heads and 33 - 448 rows, 848 of 864 points are within 3 % of the better of the two; us, general and tiles: hidden 512, 12 heads, 64 rows 3.7
   // and 6.3, 1024, 20 heads, 128 rows 6.3 and 7.7, 80 heads, 64 rows 8.9 and 7.8; 4096, 32 heads, 64 rows 11.9 and 18.1, 80 heads 25.8 and 19.4
   const int64_t workgroups = static_cast<int64_t>(heads) * 4 * ((rows + 15) / 16);
-  const int64_t general_ns = workgroups > 512 ? 3050 + workgroups * 41 / 100 + workgroups * hidden * 45 / 10000 : 3300 + hidden * (workgroups > 256 ? 186 : 110) / 100;
-  return tile_gemm_ns(rows, cols, hidden) <= general_ns;
+  return tile_gemm_ns(rows, cols, hidden) <= decode_general_ns(workgroups, hidden);
 }
 
 }  // namespace tllm

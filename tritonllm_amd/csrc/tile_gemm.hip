@@ -2,7 +2,8 @@
 // with bias. At 80 heads of 64 and a width of 2880 that is prompts of up to 1536 rows, those for which the larger tiles of
 // qkv_prefill.hip would need one more round for little (2049 - 2816, 4097 - 4864, 6145 - 6528, ... rows; qkv_prefill_tiles), and
 // decode batches from 113 rows on (qkv_decode_tiles); the plain projection where it is ahead of the library's GEMM, up to
-// 2432 rows of [2880, 4096] (linear_in_tiles in host_ops.cpp).
+// 2432 rows of [2880, 4096] (linear_in_tiles in host_ops.cpp). With a residual in the epilogue it is the out-projection of decode
+// batches from 81 rows on (out_decode_tiles: [4096, 2880] 96 rows 14.9 -> 14.0 us, 128 17.9 -> 15.1, 200 30.7 -> 16.1; [4096, 4096] 128 34.8 -> 16.6).
 //
 //   D[rows, n] = X[rows, K] . W[n, K]^T      (both operands K-contiguous, K a multiple of 64)
 //
@@ -33,6 +34,7 @@
 //   999 38.6 (49.1)   1100 40.4 (55.0)   1400 45.7 (57.1)   1536 49.9 (57)
 // [rows, 4096] x [4096, 2880] + bias (before: the library's GEMM):
 //   97 rows 13.6 (15.5)   192 15.5 (32.4)   333 17.9 (30.3)   512 20.7 (25.2)   999 32.4 (36.5)   2048 49.9 (53.4)
+#include "out_common.h"
 #include "qkv_prefill.h"
 
 namespace tllm {
@@ -61,7 +63,7 @@ struct Tile {
 };
 }  // namespace tile_gemm
 
-enum : int { kGemmLinear = 0, kGemmYarn = 1, kGemmTable = 2 };   // plain | QKV, cos / sin from YaRN parameters | ... from tables
+enum : int { kGemmLinear = 0, kGemmYarn = 1, kGemmTable = 2, kGemmResidual = 3 };   // plain | QKV, cos / sin from YaRN parameters | ... from tables | plain + residual (a.k, row stride a.k_rs)
 
 template <int N, int LPW>
 __device__ __forceinline__ void wait_slices_left(int left) {     // at most `left` (<= N) slices of LPW loads still in flight
@@ -77,6 +79,7 @@ __device__ __forceinline__ void wait_slices_left(int left) {     // at most `lef
 template <class C, int MODE, bool TURN>
 __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, YarnFreqs fr, int tiles_m, int n_blocks) {
   using namespace tile_gemm;
+  constexpr bool QKV = MODE == kGemmYarn || MODE == kGemmTable;
   constexpr int TB = C::TB, RB = C::RB, KG = C::KG, KS = C::KS, BM = C::BM, BN = C::BN, S = C::S, STAGE = C::STAGE, SLICE = C::SLICE, WSLICE = C::WSLICE;
   constexpr int LX = C::LX, LPW = C::LPW, NB = BN / 16;
   constexpr int NMF = TB * RB, NRD = TB + RB;               // MFMAs and fragment reads per k32 step
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
     int B = block0 + (i >> 4);
     if (B >= n_blocks) B = n_blocks - 1;
     const int i16 = i & 15;
-    if constexpr (MODE == kGemmLinear) return 16 * B + i16;
+    if constexpr (!QKV) return 16 * B + i16;
     else return (B >> 2) * 64 + 8 * (B & 3) + 2 * (i16 >> 2) + (i16 & 1) + 32 * ((i16 >> 1) & 1);
   };
 
@@ -207,6 +210,18 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
     const bf16* bp = a.bias ? a.bias : a.W;                          // absent: a valid address instead of a branch
     bias_raw = bp[weight_row(tid < BN ? tid : BN - 1)];
   }
+  // ... as does the residual of the thread's first sixteen outputs, where the registers allow it (the epilogue's row and block of i = tid)
+  constexpr bool RES = MODE == kGemmResidual, RES_EARLY = RES && BM == 64;
+  const bool res_vec = RES && reinterpret_cast<uintptr_t>(a.k) % 16 == 0 && a.k_rs % 8 == 0;
+  bf16x8 res_early[2];
+  if constexpr (RES_EARLY) {
+    const int b = (tid >> 4) % NB, tbw = (tid >> 4) / NB, r = 16 * (TB * (tbw / C::BP) + tbw % C::BP) + (tid & 15);
+    const int64_t grow = row0 + r < a.rows ? row0 + r : a.rows - 1;
+    const int B = block0 + b < n_blocks ? block0 + b : n_blocks - 1;
+    const bf16* const from = res_vec ? a.k + grow * a.k_rs + 16 * B : a.x;       // (else looked at element by element, later)
+    res_early[0] = *reinterpret_cast<const bf16x8*>(from);
+    res_early[1] = *reinterpret_cast<const bf16x8*>(from + 8);
+  }
   const int first = n_iter < S ? n_iter : S;
   int ahead = rot;                                                  // the stage of K that is loaded next
   auto turn = [&](int next) { ahead = TURN ? (ahead + 1 == n_iter ? 0 : ahead + 1) : next; };
@@ -227,7 +242,7 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
   const int f = lane & 31;
   float2 csr[CSN];
   bool plain = true;
-  if (MODE != kGemmLinear && a.has_rope) {
+  if (QKV && a.has_rope) {
     int pos[RPW];
     plain = rope_positions_uniform<RPW>(ra, a.W, first_row, a.rows, pos);
 #pragma unroll
@@ -285,9 +300,9 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
 
   // ---- epilogue, BP row blocks of every wavefront at a time: the sums go to LDS as they are, and a rolled loop over (row,
   // sixteen-column block) adds the KG shares in a fixed order, adds the bias, rotates, rounds once and stores 2 x 16 bytes.
-  const int64_t slot_off = MODE == kGemmLinear ? 0 : qkv_slot(a, ra) * a.kv_slot_stride;
+  const int64_t slot_off = !QKV ? 0 : qkv_slot(a, ra) * a.kv_slot_stride;
   const bool vec_ok = (reinterpret_cast<uintptr_t>(a.q) % 16 == 0) && a.q_rs % 8 == 0 &&
-                      (MODE == kGemmLinear || ((reinterpret_cast<uintptr_t>(a.k) % 16 == 0) && (reinterpret_cast<uintptr_t>(a.v) % 16 == 0) &&
+                      (!QKV || ((reinterpret_cast<uintptr_t>(a.k) % 16 == 0) && (reinterpret_cast<uintptr_t>(a.v) % 16 == 0) &&
                                                a.k_rs % 8 == 0 && a.v_rs % 8 == 0 && a.kv_slot_stride % 8 == 0));
   f32x4* const sums = reinterpret_cast<f32x4*>(smem);
   constexpr int BP = C::BP;
@@ -295,7 +310,7 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
 #pragma unroll
   for (int pass = 0; pass < C::PASSES; ++pass) {
     __syncthreads();                                                 // the ring, or the pass before, is done with
-    if (MODE != kGemmLinear && a.has_rope && pass == 0) {
+    if (QKV && a.has_rope && pass == 0) {
       float2* const mine = cs_tab + (RPW * wave + (lane >> 5)) * CSROW + f;
       if (plain) {
 #pragma unroll
@@ -337,7 +352,29 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
       }
       bf16x8 o0, o1;                                                 // QKV: eight low dims and their partners 32 up; plain: columns 0-7, 8-15
       bf16 *d0, *d1;
-      if constexpr (MODE == kGemmLinear) {
+      if constexpr (RES) {
+        const bf16* const from = a.k + grow * a.k_rs + 16 * B;
+        bf16x8 r0, r1;
+        if (RES_EARLY && res_vec && pass == 0 && i == tid) {
+          r0 = res_early[0];
+          r1 = res_early[1];
+        } else if (res_vec) {
+          r0 = *reinterpret_cast<const bf16x8*>(from);
+          r1 = *reinterpret_cast<const bf16x8*>(from + 8);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            r0[e] = from[e];
+            r1[e] = from[8 + e];
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          v[e] += static_cast<float>(r0[e]);
+          v[8 + e] += static_cast<float>(r1[e]);
+        }
+      }
+      if constexpr (!QKV) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           o0[e] = static_cast<bf16>(v[e]);
@@ -499,6 +536,29 @@ extern "C" int tllm_linear_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_d
   const TileSize t = tile_gemm_pick(rows, out_dim, in_dim, &ns);
   return t.bm << 16 | t.bn;
 }
+
+namespace tllm {
+// What tllm_linear_bf16 takes, of K, outputs and alignment.
+bool linear_fits_tiles(const void* x, const void* W, int64_t rows, int64_t in_dim, int64_t out_dim) {
+  return rows < (1ll << 31) && in_dim >= 64 && in_dim % 64 == 0 && out_dim >= 16 && out_dim % 16 == 0 && in_dim * out_dim * 2 < (1ll << 32) &&
+         in_dim * 512 < (1ll << 32) && aligned16(x) && aligned16(W);
+}
+
+int launch_tile_gemm_out(const char* what, const OutArgs& o, hipStream_t st) {
+  QkvArgs a{};
+  a.x = o.x;
+  a.W = static_cast<const bf16*>(o.W);
+  a.bias = o.bias;
+  a.k = const_cast<bf16*>(o.res);
+  a.k_rs = o.res_rs;
+  a.q = o.out;
+  a.q_rs = o.out_rs;
+  a.rows = o.rows;
+  a.hidden = o.in_dim;
+  const int n_blocks = o.out_dim / 16;
+  return o.res ? launch_mode<kGemmResidual>(what, a, RopeArgs{}, YarnFreqs{}, n_blocks, st) : launch_mode<kGemmLinear>(what, a, RopeArgs{}, YarnFreqs{}, n_blocks, st);
+}
+}  // namespace tllm
 
 extern "C" int tllm_gemm_tile_spread(int64_t rows, int64_t in_dim, int64_t out_dim) {
   int64_t ns;
