@@ -840,6 +840,28 @@ def test_qkv_large_tiles_every_position_source(gpu, rows):
     _check_qkv_position_sources(gpu, rows, 2880, 64, 8, "prefill", seed=rows)
 
 
+@pytest.mark.parametrize("rows,hidden,tile", [(65, 192, True), (333, 64, True), (2011, 2880, False), (4000, 2880, False)])
+@pytest.mark.parametrize("length", [1, 2, 7, 64, 65, 100, 10000])
+def test_qkv_positions_of_several_sequences(gpu, rows, hidden, tile, length):
+    """Sequences of every length beside what a wavefront counts through (8 or 16 rows), without a positions tensor, up to the last position
+    there is; then one step further, where the last row of a whole sequence wraps around."""
+    nq, nkv = (8, 2) if tile else (64, 8)
+    assert bool(_lib.lib().tllm_qkv_gemm_tile(1, rows, hidden, nq, nkv, 64)) == tile
+    g = torch.Generator().manual_seed(rows + length)
+    x = torch.randn(rows, hidden, generator=g).bfloat16()
+    w = (0.05 * torch.randn((nq + 2 * nkv) * 64, hidden, generator=g)).bfloat16()
+    plain = O.linear_ref(x, w, torch.zeros(w.shape[0]).bfloat16())
+    used, n = min(length, rows), (nq + nkv) * 64
+    for first in (4096 - used, 4097 - used):
+        want = plain.clone()
+        pos = (first + torch.arange(rows) % length) % 4096
+        want[:, :n] = O.rope_rotate_ref(plain[:, :n].reshape(rows, nq + nkv, 64), *O.yarn_cos_sin(pos)).reshape(rows, n)
+        got = T.qkv_rope_forward(x.to(gpu), w.to(gpu), torch.zeros(w.shape[0], dtype=torch.bfloat16, device=gpu), nq, nkv, 64, mode="prefill",
+                                 yarn=T.gpt_oss_yarn(), offset=torch.tensor([first], device=gpu), tokens_per_batch=length, max_context_length=4096)
+        for have, part in zip(got, torch.split(want, (nq * 64, nkv * 64, nkv * 64), dim=1)):
+            close(have, part)
+
+
 @pytest.mark.parametrize("batch,hidden,nq,nkv,tiles", [(100, 2880, 64, 8, False), (131, 2880, 64, 8, True), (41, 4096, 64, 8, True), (40, 512, 8, 2, False)])
 @pytest.mark.parametrize("how", ["offset", "positions"])
 def test_qkv_cache_form_of_large_batches(gpu, batch, hidden, nq, nkv, tiles, how):

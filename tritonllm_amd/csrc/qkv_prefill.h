@@ -10,8 +10,10 @@ namespace tllm {
 __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 
 // Rotary positions of N consecutive rows starting at row g0 (the same in every lane; rows past the last one repeat it), as
-// they are when all of them lie in [0, max_ctx) -- which the return value says -- and no row belongs to a second sequence.
-// Otherwise (wrap-around, several sequences without a positions tensor) the caller fills its table with rope_position(), in
+// they are when all of them lie in [0, max_ctx), which the return value says. Without a positions tensor one 32-bit division
+// finds the first row's place in its sequence and the others follow by counting (a decode batch: every row is one; with a table filled
+// row by row 128 rows of 2880 took 18.2 us and take 16.9, 200 rows 20.7 and 18.7, 33 rows of 4096 17.6 and 16.1).
+// Otherwise (wrap-around, more than 2^31 rows) the caller fills its table with rope_position(), in
 // a rolled loop: the 64-bit divisions inlined per row were 32 KB of code to fetch, executed or not, at about 1 us per 8 KB.
 // Read through the scalar cache: positions and offset were written before this kernel started and nothing writes them while
 // it runs, and a scalar load does not involve the vector-memory counter the look-ahead loads are waited for with.
@@ -23,16 +25,22 @@ __device__ __forceinline__ bool rope_positions_uniform(const RopeArgs& r, const 
   const_i64_ptr po = reinterpret_cast<const_i64_ptr>(reinterpret_cast<uintptr_t>(r.offset ? static_cast<const void*>(r.offset) : any_valid));
   const int64_t off_ld = po[0];
   const int64_t off = r.offset ? off_ld : 0;
+  const bool counts = rows < (1ll << 31);
+  // a sequence longer than the batch is as good as one that ends with it
+  const unsigned length = static_cast<unsigned>(r.tokens_per_batch < rows ? r.tokens_per_batch : rows);
+  const int64_t start = g0 < rows ? g0 : rows - 1;
+  unsigned within = counts ? static_cast<unsigned>(start) % length : 0;
   uint64_t most = 0;
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     const int64_t gi = g0 + j < rows ? g0 + j : rows - 1;
     const int64_t ld = pp[r.positions ? gi : 0];
-    const uint64_t q = static_cast<uint64_t>(r.positions ? ld : off + gi);
+    const uint64_t q = static_cast<uint64_t>(r.positions ? ld : off + static_cast<int64_t>(within));
+    if (g0 + j + 1 < rows) within = within + 1 == length ? 0 : within + 1;
     pos[j] = static_cast<int>(q);
     if (q > most) most = q;
   }
-  return most < static_cast<uint64_t>(r.max_ctx) && most < (1ull << 31) && (r.positions || rows <= r.tokens_per_batch);
+  return most < static_cast<uint64_t>(r.max_ctx) && most < (1ull << 31) && (r.positions || counts);
 }
 
 // (cos, sin) of frequency f at position p in [0, max_ctx)
