@@ -219,6 +219,8 @@ int tllm_linear_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim);
 int tllm_out_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim);
 /* Diagnostic: whether that tile's launch (or the QKV projection's, out_dim = 64 x heads) spreads its row tiles' walks over K. */
 int tllm_gemm_tile_spread(int64_t rows, int64_t in_dim, int64_t out_dim);
+/* Diagnostic: how many row tiles that launch takes before the next column of tiles. */
+int tllm_gemm_tile_group(int64_t rows, int64_t in_dim, int64_t out_dim);
 /* Diagnostic: wavefronts that stream the weight in a workgroup of the general-shape decode projections (4, 2 or 1). */
 int tllm_decode_general_streams(int64_t rows, int64_t in_dim, int64_t out_dim, int fp8);
 

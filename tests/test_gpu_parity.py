@@ -921,6 +921,19 @@ def test_linear_walks_spread_over_k(gpu, bm, bn, rows, n, k):
     assert torch.equal(out[rows - 1].float().cpu()[w[:, k - 1] != 0], (w[:, k - 1].float() * float("inf"))[w[:, k - 1] != 0])
 
 
+@pytest.mark.parametrize("rows,n,k,tiles_m,group", [(1024, 1040, 2048, 16, 16), (1025, 1040, 2048, 17, 8), (1536, 1040, 2048, 24, 8), (1551, 1040, 2048, 25, 8),
+                                                    (2048, 1024, 64, 32, 32), (2049, 1024, 64, 33, 8), (2177, 2064, 1088, 18, 8)])
+def test_linear_row_tiles_in_groups(gpu, rows, n, k, tiles_m, group):
+    """Either side of the rules, a last group of one row tile, of two and of all eight, a ragged last column."""
+    L = _lib.lib()
+    assert -(-rows // (L.tllm_linear_gemm_tile(rows, k, n) >> 16)) == tiles_m and L.tllm_gemm_tile_group(rows, k, n) == group
+    g = torch.Generator().manual_seed(rows + n + k)
+    x, w, b = torch.randn(rows, k, generator=g).bfloat16(), (0.05 * torch.randn(n, k, generator=g)).bfloat16(), (0.05 * torch.randn(n, generator=g)).bfloat16()
+    xg, wg, bg, out = x.to(gpu), w.to(gpu), b.to(gpu), torch.full((rows, n), 7.0, dtype=torch.bfloat16, device=gpu)
+    assert L.tllm_linear_bf16(xg.data_ptr(), wg.data_ptr(), bg.data_ptr(), out.data_ptr(), n, rows, k, n, torch.cuda.current_stream().cuda_stream) == 0
+    close(out, O.linear_ref(x, w, b))
+
+
 @pytest.mark.parametrize("rows", [128, 192, 333, 513, 640])
 def test_qkv_walks_spread_over_k(gpu, rows):
     assert _lib.lib().tllm_gemm_tile_spread(rows, 2880, 5120) == 1

@@ -54,6 +54,7 @@ SIGNATURES = {
     "tllm_qkv_gemm_tile": (_i32, [_i32, _i64, _i64, _i32, _i32, _i32]),
     "tllm_linear_gemm_tile": (_i32, [_i64, _i64, _i64]),
     "tllm_out_gemm_tile": (_i32, [_i64, _i64, _i64]),
+    "tllm_gemm_tile_group": (_i32, [_i64, _i64, _i64]),
     "tllm_gemm_tile_spread": (_i32, [_i64, _i64, _i64]),
     "tllm_decode_general_streams": (_i32, [_i64, _i64, _i64, _i32]),
     "tllm_linear_bf16": (_i32, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),

@@ -77,7 +77,7 @@ __device__ __forceinline__ void wait_slices_left(int left) {     // at most `lef
 
 // TURN: the row tiles begin their walks over K at different places (tile_gemm_spread).
 template <class C, int MODE, bool TURN>
-__global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, YarnFreqs fr, int tiles_m, int n_blocks) {
+__global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, YarnFreqs fr, int tiles_m, int tiles_n, int group, int n_blocks) {
   using namespace tile_gemm;
   constexpr bool QKV = MODE == kGemmYarn || MODE == kGemmTable;
   constexpr int TB = C::TB, RB = C::RB, KG = C::KG, KS = C::KS, BM = C::BM, BN = C::BN, S = C::S, STAGE = C::STAGE, SLICE = C::SLICE, WSLICE = C::WSLICE;
@@ -90,10 +90,13 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
   const int m16 = lane & 15, g = lane >> 4;
 
   // Consecutive block ids go to the eight XCDs in turn: give each XCD a contiguous run of tiles, row tiles fastest, so
-  // that the tiles that read the same weight columns share an L2 and the weight leaves HBM once.
+  // that the tiles that read the same weight columns share an L2 and the weight leaves HBM once. Of many row tiles `group` at a
+  // time, so that an XCD's tiles -- about a rectangle then -- share the rows as well (tile_gemm_group).
   const int tiles = gridDim.x, xcd = blockIdx.x & 7, per = tiles >> 3, extra = tiles & 7;
   const int id = xcd * per + (xcd < extra ? xcd : extra) + (blockIdx.x >> 3);
-  const int tile_m = id % tiles_m, tile_n = id / tiles_m;
+  const int in_group = group * tiles_n, grp = id / in_group, first_m = grp * group;
+  const int group_m = tiles_m - first_m < group ? tiles_m - first_m : group, tile_n = (id - grp * in_group) / group_m;
+  const int tile_m = first_m + (id - grp * in_group) % group_m;
   const int64_t row0 = static_cast<int64_t>(tile_m) * BM;
   const int block0 = tile_n * NB;
   const int n_slices = a.hidden / BK, n_iter = (n_slices + KS - 1) / KS;
@@ -420,14 +423,22 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
 }
 
 namespace {
+// Row tiles that a column of tiles takes before the next column begins. All of them, up to 16: the rows that an XCD's 32 tiles of a round
+// read are then few enough. Beyond, eight; us, all and eight, 17 - 50 row tiles: [rows, 2880] x [2880, 5120] 2300 rows 81.4 / 76.9, 2800 90.5 /
+// 86.3, 4300 142.9 / 132.6, 6300 190.6 / 180.5; 2880 x 1024 1411 rows 16.7 / 15.1, 2500 24.5 / 20.6; 4096 x 5120 2300 99.6 / 91.2 (six and four
+// the same within 1 %; with fewer row tiles 4096 x 2880 1100 rows 36.4 / 37.8, 2048 50.9 / 50.3). An operand that is small anyway has
+// nothing to gain before the rows are many: 1024 x 1024 1411 rows 8.2 / 8.3, 2300 11.3 / 10.8.
+int64_t tile_gemm_group(int64_t tiles_m, int64_t weight) { return tiles_m > (weight > 2000000 ? 16 : 32) ? 8 : tiles_m; }
+
 template <class C, int MODE, bool TURN>
 int launch_one(const char* what, const QkvArgs& a, const RopeArgs& ra, const YarnFreqs& fr, int n_blocks, hipStream_t st) {
   static std::atomic<uint64_t> done{0};
   const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(tile_gemm_kernel<C, MODE, TURN>), C::SMEM, done);
   TLLM_REQUIRE(e == hipSuccess, TLLM_E_LAUNCH, "%s: cannot raise LDS limit: %s", what, hipGetErrorString(e));
   const int64_t tiles_m = (a.rows + C::BM - 1) / C::BM, tiles_n = (n_blocks * 16 + C::BN - 1) / C::BN;
+  const int64_t group = tile_gemm_group(tiles_m, static_cast<int64_t>(n_blocks) * 16 * a.hidden);
   TLLM_REQUIRE(tiles_m * tiles_n < (1ll << 31), TLLM_E_SHAPE, "%s: too many tiles", what);
-  hipLaunchKernelGGL((tile_gemm_kernel<C, MODE, TURN>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), C::SMEM, st, a, ra, fr, (int)tiles_m, n_blocks);
+  hipLaunchKernelGGL((tile_gemm_kernel<C, MODE, TURN>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), C::SMEM, st, a, ra, fr, (int)tiles_m, (int)tiles_n, (int)group, n_blocks);
   return check_launch(what);
 }
 
@@ -559,6 +570,12 @@ int launch_tile_gemm_out(const char* what, const OutArgs& o, hipStream_t st) {
   return o.res ? launch_mode<kGemmResidual>(what, a, RopeArgs{}, YarnFreqs{}, n_blocks, st) : launch_mode<kGemmLinear>(what, a, RopeArgs{}, YarnFreqs{}, n_blocks, st);
 }
 }  // namespace tllm
+
+extern "C" int tllm_gemm_tile_group(int64_t rows, int64_t in_dim, int64_t out_dim) {
+  int64_t ns;
+  const int64_t bm = tile_gemm_pick(rows, out_dim, in_dim, &ns).bm;
+  return static_cast<int>(tile_gemm_group((rows + bm - 1) / bm, out_dim * in_dim));
+}
 
 extern "C" int tllm_gemm_tile_spread(int64_t rows, int64_t in_dim, int64_t out_dim) {
   int64_t ns;
