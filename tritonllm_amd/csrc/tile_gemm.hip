@@ -94,9 +94,15 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
   // time, so that an XCD's tiles -- about a rectangle then -- share the rows as well (tile_gemm_group).
   const int tiles = gridDim.x, xcd = blockIdx.x & 7, per = tiles >> 3, extra = tiles & 7;
   const int id = xcd * per + (xcd < extra ? xcd : extra) + (blockIdx.x >> 3);
-  const int in_group = group * tiles_n, grp = id / in_group, first_m = grp * group;
-  const int group_m = tiles_m - first_m < group ? tiles_m - first_m : group, tile_n = (id - grp * in_group) / group_m;
-  const int tile_m = first_m + (id - grp * in_group) % group_m;
+  // (The second division only where there are groups: it is on the first loads' way, 97 rows of [4096, 2880] 13.7 us without it, 14.0 with.)
+  int first_m = 0, group_m = tiles_m, in_group = id;
+  if (group < tiles_m) {
+    const int grp = id / (group * tiles_n);
+    first_m = grp * group;
+    in_group -= first_m * tiles_n;
+    group_m = tiles_m - first_m < group ? tiles_m - first_m : group;
+  }
+  const int tile_n = in_group / group_m, tile_m = first_m + in_group % group_m;
   const int64_t row0 = static_cast<int64_t>(tile_m) * BM;
   const int block0 = tile_n * NB;
   const int n_slices = a.hidden / BK, n_iter = (n_slices + KS - 1) / KS;
