@@ -972,6 +972,19 @@ def test_linear_hands_over_to_the_library_where_that_is_ahead(gpu, k, n, tiles, 
     assert [took(rows) for rows in tiles] == [True] * len(tiles) and [took(rows) for rows in library] == [False] * len(library)
 
 
+@pytest.mark.parametrize("rows,k,n,tiles", [(2433, 192, 2880, True), (2560, 192, 2880, True), (2561, 192, 2880, False), (1920, 128, 4080, True),
+                                            (1921, 128, 4080, True), (2049, 128, 4080, False), (2433, 128, 3072, False)])
+def test_linear_one_round_of_the_widest_tiles(gpu, rows, k, n, tiles):
+    """Outputs that are no multiple of 128 stay on GEMM tiles while 128 x 256 ones cover them in one round."""
+    g = torch.Generator().manual_seed(rows + n)
+    x, w = torch.randn(rows, k, generator=g).bfloat16(), (0.05 * torch.randn(n, k, generator=g)).bfloat16()
+    b = (0.05 * torch.randn(n, generator=g)).bfloat16()
+    got = host().linear(x.to(gpu), w.to(gpu), b.to(gpu))
+    assert (got is not None) == tiles
+    if tiles:
+        close(got, O.linear_ref(x, w, b))
+
+
 def test_linear_leaves_torch_its_hooks(gpu):
     """OUT.forward under what F.linear takes part in: vmap, forward-mode derivatives, autocast, tracing, symbolic tracing, a
     dispatch mode, a tensor subclass; a strided operand and one that is not 16-byte aligned."""

@@ -458,14 +458,18 @@ bool plain_operand(PyObject* o, c10::DeviceIndex device) {
 
 // Whether a GEMM tile is ahead of the library's GEMM. Up to tiles of 128 x 224 covering the result in one round of the 256 CUs
 // and about 2500 rows it mostly is ([2880, 4096] weight, us: 97 rows 13.9 and 15.4, 192 rows 18.8 and 32, 999 rows 33.9 and 36.6,
-// 2400 rows 53.0 and 54.8; behind that 2500 rows 57.4 and 55.9, 2700 67.8 and 58.2, 4096 103 and 83; other weights 3000 rows
-// 0.84 - 0.92 of the library's rate). Where the tiles are few and K is long the library shares K out between workgroups: from a K of
+// 2400 rows 53.0 and 54.8; behind two rounds 2700 67.8 and 58.2, 4096 103 and 83; other weights 3000 rows 0.84 - 0.92 of the
+// library's rate). Tiles of 128 x 256 are ahead as long as they are one round if the outputs are no multiple of 128, which the library's
+// own tiles would fit ([2880, 4096] 2500 rows 55.3 and 58.5, K = 2048 33.0 and 36.3, 512 17.0 and 21.5; [4400, 4096] 1664 55.9 and 59.7; [8176,
+// 2880] 1024 44.5 and 47.8; but [3072, 4096] 2500 55.7 and 53.9, [2048, 4096] 2560 43.8 and 41.4), up to weights of about 25 M elements
+// ([6000, 4096] 1280 rows 55.9 and 59.4, [6992, 4096] 1092 62.1 and 58.6). Where the tiles are few and K is long the library shares K out between workgroups: from a K of
 // 50 per tile on (32 above 4096) it is ahead ([512, 2048] 48 rows 5.7 and 7.4, [1024, 8192] 48 rows 11.9 and 17.2, [2880, 5120]
 // 8 rows 10.5 and 15.5), with 25 - 64 rows of a K of 2900 and more from 30 on ([2880, 4096] 48 rows 13.1 and 14.9). And it has
 // a kernel for a few rows of a small weight ([512, 512] 16 rows 4.1 and 4.7, [1024, 1024] 4.6 and 5.8). Of 1600 calls of a K of
 // 64 .. 8192 and 128 .. 8192 outputs measured, 85 are 3 % slower so than with the library, 353 without the latter three.
 bool linear_in_tiles(int64_t rows, int64_t k, int64_t out) {
-  if (rows > 2560 || ((rows + 127) / 128) * ((out + 223) / 224) > 256) return false;
+  const int64_t widest = out % 128 && out * k <= 25000000 ? 256 : 224;
+  if (rows > 2560 || ((rows + 127) / 128) * ((out + widest - 1) / widest) > 256) return false;
   const int tile = tllm_linear_gemm_tile(rows, k, out);
   const int64_t bm = tile >> 16, bn = tile & 0xffff, tiles = ((rows + bm - 1) / bm) * ((out + bn - 1) / bn);
   if (k >= 1024 && k >= (k > 4096 ? 32 : 50) * tiles) return false;

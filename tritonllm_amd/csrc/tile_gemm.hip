@@ -2,7 +2,7 @@
 // with bias. At 80 heads of 64 and a width of 2880 that is prompts of up to 1536 rows, those for which the larger tiles of
 // qkv_prefill.hip would need one more round for little (2049 - 2816, 4097 - 4864, 6145 - 6528, ... rows; qkv_prefill_tiles), and
 // decode batches from 113 rows on (qkv_decode_tiles); the plain projection where it is ahead of the library's GEMM, up to
-// 2432 rows of [2880, 4096] (linear_in_tiles in host_ops.cpp). With a residual in the epilogue it is the out-projection of decode
+// 2560 rows of [2880, 4096] (linear_in_tiles in host_ops.cpp). With a residual in the epilogue it is the out-projection of decode
 // batches from 81 rows on (out_decode_tiles: [4096, 2880] 96 rows 14.9 -> 14.0 us, 128 17.9 -> 15.1, 200 30.7 -> 16.1; [4096, 4096] 128 34.8 -> 16.6).
 //
 //   D[rows, n] = X[rows, K] . W[n, K]^T      (both operands K-contiguous, K a multiple of 64)
