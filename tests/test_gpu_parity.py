@@ -862,6 +862,32 @@ def test_qkv_positions_of_several_sequences(gpu, rows, hidden, tile, length):
             close(have, part)
 
 
+@pytest.mark.parametrize("rows,hidden,tile", [(97, 192, True), (2011, 2880, False)])
+def test_qkv_positions_out_of_range(gpu, rows, hidden, tile):
+    """Positions that wrap around -- one step too far, negative, wide of 32 bits -- at the first row, inside and in the last run of rows that
+    a wavefront reads, beside rows that do not; and offsets like that."""
+    nq, nkv = (8, 2) if tile else (64, 8)
+    assert bool(_lib.lib().tllm_qkv_gemm_tile(1, rows, hidden, nq, nkv, 64)) == tile
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, hidden, generator=g).bfloat16()
+    w = (0.05 * torch.randn((nq + 2 * nkv) * 64, hidden, generator=g)).bfloat16()
+    plain, n = O.linear_ref(x, w, torch.zeros(w.shape[0]).bfloat16()), (nq + nkv) * 64
+    sources = []
+    for odd in (4096, -1, (1 << 32) + 7, (1 << 62) + 5, -(1 << 31)):
+        pos = torch.arange(rows) % 300
+        pos[[0, rows // 2, rows - 1]] = odd
+        sources.append((dict(positions=pos.to(gpu)), pos % 4096))
+    for first in (-3, (1 << 32) - 2, 1 << 40):
+        sources.append((dict(offset=torch.tensor([first], device=gpu)), (first + torch.arange(rows)) % 4096))
+    for source, pos in sources:
+        want = plain.clone()
+        want[:, :n] = O.rope_rotate_ref(plain[:, :n].reshape(rows, nq + nkv, 64), *O.yarn_cos_sin(pos)).reshape(rows, n)
+        got = T.qkv_rope_forward(x.to(gpu), w.to(gpu), torch.zeros(w.shape[0], dtype=torch.bfloat16, device=gpu), nq, nkv, 64, mode="prefill",
+                                 yarn=T.gpt_oss_yarn(), max_context_length=4096, **source)
+        for have, part in zip(got, torch.split(want, (nq * 64, nkv * 64, nkv * 64), dim=1)):
+            close(have, part)
+
+
 @pytest.mark.parametrize("batch,hidden,nq,nkv,tiles", [(100, 2880, 64, 8, False), (131, 2880, 64, 8, True), (41, 4096, 64, 8, True), (40, 512, 8, 2, False)])
 @pytest.mark.parametrize("how", ["offset", "positions"])
 def test_qkv_cache_form_of_large_batches(gpu, batch, hidden, nq, nkv, tiles, how):

@@ -294,7 +294,7 @@ __global__ __launch_bounds__(512) void qkv_prefill_quads_kernel(QkvArgs a, RopeA
   bool plain = true;
   if (a.has_rope) {
     int pos[2 * CSN];
-    plain = rope_positions_uniform<2 * CSN>(ra, a.W, first_row, a.rows, pos);
+    plain = rope_positions_uniform<2 * CSN>(ra, first_row, a.rows, pos);
     // TABLE: the youngest loads of the prologue: every wait below is for older loads and so at most stricter than it
     // needs to be until these have landed, which they have by the loop's second slice.
 #pragma unroll

@@ -243,8 +243,8 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
   // cos / sin of (row, frequency), computed while the first slices arrive and kept in registers. Wavefront w: rows BM / 8 w
   // .. of the tile; lane: frequency lane % 32, rows 2 j + lane / 32 of those. The rows' positions come through the scalar
   // cache and are used as they are when all of them lie in [0, max_ctx), which one comparison of their unsigned maximum
-  // says; otherwise (wrap-around, several sequences without a positions tensor) the epilogue fills the table in a rolled
-  // loop: the 64-bit divisions inlined here would be 30 KB of code to fetch, executed or not.
+  // says; otherwise (wrap-around) the epilogue fills the table in a rolled loop: the 64-bit divisions inlined here would be 30 KB
+  // of code to fetch, executed or not.
   constexpr int RPW = BM / 8, CSN = RPW / 2;                // rows of a wavefront: 8 or 16
   static_assert(RPW == 8 || RPW == 16, "one batch of scalar loads");
   const int64_t first_row = row0 + RPW * wave;
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(512) void tile_gemm_kernel(QkvArgs a, RopeArgs ra, 
   bool plain = true;
   if (QKV && a.has_rope) {
     int pos[RPW];
-    plain = rope_positions_uniform<RPW>(ra, a.W, first_row, a.rows, pos);
+    plain = rope_positions_uniform<RPW>(ra, first_row, a.rows, pos);
 #pragma unroll
     for (int j = 0; j < CSN; ++j) csr[j] = rope_cos_sin_at<MODE == kGemmTable>(ra, fr, plain ? (lane < 32 ? pos[2 * j] : pos[2 * j + 1]) : 0, f);
   }
