@@ -308,6 +308,23 @@ def test_decode_general_streaming_wavefronts_follow_the_grid():
     assert [streams(8, k, 5120, fp8) for fp8 in (0, 1) for k in (128, 256, 512, 1024)] == [1, 2, 4, 4, 1, 1, 2, 4]
 
 
+def test_walks_spread_only_behind_a_filled_row_tile():
+    """The walks of a launch's row tiles are spread over K where the last row tile is filled far enough for the number of them, and for
+    widths and weights where that was measured to be ahead."""
+    spread = _lib.lib().tllm_gemm_tile_spread
+
+    def rows_of(k, n, rows):
+        return [r for r in rows if spread(r, k, n)]
+
+    assert rows_of(2880, 5120, (111, 112, 128, 150, 151, 192, 193, 200, 219, 220, 256)) == [112, 128, 192, 220, 256]
+    assert rows_of(5120, 2880, (113, 128, 130, 144, 159, 160, 192, 193, 219, 220, 256, 257, 271, 272, 320, 321, 327, 328, 385)) == [
+        113, 128, 160, 192, 220, 256, 272, 320, 328, 385]
+    assert rows_of(5120, 2560, (160, 167, 168, 192)) == [168, 192]             # 32 columns
+    assert rows_of(8192, 1536, (192, 256, 300, 600)) == []
+    assert rows_of(1024, 8192, (128, 200, 256, 300)) == [128]
+    assert rows_of(2880, 5120, (513, 640)) == [513, 640] and rows_of(2048, 8192, (256, 640)) == []
+
+
 def test_qkv_prefill_tiles_at_other_widths():
     """A prompt's route at K other than 2880: the fixed part of a launch counts once, whatever K is."""
     tile = _lib.lib().tllm_qkv_gemm_tile

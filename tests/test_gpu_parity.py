@@ -931,7 +931,7 @@ def test_linear_every_gemm_tile(gpu, bm, bn, rows, n, k):
 
 
 @pytest.mark.parametrize("bm,bn,rows,n,k", [(64, 32, 113, 2880, 4096), (64, 32, 128, 2880, 4160), (64, 48, 128, 5120, 2880), (64, 64, 152, 5120, 2880),
-                                            (64, 80, 193, 5120, 2880), (64, 96, 450, 2880, 4096), (64, 128, 300, 5120, 2880), (64, 160, 500, 5120, 2880),
+                                            (64, 80, 221, 5120, 2880), (64, 96, 450, 2880, 4096), (64, 128, 300, 5120, 2880), (64, 160, 500, 5120, 2880),
                                             (64, 192, 513, 5120, 2880), (128, 96, 600, 4096, 2880), (128, 128, 595, 5120, 2880)])
 def test_linear_walks_spread_over_k(gpu, bm, bn, rows, n, k):
     """Tiles whose row tiles begin at different places in K: an odd number of slices where a stage has two, so that the stage without
@@ -1361,9 +1361,9 @@ def test_out_residual_general_stream(gpu, in_dim, out_dim, rows, fp8):
 
 @pytest.mark.parametrize("bm,bn,spread,rows,in_dim,out_dim", [
     (64, 32, 0, 129, 4096, 48), (64, 32, 1, 113, 2880, 2880), (64, 48, 0, 113, 192, 5120), (64, 48, 1, 113, 2048, 5120), (64, 64, 0, 129, 192, 5120),
-    (64, 64, 1, 113, 1088, 8192), (64, 80, 0, 2307, 192, 400), (64, 80, 1, 193, 2048, 5120), (64, 96, 0, 1411, 64, 1024), (64, 96, 1, 257, 2112, 4096),
+    (64, 64, 1, 113, 1088, 8192), (64, 80, 0, 2307, 192, 400), (64, 80, 1, 221, 2048, 5120), (64, 96, 0, 1411, 64, 1024), (64, 96, 1, 273, 2112, 4096),
     (64, 128, 0, 193, 64, 8192), (64, 128, 1, 153, 1088, 8192), (64, 160, 0, 515, 64, 4032), (64, 160, 1, 515, 2112, 4032), (64, 192, 0, 257, 64, 8192),
-    (64, 192, 1, 257, 1088, 8192), (128, 96, 0, 2307, 64, 1024), (128, 96, 1, 640, 2112, 4032), (128, 128, 0, 333, 64, 8192), (128, 128, 1, 640, 2048, 5120),
+    (64, 192, 1, 273, 1600, 8192), (128, 96, 0, 2307, 64, 1024), (128, 96, 1, 640, 2112, 4032), (128, 128, 0, 333, 64, 8192), (128, 128, 1, 640, 2048, 5120),
     (128, 160, 0, 771, 64, 5120), (128, 192, 0, 515, 64, 8192), (128, 224, 0, 1411, 64, 4096), (128, 256, 0, 771, 64, 8192), (64, 32, 0, 81, 4096, 2880),
     (64, 32, 1, 128, 4096, 2880), (64, 32, 0, 33, 4096, 4032)])
 def test_out_residual_in_gemm_tiles(gpu, bm, bn, spread, rows, in_dim, out_dim):

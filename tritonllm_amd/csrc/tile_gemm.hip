@@ -480,18 +480,26 @@ TileSize tile_gemm_pick(int64_t rows, int64_t cols, int64_t k, int64_t* ns) {
 namespace {
 // Whether the row tiles of a launch begin their walks over K at places spread over it (tile m of M at m / M). In step, the
 // workgroups that share weight columns all wait for the same lines from memory; spread, each finds most of K in its XCD's L2, where
-// another one has been. It pays while an XCD's share of the weight stays in its 4 MB (weights of 8 - 16 M elements) and costs beyond,
-// and with rows 4 or 8 KB apart below 10 M; us, in step and spread: [rows, 4096] x [4096, 2880] 128 rows 16.2 / 14.6, 256 18.3 / 15.7, 500
-// 24.4 / 20.3, 1000 33.7 / 32.4; [rows, 2880] x [2880, 5120] 192 16.2 / 14.4, 512 28.9 / 25.9; 6144 x 2048 640 rows 34.7 / 29.1; and
-// 4096 x 5120 256 rows 23.4 / 29.0, 2048 x 4096 230 rows 10.6 / 11.1, 1024 x 1024 as long either way.
+// another one has been. It pays while an XCD's share of the weight stays in its 4 MB (16 M elements; below 8 M, with rows 4 or 8 KB
+// apart below 10 M, in step was as fast with the weights measured first). 700 MB of weights in turn, so that each comes from memory, in
+// step / spread, us: [rows, 4096] x [4096, 2880] 128 rows 16.4 / 15.4, 256 18.9 / 16.4, 450 22.2 / 20.4, 640 29.8 / 25.3; [rows, 2880] x [2880,
+// 5120] 192 17.5 / 15.2, 300 23.1 / 20.0, 640 30.6 / 27.1; 6144 x 2048 640 35.9 / 29.5; and 4096 x 5120 256 rows 24.6 / 29.0, 8192 x 2048 513 34.9 /
+// 42.1, 8192 x 1536 300 24.7 / 27.0, 1024 x 8192 256 11.5 / 12.0. A weight that stays in the 256 MB behind the L2 from one call to the
+// next has less to gain: 2880 x 2880 256 rows, 200 MB in turn, 11.5 / 12.6, 2048 x 5120 11.3 / 13.0.
 // In step, a last row tile that is mostly empty is ahead of the others and fetches for them, so that spreading wants one that is
-// filled: two row tiles, 97 rows (33 in the last) 13.8 / 14.4, 113 (49) 15.1 / 14.5; three, 160 (32) 16.6 / 15.6; from four on any
-// (230 16.8 / 15.5). 128-row tiles up to 128 columns: 5 tiles of 2880 x 5120 640 rows 29.9 / 27.2, six of them (720) 28.8 / 29.4,
-// 2880 x 4096 720 rows 27.5 / 25.0; 1300 rows (20 in the last) 35.5 / 38.
+// filled, the more the fewer row tiles there are and the fewer columns a tile has. In step / spread, mean and worst of 39 weights: two
+// row tiles, 113 rows (49 in the last) 1.018, 0.98; three, 160 (32) of 48 columns 1.014, 0.98, 168 (40) of 32 columns 1.007, 0.97; four, 200
+// (8) 0.985, 0.91, 220 (28) 1.038, 0.98; five, 257 (1) 1.006, 0.90, 272 (16) 1.045, 0.97; six, 330 (10) 1.058, 0.96; 256 1.14, 640 1.16.
+// 128-row tiles up to 128 columns: 5 tiles of 2880 x 5120 640 rows 30.6 / 27.1, six of them (720) 29.8 / 29.4, 2880 x 4096 720 rows 28.5 /
+// 26.0; 4096 x 2880 1300 rows (20 in the last) 35.7 / 38.8.
+// The order in which a row's products are summed then depends on its row tile: equal rows of one call agree to rounding, not to the bit.
 bool tile_gemm_spread(int64_t rows, int64_t cols, int64_t k, TileSize t) {
   const int64_t last = (rows - 1) % t.bm + 1, tiles_m = (rows + t.bm - 1) / t.bm, weight = cols * k;
-  if (tiles_m < 2 || weight < 8000000 || weight > 16000000 || (weight < 10000000 && k % 2048 == 0)) return false;
-  if (t.bm == 64) return tiles_m >= 4 || last >= (tiles_m == 3 ? 24 : 48);
+  if (tiles_m < 2 || weight < 8000000 || weight > 16000000 || (weight < 10000000 && k % 2048 == 0) || k > 6144) return false;
+  if (t.bm == 64) {
+    if (tiles_m <= 3) return last >= (tiles_m == 2 ? 48 : t.bn == 32 ? 40 : t.bn == 48 ? 32 : 24);
+    return k >= 1536 && last >= (tiles_m == 4 ? 28 : tiles_m == 5 ? 16 : tiles_m == 6 ? 8 : 1);
+  }
   return t.bn <= 128 && last >= 80 && (tiles_m <= 5 || weight <= 12000000);
 }
 
