@@ -246,6 +246,8 @@ int tllm_out_residual_decode_bf16(const void* x, const void* W, const float* w_s
 /* Diagnostic: whether tllm_unembedding_decode_bf16 takes up to 128 rows per pass over the weight for these sizes (1), or up
  * to 32 (0). No counterpart in the reference. */
 int tllm_unembedding_decode_tiled(int64_t rows, int fp8, int64_t hidden, int64_t vocab);
+/* Diagnostic: the units of sixteen vocabulary rows in such a pass's widest tile, 0 where there is none. */
+int tllm_unembedding_tile_units(int64_t rows, int fp8, int64_t hidden, int64_t vocab);
 /* Decode-size unembedding over the whole vocabulary, logits[r, v] = sum_k x[r, k] * W[v, k] (fp32 accumulate, one
  * RNE to bf16); replaces unembedding_decode_forward(hidden, weight), triton_kernels.py:163-197 (kernel :111-160),
  * and with w_scale != NULL unembedding_decode_fp8_forward :271-302 (W = fp8 e4m3 bytes, one fp32 scale per

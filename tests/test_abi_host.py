@@ -336,6 +336,16 @@ def test_qkv_prefill_tiles_at_other_widths():
         [True, True, False, False, True, True, False, False, True, False]
 
 
+def test_logits_tiles_have_a_kernel_of_about_their_width():
+    """fp8 tiles of 17 - 20 units beside more than 64 rows: one tile more where that leaves tiles of up to 15, one tile stays one."""
+    units = _lib.lib().tllm_unembedding_tile_units
+    assert [units(rows, 1, 2880, 151936) for rows in (64, 65, 96, 97, 128, 200)] == [19, 19, 19, 13, 13, 13]
+    assert [units(rows, 1, 2048, 234000) for rows in (64, 96, 97)] == [20, 15, 15]
+    assert [units(rows, 1, 2880, 70000) for rows in (96, 97, 128)] == [18, 18, 18] and units(96, 1, 2880, 163000) == 20
+    assert [units(rows, 1, 2880, 201088) for rows in (64, 128)] == [25, 25] and [units(rows, 0, 2880, 201088) for rows in (49, 128)] == [17, 17]
+    assert units(8, 0, 2880, 201088) == 0
+
+
 def test_logits_of_a_small_vocabulary_stay_in_passes():
     tiled = _lib.lib().tllm_unembedding_decode_tiled
     assert [tiled(rows, 0, hidden, vocab) for rows, hidden, vocab in ((9, 4096, 1000), (16, 4096, 4000), (33, 2880, 1000), (64, 2880, 4096))] == [0] * 4

@@ -1598,7 +1598,8 @@ def test_unembedding_more_than_16_rows_one_pass_over_the_weight(gpu, rows, vocab
 @pytest.mark.parametrize("rows,vocab,hidden", [(9, 40, 4096), (24, 3001, 4096), (33, 20, 2880), (48, 70003, 2880), (65, 40000, 2880), (96, 5001, 64),
                                                 (97, 33001, 2880), (128, 9000, 2880), (128, 3001, 128), (131, 5000, 2880), (300, 2050, 192), (17, 40, 4096),
                                                 (65, 20, 2880), (20, 70001, 3200), (40, 65000, 128), (50, 81000, 192), (70, 100003, 64), (128, 75000, 128),
-                                                (90, 114000, 128), (128, 201088, 64)])
+                                                (90, 114000, 128), (128, 201088, 64), (97, 151936, 64), (128, 70000, 128), (96, 234000, 64),
+                                                (66, 8193, 128)])
 def test_unembedding_logits_in_tiles(gpu, rows, vocab, hidden):
     """More rows than the kernels that keep them in LDS take: tiles of the vocabulary with the activations streamed next to
     the weight. One to four row blocks per wavefront, several chunks of rows, workgroups with no vocabulary, one unit, many

@@ -60,6 +60,7 @@ SIGNATURES = {
     "tllm_linear_bf16": (_i32, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "tllm_out_residual_decode_bf16": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp]),
     "tllm_unembedding_decode_tiled": (_i32, [_i64, _i32, _i64, _i64]),
+    "tllm_unembedding_tile_units": (_i32, [_i64, _i32, _i64, _i64]),
     "tllm_unembedding_decode_bf16": (_i32, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "tllm_unembedding_argmax_workspace_bytes": (_i64, [_i64]),
     "tllm_unembedding_argmax_bf16": (_i32, [_vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _vp]),

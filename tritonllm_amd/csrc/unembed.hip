@@ -718,6 +718,10 @@ int unembed_launch(const char* who, const UnembedArgs& a, bool w8, hipStream_t s
 
 extern "C" int tllm_unembedding_decode_tiled(int64_t rows, int fp8, int64_t hidden, int64_t vocab) { return unembed_tiled(rows, fp8 != 0, hidden, vocab); }
 
+extern "C" int tllm_unembedding_tile_units(int64_t rows, int fp8, int64_t hidden, int64_t vocab) {
+  return rows > 0 && hidden > 0 && vocab > 0 && unembed_tiled(rows, fp8 != 0, hidden, vocab) ? unembed_tile_units(rows, fp8 != 0, vocab) : 0;
+}
+
 extern "C" int tllm_unembedding_decode_bf16(const void* x, const void* W, const float* w_scale, void* logits, int64_t logits_row_stride,
                                             int64_t rows, int64_t hidden, int64_t vocab, void* stream) {
   int rc = unembed_check("unembedding_decode", x, W, w_scale != nullptr, rows, hidden, vocab);

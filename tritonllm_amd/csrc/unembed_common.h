@@ -22,6 +22,7 @@ constexpr int kUnembedGrid = 256;      // one workgroup per CU
 
 // Logits of up to 128 rows per pass over the weight (unembed_tiles.hip): which calls it can take, and the launch.
 bool unembed_tiles_fit(int64_t rows, bool w8, int64_t hidden, int64_t vocab);
+int unembed_tile_units(int64_t rows, bool w8, int64_t vocab);          // of its widest tile
 int launch_unembed_tiles(const char* who, const UnembedArgs& a, bool w8, hipStream_t st);
 
 }  // namespace tllm

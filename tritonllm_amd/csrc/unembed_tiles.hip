@@ -40,6 +40,11 @@ struct Shape {
   static constexpr int XBYTES = MB * 16 * 128, TAIL = W8 ? MAX_RUN * 16 * 4 : 0;
   static constexpr int LU = W8 ? 1 : 2;                      // loads of 1 KB per unit and stage
   static constexpr int LMAX = (4 * UB * LU + MB * 2 + NW - 1) / NW;         // most loads of a wavefront per stage
+  // Every wavefront has LMAX loads, the last one of the stage again where there are fewer (the same bytes to the same place). A
+  // stage of a narrow fp8 tile is 4 - 24 KB, and the tests and branches around its loads took 2 - 9 % of its time, us with and without:
+  // [rows, 2048] x [65000, 2048] 49 rows 34.6 / 33.8, [50257, 2048] 65 rows 36.7 / 35.5, [65000, 768] 64 rows 18.4 / 18.0, one or two units per
+  // CU 5 - 9 %; wider tiles (201088 33 rows 135.4 / 139.1) gain nothing, bf16's have twice the bytes.
+  static constexpr bool EVEN = W8 && UB <= 4;
   static constexpr int most(int stages) {                    // units of the widest tile of which so many stages fit
     const int fit = ((LDS - TAIL) / stages - XBYTES) / UBYTES;
     return fit < 4 * UB ? fit : 4 * UB;
@@ -89,14 +94,15 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
   // eight repeat it; never stored). bf16: eight rows of 128 bytes per load, chunk position L % 8 holds chunk (L % 8) ^ swz(row).
   // fp8: sixteen rows of 64 bytes, position L % 4 holds chunk (L % 4) ^ (row / 4).
   const int w_loads = width * LU, loads = w_loads + (nrows + 7) / 8;
-  const int mine = wave < loads ? (loads - wave + NW - 1) / NW : 0;         // this wavefront's
+  const int mine = wave < loads ? (loads - wave + NW - 1) / NW : 0;         // this wavefront's (EVEN: LMAX)
+  auto load_of = [&](int j) { return C::EVEN && wave + NW * j >= loads ? loads - 1 : wave + NW * j; };
   const int run_rows = a.vocab - u0 * 16 < run * 16 ? a.vocab - u0 * 16 : run * 16;
   unsigned off[LMAX];
   auto offsets = [&](int tile) {
     const int left = run - tile * width, here = left < width ? left : width;
 #pragma unroll
     for (int j = 0; j < LMAX; ++j) {
-      const int t = wave + NW * j;
+      const int t = load_of(j);
       if (t < w_loads) {
         const int u = t / LU, unit = tile * width + (u < here ? u : here - 1);
         const int r = W8 ? lane >> 2 : 8 * (t % LU) + (lane >> 3);
@@ -122,10 +128,12 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
     const unsigned char* const xb = x_base + static_cast<int64_t>(l_k) * (BK * 2);
 #pragma unroll
     for (int j = 0; j < LMAX; ++j) {
-      const int t = wave + NW * j;
+      const int t = load_of(j);
       const unsigned d = dst + t * 1024 + (t < w_loads ? 0 : wbytes - w_loads * 1024);
       // a slice of an fp8 row is half a line, so its line is needed again one stage on: no streaming hint
-      if constexpr (W8) {
+      if constexpr (C::EVEN) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(d), "v"(off[j]), "s"(t < w_loads ? wb : xb) : "memory", "m0");
+      } else if constexpr (W8) {
         asm volatile("s_mov_b32 m0, %0\n\ts_cmp_lt_i32 %3, %4\n\ts_cbranch_scc0 .Lskip%=\n\tglobal_load_lds_dwordx4 %1, %2\n.Lskip%=:" ::"s"(d), "v"(off[j]),
                      "s"(t < w_loads ? wb : xb), "s"(t), "s"(loads)
                      : "memory", "m0", "scc");
@@ -182,7 +190,8 @@ __global__ __launch_bounds__(512) void unembed_tiles_kernel(UnembedArgs a, int c
       // This wavefront's share of the stage has landed (the S - 2 stages behind it may be in flight; stores of the tile
       // before are younger than all of them, which makes the wait longer, never shorter), then everyone's; and everyone has
       // read the slot that the next loads go into.
-      wait_stages<LMAX, S - 2>(mine);
+      if constexpr (C::EVEN) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * LMAX) : "memory");
+      else wait_stages<LMAX, S - 2>(mine);
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       const unsigned char* const st = smem + c_slot * stage_bytes;
       bf16x8 fx[2][TB], fw[2][UB];
@@ -258,15 +267,30 @@ int launch_one(const char* who, const UnembedArgs& a, int chunk_rows, int chunks
 // as fit it: units past the tile's width are multiplied as well, and a CU that holds a third of a tile wants more stages on
 // their way ([rows, 2880] x [8192, 2880], two units per CU, 49 / 128 rows 34 / 47 -> 20 / 30; 2048 wide, 32000 34 / 41 -> 31 / 35).
 template <int MB, bool W8>
+int tile_units(int64_t vocab) {
+  using unembed_tiles::Shape;
+  const int run = static_cast<int>(((vocab + 15) / 16 + kUnembedGrid - 1) / kUnembedGrid);
+  constexpr int widest = Shape<MB, W8, W8 ? 7 : 5>::most(3);
+  const int tiles = (run + widest - 1) / widest;
+  const int slots = (run + tiles - 1) / tiles;
+  // fp8: for tiles of 17 - 20 units more than 64 rows leave no room for five stages (from 19, 17 units on at up to 96, 128 rows), and the kernel for 28
+  // multiplies eight and more units for nothing. As one tile more: [rows, 2880] x [151936, 2880] 97 rows 147 -> 139 us, 200 rows 285 -> 271, 2048 wide
+  // 109 -> 101, 213 -> 198; 96 rows of [234000, 2048] 146 -> 141. One tile stays one (70000 97 rows 72, two 80), and up to 96 rows two stay two
+  // (163000 96 rows 135 and 141).
+  if (W8 && slots > 16 && slots > Shape<MB, W8, 5>::most(5) && slots <= 20 && tiles > (MB == 8 ? 1 : 2)) return (run + tiles) / (tiles + 1);
+  return slots;
+}
+
+template <int MB, bool W8>
 int launch_shape(const char* who, const UnembedArgs& a, int chunk_rows, int chunks, hipStream_t st) {
   using unembed_tiles::Shape;
-  const int run = ((a.vocab + 15) / 16 + kUnembedGrid - 1) / kUnembedGrid;
   constexpr int BIG = W8 ? 7 : 5;
-  constexpr int widest = Shape<MB, W8, BIG>::most(3);
-  const int tiles = (run + widest - 1) / widest, slots = (run + tiles - 1) / tiles;
+  const int slots = tile_units<MB, W8>(a.vocab);
   if (slots <= 8) return launch_one<MB, W8, 2, MB <= 4 ? 6 : 5>(who, a, chunk_rows, chunks, slots, st);
   if (slots <= 16) return launch_one<MB, W8, 4, W8 ? (MB == 2 ? 7 : MB == 4 ? 6 : MB == 6 ? 5 : 4) : MB <= 4 ? 4 : 3>(who, a, chunk_rows, chunks, slots, st);
-  if (W8 && slots <= Shape<MB, W8, 5>::most(5)) return launch_one<MB, W8, 5, 5>(who, a, chunk_rows, chunks, slots, st);
+  if constexpr (W8) {
+    if (slots <= Shape<MB, W8, 5>::most(5)) return launch_one<MB, W8, 5, 5>(who, a, chunk_rows, chunks, slots, st);
+  }
   if (slots <= Shape<MB, W8, BIG>::most(4)) return launch_one<MB, W8, BIG, 4>(who, a, chunk_rows, chunks, slots, st);
   return launch_one<MB, W8, BIG, 3>(who, a, chunk_rows, chunks, slots, st);
 }
@@ -276,6 +300,12 @@ int launch_shape(const char* who, const UnembedArgs& a, int chunk_rows, int chun
 bool unembed_tiles_fit(int64_t rows, bool w8, int64_t hidden, int64_t vocab) {
   const int64_t run = (vocab + 15) / 16 / kUnembedGrid + 1;                      // units of the longest run
   return (!w8 || run <= unembed_tiles::MAX_RUN) && run * 16 * hidden * 2 < (1ll << 32) && hidden * 256 < (1ll << 32) && (rows + 127) / 128 <= 65535;
+}
+
+int unembed_tile_units(int64_t rows, bool w8, int64_t vocab) {
+  const int64_t chunks = (rows + 127) / 128, mb = ((rows + chunks - 1) / chunks + 31) / 32 * 2;
+  if (w8) return mb == 2 ? tile_units<2, true>(vocab) : mb == 4 ? tile_units<4, true>(vocab) : mb == 6 ? tile_units<6, true>(vocab) : tile_units<8, true>(vocab);
+  return mb == 2 ? tile_units<2, false>(vocab) : mb == 4 ? tile_units<4, false>(vocab) : mb == 6 ? tile_units<6, false>(vocab) : tile_units<8, false>(vocab);
 }
 
 int launch_unembed_tiles(const char* who, const UnembedArgs& a, bool w8, hipStream_t st) {
