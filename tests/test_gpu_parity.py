@@ -1295,7 +1295,7 @@ def _out_inputs(rows, seed, in_dim=4096, out_dim=2880):
                 b=(0.02 * torch.randn(out_dim, generator=g)).bfloat16(), r=torch.randn(rows, out_dim, generator=g).bfloat16())
 
 
-@pytest.mark.parametrize("rows", [1, 8, 9, 11, 12, 13, 16, 17, 20, 21, 24, 25, 28, 29, 32, 33, 41, 45, 49, 52, 53, 56, 57, 64, 65, 70, 96, 97, 113, 128, 129, 161, 300])
+@pytest.mark.parametrize("rows", [1, 8, 9, 11, 12, 13, 16, 17, 20, 21, 24, 25, 28, 29, 32, 33, 41, 45, 49, 52, 53, 56, 57, 64, 65, 70, 73, 80, 96, 97, 113, 128, 129, 161, 300])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_out_residual_decode_parity(gpu, rows, fp8):
     d = _out_inputs(rows, 600 + rows)
@@ -1311,6 +1311,19 @@ def test_out_residual_decode_parity(gpu, rows, fp8):
     assert out.shape == (rows, 1, 2880) and out.data_ptr() == res.data_ptr()          # written into the residual, as the reference does
     assert not torch.equal(res, res_before)
     close(out.view(rows, 2880), want)
+
+
+@pytest.mark.parametrize("rows,out_dim", [(49, 1536), (65, 1536), (97, 1536), (113, 2304), (128, 1536), (128, 2304)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_out_residual_narrow_outputs(gpu, rows, out_dim, fp8):
+    """Two to four chunks of 24, 28 and 32 rows beside one pass over the weight: with a bf16 weight only narrower outputs than 2880 have
+    four, and with fp8 the walks over K are spread over its phases from 2048 outputs on."""
+    assert _lib.lib().tllm_out_gemm_tile(rows, 4096, out_dim) == 0
+    d = _out_inputs(rows, 900 + rows, out_dim=out_dim)
+    w, ws = T.quantize_fp8_rows(d["w"].to(gpu)) if fp8 else (d["w"].to(gpu), None)
+    out = T.out_residual_decode_forward(d["x"].view(rows, 1, 4096).to(gpu), w, d["b"].to(gpu), d["r"].view(rows, 1, out_dim).to(gpu), weight_scale=ws)
+    want = O.dequant_fp8_ref(w.cpu(), ws.cpu()) if fp8 else d["w"]
+    close(out.view(rows, out_dim), O.out_residual_ref(d["x"], want, d["b"], d["r"]))
 
 
 @pytest.mark.parametrize("rows", [1, 5, 8, 13, 32, 37])

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(384) void out_decode_r32_kernel(OutArgs a, int vec8
   auto lds_addr = [](const void* p) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>(p)); };
   auto x_region = [&](int p) { return myring + (p % XRING) * XPH; };
   auto w_region = [&](int p) { return myring + XRING * XPH + (p % WRING) * WPH; };
-  // SPREAD: the workgroups that share an XCD's L2 begin their walks over K at different phases
+  // SPREAD (fp8): the workgroups that share an XCD's L2 begin their walks over K at different phases
   const int rot = static_cast<int>(blockIdx.x >> 3) & (NPH - 1);
   auto turned = [&](int p) { return SPREAD ? (p + rot) & (NPH - 1) : p; };
   auto issue_x = [&](int p) {
@@ -308,30 +308,33 @@ void launch_out_decode_r32(dim3 grid, hipStream_t st, const OutArgs& a) {
   // up to four chunks per workgroup: the weight is then read once for up to 128 rows
   const int cpw = chunks < 4 ? static_cast<int>(chunks) : 4;
   const dim3 g2(grid.x, (chunks + cpw - 1) / cpw);
-  // Where the activations are most of what a CU takes in, its neighbours do not ask their L2 for the same lines of them at the same time
-  // (64 rows 12.0 -> 11.8 us, 96 16.1 -> 14.9, 128 19.7 -> 17.8; fp8 64 10.4 -> 9.8, 128 18.1 -> 16.0). With fewer rows what counts is that
-  // all ask memory for the same part of their weight rows at a time (9 rows 6.6, spread 7.1; 49 rows 11.1 and 11.4).
-  const bool spread = a.rows > (a.w_scale ? 52 : 56);
-#define TLLM_OUT32(XB, SPREAD)                                                                                                   \
-  do {                                                                                                                           \
-    if (a.w_scale) hipLaunchKernelGGL((out_decode_r32_kernel<XB, true, SPREAD>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks);   \
-    else hipLaunchKernelGGL((out_decode_r32_kernel<XB, false, SPREAD>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks);            \
-  } while (0)
-  if (spread) {                                             // (more than 52 rows: chunks of 22 and more)
-    if (xb <= 6) TLLM_OUT32(6, true);
-    else if (xb == 7) TLLM_OUT32(7, true);
-    else TLLM_OUT32(8, true);
+  // fp8 weight: where the activations are most of what a CU takes in and there are outputs enough for most CUs, neighbours do not ask
+  // their L2 for the same lines of them at the same time ([2880, 4096] in step / spread, us: 56 rows 9.10 / 8.81, 64 10.0 / 9.45, 128 15.8 / 15.0,
+  // 256 32.8 / 28.4; 2304 outputs 64 rows 8.89 / 8.70, 65 9.64 / 9.68; 1536 57 rows 8.19 / 8.26, 96 10.6 / 10.7). With fewer rows, and with a
+  // bf16 weight, twice the bytes, up to the rows that go to GEMM tiles, what counts is that all ask memory for the same part of their
+  // weight rows at a time (bf16 57 rows 10.9 / 11.3, 80 12.8 / 13.2; 2304 outputs 97 rows 13.7 / 14.0).
+  if (a.w_scale && a.rows > 52 && a.out_dim >= 2048) {        // (chunks of 22 and more)
+#define TLLM_OUT32(XB) hipLaunchKernelGGL((out_decode_r32_kernel<XB, true, true>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks)
+    if (xb <= 6) TLLM_OUT32(6);
+    else if (xb == 7) TLLM_OUT32(7);
+    else TLLM_OUT32(8);
+#undef TLLM_OUT32
     return;
   }
+#define TLLM_OUT32(XB)                                                                                                          \
+  do {                                                                                                                          \
+    if (a.w_scale) hipLaunchKernelGGL((out_decode_r32_kernel<XB, true, false>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks);   \
+    else hipLaunchKernelGGL((out_decode_r32_kernel<XB, false, false>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks);            \
+  } while (0)
   switch (xb) {
-    case 1: TLLM_OUT32(1, false); break;
-    case 2: TLLM_OUT32(2, false); break;
-    case 3: TLLM_OUT32(3, false); break;
-    case 4: TLLM_OUT32(4, false); break;
-    case 5: TLLM_OUT32(5, false); break;
-    case 6: TLLM_OUT32(6, false); break;
-    case 7: TLLM_OUT32(7, false); break;
-    default: TLLM_OUT32(8, false); break;
+    case 1: TLLM_OUT32(1); break;
+    case 2: TLLM_OUT32(2); break;
+    case 3: TLLM_OUT32(3); break;
+    case 4: TLLM_OUT32(4); break;
+    case 5: TLLM_OUT32(5); break;
+    case 6: TLLM_OUT32(6); break;
+    case 7: TLLM_OUT32(7); break;
+    default: TLLM_OUT32(8); break;
   }
 #undef TLLM_OUT32
 }
