@@ -316,6 +316,9 @@ int tllm_attention_decode_bf16(const void* q, const void* k, const void* v, cons
 /* Diagnostic: groups of wavefronts that share a workgroup's key blocks out for these arguments (4, 2, or 1: none do). No
  * counterpart in the reference. */
 int tllm_attention_prefill_key_groups(int64_t batch, int64_t n_q, int64_t n_kv_ctx, int n_kv_heads, int group, int window);
+/* Diagnostic: the workgroup that it takes: queries << 16 | query heads << 8 | key groups, with 1 << 24 where it walks the keys in
+ * chunks of 32 keys x one head. */
+int tllm_attention_prefill_shape(int64_t batch, int64_t n_q, int64_t n_kv_ctx, int n_kv_heads, int group, int window);
 /* Prefill attention with sinks and an optional sliding window: n_q query positions per batch row against the keys
  * written so far. Replaces attention (attention_tt.py:167-242, kernel :17-164; definition attention_ref.py:4-42).
  * q [batch, n_q, n_kv_heads * group, 64] with batch / token strides in elements (heads adjacent: the layout the QKV

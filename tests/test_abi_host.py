@@ -288,6 +288,22 @@ def test_attention_prefill_shape_planning():
     assert groups(1, 777, 777, 8, 8, 0) == 1
 
 
+def test_attention_prefill_shapes():
+    """In chunks behind more than six blocks of keys, with a window from 322 on; workgroups of few heads while those of four are few."""
+    shape = _lib.lib().tllm_attention_prefill_shape
+
+    def of(b, n, n_kv, group=8, window=0):
+        s = shape(b, n, n_kv, 8, group, window)
+        return s >> 24, s >> 16 & 255, s >> 8 & 255, s & 255
+
+    assert [of(3, 333, n)[0] for n in (384, 385)] == [0, 1] and [of(1, 2048, 2048, window=w)[0] for w in (128, 321, 322)] == [0, 0, 1]
+    assert of(2, 600, 600) == (1, 64, 2, 1)
+    assert of(3, 450, 450) == (1, 64, 4, 1) and of(3, 333, 333) == (0, 64, 2, 1)
+    assert [of(1, n, n) for n in (1536, 2048)] == [(1, 64, 2, 1), (1, 64, 4, 1)]
+    assert of(9, 650, 700, 2) == (1, 128, 2, 1) and of(8, 650, 700, 2, 128) == (0, 128, 2, 1) and of(2, 1000, 1100, 5) == (1, 128, 1, 1)
+    assert of(1, 97, 1597) == (0, 64, 1, 4) and shape(0, 1, 1, 8, 8, 0) == 0
+
+
 def test_qkv_decode_tiles_or_the_general_kernel():
     """Decode batches of more than 32 rows at widths other than 2880: GEMM tiles only where the general kernel's passes over the
     weight cost more than a tile's fixed time."""

@@ -1929,23 +1929,43 @@ def test_attention_prefill_full_prompt(gpu):
 
 @pytest.mark.parametrize("sliding_window", [None, 128])
 def test_attention_prefill_large_launch_ragged(gpu, sliding_window):
-    """Enough workgroups for the 128-query x two-heads-per-wavefront shape (the library picks the workgroup shape from
+    """Enough workgroups for 64 queries x four heads, two per wavefront (the library picks the workgroup shape from
     the size of the launch), with a ragged last tile, a later chunk of the prompt and keys beyond the last query."""
     _attn_prefill_case(gpu, 4, 600, 700, sliding_window, 77, start_dtype=torch.int64, seed=41)
 
 
-@pytest.mark.parametrize("batch_size,num_queries,num_keys,start_q,window,kv", [
-    (1, 777, 777, 0, None, dict()),                                            # 64 queries x 2 heads, one per wavefront
-    (1, 833, 1200, 310, 257, dict()),                                          # the window's edge inside blocks; keys beyond the last query
-    (1, 600, 448, 0, None, dict(with_sinks=False)),                            # as short as walks in chunks get; queries past the keys
-    (4, 600, 700, 77, 400, dict()),                                            # 64 queries x 4 heads, two per wavefront
-    (3, 449, 640, 191, 321, dict(groups=4, kv_heads=16)),
-    (8, 650, 700, 49, None, dict(groups=2)), (6, 700, 777, 40, 350, dict(groups=6, kv_heads=4)),      # 128 queries x 2 heads
-    (2, 1000, 1100, 100, 300, dict(groups=5)),                                 # 128 queries x 1 head
+def _prefill_shape(*sizes):
+    shape = _lib.lib().tllm_attention_prefill_shape(*sizes)
+    return shape >> 24, shape >> 16 & 255, shape >> 8 & 255, shape & 255          # in chunks, queries, query heads, key groups
+
+
+@pytest.mark.parametrize("batch_size,num_queries,num_keys,start_q,window,kv,shape", [
+    (1, 777, 777, 0, None, dict(), (64, 2)),                                   # one head per wavefront
+    (1, 833, 1200, 310, 322, dict(), (64, 2)),                                 # the window's edge inside blocks; keys beyond the last query
+    (2, 450, 1100, 520, 400, dict(), (64, 2)),
+    (1, 600, 448, 0, None, dict(with_sinks=False), (64, 2)),                   # as short as walks in chunks get; queries past the keys
+    (8, 128, 2048, 0, None, dict(), (64, 2)), (5, 60, 1500, 700, None, dict(kv_heads=16), (64, 2)),       # a cache larger than what is walked
+    (4, 600, 700, 77, 400, dict(), (64, 4)),                                   # two per wavefront
+    (3, 449, 640, 191, 333, dict(groups=4, kv_heads=16), (64, 4)),
+    (9, 650, 700, 49, None, dict(groups=2), (128, 2)), (6, 700, 777, 40, 350, dict(groups=6, kv_heads=4), (128, 2)),
+    (2, 1000, 1100, 100, 400, dict(groups=5), (128, 1)), (1, 777, 900, 123, None, dict(groups=7), (128, 1)),
 ], ids=str)
-def test_attention_prefill_chunks(gpu, batch_size, num_queries, num_keys, start_q, window, kv):
-    """Walks of more than six key blocks, which run in chunks of 32 keys x one head."""
-    assert _lib.lib().tllm_attention_prefill_key_groups(batch_size, num_queries, num_keys, kv.get("kv_heads", 8), kv.get("groups", 8), window or 0) == 1
+def test_attention_prefill_chunks(gpu, batch_size, num_queries, num_keys, start_q, window, kv, shape):
+    """Keys of more than six blocks and no narrower window: in chunks of 32 keys x one head, in every shape of workgroup."""
+    assert _prefill_shape(batch_size, num_queries, num_keys, kv.get("kv_heads", 8), kv.get("groups", 8), window or 0) == (1, *shape, 1)
+    _attn_prefill_case(gpu, batch_size, num_queries, num_keys, window, start_q, seed=num_queries + num_keys, **kv)
+
+
+@pytest.mark.parametrize("batch_size,num_queries,num_keys,start_q,window,kv,shape", [
+    (1, 833, 1200, 310, 257, dict(), (64, 2)), (3, 449, 640, 191, 321, dict(groups=4, kv_heads=16), (64, 4)),
+    (4, 600, 700, 77, 128, dict(), (64, 4)),
+    (8, 650, 700, 49, 128, dict(groups=2), (128, 2)), (8, 380, 384, 4, None, dict(groups=2, kv_heads=16), (128, 2)),
+    (6, 700, 777, 40, 130, dict(groups=6, kv_heads=4), (128, 2)),
+    (2, 1000, 1100, 100, 300, dict(groups=5), (128, 1)),
+], ids=str)
+def test_attention_prefill_short_walks(gpu, batch_size, num_queries, num_keys, start_q, window, kv, shape):
+    """Up to six blocks of keys, or a window of up to 321, in every shape of workgroup."""
+    assert _prefill_shape(batch_size, num_queries, num_keys, kv.get("kv_heads", 8), kv.get("groups", 8), window or 0) == (0, *shape, 1)
     _attn_prefill_case(gpu, batch_size, num_queries, num_keys, window, start_q, seed=num_queries + num_keys, **kv)
 
 

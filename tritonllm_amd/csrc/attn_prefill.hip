@@ -438,11 +438,11 @@ __global__ __launch_bounds__(NW * 64, KG > 2 ? NW / 4 : NW / 2) void attn_prefil
 //     own four (16 x 16 x 32 ones do eight times the multiplications: 8192 queries 526 us, so 523, without any sums 496).
 //   * One barrier per block, in the middle of the block before: four stages, up to three blocks in flight. What happens rarely
 //     is laid out behind the loop, so that the loop's branches fall through.
-// 8192 queries 564 -> 523 us (1.17 M -> 0.95 M cycles, but the clock under this load falls from 2.08 to 1.8 GHz: what bounds it
-// now is power, and 345 cycles of issue per chunk, of which 16 x 13 are the exponentials and their arguments), 2048 queries
-// 50.5 -> 46.6, 2000 behind 2000 116 -> 107, 600 behind 2000 49 -> 40, 777 queries 15.9 -> 13.6. Walks of up to six blocks
-// and windows of up to 256 keys stay with the kernel above: what they pay is the first and the last block, and that one is lighter there
-// (8192 queries, window of 128: 65 us here, 50 there).
+// 8192 queries 564 -> 523 us (on other GPUs 571 -> 550; 1.17 M -> 0.95 M cycles, but the clock under this load falls from 2.08 to 1.8 GHz:
+// what bounds it now is power, and 345 cycles of issue per chunk, of which 16 x 13 are the exponentials and their arguments), 2048 queries
+// 50.5 - 53 -> 46.6 - 49.6, 2000 behind 2000 116 -> 107, 600 behind 2000 49 -> 40, 777 queries 15.9 -> 13.6. Windows of up to 321 keys and caches
+// of up to six blocks stay with the kernel above: what short walks pay is the first and the last block, and that one is lighter there (8192 queries,
+// window of 128: 65 us here, 50 there).
 template <int NH, int QG, int NW>
 __global__ __launch_bounds__(NW * 64, NW / 2) void attn_prefill_chunks_kernel(AttnPrefillArgs a) {
   constexpr int PBM = 32 * QG;                    // queries per workgroup
@@ -845,7 +845,8 @@ static int launch_prefill_chunks(const AttnPrefillArgs& a, hipStream_t st) {
   return check_launch("attention_prefill");
 }
 
-// Blocks that the longest walk over the keys can have.
+// Blocks that the longest walk of 64 queries over the keys can have: the host knows the size of the cache and the window, not where in the
+// cache the queries start (and counts from an aligned start).
 static int64_t longest_walk(int64_t n_kv_ctx, int window) {
   const int64_t all = (n_kv_ctx + PBN - 1) / PBN, seen = (static_cast<int64_t>(window) + 126) / PBN;
   return window > 0 && seen < all ? seen : all;
@@ -860,20 +861,49 @@ static int64_t longest_walk(int64_t n_kv_ctx, int window) {
 // A walk has to be long enough to pay for the meeting at its end: more than one block (16 or 64 queries alone 5.5 us, shared
 // out 6.1; two blocks, 97 queries, 6.6 and 6.3), and at two workgroups per CU more than three (eight prompts of 64 6.2 and
 // 7.5, four of 128 6.9 and 7.6, window of 128: 400 queries 8.2 and 9.4, 512 8.3 and 9.5; five blocks, 300 queries, 9.4 and 8.9).
-// Otherwise 64 queries x 4 heads with two heads per wavefront, or, where those are too few workgroups, 64 queries x 2 heads with
-// one per wavefront: twice the workgroups, and the longest of them -- it sets the time of a small launch -- takes about half as
-// long per key block. The line, with few / many heads in us. Short walks (window of 128): 2 x 500 queries (256 of the
-// workgroups with four heads) 10.4 / 11.1, 1100 (288) 13.6 / 13.0, 2048 18.4 / 16.4, 8192 60.7 / 50.1. Five or six blocks: 3 x 333
-// (288) 12.8 / 14.3, 4 x 384 (384) 16.8 / 15.9, 5 x 300 (400) 15.7 / 14.6. Walks in chunks of up to 12 blocks: 3 x 450 (384)
-// 17.9 / 16.8, 2 x 600 (320) 16.9 / 18.9; longer ones: 1536 (384) 31.1 / 34.9, 1900 (480) 43.6 / 43.7, with 300 keys before
-// 54.2 / 51.9, 4096 156 / 147. (128 queries x 2 heads, which they replace, are never ahead: an 8192 window 55.8 and 50.1, 3000
-// queries 90.9 and 88.1.) Groups that are no multiple of four take 128 x 2, odd ones 128 x 1.
 extern "C" int tllm_attention_prefill_key_groups(int64_t batch, int64_t n_q, int64_t n_kv_ctx, int n_kv_heads, int group, int window) {
   const int64_t wgs64 = (n_q + 63) / 64 * batch * n_kv_heads * group;
   const int64_t span = window > 0 && window < n_kv_ctx - n_q ? n_q + window : n_kv_ctx;     // most keys there can be to visit
   const int64_t walk = longest_walk(n_kv_ctx, window);
   if (wgs64 <= 256 && span > 192) return 4;
   return wgs64 <= 512 && walk > (wgs64 <= 256 ? 1 : 3) ? 2 : 1;
+}
+
+// Otherwise 64 queries x 4 heads with two heads per wavefront, or, where those are too few workgroups, 64 queries x 2 heads with
+// one per wavefront: twice the workgroups, and the longest of them -- it sets the time of a small launch -- takes about half as
+// long per key block. The line, with few / many heads in us. Short walks (window of 128): 2 x 500 queries (256 of the
+// workgroups with four heads) 10.4 / 11.1, 1100 (288) 13.6 / 13.0, 2048 18.4 / 16.4, 8192 60.7 / 50.1. Five or six blocks: 3 x 333
+// (288) 12.8 / 14.3, 4 x 384 (384) 16.8 / 15.9, 5 x 300 (400) 15.7 / 14.6. Walks in chunks of up to 12 blocks: 2 x 600 (320) 17.7 /
+// 19.9, 2 x 700 (352) 20.7 / 21.9, 3 x 450 (384) 18.2 / 17.9, with 300 keys before 25.9 / 26.8; longer ones: 1536 (384) 31.1 / 34.9, 1900 (480) 43.6 /
+// 43.7, with 300 keys before 54.2 / 51.9, 4096 156 / 147. (128 queries x 2 heads, which they replace, are never ahead: an 8192 window 55.8 and 50.1, 3000
+// queries 90.9 and 88.1.) Groups that are no multiple of four take 128 x 2, odd ones 128 x 1.
+// In chunks where the cache has more than six blocks, which a prompt may not walk. Of 294 batches of 1 - 16 prompts of 64 - 1300 tokens behind
+// 0 - 1000, in caches of their own length and of 4096, what is chosen here takes 0.91 of the time it took without chunks and with 128 queries x 2
+// heads, in the mean; one head per wavefront in chunks takes 0.94 - 0.975 of the other kernel's where walks are three to six blocks (4 x 300 in a
+// cache of 4096 15.3 / 14.4, 2 x 384 11.8 / 10.8, 8 x 128 9.07 / 8.82). Behind by more than 1 % are 3 x 333 (13.8 / 14.0), 3 x 384 (14.3 / 14.6), 2 x 600 (17.0 / 17.7) and 2 x 700 (20.2 / 20.7; with 100 keys before 23.9 / 22.3 and
+// 26.6 / 24.4), and with five heads 8 x 128 (9.16 / 9.34).
+namespace {
+struct PrefillShape {
+  int queries, heads, key_groups;      // of a workgroup
+  bool chunks;
+};
+
+PrefillShape prefill_shape(int64_t batch, int64_t n_q, int64_t n_kv_ctx, int n_kv_heads, int group, int window) {
+  const int key_groups = tllm_attention_prefill_key_groups(batch, n_q, n_kv_ctx, n_kv_heads, group, window);
+  if (key_groups > 1) return {64, 1, key_groups, false};
+  const int64_t walk = longest_walk(n_kv_ctx, window);
+  const bool chunks = walk > 6;
+  if (group % 2 != 0) return {128, 1, 1, chunks};
+  const int64_t wgs4 = (n_q + 63) / 64 * batch * n_kv_heads * group / 4;
+  if (wgs4 < (chunks ? (walk <= 12 ? 336 : 432) : (walk <= 4 ? 272 : 320))) return {64, 2, 1, chunks};
+  return group % 4 == 0 ? PrefillShape{64, 4, 1, chunks} : PrefillShape{128, 2, 1, chunks};
+}
+}  // namespace
+
+extern "C" int tllm_attention_prefill_shape(int64_t batch, int64_t n_q, int64_t n_kv_ctx, int n_kv_heads, int group, int window) {
+  if (batch < 1 || n_q < 1 || n_kv_ctx < 1 || n_kv_heads < 1 || group < 1 || window < 0) return 0;
+  const PrefillShape p = prefill_shape(batch, n_q, n_kv_ctx, n_kv_heads, group, window);
+  return (p.chunks ? 1 << 24 : 0) | p.queries << 16 | p.heads << 8 | p.key_groups;
 }
 
 extern "C" int tllm_attention_prefill_bf16(const void* q, const void* k, const void* v, const void* sinks, void* out, int64_t q_batch_stride,
@@ -923,14 +953,11 @@ extern "C" int tllm_attention_prefill_bf16(const void* q, const void* k, const v
   const int64_t wgs128 = (n_q + 127) / 128 * batch * n_kv_heads * (group % 2 == 0 ? group / 2 : group);
   TLLM_REQUIRE(batch < (1ll << 24) && wgs128 < (1ll << 31), TLLM_E_SHAPE, "attention_prefill: %lld workgroups are too many for one launch", (long long)wgs128);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int key_groups = tllm_attention_prefill_key_groups(batch, n_q, n_kv_ctx, n_kv_heads, group, window);
-  if (key_groups == 4) return launch_prefill<1, 2, 4, 8>(a, st);
-  if (key_groups == 2) return launch_prefill<1, 2, 2, 4>(a, st);
-  const int64_t walk = longest_walk(n_kv_ctx, window);
-  const bool chunks = walk > 6;
-  if (group % 2 != 0) return chunks ? launch_prefill_chunks<1, 4, 4>(a, st) : launch_prefill<1, 4, 1, 4>(a, st);
-  const int64_t wgs4 = (n_q + 63) / 64 * batch * n_kv_heads * group / 4;
-  if (wgs4 < (chunks ? (walk <= 12 ? 336 : 432) : (walk <= 4 ? 272 : 320))) return chunks ? launch_prefill_chunks<1, 2, 4>(a, st) : launch_prefill<1, 2, 1, 4>(a, st);
-  if (group % 4 == 0) return chunks ? launch_prefill_chunks<2, 2, 4>(a, st) : launch_prefill<2, 2, 1, 4>(a, st);
-  return chunks ? launch_prefill_chunks<2, 4, 4>(a, st) : launch_prefill<2, 4, 1, 4>(a, st);
+  const PrefillShape p = prefill_shape(batch, n_q, n_kv_ctx, n_kv_heads, group, window);
+  if (p.key_groups == 4) return launch_prefill<1, 2, 4, 8>(a, st);
+  if (p.key_groups == 2) return launch_prefill<1, 2, 2, 4>(a, st);
+  if (p.heads == 1) return p.chunks ? launch_prefill_chunks<1, 4, 4>(a, st) : launch_prefill<1, 4, 1, 4>(a, st);
+  if (p.heads == 4) return p.chunks ? launch_prefill_chunks<2, 2, 4>(a, st) : launch_prefill<2, 2, 1, 4>(a, st);
+  if (p.queries == 64) return p.chunks ? launch_prefill_chunks<1, 2, 4>(a, st) : launch_prefill<1, 2, 1, 4>(a, st);
+  return p.chunks ? launch_prefill_chunks<2, 4, 4>(a, st) : launch_prefill<2, 4, 1, 4>(a, st);
 }
