@@ -297,7 +297,7 @@ def test_attention_prefill_shapes():
         return s >> 24, s >> 16 & 255, s >> 8 & 255, s & 255
 
     assert [of(3, 333, n)[0] for n in (384, 385)] == [0, 1] and [of(1, 2048, 2048, window=w)[0] for w in (128, 321, 322)] == [0, 0, 1]
-    assert of(2, 600, 600) == (1, 64, 2, 1)
+    assert of(2, 700, 700) == of(2, 600, 600) == (1, 64, 2, 1)              # 352 and 320 workgroups of four heads
     assert of(3, 450, 450) == (1, 64, 4, 1) and of(3, 333, 333) == (0, 64, 2, 1)
     assert [of(1, n, n) for n in (1536, 2048)] == [(1, 64, 2, 1), (1, 64, 4, 1)]
     assert of(9, 650, 700, 2) == (1, 128, 2, 1) and of(8, 650, 700, 2, 128) == (0, 128, 2, 1) and of(2, 1000, 1100, 5) == (1, 128, 1, 1)

@@ -895,7 +895,7 @@ PrefillShape prefill_shape(int64_t batch, int64_t n_q, int64_t n_kv_ctx, int n_k
   const bool chunks = walk > 6;
   if (group % 2 != 0) return {128, 1, 1, chunks};
   const int64_t wgs4 = (n_q + 63) / 64 * batch * n_kv_heads * group / 4;
-  if (wgs4 < (chunks ? (walk <= 12 ? 336 : 432) : (walk <= 4 ? 272 : 320))) return {64, 2, 1, chunks};
+  if (wgs4 < (chunks ? (walk <= 12 ? 368 : 432) : (walk <= 4 ? 272 : 320))) return {64, 2, 1, chunks};
   return group % 4 == 0 ? PrefillShape{64, 4, 1, chunks} : PrefillShape{128, 2, 1, chunks};
 }
 }  // namespace
