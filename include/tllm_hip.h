@@ -338,6 +338,8 @@ int tllm_attention_prefill_bf16(const void* q, const void* k, const void* v, con
  * e8m0 bytes (bias 127); out [n_blocks][32] bf16 = FP4[nibble] * 2^(scale - 127), formed in fp32 and rounded once, as
  * torch.ldexp does on the reference's bf16 tensor. Bit-exact. */
 int tllm_mxfp4_dequant_bf16(const void* blocks, const void* scales, void* out, int64_t n_blocks, void* stream);
+/* Diagnostic: threads of the largest launch that it makes; a grid holds fewer than 2^32. */
+int64_t tllm_mxfp4_launch_threads(int64_t n_blocks);
 
 #ifdef __cplusplus
 }

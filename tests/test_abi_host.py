@@ -226,6 +226,12 @@ def test_mxfp4_argument_errors():
     assert "aligned" in _err()
 
 
+def test_mxfp4_launches_hold_fewer_threads_than_a_grid_may():
+    threads = _lib.lib().tllm_mxfp4_launch_threads
+    assert [threads(n) for n in (0, 1, 128, 129)] == [0, 256, 256, 512]
+    assert all(threads(n) < 1 << 32 for n in ((1 << 31) - 128, 1 << 31, 1 << 33, 1 << 40))
+
+
 def test_attention_prefill_argument_errors():
     """Argument checks of the prefill attention entry point happen before anything touches the GPU."""
     f = _lib.lib().tllm_attention_prefill_bf16

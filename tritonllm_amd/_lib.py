@@ -78,6 +78,7 @@ SIGNATURES = {
     "tllm_attention_prefill_bf16": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _i32,
                                            _f32, _i32, _vp, _i32, _vp]),
     "tllm_mxfp4_dequant_bf16": (_i32, [_vp, _vp, _vp, _i64, _vp]),
+    "tllm_mxfp4_launch_threads": (_i64, [_i64]),
     "tllm_qkv_rope_decode_w8_bf16": (_i32, [_vp, _vp, _i32, _f32, _vp, _vp] + _QKV_SIG[2:]),
 }
 

@@ -28,6 +28,8 @@ typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4;
 // 8 / 16 dwords per lane take 247 / 224 / 226 / 225 / 239 / 252 us, ordinary stores at eight 245 (239), a contiguous eighth of the
 // output per XCD 242, a resident grid 249.
 constexpr int MX_UNROLL = 2;
+// Blocks of a launch: a grid holds fewer than 2^32 threads, this one 2^31 (16 GB of blocks, 64 GB of output).
+constexpr int64_t MX_LAUNCH = 1ll << 30;
 
 __global__ __launch_bounds__(256) void mxfp4_dequant_kernel(const unsigned* __restrict__ blocks, const unsigned char* __restrict__ scales,
                                                             u32x4* __restrict__ out, int64_t n_dwords) {
@@ -79,10 +81,20 @@ extern "C" int tllm_mxfp4_dequant_bf16(const void* blocks, const void* scales, v
   if (n_blocks == 0) return TLLM_OK;
   TLLM_REQUIRE(blocks && scales && out, TLLM_E_ARG, "mxfp4_dequant: null pointer");
   TLLM_REQUIRE(aligned16(blocks) && aligned16(out), TLLM_E_ALIGN, "mxfp4_dequant: blocks and out must be 16-byte aligned");
-  const int64_t n_dwords = n_blocks * 4;
-  const int64_t wgs = (n_dwords + 256 * MX_UNROLL - 1) / (256 * MX_UNROLL);
-  TLLM_REQUIRE(wgs < (1ll << 31), TLLM_E_SHAPE, "mxfp4_dequant: %lld blocks are too many for one launch", (long long)n_blocks);
-  hipLaunchKernelGGL(mxfp4_dequant_kernel, dim3((unsigned)wgs), dim3(256), 0, static_cast<hipStream_t>(stream), (const unsigned*)blocks,
-                     (const unsigned char*)scales, (u32x4*)out, n_dwords);
-  return check_launch("mxfp4_dequant");
+  TLLM_REQUIRE(n_blocks < (1ll << 40), TLLM_E_SHAPE, "mxfp4_dequant: %lld blocks are too many", (long long)n_blocks);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  for (int64_t at = 0; at < n_blocks; at += MX_LAUNCH) {
+    const int64_t n_dwords = (n_blocks - at < MX_LAUNCH ? n_blocks - at : MX_LAUNCH) * 4;
+    hipLaunchKernelGGL(mxfp4_dequant_kernel, dim3((unsigned)((n_dwords + 256 * MX_UNROLL - 1) / (256 * MX_UNROLL))), dim3(256), 0, st,
+                       static_cast<const unsigned*>(blocks) + at * 4, static_cast<const unsigned char*>(scales) + at, static_cast<u32x4*>(out) + at * 4, n_dwords);
+    const int rc = check_launch("mxfp4_dequant");
+    if (rc != TLLM_OK) return rc;
+  }
+  return TLLM_OK;
+}
+
+extern "C" int64_t tllm_mxfp4_launch_threads(int64_t n_blocks) {
+  if (n_blocks < 1) return 0;
+  const int64_t n_dwords = (n_blocks < MX_LAUNCH ? n_blocks : MX_LAUNCH) * 4;
+  return (n_dwords + 256 * MX_UNROLL - 1) / (256 * MX_UNROLL) * 256;
 }
