@@ -101,11 +101,9 @@ extern "C" int tllm_out_residual_decode_bf16(const void* x, const void* W, const
   if (!w_scale && rows <= (wide ? 32ll : 16ll) * 65535 && out_decode_tiles(rows, in_dim, out_dim) && linear_fits_tiles(x, W, rows, in_dim, out_dim))
     return launch_tile_gemm_out("out_residual_decode", a, st);
   if (wide && aligned16(x) && aligned16(W)) {
-    const int64_t chunks = (rows + 31) / 32;
-    TLLM_REQUIRE(chunks <= 65535, TLLM_E_SHAPE, "out_residual_decode: rows %lld too many for the decode kernel", (long long)rows);
-    const dim3 grid((unsigned)(out_dim / 12), (unsigned)chunks);
-    if (rows <= 8) launch_out_decode_r8(grid, st, a);
-    else launch_out_decode_r32(grid, st, a);
+    TLLM_REQUIRE((rows + 31) / 32 <= 65535, TLLM_E_SHAPE, "out_residual_decode: rows %lld too many for the decode kernel", (long long)rows);
+    if (rows <= 8) launch_out_decode_r8(dim3((unsigned)(out_dim / 12)), st, a);
+    else launch_out_decode_r32(st, a);
     return check_launch("out_residual_decode");
   }
   // [4096, 4096] weight, 8 rows: 7.1 us; out_generic_kernel 89.7 (it reads the weight once per row, two bytes a lane)

@@ -297,7 +297,7 @@ __global__ __launch_bounds__(384) void out_decode_r32_kernel(OutArgs a, int vec8
 }
 
 // in_dim 4096, out_dim % 12 == 0, bf16 weight or (a.w_scale != null) fp8; grid = (out_dim / 12, ceil(rows / 32))
-void launch_out_decode_r32(dim3 grid, hipStream_t st, const OutArgs& a) {
+void launch_out_decode_r32(hipStream_t st, const OutArgs& a) {
   auto al8 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 8 == 0; };
   const int vec8 = al8(a.out) && a.out_rs % 4 == 0 && (a.res == nullptr || (al8(a.res) && a.res_rs % 4 == 0)) && (a.bias == nullptr || al8(a.bias));
   // As few chunks as will do, of as few rows as will do, a multiple of four: a chunk of XB four-row blocks loads all of them, real rows or
@@ -307,14 +307,14 @@ void launch_out_decode_r32(dim3 grid, hipStream_t st, const OutArgs& a) {
   const unsigned chunks = static_cast<unsigned>((a.rows + 4 * xb - 1) / (4 * xb));
   // up to four chunks per workgroup: the weight is then read once for up to 128 rows
   const int cpw = chunks < 4 ? static_cast<int>(chunks) : 4;
-  const dim3 g2(grid.x, (chunks + cpw - 1) / cpw);
+  const dim3 grid((unsigned)(a.out_dim / r32o::RW), (chunks + cpw - 1) / cpw);
   // fp8 weight: where the activations are most of what a CU takes in and there are outputs enough for most CUs, neighbours do not ask
   // their L2 for the same lines of them at the same time ([2880, 4096] in step / spread, us: 56 rows 9.10 / 8.81, 64 10.0 / 9.45, 128 15.8 / 15.0,
   // 256 32.8 / 28.4; 2304 outputs 64 rows 8.89 / 8.70, 65 9.64 / 9.68; 1536 57 rows 8.19 / 8.26, 96 10.6 / 10.7). With fewer rows, and with a
   // bf16 weight, twice the bytes, up to the rows that go to GEMM tiles, what counts is that all ask memory for the same part of their
   // weight rows at a time (bf16 57 rows 10.9 / 11.3, 80 12.8 / 13.2; 2304 outputs 97 rows 13.7 / 14.0).
   if (a.w_scale && a.rows > 52 && a.out_dim >= 2048) {        // (chunks of 22 and more)
-#define TLLM_OUT32(XB) hipLaunchKernelGGL((out_decode_r32_kernel<XB, true, true>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks)
+#define TLLM_OUT32(XB) hipLaunchKernelGGL((out_decode_r32_kernel<XB, true, true>), grid, dim3(384), 0, st, a, vec8, cpw, (int)chunks)
     if (xb <= 6) TLLM_OUT32(6);
     else if (xb == 7) TLLM_OUT32(7);
     else TLLM_OUT32(8);
@@ -323,8 +323,8 @@ void launch_out_decode_r32(dim3 grid, hipStream_t st, const OutArgs& a) {
   }
 #define TLLM_OUT32(XB)                                                                                                          \
   do {                                                                                                                          \
-    if (a.w_scale) hipLaunchKernelGGL((out_decode_r32_kernel<XB, true, false>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks);   \
-    else hipLaunchKernelGGL((out_decode_r32_kernel<XB, false, false>), g2, dim3(384), 0, st, a, vec8, cpw, (int)chunks);            \
+    if (a.w_scale) hipLaunchKernelGGL((out_decode_r32_kernel<XB, true, false>), grid, dim3(384), 0, st, a, vec8, cpw, (int)chunks);   \
+    else hipLaunchKernelGGL((out_decode_r32_kernel<XB, false, false>), grid, dim3(384), 0, st, a, vec8, cpw, (int)chunks);            \
   } while (0)
   switch (xb) {
     case 1: TLLM_OUT32(1); break;
