@@ -217,7 +217,8 @@ int tllm_qkv_rope_prefill_bf16(const void* x, const void* W, const void* b,
 int tllm_qkv_gemm_tile(int prefill, int64_t rows, int64_t hidden, int n_q_heads, int n_kv_heads, int head_dim);
 int tllm_linear_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim);
 int tllm_out_gemm_tile(int64_t rows, int64_t in_dim, int64_t out_dim);
-/* Diagnostic: whether that tile's launch (or the QKV projection's, out_dim = 64 x heads) spreads its row tiles' walks over K. */
+/* Diagnostic: whether that tile's launch (or the QKV projection's, out_dim = 64 x heads) spreads its row tiles' walks over K. A row's
+ * products are then summed in an order that depends on its row tile: equal rows of x agree to fp32 rounding, not to the bit. */
 int tllm_gemm_tile_spread(int64_t rows, int64_t in_dim, int64_t out_dim);
 /* Diagnostic: how many row tiles that launch takes before the next column of tiles. */
 int tllm_gemm_tile_group(int64_t rows, int64_t in_dim, int64_t out_dim);
@@ -253,7 +254,7 @@ int tllm_unembedding_tile_units(int64_t rows, int fp8, int64_t hidden, int64_t v
  * and with w_scale != NULL unembedding_decode_fp8_forward :271-302 (W = fp8 e4m3 bytes, one fp32 scale per
  * vocabulary row, as quantised by :261-268). x [rows, hidden] bf16 dense, W [vocab, hidden] dense, logits
  * [rows, vocab] with logits_row_stride elements between rows. hidden must be a multiple of 64. One pass over the
- * weight serves up to 32 rows; more rows take one pass per 32. */
+ * weight serves up to 128 rows where tllm_unembedding_decode_tiled says so, up to 32 (8 in wide models) otherwise; more rows take more passes. */
 int tllm_unembedding_decode_bf16(const void* x, const void* W, const float* w_scale, void* logits,
                                  int64_t logits_row_stride, int64_t rows, int64_t hidden, int64_t vocab, void* stream);
 

@@ -457,8 +457,8 @@ bool plain_operand(PyObject* o, c10::DeviceIndex device) {
 }
 
 // Whether a GEMM tile is ahead of the library's GEMM. Up to tiles of 128 x 224 covering the result in one round of the 256 CUs
-// and about 2500 rows it mostly is ([2880, 4096] weight, us: 97 rows 13.9 and 15.4, 192 rows 18.8 and 32, 999 rows 33.9 and 36.6,
-// 2400 rows 53.0 and 54.8; behind two rounds 2700 67.8 and 58.2, 4096 103 and 83; other weights 3000 rows 0.84 - 0.92 of the
+// and about 2500 rows it mostly is ([2880, 4096] weight, us: 97 rows 13.8 and 15.5, 192 rows 16.5 and 32, 999 rows 29.8 and 35.4,
+// 2400 rows 53.2 and 55.6; behind two rounds 2700 68.6 and 58.5, 4096 94 and 75; other weights 3000 rows 0.84 - 0.92 of the
 // library's rate). Tiles of 128 x 256 are ahead as long as they are one round if the outputs are no multiple of 128, which the library's
 // own tiles would fit ([2880, 4096] 2500 rows 55.3 and 58.5, K = 2048 33.0 and 36.3, 512 17.0 and 21.5; [4400, 4096] 1664 55.9 and 59.7; [8176,
 // 2880] 1024 44.5 and 47.8; but [3072, 4096] 2500 55.7 and 53.9, [2048, 4096] 2560 43.8 and 41.4), up to weights of about 25 M elements

@@ -45,8 +45,8 @@ __global__ __launch_bounds__(256) void out_generic_kernel(OutArgs a) {
 }
 
 // From where on GEMM tiles are ahead, us, decode kernel / tiles. The kernel for 4096 wide inputs reads its weight once for up to 128 rows in
-// chunks that follow each other, which is what it takes: [4096, 2880] 72 rows 12.8 / 13.2, 80 13.5 / 13.2, 96 14.9 / 13.8, 128 17.9 / 15.0, 192
-// 26.8 / 16.0, 400 51.2 / 19.5. Narrower outputs leave it as many CUs as it has workgroups of twelve columns, and each its own share of the
+// chunks that follow each other, which is what it takes: [4096, 2880] 72 rows 12.2 / 13.2, 80 12.8 / 13.2, 96 14.5 / 13.8, 128 17.3 / 15.1, 192
+// 27.8 / 16.3, 400 56.9 / 19.6. Narrower outputs leave it as many CUs as it has workgroups of twelve columns, and each its own share of the
 // memory: 1536 columns 96 rows 12.3 / 13.2, 128 15.1 / 15.4, 144 15.1 / 12.8; 2304 columns 96 rows 13.4 / 13.5, 144 17.5 / 13.1. More than 256
 // workgroups take two rounds: 4032 columns 40 rows 16.0 / 14.5, 96 rows 25.0 / 14.1.
 // Any other width, as in qkv_decode_tiles: of 420 points at widths of 512 - 6144, 512 - 5120 columns and 16 - 400 rows 397 within 3 % of the

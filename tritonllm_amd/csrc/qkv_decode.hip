@@ -122,7 +122,7 @@ bool qkv_decode_tiles(int64_t rows, int64_t hidden, int heads, int head_dim) {
   if (!qkv_tiles_fit(rows, hidden, heads, head_dim)) return false;
   const int64_t cols = static_cast<int64_t>(heads) * 64;
   // the rows kernel takes 6.4 us and 1.4 per block of 16 rows (97 rows 15.9, 128 rows 17.5, 256 rows 26.6): from about a
-  // hundred rows a GEMM tile is ahead of it (97 rows 16.1, 128 rows 16.2, 256 rows 21.2)
+  // hundred rows a GEMM tile is ahead of it (97 rows 15.7, 128 rows 16.5, 256 rows 18.6)
   if (hidden == 2880) return tile_gemm_ns(rows, cols, hidden) < 6400 + 1400 * ((rows + 15) / 16);
   // Beyond 32 rows the general kernel reads the weight a third time, which costs little while its workgroups -- sixteen weight
   // rows x sixteen rows -- are on the machine together (decode_general_ns).

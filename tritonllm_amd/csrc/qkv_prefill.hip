@@ -677,8 +677,8 @@ int prefill_tile_height(int64_t rows, int heads, int64_t* rounds128, int64_t* ro
 }  // namespace
 
 // Up to about 1500 rows (of 5120 columns) smaller tiles fill the machine in less than a round of these (tile_gemm.hip: 1536
-// rows 50.9 against 57 us, 999 rows 39.8 against 49.1, 97 rows 16.1 against 51), and a little above a whole number of rounds
-// they need less than the round more (2300 rows 76.9 against 85.7, 4300 132.6 against 144.9).
+// rows 47 - 50 against 57 us, 999 rows 37 - 39 against 49, 97 rows 15.7 against 51), and a little above a whole number of rounds
+// they need less than the round more (2300 rows 71 - 77 against 86, 4300 128 - 133 against 145).
 bool qkv_prefill_tiles(int64_t rows, int64_t hidden, int heads, int head_dim) {
   if (!prefill_fits(hidden, heads, head_dim)) return false;
   int64_t rounds128, rounds256;

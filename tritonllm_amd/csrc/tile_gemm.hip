@@ -3,7 +3,7 @@
 // qkv_prefill.hip would need one more round for little (2049 - 2816, 4097 - 4864, 6145 - 6528, ... rows; qkv_prefill_tiles), and
 // decode batches from 113 rows on (qkv_decode_tiles); the plain projection where it is ahead of the library's GEMM, up to
 // 2560 rows of [2880, 4096] (linear_in_tiles in host_ops.cpp). With a residual in the epilogue it is the out-projection of decode
-// batches from 81 rows on (out_decode_tiles: [4096, 2880] 96 rows 14.9 -> 14.0 us, 128 17.9 -> 15.1, 200 30.7 -> 16.1; [4096, 4096] 128 34.8 -> 16.6).
+// batches from 81 rows on (out_decode_tiles: [4096, 2880] 96 rows 14.5 -> 13.8 us, 128 17.3 -> 15.1, 200 30.6 -> 16.3; [4096, 4096] 128 33.6 -> 16.7).
 //
 //   D[rows, n] = X[rows, K] . W[n, K]^T      (both operands K-contiguous, K a multiple of 64)
 //
@@ -30,10 +30,10 @@
 // multiple of sixteen columns will do as a tile.
 //
 // [rows, 2880] x [2880, 5120] + bias + rotary, us (before: the many-row decode kernel up to 448 rows, 128 x 320 tiles above):
-//   128 rows 15.9 (17.5)   192 16.1 (22.1)   256 18.4 (26.6)   333 21.0 (32.3)   512 25.9 (54.0)   777 32.5 (50.9)
-//   999 38.6 (49.1)   1100 40.4 (55.0)   1400 45.7 (57.1)   1536 49.9 (57)
+//   128 rows 16.5 (17.5)   192 16.7 (22.1)   256 18.6 (26.6)   333 21.4 (32.3)   512 25.0 (54.0)   777 31.3 (50.9)
+//   999 36.9 (49.1)   1100 38.8 (55.0)   1400 43.7 (57.1)   1536 47.4 (57)
 // [rows, 4096] x [4096, 2880] + bias (before: the library's GEMM):
-//   97 rows 13.6 (15.5)   192 15.5 (32.4)   333 17.9 (30.3)   512 20.7 (25.2)   999 32.4 (36.5)   2048 49.9 (53.4)
+//   97 rows 13.8 (15.5)   192 16.5 (32.2)   333 19.0 (29.9)   512 20.5 (25.1)   999 29.8 (35.4)   2048 49.3 (49.7)
 #include "out_common.h"
 #include "qkv_prefill.h"
 
@@ -452,9 +452,10 @@ int launch_one(const char* what, const QkvArgs& a, const RopeArgs& ra, const Yar
 // arrive with (2.15 ns per row and slice of 64 K, the same within 5 % from 64 x 32 to 128 x 160), plus launch, first
 // slice and epilogue, which grow with the tile (5.3 us at 64 x 32, 9 at 128 x 160); a CU holds one tile at a time. Measured on
 // [rows, 2880] x [2880, 5120], us, chosen tile against the neighbouring ones:
-//   97 rows   64 x 48 16.1   64 x 64 17.2   64 x 32 24.5        256 rows  64 x 80 21.2    64 x 64 34.2    64 x 128 25.3
-//   333 rows  64 x 128 23.2  64 x 160 27.1  64 x 96 36.3        512 rows  64 x 160 29.6   128 x 128 33.7  64 x 128 47.5
-//   777 rows  128 x 160 33.9 128 x 192 36.3 64 x 160 52.2       999 rows  128 x 160 39.8  128 x 192 41.1  128 x 128 64.2
+//   97 rows   64 x 48 15.7   64 x 64 16.9   64 x 32 23.8        256 rows  64 x 80 18.6    64 x 64 28.6    64 x 128 21.5
+//   333 rows  64 x 128 21.4  64 x 160 23.5  64 x 96 32.1        512 rows  64 x 160 24.8   128 x 128 27.6  64 x 128 37.8
+//   777 rows  128 x 160 31.3 128 x 192 34.3 64 x 160 43.4       999 rows  128 x 160 37.4  128 x 192 39.1  128 x 128 60.7
+// (It knows neither walks that are spread over K, 8 % less in the mean, nor groups of row tiles; both came after it was fitted.)
 constexpr TileSize kTiles[] = {{64, 32}, {64, 48}, {64, 64}, {64, 80}, {64, 96}, {64, 128}, {64, 160}, {64, 192}, {128, 96}, {128, 128}, {128, 160}, {128, 192}, {128, 224}, {128, 256}};
 
 int64_t tile_ns(int64_t rows, int64_t cols, int64_t k, TileSize t) {

@@ -10,16 +10,16 @@
 // evenly: 50 units per CU are three tiles of seventeen, not two of twenty and one of ten), and the ring of S stages -- global
 // memory straight into LDS, 16-byte chunks XOR-swizzled by row -- runs on across tiles, so that 64-96 KB of the weight are in
 // flight per CU from the first instruction to the last. The activations (737 KB at 128 rows) come from the L2, once per tile.
-// A CU takes in 33-35 GB/s of this stream, whatever mixture of the two it is (its loads come back in order, the weight's from
-// memory among them), so what counts is bytes: few tall tiles, no row of either operand that is not needed, the loads of a
-// stage dealt to the wavefronts one by one. Wavefronts: four over the vocabulary x two over the batch rows, on
+// A CU takes in 28 GB/s of this stream, weight and activations together (fp8 21; 5.5 MB at 49 rows, 6.7 at 128; its loads come back in
+// order, the weight's from memory among them), and more bytes take longer if not in proportion (7.4 MB at 49 rows 34 GB/s): few tall tiles, no row
+// of either operand that is not needed, the loads of a stage dealt to the wavefronts one by one. Wavefronts: four over the vocabulary x two over the batch rows, on
 // v_mfma_f32_16x16x32_bf16 with the vocabulary on M, so that a lane ends up with four consecutive logits of a row. One barrier
 // per stage.
 //
 // [rows, 2880] x [201088, 2880], us (in brackets four tiles of thirteen units whose stages had room and loads for sixteen; in
 // chunks of 32 rows, of 8 where the width is 4096; a read of the weight alone: 174):
 //   bf16   33 rows 198 (205, 377)   49 200 (218, 382)   64 205 (228, 386)   96 219 (245, 586)   128 240 (262, 782)   200 465 (510, 1370)
-//   fp8    33 rows 133 (143, 240)   49 139 (148, 251)   64 144 (153, 253)   96 157 (177, 372)   128 178 (205, 491)
+//   fp8    33 rows 133 (143, 240)   49 139 (148, 251)   64 144 (153, 253)   96 157 (177, 372)   128 171 - 178 (193 - 205, 491)
 //   4096 wide, bf16: 9 rows 262 (257, 520; on another GPU 283 and 288)   32 275 (285, 1035)   49 273 (294)   128 313 (344, 4098)
 #include <atomic>
 
