@@ -947,6 +947,26 @@ def test_linear_walks_spread_over_k(gpu, bm, bn, rows, n, k):
     assert torch.equal(out[rows - 1].float().cpu()[w[:, k - 1] != 0], (w[:, k - 1].float() * float("inf"))[w[:, k - 1] != 0])
 
 
+@pytest.mark.parametrize("rows,n,k", [(200, 5120, 2880), (333, 5120, 2880), (640, 4096, 2880)])
+def test_linear_equal_rows(gpu, rows, n, k):
+    """Equal rows have equal results where row tiles walk K in step, and always within a row tile; between tiles whose walks are spread the fp32
+    sums differ in their order, by up to 2 k u of the sum of the products' magnitudes, which can move a bf16 result by that and one place."""
+    L = _lib.lib()
+    spread = L.tllm_gemm_tile_spread(rows, k, n)
+    assert spread == (rows != 200)
+    g = torch.Generator().manual_seed(rows)
+    x, w = torch.randn(1, k, generator=g).bfloat16(), (0.02 * torch.randn(n, k, generator=g)).bfloat16()
+    xg, wg, out = x.expand(rows, k).contiguous().to(gpu), w.to(gpu), torch.empty(rows, n, dtype=torch.bfloat16, device=gpu)
+    assert L.tllm_linear_bf16(xg.data_ptr(), wg.data_ptr(), None, out.data_ptr(), n, rows, k, n, torch.cuda.current_stream().cuda_stream) == 0
+    out, bm = out.cpu(), L.tllm_linear_gemm_tile(rows, k, n) >> 16
+    tiles = out[::bm]
+    assert torch.equal(out, tiles.repeat_interleave(bm, 0)[:rows])
+    if not spread:
+        assert torch.equal(tiles, tiles[:1].expand_as(tiles))
+    sums = 2 * k * 2.0 ** -24 * (x.float().abs() @ w.float().abs().T)
+    assert ((tiles.float() - tiles[:1].float()).abs() <= sums + 2.0 ** -7 * tiles[:1].float().abs()).all()
+
+
 @pytest.mark.parametrize("rows,n,k,tiles_m,group", [(1024, 1040, 2048, 16, 16), (1025, 1040, 2048, 17, 8), (1536, 1040, 2048, 24, 8), (1551, 1040, 2048, 25, 8),
                                                     (2048, 1024, 64, 32, 32), (2049, 1024, 64, 33, 8), (2177, 2064, 1088, 18, 8)])
 def test_linear_row_tiles_in_groups(gpu, rows, n, k, tiles_m, group):
